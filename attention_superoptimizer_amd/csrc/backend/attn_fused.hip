@@ -38,6 +38,7 @@
 // programs include as well.
 #include "common.h"
 #include "tb_program.h"
+#include "attn_tiles.h"
 #include <atomic>
 #include <cstdlib>
 #include <string>
@@ -188,8 +189,7 @@ bool match(DevProgram const &P, Match &M, bool pieces = false) {
   M.D = tq.cols;
   M.NK = tk.cols;
   M.DV = tv.cols;
-  // query tiles of whole 16-row groups, or a single group of 8 rows (padded with zero rows)
-  if (tk.rows != M.D || tv.rows != M.NK || (M.m % 16 != 0 && M.m != 8)) {
+  if (tk.rows != M.D || tv.rows != M.NK) {
     return false;
   }
   // Q must be loop invariant; all tiles reachable with 16-byte accesses
@@ -280,6 +280,35 @@ bool merge_column_pieces(DevProgram const &P, Match &M, DevProgram &Q, int &copi
       return false;
     }
     M.DV = 64;
+    return true;
+  }
+  return false;
+}
+
+// A plan that cuts the query rows into tiles along a grid dimension K and V do not move with: row
+// r of block i is row i m + r of one tall tile (every row is worked on by itself), so Q becomes
+// that program -- grid dimension of extent 1, G m rows -- and no row group is left half empty at
+// the end of every tile.  False when P is not of this shape.
+bool merge_row_blocks(DevProgram const &P, Match &M, DevProgram &Q) {
+  for (int g = 0; g < 3; g++) {
+    int const G = P.grid[g];
+    if (G < 2 || (long long)G * M.m > (1 << 24)) {
+      continue;
+    }
+    auto still = [&](DevOp const &op) { return !op.row_bs[g] && !op.col_bs[g] && !op.g_bs[g]; };
+    auto stacked = [&](DevOp const &op) { return op.row_bs[g] == M.m && !op.col_bs[g] && !op.g_bs[g]; };
+    if (!still(P.ops[M.k]) || !still(P.ops[M.v]) || !stacked(P.ops[M.q]) || !stacked(P.ops[M.out_o]) ||
+        (M.out_r >= 0 && !stacked(P.ops[M.out_r]))) {
+      continue;
+    }
+    Q = P;
+    Q.grid[g] = 1;
+    for (int o : {M.q, M.out_o, M.out_r}) {
+      if (o >= 0) {
+        Q.ops[o].row_bs[g] = 0;
+      }
+    }
+    M.m *= G;
     return true;
   }
   return false;
@@ -615,12 +644,23 @@ static bool choose_stream(DevProgram const &P, Match const &M, StreamShape &st) 
   return true;
 }
 
+std::string attn_params_literal(AttnParams const &A) { return literal(A); }
+
+static bool choose_tiles(DevProgram const &P, Match const &M, TilesShape &t) {
+  State &s = state();
+  long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
+  return choose_attn_tiles(M.D, M.DV, M.NK, M.m, M.has_div, M.kv_colmajor, blocks, P.forloop_range, s.max_lds, t) &&
+         (long long)P.grid[0] * t.split <= 2147483647LL;
+}
+
 bool attention_applicable(DevProgram const &P) {
   Match M;
   DirectShape d;
   StreamShape st;
+  TilesShape tiles;
   int lds = 0;
-  if (match(P, M) && (shape_supported(M) || choose_stream(P, M, st) || choose_direct(P, M, d, lds))) {
+  if (match(P, M) && (shape_supported(M) || choose_stream(P, M, st) || choose_direct(P, M, d, lds) ||
+                      choose_tiles(P, M, tiles))) {
     return true;
   }
   DevProgram merged;
@@ -635,12 +675,29 @@ int try_launch_attention(DevProgram const &P0) {
   int r_copies = 1, r_copy_stride = 0;
   // as the plan states it, or (value tiles narrower than 64 columns) with its column pieces merged
   bool pieces = !match(P0, M);
+  TilesShape tiles_shape;
+  bool tiles = false;
   if (!pieces) {
     DirectShape probe;
     StreamShape probe_stream;
     int probe_lds = 0;
     pieces = !shape_supported(M) && !choose_stream(P0, M, probe_stream) &&
              !choose_direct(P0, M, probe, probe_lds);
+    if (pieces) {
+      // sizes the kernels of whole tiles are not built for: any-size kernel, row tiles joined
+      Match T = M;
+      DevProgram tall;
+      bool const joined = merge_row_blocks(P0, T, tall);
+      tiles = choose_tiles(joined ? tall : P0, T, tiles_shape);
+      if (tiles) {
+        pieces = false;
+        M = T;
+        if (joined) {
+          merged = tall;
+          run = &merged;
+        }
+      }
+    }
   }
   if (pieces) {
     if (!merge_column_pieces(P0, M, merged, r_copies, r_copy_stride)) {
@@ -651,10 +708,10 @@ int try_launch_attention(DevProgram const &P0) {
   DevProgram const &P = *run;
   DirectShape dshape;
   int direct_lds = 0;
-  bool const direct = choose_direct(P, M, dshape, direct_lds);
+  bool const direct = !tiles && choose_direct(P, M, dshape, direct_lds);
   StreamShape stream_probe;
-  bool const stream = !pieces && choose_stream(P, M, stream_probe);
-  if (!direct && !stream && (pieces || !shape_supported(M))) {
+  bool const stream = !tiles && !pieces && choose_stream(P, M, stream_probe);
+  if (!tiles && !direct && !stream && (pieces || !shape_supported(M))) {
     return 0;  // (only the direct-staging variant stores copies of the row sums)
   }
   State &s = state();
@@ -692,6 +749,29 @@ int try_launch_attention(DevProgram const &P0) {
         A.perm[n++] = d;
       }
     }
+  }
+  // ---- any tile size
+  if (tiles) {
+    A.split = tiles_shape.split;
+    A.rows = M.m;
+    A.stages = M.NK;
+    A.lds_stage_bytes = 0;
+    if (A.k.d_cols >= (1 << 24) || A.v.d_cols >= (1 << 24)) {
+      return 0;  // (offsets inside a tile are 32-bit: up to 128 rows of the tensor)
+    }
+    dim3 const grid(P.grid[0] * A.split, P.grid[1], P.grid[2]);
+    if (!set_grid_magics(A, grid)) {
+      return 0;
+    }
+    int const rc = launch_attn_tiles(A, grid, M.D, M.has_div, M.kv_colmajor, tiles_shape);
+    if (rc == 1) {
+      s.last().kernel_id = MI355_KERNEL_F16_ATTENTION;
+      s.last().workgroups = grid.x * grid.y * grid.z;
+      s.last().threads = 64 * tiles_shape.ip;
+      s.last().lds_bytes = tiles_shape.lds;
+      s.last().row_split = A.split;
+    }
+    return rc;
   }
   // ---- throughput variant
   {

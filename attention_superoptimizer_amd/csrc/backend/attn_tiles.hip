@@ -1,0 +1,123 @@
+// Launches of attn_tiles_kernel (include/mi355_kernels/attention_tiles.h): which instantiation an
+// attention plan of any tile size gets.  Recognition and the parameter block are attn_fused.hip's.
+#include "common.h"
+#include "tb_program.h"
+#include "attn_tiles.h"
+#include <algorithm>
+#include <atomic>
+#include <string>
+
+#include "mi355_kernels/attention_tiles.h"
+
+namespace mi355 {
+
+namespace {
+
+template <int D, bool HAS_DIV, bool CM, int RPW, int CHB>
+int launch_tiles_one(AttnParams const &A, dim3 grid, int ip, int lds) {
+  if (EmitSink *sink = emit_sink()) {
+    sink->headers |= 8u;
+    emit_launch(*sink, "attn_tiles_kernel",
+                emit_fmt("%d, %s, %s, %d, %d", D, HAS_DIV ? "true" : "false", CM ? "true" : "false", RPW, CHB), grid, 64 * ip, lds,
+                attn_params_literal(A));
+    return 1;
+  }
+  auto *fn = attn_tiles_kernel<D, HAS_DIV, CM, RPW, CHB>;
+  static std::atomic<int> granted{0};  // per instantiation
+  if (lds > 65536 && granted.load(std::memory_order_acquire) < lds) {
+    MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  state().max_lds));
+    granted.store(state().max_lds, std::memory_order_release);
+  }
+  fn<<<grid, 64 * ip, lds, state().stream()>>>(A);
+  MI355_HIP(hipGetLastError());
+  return 1;
+}
+
+template <int D, bool HAS_DIV, bool CM>
+int launch_tiles_shape(AttnParams const &A, dim3 grid, int rpw, int chb, int ip, int lds) {
+  if constexpr (D == 64) {
+    switch (rpw * 10 + chb) {
+      case 14: return launch_tiles_one<D, HAS_DIV, CM, 1, 4>(A, grid, ip, lds);
+      case 18: return launch_tiles_one<D, HAS_DIV, CM, 1, 8>(A, grid, ip, lds);
+      case 24: return launch_tiles_one<D, HAS_DIV, CM, 2, 4>(A, grid, ip, lds);
+      case 28: return launch_tiles_one<D, HAS_DIV, CM, 2, 8>(A, grid, ip, lds);
+      case 44: return launch_tiles_one<D, HAS_DIV, CM, 4, 4>(A, grid, ip, lds);
+      default: break;
+    }
+    if constexpr (HAS_DIV) {
+      return rpw * 10 + chb == 48 ? launch_tiles_one<D, HAS_DIV, CM, 4, 8>(A, grid, ip, lds) : 0;
+    }
+    return 0;
+  }
+  switch (rpw * 10 + chb) {
+    case 14: return launch_tiles_one<D, HAS_DIV, CM, 1, 4>(A, grid, ip, lds);
+    case 24: return launch_tiles_one<D, HAS_DIV, CM, 2, 4>(A, grid, ip, lds);
+    default: return 0;
+  }
+}
+
+}  // namespace
+
+bool choose_attn_tiles(int D, int DV, int NK, int m, bool has_div, bool cm, long long blocks, int F, int max_lds,
+                       TilesShape &t) {
+  if (D != DV || (D != 64 && D != 128) || NK % 16 != 0 || NK < 16 || m < 1) {
+    return false;
+  }
+  int const nb = NK / 16;
+  t.chb = D == 64 && nb > 4 ? 8 : 4;
+  if (has_div && nb > t.chb) {
+    return false;  // the division needs the row sum of the whole tile before P.V
+  }
+  // Row groups per wavefront: as many as still leave a workgroup for every compute unit (each K / V
+  // operand then feeds that many matrix instructions), unless rounding the row groups up to
+  // whole wavefronts would add more than a third of work.
+  int const groups = (m + 15) / 16;
+  t.rpw = 1;
+  for (int r : {4, 2}) {
+    if (r == 4 && D == 128) {
+      continue;
+    }
+    int const slabs = (groups + r - 1) / r;
+    if (groups >= r && 3 * slabs * r <= 4 * groups && blocks * slabs >= 192) {
+      t.rpw = r;
+      break;
+    }
+  }
+  t.split = (groups + t.rpw - 1) / t.rpw;
+  if (t.rpw == 4 && !has_div) {
+    t.chb = 4;  // (two chunks of a longer key tile: eight blocks beside four row groups would spill)
+  }
+  // Iteration lanes: one wavefront per iteration up to what the instantiation allows, evened out
+  // over the rounds.
+  int const most = attn_tiles_lanes(D, t.rpw, t.chb);
+  int const slot = (16 * t.rpw * (DV + 8) + 16 * t.rpw) * 2, strips = cm ? 0 : (D * 40 + 32 * (DV + 8)) * 2;
+  for (int cap = most; cap >= 1; cap--) {
+    int const rounds = (F + cap - 1) / cap;
+    t.ip = (F + rounds - 1) / rounds;
+    t.lds = (rounds > 1 ? 2 : 1) * t.ip * slot + t.ip * strips;
+    if (t.lds <= max_lds) {
+      return true;
+    }
+  }
+  return false;
+}
+
+int launch_attn_tiles(AttnParams const &A, dim3 grid, int D, bool has_div, bool cm, TilesShape const &t) {
+  if (D == 64) {
+    if (has_div) {
+      return cm ? launch_tiles_shape<64, true, true>(A, grid, t.rpw, t.chb, t.ip, t.lds)
+                : launch_tiles_shape<64, true, false>(A, grid, t.rpw, t.chb, t.ip, t.lds);
+    }
+    return cm ? launch_tiles_shape<64, false, true>(A, grid, t.rpw, t.chb, t.ip, t.lds)
+              : launch_tiles_shape<64, false, false>(A, grid, t.rpw, t.chb, t.ip, t.lds);
+  }
+  if (has_div) {
+    return cm ? launch_tiles_shape<128, true, true>(A, grid, t.rpw, t.chb, t.ip, t.lds)
+              : launch_tiles_shape<128, true, false>(A, grid, t.rpw, t.chb, t.ip, t.lds);
+  }
+  return cm ? launch_tiles_shape<128, false, true>(A, grid, t.rpw, t.chb, t.ip, t.lds)
+            : launch_tiles_shape<128, false, false>(A, grid, t.rpw, t.chb, t.ip, t.lds);
+}
+
+}  // namespace mi355
