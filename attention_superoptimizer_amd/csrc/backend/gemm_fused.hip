@@ -45,6 +45,7 @@
 #include <algorithm>
 #include <string>
 
+#include "gemm_tiles.h"
 #include "mi355_kernels/gemm.h"
 
 namespace mi355 {
@@ -118,7 +119,10 @@ struct GMatch {
   bool lora;
   int a0, a1, b0, b1, la, lb;  // load op indices (-1 when absent)
   int o0, o1;                  // output op indices
-  int M, KT;
+  int M, KT, NC, rank;         // rows, k extent and columns of the tiles; lora rank (0: no lora)
+  // the sizes gemm_fused_kernel is built for (64 columns, k up to 512, up to 64 rows, rank 16);
+  // anything else runs on gemm_tiles_kernel
+  bool whole;
   // every weight-side operand (b0, b1, la, lb) is a DmemColumnMajor tensor, as the reference's
   // plans declare their weights (cpp_examples/lora.cc:36-41): k is contiguous in memory
   bool wcm;
@@ -145,6 +149,7 @@ bool gmatch(DevProgram const &P, GMatch &G) {
   G.pro = PRO_NONE;
   G.nb = 1;
   G.lora = false;
+  G.rank = 0;
   DevOp const *o = P.ops + nl;
   int const n = P.num_ops - nl;
   auto L = [&](int tensor) { return loader_of(P, nl, tensor); };
@@ -198,7 +203,8 @@ bool gmatch(DevProgram const &P, GMatch &G) {
     }
     DevTensor const &ta = P.t[P.ops[G.la].dst], &tb = P.t[P.ops[G.lb].dst];
     DevOp const &lb = P.ops[G.lb];
-    if (ta.cols != 16 || tb.rows != 16 || tb.cols != 64 || lb.row_fs != 0 || lb.col_fs != 0 ||
+    G.rank = ta.cols;
+    if (tb.rows != G.rank || (G.rank != 8 && G.rank != 16 && G.rank != 32) || lb.row_fs != 0 || lb.col_fs != 0 ||
         lb.g_fs != 0 || !P.ops[G.la].galign || !lb.galign) {
       return false;
     }
@@ -223,14 +229,16 @@ bool gmatch(DevProgram const &P, GMatch &G) {
   DevTensor const &ta = P.t[P.ops[G.a0].dst], &tb = P.t[P.ops[G.b0].dst];
   G.M = ta.rows;
   G.KT = ta.cols;
-  if (tb.rows != G.KT || tb.cols != 64 || G.KT % 32 != 0 || G.KT < 64 || G.KT > 512 ||
-      !(G.M == 8 || (G.M % 16 == 0 && G.M <= 64))) {
+  G.NC = tb.cols;
+  if (tb.rows != G.KT || G.NC % 16 != 0 || G.KT % 32 != 0 || G.M < 1 || G.M > 256) {
     return false;
   }
-  if (G.lora && (G.M != 16 || ta.rows != 16)) {
+  G.whole = G.NC == 64 && G.KT >= 64 && G.KT <= 512 && G.M <= (G.pro == PRO_NONE && G.nb == 1 && !G.lora ? 64 : 16) &&
+            (!G.lora || G.rank == 16);
+  if (G.nb == 2 && (P.t[P.ops[G.b1].dst].rows != G.KT || P.t[P.ops[G.b1].dst].cols != G.NC)) {
     return false;
   }
-  if (G.nb == 2 && (P.t[P.ops[G.b1].dst].rows != G.KT || P.t[P.ops[G.b1].dst].cols != 64)) {
+  if (G.lora && P.t[P.ops[G.lb].dst].cols != G.NC) {
     return false;
   }
   for (int i : {G.a0, G.a1, G.b0, G.b1, G.la, G.lb}) {
@@ -314,7 +322,7 @@ int launch_lanes_kt(LaneParams const &L, int grid, int threads, int lds) {
 
 int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) {
   State &s = state();
-  if (s.gemm_mode == 1 || !(G.KT == 64 || G.KT == 128 || G.KT == 256)) {
+  if (s.gemm_mode == 1 || s.gemm_mode == 3 || !G.whole || !(G.KT == 64 || G.KT == 128 || G.KT == 256)) {
     return 0;
   }
   long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
@@ -388,6 +396,8 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
 
 }  // namespace
 
+std::string gemm_params_literal(GemmParams const &A, char const *var) { return literal(A, var); }
+
 bool gemm_applicable(DevProgram const &P) {
   GMatch G;
   return gmatch(P, G);
@@ -420,7 +430,10 @@ int try_launch_gemm(DevProgram const &P) {
   if (int const rc = try_launch_lanes(P, G, A)) {
     return rc;
   }
-  int const mt = (G.M + 15) / 16;
+  if (!G.whole || s.gemm_mode == 3) {
+    return launch_gemm_tiles(A, TileGemmPlan{{P.grid[0], P.grid[1], P.grid[2]}, G.pro, G.nb, G.rank, G.NC, G.wcm});
+  }
+  int const mt = G.M <= 16 ? 1 : (G.M <= 32 ? 2 : 4);
   long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
   // Ranges per block: the split that minimises (rounds of resident workgroups) x
   // (iterations per workgroup + a fixed cost per workgroup + the combine's cost per range),

@@ -278,7 +278,7 @@ extern "C" int mi355_set_option(int option, int value) {
     state().direct_lanes = value;
     return MI355_OK;
   }
-  if (option == MI355_OPT_GEMM_MODE && value >= 0 && value <= 2) {
+  if (option == MI355_OPT_GEMM_MODE && value >= 0 && value <= 3) {
     state().gemm_mode = value;
     return MI355_OK;
   }

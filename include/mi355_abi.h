@@ -130,8 +130,9 @@ typedef struct mi355_launch_info {
  * launch with the output tile cut into 16 x 16 pieces for plans that would otherwise leave
  * most of the chip idle; the for-loop cut into ranges, plus a launch that adds them, for
  * plans whose traffic, not the launch, sets the time); 1 = always the range-splitting kernel; 2 = the one-launch
- * kernel wherever it applies.  Both keep the accumulation order of the sequential loop;
- * results agree to the last bit.  A measurement knob that the tests use to cover both. */
+ * kernel wherever it applies; 3 = the kernel for tiles of any size, which otherwise runs the
+ * plans the other two are not built for.  All keep the accumulation order of the sequential
+ * loop.  A measurement knob that the tests use to cover them. */
 #define MI355_OPT_GEMM_MODE 7
 /* F16_MATMUL_ROUTE: what runs a kernel-level fp16 matmul (mi355_f16_matmul,
  * mi355_f16_matmul_layout).  0 = this library's kernels (default); 1 = the vendor's BLAS
