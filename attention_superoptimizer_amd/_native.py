@@ -112,6 +112,9 @@ ABI = {
     "mi355_customized_fp_batch": (_ci, [_pplan, _ci, _pvp, _pvp]),
     "mi355_plan_extents": (_ci, [_pplan, _pll, _pll, _pi, _pi]),
     "mi355_customized_run": (_ci, [_pplan, _pvp, _pvp]),
+    "mi355_prepare": (_ci, [_pplan, _pvp, _pvp, _ci, _pvp]),
+    "mi355_prepared_run": (_ci, [_vp]),
+    "mi355_prepared_free": (_ci, [_vp]),
     "mi355_customized_profile": (_ci, [_pplan, _pvp, _pvp, _ci, _ci, _ci, _pf]),
     "mi355_last_launch": (_ci, [ctypes.POINTER(Mi355LaunchInfo)]),
     "mi355_phase_trace_read": (_ci, [ctypes.POINTER(ctypes.c_ulonglong), _sz]),
@@ -158,6 +161,7 @@ FACADE = {
     "mirage_op_fingerprint": (_ci, [_vp, _ci]),
     "mirage_op_profile": (ctypes.c_float, [_vp, _ci]),
     "mirage_op_execute": (_ci, [_vp, _ci]),
+    "mirage_graph_execute": (_ci, [_vp]),
     "mirage_op_lowered": (_ci, [_vp, _ci, _ci, _pplan, _pi]),
     "mirage_tensor_info": (_ci, [_vp, _pi, _pi, _pi, _pi, _pll]),
     "mirage_tensor_ptr": (_vp, [_vp, _ci]),

@@ -39,7 +39,6 @@
 #include "common.h"
 #include "tb_program.h"
 #include "attn_tiles.h"
-#include <atomic>
 #include <cstdlib>
 #include <string>
 
@@ -328,14 +327,8 @@ int launch_direct_one(AttnParams const &A, dim3 grid, int lds, bool dry) {
     return 1;
   }
   auto go = [&](auto *fn) -> int {
-    static std::atomic<int> granted{0};  // per instantiation
-    if (lds > 65536 && lds > granted) {
-      MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fn),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, state().max_lds));
-      granted = state().max_lds;
-    }
-    fn<<<grid, 64 * IP, lds, state().stream()>>>(A);
-    MI355_HIP(hipGetLastError());
+    MI355_GRANT_LDS(fn, lds);
+    MI355_HIP(launch_kernel(fn, grid, 64 * IP, lds, state().stream(), A));
     return 1;
   };
   if (SPI == 1 && IPS == 1 && A.trace != nullptr) {
@@ -409,14 +402,8 @@ int launch_one(AttnParams const &A, dim3 grid, int lds) {
     return 1;
   }
   auto *fn = attn_fused_kernel<D, NK, DV, HAS_DIV, RG, IP, CM>;
-  static std::atomic<int> granted{0};  // per instantiation
-  if (lds > 65536 && lds > granted) {
-    MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fn),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, state().max_lds));
-    granted = state().max_lds;
-  }
-  fn<<<grid, 64 * RG * IP, lds, state().stream()>>>(A);
-  MI355_HIP(hipGetLastError());
+  MI355_GRANT_LDS(fn, lds);
+  MI355_HIP(launch_kernel(fn, grid, 64 * RG * IP, lds, state().stream(), A));
   return 1;
 }
 
@@ -456,12 +443,8 @@ int launch_stream_one(AttnParams const &A, dim3 grid, int lds) {
     return 1;
   }
   auto *fn = attn_stream_kernel<D, NK, DV, HAS_DIV, RG, RPW, CM, SPI>;
-  if (lds > 65536) {
-    MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fn),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-  }
-  fn<<<grid, 64 * RG, lds, state().stream()>>>(A);
-  MI355_HIP(hipGetLastError());
+  MI355_GRANT_LDS(fn, lds);
+  MI355_HIP(launch_kernel(fn, grid, 64 * RG, lds, state().stream(), A));
   return 1;
 }
 
@@ -683,7 +666,7 @@ int try_launch_attention(DevProgram const &P0) {
     int probe_lds = 0;
     pieces = !shape_supported(M) && !choose_stream(P0, M, probe_stream) &&
              !choose_direct(P0, M, probe, probe_lds);
-    if (pieces) {
+    if (pieces || state().any_size_kernels) {
       // sizes the kernels of whole tiles are not built for: any-size kernel, row tiles joined
       Match T = M;
       DevProgram tall;

@@ -4,7 +4,6 @@
 #include "tb_program.h"
 #include "attn_tiles.h"
 #include <algorithm>
-#include <atomic>
 #include <string>
 
 #include "mi355_kernels/attention_tiles.h"
@@ -23,14 +22,8 @@ int launch_tiles_one(AttnParams const &A, dim3 grid, int ip, int lds) {
     return 1;
   }
   auto *fn = attn_tiles_kernel<D, HAS_DIV, CM, RPW, CHB>;
-  static std::atomic<int> granted{0};  // per instantiation
-  if (lds > 65536 && granted.load(std::memory_order_acquire) < lds) {
-    MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  state().max_lds));
-    granted.store(state().max_lds, std::memory_order_release);
-  }
-  fn<<<grid, 64 * ip, lds, state().stream()>>>(A);
-  MI355_HIP(hipGetLastError());
+  MI355_GRANT_LDS(fn, lds);
+  MI355_HIP(launch_kernel(fn, grid, 64 * ip, lds, state().stream(), A));
   return 1;
 }
 

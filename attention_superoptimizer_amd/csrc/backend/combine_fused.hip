@@ -227,7 +227,7 @@ int try_launch_combine(DevProgram const &P) {
   hipStream_t const q = s.stream();
 #define MI355_COMBINE_CASE(VECV, MODEV, BATCHV)                                  \
   if ((M.vec == 8 ? 8 : 4) == VECV && M.mode == MODEV && batch == BATCHV) {      \
-    combine_fused_kernel<VECV, MODEV, BATCHV><<<grid, 256, 0, q>>>(A);           \
+    MI355_HIP(launch_kernel(combine_fused_kernel<VECV, MODEV, BATCHV>, grid, 256, 0, q, A)); \
   }
   MI355_COMBINE_CASE(8, SUM_THEN_DIV, 4)
   MI355_COMBINE_CASE(8, DIV_THEN_SUM, 4)
@@ -242,7 +242,6 @@ int try_launch_combine(DevProgram const &P) {
   MI355_COMBINE_CASE(4, DIV_THEN_SUM, 16)
   MI355_COMBINE_CASE(4, DIV_THEN_SAVE, 16)
 #undef MI355_COMBINE_CASE
-  MI355_HIP(hipGetLastError());
   s.last().kernel_id = MI355_KERNEL_F16_COMBINE;
   s.last().workgroups = (int)(grid.x * grid.y * grid.z);
   s.last().threads = 256;

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "mi355_abi.h"
+#include "launch.h"
 #include <hip/hip_runtime.h>
 #include <cstdarg>
 #include <cstdint>
@@ -88,6 +89,7 @@ struct State {
   int direct_lanes = 0;      // MI355_OPT_DIRECT_LANES
   int gemm_mode = 0;         // MI355_OPT_GEMM_MODE
   int f16_matmul_route = 0;  // MI355_OPT_F16_MATMUL_ROUTE
+  int any_size_kernels = 0;  // MI355_OPT_ANY_SIZE_KERNELS
   // phase timestamps of the direct-staging attention kernel (MI355_OPT_PHASE_TRACE): while
   // set, launches of that kernel record six wall-clock stamps per wavefront here
   unsigned long long *phase_trace = nullptr;        // null while tracing is off
@@ -110,14 +112,26 @@ struct State {
 
 State &state();
 
+// Raises the dynamic LDS limit of a kernel to what the device has, once per kernel: the call costs
+// the host several microseconds.  A launch that requests at most 64 KB needs none.
+int grant_lds(void const *fn, int lds);
+#define MI355_GRANT_LDS(fn, lds)                                                \
+  do {                                                                          \
+    if (int rc_ = ::mi355::grant_lds(reinterpret_cast<void const *>(fn), lds)) { \
+      return rc_;                                                               \
+    }                                                                           \
+  } while (0)
+
 // Matrix-core fingerprint matmul (fp_mfma.hip): whether a single matmul is large enough to
 // repay the extra launch that splits its operands into residue planes, and its launch.
 bool mfma_matmul_pays(int batch, int m, int n, int k);
 int launch_mfma_matmul(uint16_t const *A, uint16_t const *B, uint16_t *C, int batch, int m, int n,
                        int k);
 int sync_all_queues();
-// Drops what mi355_customized_profile keeps of its last call per queue (tb_interp.hip).
+// Drops what mi355_customized_profile keeps of its last call per queue and the launches of prepared
+// operators (tb_interp.hip); options_generation() counts how often.
 void drop_profile_replays();
+unsigned options_generation();
 // The vendor library's GEMM on the calling thread's queue (vendor_gemm.cc): row-major C =
 // A . B for `batch` matrices, each operand in either storage order; MI355_ERR_UNSUPPORTED
 // when the library cannot be loaded.  vendor_gemm_release drops its per-queue handles.

@@ -293,20 +293,6 @@ __global__ __launch_bounds__(kThreads) void fp_gemm_multi_kernel(
                      x / P.grid[0]);
 }
 
-template <int TPT>
-int raise_lds(int lds_total) {
-  static std::atomic<int> granted_single{0}, granted_multi{0};
-  State &s = state();
-  if (lds_total > 65536 && (granted_single < s.max_lds || granted_multi < s.max_lds)) {
-    MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fp_gemm_kernel<TPT>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, s.max_lds));
-    MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fp_gemm_multi_kernel<TPT>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, s.max_lds));
-    granted_single = granted_multi = s.max_lds;
-  }
-  return MI355_OK;
-}
-
 }  // namespace
 
 // Recognises the family in a lowered uint16 program; on success marks it (fused = 4),
@@ -405,21 +391,9 @@ bool fp_gemm_applicable(DevProgram &P) {
 
 int launch_fp_gemm(DevProgram const &P, hipStream_t stream) {
   dim3 grid(P.grid[0] * P.splits, P.grid[1], P.grid[2]);
-  switch (P.fg[3]) {
-    case 1:
-      if (int rc = raise_lds<1>(P.lds_bytes)) return rc;
-      fp_gemm_kernel<1><<<grid, kThreads, P.lds_bytes, stream>>>(P);
-      break;
-    case 2:
-      if (int rc = raise_lds<2>(P.lds_bytes)) return rc;
-      fp_gemm_kernel<2><<<grid, kThreads, P.lds_bytes, stream>>>(P);
-      break;
-    default:
-      if (int rc = raise_lds<4>(P.lds_bytes)) return rc;
-      fp_gemm_kernel<4><<<grid, kThreads, P.lds_bytes, stream>>>(P);
-      break;
-  }
-  MI355_HIP(hipGetLastError());
+  auto *fn = P.fg[3] == 1 ? fp_gemm_kernel<1> : (P.fg[3] == 2 ? fp_gemm_kernel<2> : fp_gemm_kernel<4>);
+  MI355_GRANT_LDS(fn, P.lds_bytes);
+  MI355_HIP(launch_kernel(fn, grid, kThreads, P.lds_bytes, stream, P));
   return MI355_OK;
 }
 
@@ -427,21 +401,9 @@ int launch_fp_gemm_multi(DevProgram const *progs, int const *first_block, int n,
                          int staging_bytes, hipStream_t stream) {
   int const program_off = (staging_bytes + 15) / 16 * 16;
   int const lds_total = program_off + (int)sizeof(DevProgram);
-  switch (tpt) {
-    case 1:
-      if (int rc = raise_lds<1>(lds_total)) return rc;
-      fp_gemm_multi_kernel<1><<<blocks, kThreads, lds_total, stream>>>(progs, first_block, n, program_off);
-      break;
-    case 2:
-      if (int rc = raise_lds<2>(lds_total)) return rc;
-      fp_gemm_multi_kernel<2><<<blocks, kThreads, lds_total, stream>>>(progs, first_block, n, program_off);
-      break;
-    default:
-      if (int rc = raise_lds<4>(lds_total)) return rc;
-      fp_gemm_multi_kernel<4><<<blocks, kThreads, lds_total, stream>>>(progs, first_block, n, program_off);
-      break;
-  }
-  MI355_HIP(hipGetLastError());
+  auto *fn = tpt == 1 ? fp_gemm_multi_kernel<1> : (tpt == 2 ? fp_gemm_multi_kernel<2> : fp_gemm_multi_kernel<4>);
+  MI355_GRANT_LDS(fn, lds_total);
+  MI355_HIP(launch_kernel(fn, blocks, kThreads, lds_total, stream, progs, first_block, n, program_off));
   return MI355_OK;
 }
 

@@ -1001,8 +1001,7 @@ static int launch_split_jobs(SplitJob *jobs, int count, hipStream_t stream) {
     }
     S.count = group;
     S.tables = tables();
-    fp_split_planes_kernel<<<blocks, kThreads, 0, stream>>>(S);
-    MI355_HIP(hipGetLastError());
+    MI355_HIP(launch_kernel(fp_split_planes_kernel, blocks, kThreads, 0, stream, S));
   }
   return MI355_OK;
 }
@@ -1434,8 +1433,7 @@ int launch_fp_mfma_gemm(DevProgram const &P, hipStream_t stream) {
     return rc;
   }
   dim3 grid(P.grid[0] / P.pl_group[0] * P.splits, P.grid[1] / P.pl_group[1], P.grid[2]);
-  fp_mfma_gemm_kernel<<<grid, kThreads, 0, stream>>>(P, tables());
-  MI355_HIP(hipGetLastError());
+  MI355_HIP(launch_kernel(fp_mfma_gemm_kernel, grid, kThreads, 0, stream, P, tables()));
   return MI355_OK;
 }
 

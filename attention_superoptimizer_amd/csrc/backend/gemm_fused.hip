@@ -268,12 +268,8 @@ int launch_kt(GemmParams const &A, dim3 grid, int lds) {
   }
   State &s = state();
   auto go = [&](auto *fn) -> int {
-    if (lds > 65536) {
-      MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fn),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    }
-    fn<<<grid, 256, lds, s.stream()>>>(A);
-    MI355_HIP(hipGetLastError());
+    MI355_GRANT_LDS(fn, lds);
+    MI355_HIP(launch_kernel(fn, grid, 256, lds, s.stream(), A));
     return 1;
   };
   if (A.KT <= 64) {
@@ -300,12 +296,8 @@ int launch_lanes_kt(LaneParams const &L, int grid, int threads, int lds) {
   }
   State &s = state();
   auto go = [&](auto *fn) -> int {
-    if (lds > 65536) {
-      MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fn),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    }
-    fn<<<grid, threads, lds, s.stream()>>>(L);
-    MI355_HIP(hipGetLastError());
+    MI355_GRANT_LDS(fn, lds);
+    MI355_HIP(launch_kernel(fn, grid, threads, lds, s.stream(), L));
     return 1;
   };
   switch (L.g.KT) {
@@ -322,7 +314,7 @@ int launch_lanes_kt(LaneParams const &L, int grid, int threads, int lds) {
 
 int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) {
   State &s = state();
-  if (s.gemm_mode == 1 || s.gemm_mode == 3 || !G.whole || !(G.KT == 64 || G.KT == 128 || G.KT == 256)) {
+  if (s.gemm_mode == 1 || s.any_size_kernels || !G.whole || !(G.KT == 64 || G.KT == 128 || G.KT == 256)) {
     return 0;
   }
   long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
@@ -430,7 +422,7 @@ int try_launch_gemm(DevProgram const &P) {
   if (int const rc = try_launch_lanes(P, G, A)) {
     return rc;
   }
-  if (!G.whole || s.gemm_mode == 3) {
+  if (!G.whole || s.any_size_kernels) {
     return launch_gemm_tiles(A, TileGemmPlan{{P.grid[0], P.grid[1], P.grid[2]}, G.pro, G.nb, G.rank, G.NC, G.wcm});
   }
   int const mt = G.M <= 16 ? 1 : (G.M <= 32 ? 2 : 4);
@@ -494,12 +486,7 @@ int try_launch_gemm(DevProgram const &P) {
                 literal(A, "P"));
   } else if (rc == 1 && ksplit > 1) {
     dim3 cgrid(P.grid[0], P.grid[1], P.grid[2]);
-    if (G.nb == 1) {
-      gemm_combine_kernel<1><<<cgrid, 256, 0, s.stream()>>>(A);
-    } else {
-      gemm_combine_kernel<2><<<cgrid, 256, 0, s.stream()>>>(A);
-    }
-    MI355_HIP(hipGetLastError());
+    MI355_HIP(launch_kernel(G.nb == 1 ? gemm_combine_kernel<1> : gemm_combine_kernel<2>, cgrid, 256, 0, s.stream(), A));
   }
   if (rc == 1) {
     s.last().kernel_id = MI355_KERNEL_F16_GEMM;

@@ -5,7 +5,6 @@
 #include "gemm_tiles.h"
 #include "tb_program.h"
 #include <algorithm>
-#include <atomic>
 #include <string>
 
 namespace mi355 {
@@ -31,14 +30,8 @@ int launch_one(TileGemmParams const &L, dim3 grid, int threads, int lds) {
     return 1;
   }
   auto *fn = gemm_tiles_kernel<MT, CT, NB, PRO, LORA, WCM>;
-  static std::atomic<int> granted{0};  // per instantiation
-  if (lds > 65536 && granted.load(std::memory_order_acquire) < lds) {
-    MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  state().max_lds));
-    granted.store(state().max_lds, std::memory_order_release);
-  }
-  fn<<<grid, threads, lds, state().stream()>>>(L);
-  MI355_HIP(hipGetLastError());
+  MI355_GRANT_LDS(fn, lds);
+  MI355_HIP(launch_kernel(fn, grid, threads, lds, state().stream(), L));
   return 1;
 }
 
@@ -59,9 +52,15 @@ int launch_gemm_tiles(GemmParams const &A, TileGemmPlan const &p) {
   int const F = A.forloop_range;
   long long const blocks = (long long)p.grid[0] * p.grid[1] * p.grid[2];
   int const groups = (A.M + 15) / 16;
-  // Rows: one slab of up to 64 (the weights stream once); the members with a prologue or a second
-  // product keep at most 32 rows in registers.
-  int const mt = groups <= 1 ? 1 : (groups == 2 || !plain ? 2 : 4);
+  // Rows: as many as one slab can hold (64; 32 for the members with a prologue or a second product),
+  // so that the weights stream once, while that leaves a workgroup for every compute unit; fewer
+  // otherwise: the slabs then re-read weights of a few MB from the L2, which costs less than an idle
+  // chip (38 rows x 48 columns x 12 blocks, for-loop 24: 9.9 us in 36 workgroups, 6.7 in 108).  A
+  // lora slab also repeats X.A, so it is cut later.
+  int mt = groups <= 1 ? 1 : (groups == 2 || !plain ? 2 : 4);
+  while (mt > 1 && blocks * ((groups + mt - 1) / mt) * (p.cols / 16) < (lora ? 128 : 256)) {
+    mt /= 2;
+  }
   int const slabs = (groups + mt - 1) / mt;
   // Columns: 32 per workgroup where that still leaves two workgroups for every compute unit (half
   // the activation traffic, and 64-byte rows of a row-major weight strip), else 16.
@@ -78,11 +77,14 @@ int launch_gemm_tiles(GemmParams const &A, TileGemmPlan const &p) {
   if (gx * (unsigned)std::max(L.strips, L.slabs) >= (1ull << 32) || gx > 2147483647ull) {
     return 0;  // (the magics are exact below 2^32)
   }
-  // Lanes: a wavefront per iteration up to eight.  A round is the whole for-loop while its slots
+  // Lanes: a wavefront per iteration up to what the instantiation allows, sixteen only while there
+  // are fewer than two workgroups for every compute unit (16 rows x 128 columns x 119 blocks: 13.6 us
+  // with eight lanes, 15.8 with sixteen).  A round is the whole for-loop while its slots
   // take at most 64 KB (two workgroups per compute unit), else as many whole sets of lanes as fit
   // half of that, double buffered.
   int const slot = p.nb * 16 * mt * (16 * ct + 4) * 2;
-  int const sets = (F + 7) / 8, ip = (F + sets - 1) / sets;
+  int const most = gx * p.grid[1] * p.grid[2] < 512 ? gemm_tiles_lanes(mt, ct, p.nb, p.pro, lora) : 8;
+  int const sets = (F + most - 1) / most, ip = (F + sets - 1) / sets;
   L.round = (long long)F * slot <= 65536 ? F : std::max(1, 32768 / (ip * slot)) * ip;
   if (L.round > F) {
     L.round = F;

@@ -6,6 +6,8 @@
 #include "common.h"
 #include <atomic>
 #include <cstring>
+#include <mutex>
+#include <unordered_set>
 #include <vector>
 
 namespace mi355 {
@@ -26,6 +28,20 @@ int fail(int code, char const *fmt, ...) {
 }
 
 thread_local int tls_queue = 0;
+
+int grant_lds(void const *fn, int lds) {
+  if (lds <= 65536) {
+    return MI355_OK;
+  }
+  static std::mutex m;
+  static std::unordered_set<void const *> granted;
+  std::lock_guard<std::mutex> lock(m);
+  if (granted.count(fn) == 0) {
+    MI355_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, state().max_lds));
+    granted.insert(fn);
+  }
+  return MI355_OK;
+}
 
 int sync_all_queues() {
   State &s = state();
@@ -278,12 +294,16 @@ extern "C" int mi355_set_option(int option, int value) {
     state().direct_lanes = value;
     return MI355_OK;
   }
-  if (option == MI355_OPT_GEMM_MODE && value >= 0 && value <= 3) {
+  if (option == MI355_OPT_GEMM_MODE && value >= 0 && value <= 2) {
     state().gemm_mode = value;
     return MI355_OK;
   }
   if (option == MI355_OPT_F16_MATMUL_ROUTE && (value == 0 || value == 1)) {
     state().f16_matmul_route = value;
+    return MI355_OK;
+  }
+  if (option == MI355_OPT_ANY_SIZE_KERNELS && (value == 0 || value == 1)) {
+    state().any_size_kernels = value;
     return MI355_OK;
   }
   if (option == MI355_OPT_PHASE_TRACE && (value == 0 || value == 1)) {

@@ -1176,14 +1176,15 @@ static void choose_splits(DevProgram &prog, PlanExtents const &ext, int num_outp
 }
 
 // `ext_out` set: the caller decides about split for-loops itself (batched launches).
+// `interpreter`: lower for the generic interpreter whatever kernel would recognise the plan.
 static int prepare(mi355_plan const *plan, void const *const *inputs, void *const *outputs,
-                   bool f16, DevProgram &prog, PlanExtents *ext_out = nullptr) {
+                   bool f16, DevProgram &prog, PlanExtents *ext_out = nullptr, bool interpreter = false) {
   if (plan == nullptr || inputs == nullptr || outputs == nullptr) {
     return fail(MI355_ERR_INVALID, "null argument");
   }
   PlanExtents ext;
   std::string err;
-  bool const try_fused = f16 && !state().force_interpreter;
+  bool const try_fused = f16 && !state().force_interpreter && !interpreter;
   // a fused kernel keeps tiles in registers, so the interpreter's LDS need does not
   // bound it: lower without the limit first, and again with it if no fused kernel fits
   bool const declared = f16 && state().plan_smem_layout != 0;
@@ -1295,12 +1296,15 @@ static int fold_splits(DevProgram const &prog) {
     }
     long long const n = prog.part_elems[o];
     int const blocks = (int)std::min<long long>((n + 255) / 256, 2048);
-    fp_combine_splits_kernel<<<blocks, 256, 0, s.stream()>>>(
-        prog.part[o], static_cast<uint16_t *>(prog.out[o]), n, prog.part_stride[o], prog.splits);
+    MI355_HIP(launch_kernel(fp_combine_splits_kernel, blocks, 256, 0, s.stream(), prog.part[o],
+                            static_cast<uint16_t *>(prog.out[o]), n, prog.part_stride[o], prog.splits));
   }
-  MI355_HIP(hipGetLastError());
   return MI355_OK;
 }
+
+// What launch() returns when the fused kernel a program was recognised for does not take its
+// addresses (tile origins beyond 31 bits, say): the program runs on the interpreter instead.
+constexpr int kDeclined = 1;
 
 static int launch(DevProgram const &prog, bool f16) {
   State &s = state();
@@ -1327,44 +1331,44 @@ static int launch(DevProgram const &prog, bool f16) {
     int rc = prog.fused == 1   ? try_launch_attention(prog)
              : prog.fused == 2 ? try_launch_gemm(prog)
                                : try_launch_combine(prog);
-    if (rc == 1) {
-      return MI355_OK;
-    }
-    return rc < 0 ? rc : fail(MI355_ERR_UNSUPPORTED, "fused kernel declined the launch");
+    return rc == 1 ? MI355_OK : (rc < 0 ? rc : kDeclined);
   }
   dim3 grid(prog.grid[0] * (f16 ? 1 : prog.splits), prog.grid[1], prog.grid[2]);
-  // atomics: host threads of different queues may get here together (raising the limit twice
-  // is harmless, a torn flag is not)
-  static std::atomic<int> fp_lds_set{0}, f16_lds_set{0};
-  std::atomic<int> &cur = f16 ? f16_lds_set : fp_lds_set;
-  if (prog.lds_bytes > 65536 && prog.lds_bytes > cur) {
-    if (f16) {
-      MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(f16_interp_kernel),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, s.max_lds));
-    } else {
-      MI355_HIP(hipFuncSetAttribute(reinterpret_cast<void const *>(fp_interp_kernel),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, s.max_lds));
-    }
-    cur = s.max_lds;
-  }
   if (f16) {
-    f16_interp_kernel<<<grid, kInterpThreads, prog.lds_bytes, s.stream()>>>(prog, s.phase_trace);
+    MI355_GRANT_LDS(f16_interp_kernel, prog.lds_bytes);
+    MI355_HIP(launch_kernel(f16_interp_kernel, grid, kInterpThreads, prog.lds_bytes, s.stream(), prog, s.phase_trace));
   } else {
-    fp_interp_kernel<<<grid, kInterpThreads, prog.lds_bytes, s.stream()>>>(prog, s.exp_tbl,
-                                                                          s.div_p, s.div_q);
+    MI355_GRANT_LDS(fp_interp_kernel, prog.lds_bytes);
+    MI355_HIP(launch_kernel(fp_interp_kernel, grid, kInterpThreads, prog.lds_bytes, s.stream(), prog, s.exp_tbl, s.div_p,
+                            s.div_q));
     if (prog.splits > 1) {
       if (int rc = fold_splits(prog)) {
         return rc;
       }
     }
   }
-  MI355_HIP(hipGetLastError());
   s.last().kernel_id = f16 ? MI355_KERNEL_F16_INTERP : MI355_KERNEL_FP_INTERP;
   s.last().workgroups = (int)(grid.x * grid.y * grid.z);
   s.last().threads = kInterpThreads;
   s.last().lds_bytes = prog.lds_bytes;
   s.last().row_split = 1;
   return MI355_OK;
+}
+
+// One call of a customized operator: lowered and launched (or, under a recorder, recorded).
+static int run_plan(mi355_plan const *plan, void const *const *inputs, void *const *outputs, bool f16) {
+  DevProgram prog;
+  int rc = prepare(plan, inputs, outputs, f16, prog);
+  if (rc != MI355_OK) {
+    return rc;
+  }
+  rc = launch(prog, f16);
+  if (rc == kDeclined) {
+    if ((rc = prepare(plan, inputs, outputs, f16, prog, nullptr, true)) == MI355_OK) {
+      rc = launch(prog, f16);
+    }
+  }
+  return rc;
 }
 
 }  // namespace mi355
@@ -1407,12 +1411,7 @@ extern "C" int mi355_plan_extents(mi355_plan const *plan, long long *in_elems,
 extern "C" int mi355_customized_fp(mi355_plan const *plan, void const *const *inputs,
                                    void *const *outputs) {
   MI355_REQUIRE_INIT();
-  DevProgram prog;
-  int rc = prepare(plan, inputs, outputs, false, prog);
-  if (rc != MI355_OK) {
-    return rc;
-  }
-  return launch(prog, false);
+  return run_plan(plan, inputs, outputs, false);
 }
 
 // ---- the entry point that allocates nothing ----------------------------------------------
@@ -1865,26 +1864,89 @@ extern "C" int mi355_customized_fp_batch(mi355_plan const *plans, int n,
 extern "C" int mi355_customized_run(mi355_plan const *plan, void const *const *inputs,
                                     void *const *outputs) {
   MI355_REQUIRE_INIT();
-  DevProgram prog;
-  int rc = prepare(plan, inputs, outputs, true, prog);
+  return run_plan(plan, inputs, outputs, true);
+}
+
+// ---- prepared operators ------------------------------------------------------------------------
+// The kernel launches of one customized operator, recorded once and repeated: see launch.h.  They
+// hold for the queue (its scratch memory is in the arguments) and the options they were recorded
+// under; a run from another queue or after mi355_set_option records them again.
+struct mi355_prepared {
+  mi355_plan plan;
+  void const *inputs[MI355_MAX_DMEM_INPUTS];
+  void *outputs[MI355_MAX_DMEM_OUTPUTS];
+  bool fp16;
+  int queue;
+  unsigned generation;
+  LaunchList list;
+  mi355_launch_info info;
+};
+
+static int record_prepared(mi355_prepared &p) {
+  p.list.launches.clear();
+  p.queue = tls_queue;
+  p.generation = options_generation();
+  launch_recorder() = &p.list;
+  int const rc = run_plan(&p.plan, p.inputs, p.outputs, p.fp16);
+  launch_recorder() = nullptr;
+  p.info = state().last();
   if (rc != MI355_OK) {
+    p.generation = 0;  // (nothing to repeat: recorded again on the next run)
+  }
+  return rc;
+}
+
+extern "C" int mi355_prepare(mi355_plan const *plan, void const *const *inputs, void *const *outputs, int fingerprint,
+                             mi355_prepared **prepared) {
+  MI355_REQUIRE_INIT();
+  if (plan == nullptr || inputs == nullptr || outputs == nullptr || prepared == nullptr ||
+      plan->num_dmem_inputs > MI355_MAX_DMEM_INPUTS || plan->num_dmem_outputs > MI355_MAX_DMEM_OUTPUTS) {
+    return fail(MI355_ERR_INVALID, "bad argument");
+  }
+  std::unique_ptr<mi355_prepared> p(new mi355_prepared{});
+  p->plan = *plan;
+  std::copy(inputs, inputs + plan->num_dmem_inputs, p->inputs);
+  std::copy(outputs, outputs + plan->num_dmem_outputs, p->outputs);
+  p->fp16 = fingerprint == 0;
+  if (int rc = record_prepared(*p)) {
     return rc;
   }
-  return launch(prog, true);
+  *prepared = p.release();
+  return MI355_OK;
+}
+
+extern "C" int mi355_prepared_run(mi355_prepared *prepared) {
+  MI355_REQUIRE_INIT();
+  if (prepared == nullptr) {
+    return fail(MI355_ERR_INVALID, "null argument");
+  }
+  mi355_prepared &p = *prepared;
+  if (p.queue != tls_queue || p.generation != options_generation()) {
+    if (int rc = record_prepared(p)) {
+      return rc;
+    }
+  }
+  State &s = state();
+  hipStream_t const q = s.stream();
+  for (RecordedLaunch &l : p.list.launches) {
+    MI355_HIP(hipLaunchKernel(l.fn, l.grid, l.block, l.args.data(), l.lds, q));
+  }
+  s.last() = p.info;
+  return MI355_OK;
+}
+
+extern "C" int mi355_prepared_free(mi355_prepared *prepared) {
+  delete prepared;
+  return MI355_OK;
 }
 
 namespace mi355 {
 namespace {
-// The kernel launches one call of launch() makes, taken from a stream capture of that call so
-// that a timed loop can repeat them without going through plan matching and parameter set-up
-// every time: with a 3.7 us kernel that host work (2.8 - 3.9 us a launch) is sometimes more than
-// the device needs and the loop then times the host.  The captured graph is never launched; it
-// owns the argument copies the node parameters point to.
+// A timed loop's launches: those of one call (see launch.h), and for long loops `kRepeats` calls'
+// worth of them as one chain of kernel nodes -- one graph launch enqueues them all, for a
+// fraction of the host time of as many kernel launches.
 struct LaunchReplay {
-  hipGraph_t graph = nullptr;
-  std::vector<hipKernelNodeParams> kernels;  // in launch order
-  // `kRepeats` calls' worth of those kernels as one chain of kernel nodes: one graph launch
-  // enqueues them all, for a fraction of the host time of as many kernel launches
+  LaunchList list;
   static constexpr int kRepeats = 256;
   hipGraph_t chain = nullptr;
   hipGraphExec_t chain_exec = nullptr;
@@ -1896,9 +1958,6 @@ struct LaunchReplay {
     if (chain != nullptr) {
       (void)hipGraphDestroy(chain);
     }
-    if (graph != nullptr) {
-      (void)hipGraphDestroy(graph);
-    }
   }
   // false (and no chain) when the runtime refuses any step: the caller launches kernel by kernel
   bool build_chain() {
@@ -1906,12 +1965,18 @@ struct LaunchReplay {
       return chain_exec != nullptr;
     }
     chain_tried = true;
-    if (kernels.empty() || hipGraphCreate(&chain, 0) != hipSuccess) {
+    if (list.launches.empty() || hipGraphCreate(&chain, 0) != hipSuccess) {
       return false;
     }
     hipGraphNode_t prev = nullptr;
     for (int r = 0; r < kRepeats; r++) {
-      for (hipKernelNodeParams const &k : kernels) {
+      for (RecordedLaunch &l : list.launches) {
+        hipKernelNodeParams k{};
+        k.func = const_cast<void *>(l.fn);
+        k.gridDim = l.grid;
+        k.blockDim = l.block;
+        k.sharedMemBytes = l.lds;
+        k.kernelParams = l.args.data();
         hipGraphNode_t node = nullptr;
         if (hipGraphAddKernelNode(&node, chain, prev == nullptr ? nullptr : &prev, prev == nullptr ? 0 : 1, &k) !=
             hipSuccess) {
@@ -1930,74 +1995,8 @@ struct LaunchReplay {
   }
 };
 
-// R.kernels filled, or left empty when the call cannot be replayed (it enqueues something other
-// than kernels, fails under capture, or capture is refused).
-int capture_launches(DevProgram const &prog, bool fp16, LaunchReplay &R) {
-  hipStream_t const q = state().stream();
-  if (hipStreamBeginCapture(q, hipStreamCaptureModeThreadLocal) != hipSuccess) {
-    (void)hipGetLastError();
-    return MI355_OK;
-  }
-  int const rc = launch(prog, fp16);
-  hipGraph_t g = nullptr;
-  hipError_t const ended = hipStreamEndCapture(q, &g);  // (always: the queue must leave capture)
-  R.graph = g;
-  if (rc != MI355_OK || ended != hipSuccess || g == nullptr) {
-    // (a call that fails under capture, e.g. because it waits for something, is made again
-    // outside it by the caller's loop, which then reports what it returns)
-    (void)hipGetLastError();
-    return MI355_OK;
-  }
-  size_t n = 0;
-  if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n == 0 || n > 16) {
-    return MI355_OK;
-  }
-  std::vector<hipGraphNode_t> nodes(n);
-  if (hipGraphGetNodes(g, nodes.data(), &n) != hipSuccess) {
-    return MI355_OK;
-  }
-  // launch order: a capture of one queue is a chain, each node depending on the one before
-  size_t ne = 0;
-  if (hipGraphGetEdges(g, nullptr, nullptr, &ne) != hipSuccess || ne != n - 1) {
-    return MI355_OK;
-  }
-  std::vector<hipGraphNode_t> from(ne), to(ne);
-  if (ne > 0 && hipGraphGetEdges(g, from.data(), to.data(), &ne) != hipSuccess) {
-    return MI355_OK;
-  }
-  std::vector<hipGraphNode_t> order;
-  for (hipGraphNode_t cand : nodes) {  // the head: no edge ends in it
-    if (std::find(to.begin(), to.end(), cand) == to.end()) {
-      order.push_back(cand);
-    }
-  }
-  if (order.size() != 1) {
-    return MI355_OK;
-  }
-  while (order.size() < n) {
-    auto const it = std::find(from.begin(), from.end(), order.back());
-    if (it == from.end()) {
-      return MI355_OK;
-    }
-    order.push_back(to[it - from.begin()]);
-  }
-  std::vector<hipKernelNodeParams> kernels;
-  for (hipGraphNode_t node : order) {
-    hipGraphNodeType type;
-    hipKernelNodeParams kp{};
-    if (hipGraphNodeGetType(node, &type) != hipSuccess || type != hipGraphNodeTypeKernel ||
-        hipGraphKernelNodeGetParams(node, &kp) != hipSuccess || kp.extra != nullptr) {
-      return MI355_OK;
-    }
-    kernels.push_back(kp);
-  }
-  R.kernels = std::move(kernels);
-  return MI355_OK;
-}
-
-// The last call each queue profiled, kept with its captured launches: a caller that warms up
-// in one call and times in the next (same plan, same tensors) pays for the capture and the
-// chain once, outside its timed call.
+// The last call each queue profiled, kept with its launches: a caller that warms up in one call and
+// times in the next (same plan, same tensors) pays for the chain once, outside its timed call.
 struct KeptReplay {
   bool fp16 = false;
   unsigned generation = 0;
@@ -2010,8 +2009,9 @@ KeptReplay g_kept[MI355_NUM_QUEUES];
 std::atomic<unsigned> g_kept_generation{1};
 }  // namespace
 
-// (options change which kernels a plan runs on: what was captured under the old ones is dropped)
+// (options change which kernels a plan runs on: what was recorded under the old ones is dropped)
 void drop_profile_replays() { g_kept_generation.fetch_add(1, std::memory_order_relaxed); }
+unsigned options_generation() { return g_kept_generation.load(std::memory_order_relaxed); }
 }  // namespace mi355
 
 extern "C" int mi355_customized_profile(mi355_plan const *plan, void const *const *inputs,
@@ -2027,7 +2027,7 @@ extern "C" int mi355_customized_profile(mi355_plan const *plan, void const *cons
     return rc;
   }
   State &s = state();
-  // What a call launches is captured once and repeated from there (kernel by kernel, or, for
+  // What a call launches is recorded once and repeated from there (kernel by kernel, or, for
   // loops of 512 launches and more, 256 calls at a time as one chain of kernel nodes), so that
   // the loop times the device and not plan matching, parameter set-up and launch calls on the
   // host.  The loop is also paced: a marker after every batch of 1024, and the host waits for
@@ -2045,18 +2045,24 @@ extern "C" int mi355_customized_profile(mi355_plan const *plan, void const *cons
     kept.generation = generation;
     std::memcpy(&kept.prog, &prog, sizeof(prog));
     kept.fp16 = fingerprint == 0;
-    if ((rc = capture_launches(prog, fingerprint == 0, *kept.replay)) != MI355_OK) {
+    launch_recorder() = &kept.replay->list;
+    rc = launch(prog, fingerprint == 0);
+    if (rc == kDeclined) {
+      kept.replay->list.launches.clear();
+      if ((rc = prepare(plan, inputs, outputs, fingerprint == 0, prog, nullptr, true)) == MI355_OK) {
+        rc = launch(prog, fingerprint == 0);
+      }
+    }
+    launch_recorder() = nullptr;
+    if (rc != MI355_OK) {
       kept.replay.reset();
       return rc;
     }
   }
   LaunchReplay &replay = *kept.replay;
   auto launch_once = [&]() -> int {
-    if (replay.kernels.empty()) {
-      return launch(prog, fingerprint == 0);
-    }
-    for (hipKernelNodeParams const &k : replay.kernels) {
-      MI355_HIP(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes, s.stream()));
+    for (RecordedLaunch &l : replay.list.launches) {
+      MI355_HIP(hipLaunchKernel(l.fn, l.grid, l.block, l.args.data(), l.lds, s.stream()));
     }
     return MI355_OK;
   };

@@ -159,6 +159,14 @@ int mirage_op_execute(void *g, int idx) {
   return 0;
 }
 
+// every operator in order
+int mirage_graph_execute(void *g) {
+  for (KNOperator *op : static_cast<kernel::Graph *>(g)->operators) {
+    kernel::execute_once(op);
+  }
+  return 0;
+}
+
 // the lowered program of a customized op, as handed to the backend
 int mirage_op_lowered(void *g, int idx, int fingerprint, mi355_plan *out, int *smem_offset) {
   KNOperator *op = static_cast<kernel::Graph *>(g)->operators.at(idx);

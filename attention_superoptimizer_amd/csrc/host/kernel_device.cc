@@ -306,7 +306,7 @@ struct LoweredOp {
   void *outputs[MI355_MAX_DMEM_OUTPUTS];
 };
 
-static LoweredOp lower(KNCustomizedOp const &op, bool fingerprint) {
+static LoweredOp lower_unchecked(KNCustomizedOp const &op, bool fingerprint) {
   mirage::threadblock::NewKernelParams p = op.bgraph.get_new_kernel_params(fingerprint);
   LoweredOp l;
   std::memset(&l, 0, sizeof(l));
@@ -333,6 +333,10 @@ static LoweredOp lower(KNCustomizedOp const &op, bool fingerprint) {
   for (int i = 0; i < p.num_dmem_outputs; i++) {
     l.outputs[i] = p.dmem_output_ptrs[i];
   }
+  return l;
+}
+
+static void check_extents(KNCustomizedOp const &op, LoweredOp const &l) {
   // every tile the program touches must lie inside its device tensor
   long long in_ext[MI355_MAX_DMEM_INPUTS], out_ext[MI355_MAX_DMEM_OUTPUTS];
   MI355_CALL(mi355_plan_extents(&l.plan, in_ext, out_ext, nullptr, nullptr));
@@ -350,6 +354,11 @@ static LoweredOp lower(KNCustomizedOp const &op, bool fingerprint) {
       oo++;
     }
   }
+}
+
+static LoweredOp lower(KNCustomizedOp const &op, bool fingerprint) {
+  LoweredOp l = lower_unchecked(op, fingerprint);
+  check_extents(op, l);
   return l;
 }
 
@@ -362,10 +371,33 @@ void lower_customized(KNCustomizedOp const &op, bool fingerprint, mi355_plan *pl
   std::memcpy(outputs, l.outputs, sizeof(l.outputs));
 }
 
+// A run of the operator repeats the launches the backend prepared for it the first time, as long
+// as its program, lowered again here, is the one they were prepared for (a layout search may have
+// changed the storage orders since): lowering is a few hundred nanoseconds, checking the extents
+// and choosing a kernel several microseconds.  One set per domain and queue: a queue is driven by one thread.
+struct KeptLaunch {
+  LoweredOp lowered;
+  mi355_prepared *prepared = nullptr;
+  ~KeptLaunch() { mi355_prepared_free(prepared); }
+};
+
+void KNCustomizedOp::launch(bool fingerprint) {
+  LoweredOp const l = lower_unchecked(*this, fingerprint);
+  static_assert(sizeof(kept) / sizeof(kept[0]) == 2 && sizeof(kept[0]) / sizeof(kept[0][0]) == MI355_NUM_QUEUES, "per queue");
+  std::shared_ptr<KeptLaunch> &k = kept[fingerprint ? 1 : 0][mi355_queue_current()];
+  if (k == nullptr || std::memcmp(&k->lowered, &l, sizeof(l)) != 0) {
+    check_extents(*this, l);
+    k = std::make_shared<KeptLaunch>();
+    k->lowered = l;
+    int const rc = mi355_prepare(&l.plan, l.inputs, l.outputs, fingerprint ? 1 : 0, &k->prepared);
+    MIRAGE_CHECK(rc == MI355_OK, mi355_last_error());
+  }
+  MI355_CALL(mi355_prepared_run(k->prepared));
+}
+
 void KNCustomizedOp::run() {
   require_device("KNCustomizedOp::run");
-  LoweredOp l = lower(*this, false);
-  MI355_CALL(mi355_customized_run(&l.plan, l.inputs, l.outputs));
+  launch(false);
 }
 
 bool KNCustomizedOp::profile(ProfileResult &result) {
@@ -387,8 +419,7 @@ bool KNCustomizedOp::profile(ProfileResult &result) {
 
 bool KNCustomizedOp::fingerprint(void) {
   require_device("KNCustomizedOp::fingerprint");
-  LoweredOp l = lower(*this, true);
-  MI355_CALL(mi355_customized_fp(&l.plan, l.inputs, l.outputs));
+  launch(true);
   return true;
 }
 

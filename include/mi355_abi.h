@@ -130,9 +130,8 @@ typedef struct mi355_launch_info {
  * launch with the output tile cut into 16 x 16 pieces for plans that would otherwise leave
  * most of the chip idle; the for-loop cut into ranges, plus a launch that adds them, for
  * plans whose traffic, not the launch, sets the time); 1 = always the range-splitting kernel; 2 = the one-launch
- * kernel wherever it applies; 3 = the kernel for tiles of any size, which otherwise runs the
- * plans the other two are not built for.  All keep the accumulation order of the sequential
- * loop.  A measurement knob that the tests use to cover them. */
+ * kernel wherever it applies.  Both keep the accumulation order of the sequential loop;
+ * results agree to the last bit.  A measurement knob that the tests use to cover both. */
 #define MI355_OPT_GEMM_MODE 7
 /* F16_MATMUL_ROUTE: what runs a kernel-level fp16 matmul (mi355_f16_matmul,
  * mi355_f16_matmul_layout).  0 = this library's kernels (default); 1 = the vendor's BLAS
@@ -143,6 +142,10 @@ typedef struct mi355_launch_info {
  * runs in its place.  Both routes accumulate in fp32 and round once; their sums differ in
  * order, so results agree to fp16 rounding, not to the bit. */
 #define MI355_OPT_F16_MATMUL_ROUTE 8
+/* ANY_SIZE_KERNELS: 1 = attention and skinny-GEMM plans run on the kernels for tiles of any size
+ * wherever those apply; 0 = only the plans the kernels of whole tiles are not built for, or
+ * slower on (default).  A measurement knob that the tests use to cover them. */
+#define MI355_OPT_ANY_SIZE_KERNELS 9
 
 /* ---- lifetime ------------------------------------------------------------
  * Replaces DeviceMemoryManager's constructor / destructor
@@ -325,12 +328,23 @@ int mi355_plan_extents(mi355_plan const *plan, long long *in_elems, long long *o
  * src/kernel/cuda/customized_kernel.cu:39-305,605-613 */
 int mi355_customized_run(mi355_plan const *plan, void const *const *inputs,
                          void *const *outputs);
+/* The same (fingerprint != 0: mi355_customized_fp) for a caller that runs one operator many
+ * times on the same tensors: mi355_prepare lowers the plan, chooses the kernels and keeps their
+ * launches (no device work), mi355_prepared_run repeats them on the calling thread's queue.
+ * Lowering, matching and parameter set-up cost the host 4 us and more per call, a repeated launch
+ * is one launch call.  A handle holds host memory only.  It follows the queue and the options: a
+ * run from another queue than the last, or after mi355_set_option, prepares again first.  One
+ * thread at a time uses a handle. */
+typedef struct mi355_prepared mi355_prepared;
+int mi355_prepare(mi355_plan const *plan, void const *const *inputs, void *const *outputs,
+                  int fingerprint, mi355_prepared **prepared);
+int mi355_prepared_run(mi355_prepared *prepared);
+int mi355_prepared_free(mi355_prepared *prepared);
 /* KNCustomizedOp::profile, customized_kernel.cu:615-653: `warmup` untimed then
  * `iters` timed launches between two events on the backend stream; *ms = mean.
- * What one call launches is captured once (a stream capture that is not executed) and
- * repeated from there: kernel by kernel, or, for 512 launches and more, 256 calls at a time
- * as one chain of kernel nodes (one graph launch); a call that enqueues anything other than
- * kernels is repeated by calling it.  So the loop times the device: plan matching and
+ * What one call launches is recorded once (as mi355_prepare does) and repeated from there:
+ * kernel by kernel, or, for 512 launches and more, 256 calls at a time as one chain of kernel
+ * nodes (one graph launch).  So the loop times the device: plan matching and
  * parameter set-up cost the host 2.8 - 3.9 us a launch here, more than a 3.5 us kernel takes.
  * The host never runs more than two batches of 1024 launches ahead of the device (a marker
  * per batch, waited for one batch later): with several thousand launches queued every

@@ -36,8 +36,13 @@ struct TileGemmParams {
 // Steps of 32 k whose loads are in flight together.
 constexpr int gemm_tiles_steps(int MT, int NB, bool LORA) { return MT == 1 && NB == 1 && !LORA ? 8 : 4; }
 
+// Most iteration lanes of a workgroup: sixteen where 128 registers hold a lane's operands.
+constexpr int gemm_tiles_lanes(int MT, int CT, int NB, int PRO, bool LORA) {
+  return MT == 1 && CT == 1 && NB == 1 && !LORA && PRO != PRO_SILU_MUL ? 16 : 8;
+}
+
 template <int MT, int CT, int NB, int PRO, bool LORA, bool WCM>
-__global__ __launch_bounds__(512) void gemm_tiles_kernel(TileGemmParams const L) {
+__global__ __launch_bounds__(64 * gemm_tiles_lanes(MT, CT, NB, PRO, LORA)) void gemm_tiles_kernel(TileGemmParams const L) {
   fetch_kernel_arguments<sizeof(TileGemmParams), 4>();  // (blockDim.x is read)
   GemmParams const &P = L.g;
   constexpr int KS = gemm_tiles_steps(MT, NB, LORA);

@@ -4,9 +4,12 @@
 
 #include "mirage/kernel/operator.h"
 #include "mirage/threadblock/graph.h"
+#include <memory>
 
 namespace mirage {
 namespace kernel {
+
+struct KeptLaunch;
 
 class KNCustomizedOp : public KNOperator {
 public:
@@ -27,6 +30,10 @@ public:
   mirage::threadblock::Graph bgraph;
 
 private:
+  // the kernel launches of run() [0] and fingerprint() [1] per backend queue, kept from one call
+  // to the next
+  std::shared_ptr<KeptLaunch> kept[2][4];
+  void launch(bool fingerprint);
   void add_output(mirage::threadblock::STensor const &stensor, int3 output_map);
 };
 

@@ -14,9 +14,9 @@ ROW, COL = "DmemRowMajor", "DmemColumnMajor"
 
 @pytest.fixture
 def any_size_kernel(abi):
-    assert abi.mi355_set_option(7, 3) == 0
+    assert abi.mi355_set_option(9, 1) == 0
     yield
-    assert abi.mi355_set_option(7, 0) == 0
+    assert abi.mi355_set_option(9, 0) == 0
 
 
 def _run(rt, spec, order, what, std=0.1):
