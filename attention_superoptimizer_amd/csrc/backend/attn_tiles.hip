@@ -29,25 +29,23 @@ int launch_tiles_one(AttnParams const &A, dim3 grid, int ip, int lds) {
 
 template <int D, bool HAS_DIV, bool CM>
 int launch_tiles_shape(AttnParams const &A, dim3 grid, int rpw, int chb, int ip, int lds) {
-  if constexpr (D == 64) {
+  switch (rpw * 10 + chb) {
+    case 12: return launch_tiles_one<D, HAS_DIV, CM, 1, 2>(A, grid, ip, lds);
+    case 14: return launch_tiles_one<D, HAS_DIV, CM, 1, 4>(A, grid, ip, lds);
+    case 22: return launch_tiles_one<D, HAS_DIV, CM, 2, 2>(A, grid, ip, lds);
+    case 24: return launch_tiles_one<D, HAS_DIV, CM, 2, 4>(A, grid, ip, lds);
+    default: break;
+  }
+  if constexpr (D == 64 && HAS_DIV) {
     switch (rpw * 10 + chb) {
-      case 14: return launch_tiles_one<D, HAS_DIV, CM, 1, 4>(A, grid, ip, lds);
+      case 16: return launch_tiles_one<D, HAS_DIV, CM, 1, 6>(A, grid, ip, lds);
       case 18: return launch_tiles_one<D, HAS_DIV, CM, 1, 8>(A, grid, ip, lds);
-      case 24: return launch_tiles_one<D, HAS_DIV, CM, 2, 4>(A, grid, ip, lds);
+      case 26: return launch_tiles_one<D, HAS_DIV, CM, 2, 6>(A, grid, ip, lds);
       case 28: return launch_tiles_one<D, HAS_DIV, CM, 2, 8>(A, grid, ip, lds);
-      case 44: return launch_tiles_one<D, HAS_DIV, CM, 4, 4>(A, grid, ip, lds);
       default: break;
     }
-    if constexpr (HAS_DIV) {
-      return rpw * 10 + chb == 48 ? launch_tiles_one<D, HAS_DIV, CM, 4, 8>(A, grid, ip, lds) : 0;
-    }
-    return 0;
   }
-  switch (rpw * 10 + chb) {
-    case 14: return launch_tiles_one<D, HAS_DIV, CM, 1, 4>(A, grid, ip, lds);
-    case 24: return launch_tiles_one<D, HAS_DIV, CM, 2, 4>(A, grid, ip, lds);
-    default: return 0;
-  }
+  return 0;
 }
 
 }  // namespace
@@ -58,29 +56,22 @@ bool choose_attn_tiles(int D, int DV, int NK, int m, bool has_div, bool cm, long
     return false;
   }
   int const nb = NK / 16;
-  t.chb = D == 64 && nb > 4 ? 8 : 4;
-  if (has_div && nb > t.chb) {
-    return false;  // the division needs the row sum of the whole tile before P.V
-  }
-  // Row groups per wavefront: as many as still leave a workgroup for every compute unit (each K / V
-  // operand then feeds that many matrix instructions), unless rounding the row groups up to
-  // whole wavefronts would add more than a third of work.
-  int const groups = (m + 15) / 16;
-  t.rpw = 1;
-  for (int r : {4, 2}) {
-    if (r == 4 && D == 128) {
-      continue;
-    }
-    int const slabs = (groups + r - 1) / r;
-    if (groups >= r && 3 * slabs * r <= 4 * groups && blocks * slabs >= 192) {
-      t.rpw = r;
-      break;
+  // Blocks of keys in registers at a time: the fewest that hold the tile, four at most (two or three
+  // wavefronts per SIMD; with eight there is one: prefill in 80-key tiles 74 us against 51).  The
+  // division needs the row sum of the whole tile before P.V, so there the tile is one chunk.
+  t.chb = nb <= 2 ? 2 : 4;
+  if (has_div && nb > 4) {
+    t.chb = nb <= 6 ? 6 : 8;
+    if (D != 64 || nb > 8) {
+      return false;
     }
   }
+  // Two row groups per wavefront (each K / V operand then feeds two matrix instructions) where that
+  // leaves a workgroup for almost every compute unit, unless rounding the row groups up to whole
+  // wavefronts would add more than a third of work.
+  int const groups = (m + 15) / 16, halves = (groups + 1) / 2;
+  t.rpw = groups >= 2 && 6 * halves <= 4 * groups && blocks * halves >= 192 ? 2 : 1;
   t.split = (groups + t.rpw - 1) / t.rpw;
-  if (t.rpw == 4 && !has_div) {
-    t.chb = 4;  // (two chunks of a longer key tile: eight blocks beside four row groups would spill)
-  }
   // Iteration lanes: one wavefront per iteration up to what the instantiation allows, evened out
   // over the rounds.
   int const most = attn_tiles_lanes(D, t.rpw, t.chb);

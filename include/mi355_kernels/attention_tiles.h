@@ -15,8 +15,8 @@
 //
 // What bounds it: the trip to memory at decode sizes (a wavefront issues all of an iteration's
 // loads before it waits for the first), the conversions and exponentials beside the matrix
-// instructions at prefill sizes.  RPW row groups share every K and V operand, which is what keeps
-// the L2 -> register traffic of a prefill down (RPW = 4: an eighth of a byte per multiply-add).
+// instructions at prefill sizes.  Two row groups share every K and V operand where there are enough
+// of them, which halves the L2 -> register traffic of a prefill.
 // Keys of a pair of 16-key blocks are permuted as in attention.h (see cm_swizzle_key) so that a
 // lane's eight values of P are consecutive keys; a lone last block keeps the plain order and takes
 // the 16 x 16 x 16 instruction.
@@ -31,7 +31,7 @@ namespace mi355 {
 // one chunk (the host checks).  AttnParams as used here: rows = query rows of a block, stages =
 // keys of a tile, lds_stage_bytes unused.
 // Most iteration lanes of a workgroup: eight where 256 registers hold a wavefront's operands.
-constexpr int attn_tiles_lanes(int D, int RPW, int CHB) { return RPW == 1 && CHB == 4 && D == 64 ? 8 : 4; }
+constexpr int attn_tiles_lanes(int D, int RPW, int CHB) { return RPW == 1 && CHB <= 4 && D == 64 ? 8 : 4; }
 
 template <int D, bool HAS_DIV, bool CM, int RPW, int CHB>
 __global__ __launch_bounds__(attn_tiles_lanes(D, RPW, CHB) * 64) void attn_tiles_kernel(AttnParams const) {
