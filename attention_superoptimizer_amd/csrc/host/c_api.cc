@@ -18,6 +18,7 @@ using kernel::KNOperator;
 namespace mirage {
 namespace kernel {
 void execute_once(KNOperator *op);
+void execute_all(Graph const &graph);
 }
 }  // namespace mirage
 
@@ -161,9 +162,7 @@ int mirage_op_execute(void *g, int idx) {
 
 // every operator in order
 int mirage_graph_execute(void *g) {
-  for (KNOperator *op : static_cast<kernel::Graph *>(g)->operators) {
-    kernel::execute_once(op);
-  }
+  kernel::execute_all(*static_cast<kernel::Graph *>(g));
   return 0;
 }
 

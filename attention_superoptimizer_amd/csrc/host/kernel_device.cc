@@ -598,5 +598,89 @@ void execute_once(KNOperator *op) {
   }
 }
 
+// ---- a whole graph: neighbouring kernel-level operators that one launch can run ------------------
+// Every tensor is still written; what a launch saves is the trip of the producer's result through
+// memory and a launch per operator.
+static bool same_shape(DTensor const &a, DTensor const &b) {
+  bool same = a.num_dims == b.num_dims;
+  for (int d = 0; same && d < a.num_dims; d++) {
+    same = a.dim[d] == b.dim[d];
+  }
+  return same;
+}
+
+// a matmul and the element-wise operator after it that reads its result
+static bool run_matmul_then(KNOperator const *mm, KNOperator const *next) {
+  bool const unary = next->op_type == KN_EXP_OP || next->op_type == KN_SILU_OP;
+  bool const binary = next->op_type == KN_ADD_OP || next->op_type == KN_MUL_OP || next->op_type == KN_DIV_OP;
+  if (mm->op_type != KN_MATMUL_OP || (!unary && !binary)) {
+    return false;
+  }
+  DTensor const &C = mm->output_tensors[0], &E = next->output_tensors[0];
+  DTensor const *X = nullptr;
+  bool x_first = false;
+  if (unary) {
+    if (next->input_tensors[0].guid != C.guid) {
+      return false;
+    }
+  } else {
+    bool const first = next->input_tensors[0].guid == C.guid, second = next->input_tensors[1].guid == C.guid;
+    if (first == second) {  // (an operator of C with itself needs C twice)
+      return false;
+    }
+    x_first = second;
+    X = &next->input_tensors[second ? 0 : 1];
+    if (!same_shape(*X, C) || column_major(*X)) {
+      return false;
+    }
+  }
+  if (!same_shape(C, E) || column_major(C) || column_major(E)) {
+    return false;
+  }
+  int batch, m, n, k;
+  matmul_extents(mm->input_tensors[0], mm->input_tensors[1], batch, m, n, k);
+  MI355_CALL(mi355_f16_matmul_then(mm->input_tensors[0].data_ptr, mm->input_tensors[1].data_ptr, C.data_ptr, batch, m, n, k,
+                                   column_major(mm->input_tensors[0]) ? 1 : 0, column_major(mm->input_tensors[1]) ? 1 : 0,
+                                   next->op_type, X == nullptr ? nullptr : X->data_ptr, x_first ? 1 : 0, E.data_ptr));
+  return true;
+}
+
+// exp, the sum of its rows and their division
+static bool is_softmax_rows(KNOperator const *e, KNOperator const *r, KNOperator const *d) {
+  if (e->op_type != KN_EXP_OP || d->op_type != KN_DIV_OP ||
+      (r->op_type != KN_REDUCTION_0_OP && r->op_type != KN_REDUCTION_1_OP && r->op_type != KN_REDUCTION_2_OP)) {
+    return false;
+  }
+  DTensor const &X = e->input_tensors[0], &E = e->output_tensors[0], &R = r->output_tensors[0], &P = d->output_tensors[0];
+  int const last = E.num_dims - 1;
+  return r->input_tensors[0].guid == E.guid && static_cast<KNReductionOp const *>(r)->reduction_dim_idx == last &&
+         R.dim[last] == 1 && d->input_tensors[0].guid == E.guid && d->input_tensors[1].guid == R.guid && same_shape(E, P) &&
+         !column_major(X) && !column_major(E) && !column_major(R) && !column_major(P);
+}
+
+static void run_softmax_rows(KNOperator const *e, KNOperator const *r, KNOperator const *d) {
+  DTensor const &X = e->input_tensors[0], &E = e->output_tensors[0], &R = r->output_tensors[0], &P = d->output_tensors[0];
+  size_t const n = (size_t)E.dim[E.num_dims - 1];
+  MI355_CALL(mi355_f16_softmax_rows(X.data_ptr, E.data_ptr, R.data_ptr, P.data_ptr, E.num_elements() / n, (int)n));
+}
+
+void execute_all(Graph const &graph) {
+  require_device("execute_all");
+  std::vector<KNOperator *> const &ops = graph.operators;
+  size_t const n = ops.size();
+  auto softmax_at = [&](size_t i) { return i + 2 < n && is_softmax_rows(ops[i], ops[i + 1], ops[i + 2]); };
+  for (size_t i = 0; i < n;) {
+    if (softmax_at(i)) {
+      run_softmax_rows(ops[i], ops[i + 1], ops[i + 2]);
+      i += 3;
+    } else if (i + 1 < n && !softmax_at(i + 1) && run_matmul_then(ops[i], ops[i + 1])) {
+      i += 2;
+    } else {
+      execute_once(ops[i]);
+      i += 1;
+    }
+  }
+}
+
 }  // namespace kernel
 }  // namespace mirage

@@ -369,6 +369,14 @@ int mi355_f16_matmul(void const *A, void const *B, void *C, int batch, int m, in
  * matrix holds element (r, c) at c * rows + r.  C is row-major (matmul_kernel.cu:74-75). */
 int mi355_f16_matmul_layout(void const *A, void const *B, void *C, int batch, int m, int n, int k,
                             int a_column_major, int b_column_major);
+/* The same, and the element-wise operator that consumes C: E = op(C) (KN_EXP_OP, KN_SILU_OP) or
+ * E = C op X (KN_ADD_OP, KN_MUL_OP, KN_DIV_OP; x_first: E = X op C) for an X of C's shape.  C and E
+ * hold what the two operators one after the other leave. */
+int mi355_f16_matmul_then(void const *A, void const *B, void *C, int batch, int m, int n, int k,
+                          int a_column_major, int b_column_major, int op, void const *X, int x_first, void *E);
+/* E = exp(X), R[row] = sum of a row of E, P = E / R for `rows` rows of n elements: what
+ * mi355_f16_unary, mi355_f16_reduce and mi355_f16_binary one after the other leave. */
+int mi355_f16_softmax_rows(void const *X, void *E, void *R, void *P, size_t rows, int n);
 /* out[b][c][r] = in[b][r][c] for `batch` [rows, cols] matrices: the row-major copy of a
  * DmemColumnMajor tensor (call it with rows = the tensor's columns and cols = its rows) for
  * the element-wise operators and reductions, which index their inputs flat as

@@ -1,0 +1,76 @@
+"""The any-shape fp16 matmul and the launches that take an operator's consumer along."""
+import numpy as np
+import pytest
+
+from attention_superoptimizer_amd import graph as G
+from helpers import assert_f16_close, normal_f16
+from oracle import evaluate as orc
+from test_gpu_f16 import _abi_matmul
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("batch,m,n,k", [
+    (1, 1, 8, 8),        # one chunk of everything
+    (2, 5, 9, 63),       # no whole stage: the partial one alone
+    (1, 17, 65, 65),     # one element past a tile, a stage and a chunk
+    (3, 15, 71, 128),    # whole stages only, ragged columns
+    (1, 3, 333, 3001),   # few tiles, long odd k: ranges of k, summed by the second launch
+    (4, 65, 191, 257),
+    (1, 300, 1001, 515),
+    (1, 1000, 4001, 75),  # the largest tiles
+    (2, 9, 7, 40),       # rows shorter than a chunk: element by element
+])
+def test_matmul_of_any_shape(rt, abi, batch, m, n, k):
+    for a_cm, b_cm in ((0, 1), (0, 0), (1, 1), (1, 0)):
+        a, b, got = _abi_matmul(rt, abi, batch, m, n, k, a_cm, b_cm, 5)
+        assert_f16_close(got, orc.f16_matmul(a, b), what=f"[{batch},{m},{k}] . [{batch},{k},{n}], A cm {a_cm}, B cm {b_cm}")
+
+
+def _execute(build, inputs, whole):
+    """Every tensor of a graph after one run: of the whole graph at once, or operator by operator."""
+    g = G.KNGraph()
+    try:
+        tensors = build(g)
+        for t, a in zip(tensors, inputs):
+            t.write_data(a)
+        if whole:
+            g.execute_all()
+        else:
+            for i in range(g.num_operators):
+                g.execute(i)
+        return [t.read_data() for t in tensors]
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("b,m,n,k", [(1, 1, 8, 16), (2, 33, 77, 65), (1, 40, 130, 3001), (1, 3, 6, 20), (1, 3600, 3700, 256)])
+@pytest.mark.parametrize("op", ["exp", "silu", "add", "mul", "div", "rdiv"])
+def test_consumer_in_the_matmul(rt, abi, op, b, m, n, k):
+    if m > 1000 and op not in ("silu", "mul"):
+        pytest.skip("the large tiles once per kind")
+
+    def build(g):
+        A, B, X = g.new_input((b, m, k)), g.new_input((b, k, n), layout="DmemColumnMajor"), g.new_input((b, m, n))
+        C = g.matmul(A, B)
+        E = g._unary(op, C) if op in ("exp", "silu") else g.div(X, C) if op == "rdiv" else g._binary(op, C, X)
+        return A, B, X, C, E
+
+    ins = [normal_f16([b, m, k], 0.2, 1), normal_f16([b, k, n], 0.2, 2), np.abs(normal_f16([b, m, n], 1.0, 3)) + np.float16(0.5)]
+    for whole, single in zip(_execute(build, ins, True), _execute(build, ins, False)):
+        np.testing.assert_array_equal(whole, single)
+
+
+@pytest.mark.parametrize("b,m,n", [(1, 1, 1), (2, 3, 7), (1, 5, 2047), (1, 5, 4097), (2, 600, 513), (1, 1024, 65), (1, 1025, 4096), (1, 2, 20001)])
+def test_softmax_rows(rt, abi, b, m, n):
+    def build(g):
+        X = g.new_input((b, m, n))
+        E = g.exp(X)
+        R = g.reduction(E, 2)
+        return X, E, R, g.div(E, R)
+
+    ins = [normal_f16([b, m, n], 0.5, 4)]
+    whole, single = _execute(build, ins, True), _execute(build, ins, False)
+    np.testing.assert_array_equal(whole[1], single[1])
+    for w, s in zip(whole[2:], single[2:]):  # (another order of the row sum)
+        assert_f16_close(w, s, rtol=2e-3, atol=1e-6, what="row sum or quotient")
