@@ -199,6 +199,7 @@ FACADE = {
 
 _backend = None
 _runtime = None
+_spec = None
 
 
 def _bind(lib, table):
@@ -233,6 +234,16 @@ def runtime():
         _bind(lib, FACADE)
         _runtime = lib
     return _runtime
+
+
+def spec():
+    """The extension that builds graph specs (linked against the runtime)."""
+    global _spec
+    if _spec is None:
+        runtime()
+        from . import _spec as module
+        _spec = module
+    return _spec
 
 
 def last_error() -> str:

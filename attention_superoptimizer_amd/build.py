@@ -2,6 +2,7 @@
 
   libmi355_backend.so   HIP kernels + the C ABI of include/mi355_abi.h
   libmirage_runtime.so  the mirage:: host API (C++) + its C facade for ctypes
+  _spec.so              CPython extension: graph specs built without a ctypes call per operator
   mirage_profile        the reference's cpp_examples/profile.cc over that API
   generated/            HIP programs written by Graph::generate_hip_program for the example
                         graphs of codegen.py, compiled as libraries and executables
@@ -12,6 +13,7 @@ from __future__ import annotations
 
 import os
 import subprocess
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 import sys
 
@@ -21,6 +23,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 BACKEND_LIB = os.path.join(HERE, "libmi355_backend.so")
 RUNTIME_LIB = os.path.join(HERE, "libmirage_runtime.so")
+SPEC_LIB = os.path.join(HERE, "_spec.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops off: packed FP32 forms have produced silent wrong results on these boxes
@@ -117,6 +120,12 @@ def build_runtime():
          ["-L" + HERE, "-lmi355_backend", "-Wl,-rpath,$ORIGIN", "-pthread"])
 
 
+def build_spec_reader():
+    """_spec: the CPython extension that reads graph specs (graph.build_from_spec)."""
+    _run(["g++", "-O2", "-fPIC", "-std=c++17", "-shared", "-I", INCLUDE, "-I", sysconfig.get_paths()["include"], "-o", SPEC_LIB,
+          os.path.join(CSRC, "python", "spec.cc"), "-L" + HERE, "-lmirage_runtime", "-lmi355_backend", "-Wl,-rpath,$ORIGIN"])
+
+
 def build_tools():
     """mirage_profile: loads a graph / checkpoint JSON, fingerprints and times it (the
     reference's cpp_examples/profile.cc)."""
@@ -141,6 +150,7 @@ def main():
     build_backend()
     if os.path.isdir(os.path.join(CSRC, "host")):
         build_runtime()
+        build_spec_reader()
         build_tools()
         build_generated()
     return 0

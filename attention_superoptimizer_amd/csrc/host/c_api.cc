@@ -5,6 +5,7 @@
 // Graph-building calls return NULL / -1 for an infeasible operator instead of
 // aborting (they go through the create_* functions).
 #include "mi355_abi.h"
+#include "mirage/c_plan.h"
 #include "mirage/kernel/device_memory_manager.h"
 #include "mirage/kernel/graph.h"
 #include "mirage/utils/hip_types.h"
@@ -23,22 +24,6 @@ void execute_all(Graph const &graph);
 }  // namespace mirage
 
 extern "C" {
-
-typedef struct mirage_c_plan {
-  int grid_dim[3];
-  int block_dim[3];
-  int forloop_range;
-  int reduction_dimx;
-  int num_inputs;
-  int input_map[4][3];
-  int forloop_dim[4];
-  int input_smem_layout[4];
-  int output_map[3];
-  int num_ops;
-  int op_type[16];
-  int op_num_operands[16];
-  int op_operands[16][2][2];
-} mirage_c_plan;
 
 void *mirage_graph_create(void) { return new kernel::Graph(); }
 

@@ -55,23 +55,25 @@ def device_ready() -> bool:
 class DTensor:
     """Handle of a mirage::kernel::DTensor owned by an operator of a KNGraph."""
 
-    def __init__(self, handle: int):
-        self._h = ctypes.c_void_p(handle)
+    __slots__ = ("_h", "dims", "data_type", "guid", "__weakref__")
+
+    def __init__(self, handle: int, dims=None, data_type=None, guid=None):
+        self._h = handle
+        if dims is None:
+            dims, data_type, guid, _ = self._info()
+        self.dims, self.data_type, self.guid = dims, data_type, guid
+
+    def _info(self):
         nd, dt, lay = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         dims = (ctypes.c_int * 4)()
         guid = ctypes.c_longlong()
         N.runtime().mirage_tensor_info(self._h, nd, dims, dt, lay, guid)
-        self.dims = tuple(dims[i] for i in range(nd.value))
-        self.data_type, self.guid = dt.value, guid.value
+        return tuple(dims[i] for i in range(nd.value)), dt.value, guid.value, lay.value
 
     @property
     def layout(self) -> int:
         """The tensor's DmemLayout now (a layout search may have changed it)."""
-        nd, dt, lay = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
-        dims = (ctypes.c_int * 4)()
-        guid = ctypes.c_longlong()
-        N.runtime().mirage_tensor_info(self._h, nd, dims, dt, lay, guid)
-        return lay.value
+        return self._info()[3]
 
     @property
     def num_elements(self) -> int:
@@ -416,25 +418,5 @@ def build_from_spec(spec: List[dict], graph: Optional[KNGraph] = None):
     """Builds a graph spec (see workloads.py) through the host API.
     Returns (graph, per-operator lists of output tensors)."""
     g = graph or KNGraph()
-    vals: List[List[DTensor]] = []
-
-    def get(ref):
-        return vals[ref[0]][ref[1]]
-
-    for op in spec:
-        k = op["op"]
-        if k == "input":
-            vals.append([g.new_input(op["dims"], DT_FLOAT16, op.get("layout", "DmemRowMajor"))])
-        elif k == "matmul":
-            vals.append([g.matmul(get(op["in"][0]), get(op["in"][1]))])
-        elif k in ("exp", "silu"):
-            vals.append([g._unary(k, get(op["in"][0]))])
-        elif k in ("add", "mul", "div"):
-            vals.append([g._binary(k, get(op["in"][0]), get(op["in"][1]))])
-        elif k == "reduction":
-            vals.append([g.reduction(get(op["in"][0]), op["dim"], op.get("size", 1))])
-        elif k == "customized":
-            vals.append(g.customized([get(r) for r in op["in"]], op["plan"]))
-        else:
-            raise ValueError(k)
-    return g, vals
+    return g, N.spec().build(g._g.value, spec if isinstance(spec, list) else list(spec), DTensor, DMEM_LAYOUT, SMEM_LAYOUT,
+                             KN_OP, TB_OP, InfeasibleOperator)
