@@ -53,8 +53,8 @@ struct State {
   size_t arena_bytes = 0;
   // device copies of the lookup tables, reference layout
   uint16_t *exp_tbl = nullptr, *div_p = nullptr, *div_q = nullptr;
-  int *flag = nullptr;        // device scratch of mi355_fp_equal: one int per queue, 64 bytes apart
-  int *flag_host = nullptr;   // pinned mirror, same layout
+  int *flag_host = nullptr;   // answers of mi355_fp_equal, pinned: one int per queue, 64 bytes apart
+  int *flag = nullptr;        // the same memory as the device addresses it
   int *queue_flag() const { return flag + 16 * tls_queue; }
   int *queue_flag_host() const { return flag_host + 16 * tls_queue; }
   int *cmp_host = nullptr;    // MI355_COMPARE_SLOTS mismatch flags of deferred compares, in
@@ -159,22 +159,57 @@ int fail(int code, char const *fmt, ...);
     }                                                                               \
   } while (0)
 
-// x mod 25651 / 227 / 113 for 32-bit x.  The compiler lowers `%` by a constant to
-// a multiply-high; kept as functions so every kernel spells it the same way.
-__device__ __forceinline__ uint32_t mod_pq(uint32_t x) { return x % FP_PQ; }
-__device__ __forceinline__ uint32_t mod_p(uint32_t x) { return x % FP_P; }
-__device__ __forceinline__ uint32_t mod_q(uint32_t x) { return x % FP_Q; }
+// Residues of a 16-bit value.  The compiler lowers `%` by a constant to 32-bit multiply-highs, which
+// run at a quarter of the rate of a 24-bit multiply; for values below 2^16 a 24-bit reciprocal is exact
+// (37118 = ceil(2^22 / 113); 36954 = floor(2^23 / 227), so the value is taken one higher).
+__device__ __forceinline__ uint32_t residue_q(uint32_t x) { return x - __umul24(__umul24(x, 37118u) >> 22, FP_Q); }
+__device__ __forceinline__ uint32_t residue_p(uint32_t x) { return x - __umul24((__umul24(x, 36954u) + 36954u) >> 23, FP_P); }
+// the residue modulo 227 in [-113, 113]: what a signed byte holds
+__device__ __forceinline__ int residue_p_signed(uint32_t x) {
+  return (int)(x - __umul24((__umul24(x, 36954u) + 36954u * 114u) >> 23, FP_P));
+}
+// Residues of any 32-bit value: one multiply-high; the quotient times the modulus by a 24-bit multiply,
+// of which only the low bits matter (a residue is below 2^8 / 2^15).
+__device__ __forceinline__ uint32_t mod_p(uint32_t x) { return (x - __umul24(x / FP_P, FP_P)) & 0xffu; }
+__device__ __forceinline__ uint32_t mod_q(uint32_t x) { return (x - __umul24(x / FP_Q, FP_Q)) & 0xffu; }
+__device__ __forceinline__ uint32_t mod_pq(uint32_t x) { return x - __umul24(x / FP_PQ, FP_PQ); }
+// The ring value with residues p modulo 227 (p < 227) and q modulo 113 (any 16-bit q).  227 is 1
+// modulo 113, so p + 227 t has residue p + t there: t = q - p.
+__device__ __forceinline__ uint32_t fp_from_residues(uint32_t p, uint32_t q) {
+  return p + __umul24(residue_q(q + 2 * FP_Q - p), FP_P);
+}
+// four of them as bytes
+__device__ __forceinline__ uint32_t pack_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  uint32_t const lo = __builtin_amdgcn_perm(b, a, 0x0c0c0400u), hi = __builtin_amdgcn_perm(d, c, 0x0c0c0400u);
+  return lo | (hi << 16);
+}
+__device__ __forceinline__ uint32_t residues_q4(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  return pack_bytes(residue_q(a), residue_q(b), residue_q(c), residue_q(d));
+}
+__device__ __forceinline__ uint32_t residues_p4(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  return pack_bytes(residue_p(a), residue_p(b), residue_p(c), residue_p(d));
+}
+__device__ __forceinline__ uint32_t residues_p4_signed(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  return pack_bytes((uint32_t)residue_p_signed(a), (uint32_t)residue_p_signed(b), (uint32_t)residue_p_signed(c),
+                    (uint32_t)residue_p_signed(d));
+}
 
-// Fingerprint value of a matmul output from its two residue sums (matrix-core kernels).
-// u * 25425 + v * 227 has residue u modulo 227 and v modulo 113 whatever the integers u and v
-// are (25425 = 113 * 225 = 1 mod 227, 227 = 1 mod 113), so the sums need not be reduced modulo
-// their own primes first: each is brought below 25651 and one more reduction finishes.
-// sum_p may be negative (operands recentred to [-113, 113]), |sum_p| < 2^31 - 2^17; adding
-// 83715 * 25651 makes it non-negative without changing a residue.  sum_q >= 0.
+// A sum of residue products, |x| < 2^31, modulo 227: one signed multiply-high (605457945 =
+// ceil(2^37 / 227) is exact below 2^31), the quotient times 227 by a 24-bit multiply of which the low
+// byte is right.  A negative multiple of 227 leaves 227.
+__device__ __forceinline__ uint32_t reduce_p(int x) {
+  uint32_t const r = (static_cast<uint32_t>(x) - __umul24(static_cast<uint32_t>(__mulhi(x, 605457945) >> 5), FP_P)) & 0xffu;
+  return r < r - FP_P ? r : r - FP_P;
+}
+// 0 <= x < 2^31 modulo 113 (1216273925 = ceil(2^37 / 113)); the general mod_q takes a fix-up more
+__device__ __forceinline__ uint32_t reduce_q(uint32_t x) {
+  return (x - __umul24(__umulhi(x, 1216273925u) >> 5, FP_Q)) & 0xffu;
+}
+// Fingerprint value of a matmul output from its two residue sums (matrix-core kernels): |sum_p| <
+// 2^31 (operands recentred to [-113, 113]), 0 <= sum_q < 2^31 - 226.
 __device__ __forceinline__ uint32_t fp_from_residue_sums(int sum_p, int sum_q) {
-  uint32_t const a = (static_cast<uint32_t>(sum_p) + 2147373465u) % FP_PQ;  // unsigned: wraps by definition
-  uint32_t const b = static_cast<uint32_t>(sum_q) % FP_PQ;
-  return (a * FP_Q_MUL_P_MOD_1 + b * FP_P_MUL_Q_MOD_1) % FP_PQ;
+  uint32_t const p = reduce_p(sum_p);
+  return p + __umul24(reduce_q(static_cast<uint32_t>(sum_q) + 2 * FP_Q - p), FP_P);
 }
 
 // The fingerprint lookup tables in device memory and the ring operations built on them
@@ -184,21 +219,20 @@ struct FpTables {
 };
 
 __device__ __forceinline__ uint32_t fp_exp_value(FpTables t, uint32_t x) {
-  // reference element_unary_kernel.cu:85-89
-  return (t.exp_tbl[x % FP_Q] * FP_Q_MUL_P_MOD_1) % FP_PQ;
+  // reference element_unary_kernel.cu:85-89: an exponential's residue modulo 113 is zero
+  return fp_from_residues(t.exp_tbl[residue_q(x)], 0u);
 }
 
 __device__ __forceinline__ uint32_t fp_div_value(FpTables t, uint32_t x, uint32_t y) {
   // reference element_binary_kernel.cu:155-160
-  uint32_t z = (x % FP_P) * t.div_p[y % FP_P] * FP_Q_MUL_P_MOD_1 +
-               (x % FP_Q) * t.div_q[y % FP_Q] * FP_P_MUL_Q_MOD_1;
-  return z % FP_PQ;
+  return fp_from_residues(residue_p(__umul24(residue_p(x), t.div_p[residue_p(y)])),
+                          __umul24(residue_q(x), t.div_q[residue_q(y)]));
 }
 
 __device__ __forceinline__ uint32_t fp_silu_value(FpTables t, uint32_t x) {
   // extension: x / (1 + exp(-x)) from the ring primitives above
-  uint32_t neg = (FP_PQ - x) % FP_PQ;
-  uint32_t den = (1u + fp_exp_value(t, neg)) % FP_PQ;
+  uint32_t neg = mod_pq(FP_PQ - x);
+  uint32_t den = mod_pq(1u + fp_exp_value(t, neg));
   return fp_div_value(t, x, den);
 }
 

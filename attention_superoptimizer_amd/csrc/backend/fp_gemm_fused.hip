@@ -26,8 +26,8 @@ typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void residues4(uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3,
                                           uint32_t &pp, uint32_t &qq) {
-  pp = (v0 % FP_P) | ((v1 % FP_P) << 8) | ((v2 % FP_P) << 16) | ((v3 % FP_P) << 24);
-  qq = (v0 % FP_Q) | ((v1 % FP_Q) << 8) | ((v2 % FP_Q) << 16) | ((v3 % FP_Q) << 24);
+  pp = residues_p4(v0, v1, v2, v3);
+  qq = residues_q4(v0, v1, v2, v3);
 }
 
 __device__ __forceinline__ long long origin(DevOp const &op, int it, int bx, int by, int bz) {

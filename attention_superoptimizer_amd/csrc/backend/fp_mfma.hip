@@ -46,13 +46,6 @@ constexpr int kMaxJobs = MI355_MAX_MATMULS;
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
-// residue mod 227 as a signed byte congruent to it, residue mod 113 as it is
-__device__ __forceinline__ uint32_t byte_p(uint32_t x) {
-  uint32_t const r = x % FP_P;
-  return (r > 113u ? r + 29u : r) & 0xffu;  // r - 227 = r + 29 (mod 256)
-}
-__device__ __forceinline__ uint32_t byte_q(uint32_t x) { return x % FP_Q; }
-
 struct SplitJob {
   uint16_t const *src;   // [slabs][rows][cols], row-major
   int8_t *plane_p, *plane_q;
@@ -132,10 +125,8 @@ __global__ __launch_bounds__(kThreads) void fp_split_planes_kernel(SplitMany con
       uint4v p, q;
 #pragma unroll
       for (int w = 0; w < 4; w++) {
-        p[w] = byte_p(v[4 * w]) | (byte_p(v[4 * w + 1]) << 8) | (byte_p(v[4 * w + 2]) << 16) |
-               (byte_p(v[4 * w + 3]) << 24);
-        q[w] = byte_q(v[4 * w]) | (byte_q(v[4 * w + 1]) << 8) | (byte_q(v[4 * w + 2]) << 16) |
-               (byte_q(v[4 * w + 3]) << 24);
+        p[w] = residues_p4_signed(v[4 * w], v[4 * w + 1], v[4 * w + 2], v[4 * w + 3]);
+        q[w] = residues_q4(v[4 * w], v[4 * w + 1], v[4 * w + 2], v[4 * w + 3]);
       }
       *reinterpret_cast<uint4v *>(J.plane_p + (size_t)u * 16) = p;  // u = ((strip * chunks + c) * 16 + r)
       *reinterpret_cast<uint4v *>(J.plane_q + (size_t)u * 16) = q;
@@ -180,10 +171,8 @@ __global__ __launch_bounds__(kThreads) void fp_split_planes_kernel(SplitMany con
     }
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-      tile[0][4 * ng + c][kq] = byte_p(v[0][c]) | (byte_p(v[1][c]) << 8) | (byte_p(v[2][c]) << 16) |
-                                (byte_p(v[3][c]) << 24);
-      tile[1][4 * ng + c][kq] = byte_q(v[0][c]) | (byte_q(v[1][c]) << 8) | (byte_q(v[2][c]) << 16) |
-                                (byte_q(v[3][c]) << 24);
+      tile[0][4 * ng + c][kq] = residues_p4_signed(v[0][c], v[1][c], v[2][c], v[3][c]);
+      tile[1][4 * ng + c][kq] = residues_q4(v[0][c], v[1][c], v[2][c], v[3][c]);
     }
     __syncthreads();
     if (n0 + out_n < J.rp) {  // rows past the last column hold zeros

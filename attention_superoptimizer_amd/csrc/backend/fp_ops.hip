@@ -35,11 +35,14 @@ __global__ void fp_fill_iota_kernel(uint16_t *fp, size_t n) {
 }
 
 __device__ __forceinline__ uint32_t uniform_value(uint64_t seed, size_t i) {
-  // v % 25651 for 64-bit v through 32-bit arithmetic: 2^32 = 15158 (mod 25651)
+  // v % 25651 for 64-bit v: 2^16, 2^32, 2^48 are 14234, 15158, 8411 modulo 25651, and the sum of the
+  // four 16-bit words times these stays below 2^32, so it is reduced once
+  typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
   uint64_t const v = splitmix64(seed + i);
-  uint32_t const hi = static_cast<uint32_t>(v >> 32) % FP_PQ;
-  uint32_t const lo = static_cast<uint32_t>(v) % FP_PQ;
-  return (hi * 15158u + lo) % FP_PQ;
+  uint32_t const lo = static_cast<uint32_t>(v), hi = static_cast<uint32_t>(v >> 32);
+  uint32_t s = __builtin_amdgcn_udot2(__builtin_bit_cast(ushort2v, lo), ushort2v{1, 14234}, 0u, false);
+  s = __builtin_amdgcn_udot2(__builtin_bit_cast(ushort2v, hi), ushort2v{15158, 8411}, s, false);
+  return mod_pq(s);
 }
 
 // eight values = one 16-byte store per thread and step (fp is 16-byte aligned)
@@ -81,9 +84,11 @@ __global__ void fp_fill_many_kernel(FillMany const F, int iota) {
   size_t const stride = (size_t)gridDim.x * blockDim.x * 8;
   for (; i < n; i += stride) {
     size_t const end = i + 8 <= n ? i + 8 : n;
-    uint32_t v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (size_t j = i; j < end; j++) {
-      v[j - i] = iota ? static_cast<uint32_t>(j % FP_PQ) : uniform_value(seed, j);
+    uint32_t v[8];  // (values past the end are computed and dropped: the registers keep fixed places)
+    uint32_t const first_iota = static_cast<uint32_t>(i % FP_PQ);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      v[j] = iota ? mod_pq(first_iota + j) : uniform_value(seed, i + j);
     }
     if (end == i + 8) {
       uint4v w = {v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16)};
@@ -92,8 +97,11 @@ __global__ void fp_fill_many_kernel(FillMany const F, int iota) {
       }
     } else {
       for (int t = 0; t < members; t++) {
-        for (size_t j = i; j < end; j++) {
-          F.ptr[first + t][j] = static_cast<uint16_t>(v[j - i]);
+#pragma unroll
+        for (int j = 0; j < 7; j++) {
+          if (i + j < end) {
+            F.ptr[first + t][i + j] = static_cast<uint16_t>(v[j]);
+          }
         }
       }
     }
@@ -103,8 +111,8 @@ __global__ void fp_fill_many_kernel(FillMany const F, int iota) {
 // ---- matmul (reference src/kernel/cuda/matmul_kernel.cu:145-173) ---------------
 __device__ __forceinline__ void residues4(uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3,
                                           uint32_t &pp, uint32_t &qq) {
-  pp = (v0 % FP_P) | ((v1 % FP_P) << 8) | ((v2 % FP_P) << 16) | ((v3 % FP_P) << 24);
-  qq = (v0 % FP_Q) | ((v1 % FP_Q) << 8) | ((v2 % FP_Q) << 16) | ((v3 % FP_Q) << 24);
+  pp = residues_p4(v0, v1, v2, v3);
+  qq = residues_q4(v0, v1, v2, v3);
 }
 
 // Block tile (16*RM) x 64 outputs, 32 k per step; thread (ty, tx) owns rows
@@ -218,9 +226,9 @@ __global__ __launch_bounds__(kThreads) void fp_matmul_kernel(uint16_t const *__r
     for (int j = 0; j < 4; j++) {
       int gc = col0 + tx * 4 + j;
       if (gc < n) {
-        uint32_t rp = accp[i][j] % FP_P, rq = accq[i][j] % FP_Q;
+        uint32_t rp = mod_p(accp[i][j]), rq = mod_q(accq[i][j]);
         C[(size_t)gr * n + gc] =
-            static_cast<uint16_t>((rp * FP_Q_MUL_P_MOD_1 + rq * FP_P_MUL_Q_MOD_1) % FP_PQ);
+            static_cast<uint16_t>(fp_from_residues(rp, rq));
       }
     }
   }
@@ -355,7 +363,7 @@ __global__ __launch_bounds__(kThreads) void fp_matmul64_kernel(uint16_t const *_
     uint32_t z[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      z[j] = ((accp[i][j] % FP_P) * FP_Q_MUL_P_MOD_1 + (accq[i][j] % FP_Q) * FP_P_MUL_Q_MOD_1) % FP_PQ;
+      z[j] = fp_from_residues(mod_p(accp[i][j]), mod_q(accq[i][j]));
     }
     uint2 out;
     out.x = z[0] | (z[1] << 16);
@@ -397,13 +405,104 @@ __global__ void fp_binary_kernel(int op, FpTables t, uint16_t const *__restrict_
     }
     uint32_t x = in1[i1], y = in2[i2], z;
     if (op == KN_ADD_OP) {
-      z = (x + y) % FP_PQ;
+      z = mod_pq(x + y);
     } else if (op == KN_MUL_OP) {
-      z = (x * y) % FP_PQ;
+      z = mod_pq(x * y);
     } else {
       z = fp_div_value(t, x, y);
     }
     out[gid] = static_cast<uint16_t>(z);
+  }
+}
+
+// exp, row sum and division in one pass (see f16_softmax_rows_kernel): E = exp(X), R = sum of a row of
+// E, P = E / R.  An exponential's residue modulo 113 is zero, and so is every sum or quotient of
+// exponentials: all three are fixed by their residues modulo 227, an element costs a table lookup and
+// one product, and the index arithmetic of a general broadcast goes.  [32, 256, 1024]: 77 us in three
+// launches before.  TPR threads own a row, CH chunks of eight elements each.
+typedef uint16_t ushort8v __attribute__((ext_vector_type(8)));
+typedef ushort8v ushort8_any __attribute__((aligned(2)));
+
+__device__ __forceinline__ void fp_store_chunk(uint16_t *row, ushort8v v, int c, int n, bool live) {
+  if (live && c + 8 <= n) {
+    *reinterpret_cast<ushort8_any *>(row + c) = v;
+  } else if (live) {
+#pragma unroll
+    for (int u = 0; u < 7; u++) {
+      if (c + u < n) {
+        row[c + u] = v[u];
+      }
+    }
+  }
+}
+
+template <int TPR, int CH>
+__global__ __launch_bounds__(kThreads) void fp_softmax_rows_kernel(FpTables t, uint16_t const *__restrict__ X,
+                                                                  uint16_t *__restrict__ E, uint16_t *__restrict__ R,
+                                                                  uint16_t *__restrict__ P, size_t rows, int n) {
+  __shared__ uint32_t exps[FP_Q];  // residue modulo 227 | the ring value << 16
+  __shared__ uint32_t parts[kThreads / 64];
+  if (threadIdx.x < FP_Q) {
+    uint32_t const p = t.exp_tbl[threadIdx.x];
+    exps[threadIdx.x] = p | (fp_from_residues(p, 0u) << 16);
+  }
+  size_t const row = blockIdx.x * (size_t)(kThreads / TPR) + threadIdx.x / TPR;
+  int const at_thread = threadIdx.x % TPR;
+  bool const live = row < rows;
+  size_t const at = (live ? row : rows - 1) * (size_t)n;
+  ushort8v v[CH];
+#pragma unroll
+  for (int i = 0; i < CH; i++) {
+    int const c = 8 * (i * TPR + at_thread);
+    if (c + 8 <= n) {
+      v[i] = *reinterpret_cast<ushort8_any const *>(X + at + c);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        v[i][u] = c + u < n ? X[at + c + u] : 0;
+      }
+    }
+  }
+  __syncthreads();
+  uint32_t sum = 0;
+#pragma unroll
+  for (int i = 0; i < CH; i++) {
+    int const c = 8 * (i * TPR + at_thread);
+    ushort8v e;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      uint32_t const x = exps[residue_q(v[i][u])];
+      e[u] = static_cast<uint16_t>(x >> 16);
+      v[i][u] = static_cast<uint16_t>(x & 0xffu);
+      sum += c + u < n ? x & 0xffu : 0u;
+    }
+    fp_store_chunk(E + at, e, c, n, live);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    sum += __shfl_xor(sum, off, 64);
+  }
+  if (TPR > 64) {
+    parts[threadIdx.x / 64] = sum;
+    __syncthreads();
+    sum = 0;
+#pragma unroll
+    for (int w = 0; w < TPR / 64; w++) {
+      sum += parts[w];
+    }
+  }
+  uint32_t const total = mod_p(sum), inverse = t.div_p[total];
+  if (at_thread == 0 && live) {
+    R[row] = static_cast<uint16_t>(fp_from_residues(total, 0u));
+  }
+#pragma unroll
+  for (int i = 0; i < CH; i++) {
+    ushort8v q;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      q[u] = static_cast<uint16_t>(fp_from_residues(residue_p(__umul24(v[i][u], inverse)), 0u));
+    }
+    fp_store_chunk(P + at, q, 8 * (i * TPR + at_thread), n, live);
   }
 }
 
@@ -439,7 +538,7 @@ __global__ void fp_binary_many_kernel(BinaryMany const B, FpTables t) {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
           uint32_t const x = h ? a[w] >> 16 : a[w] & 0xffffu, y = h ? b[w] >> 16 : b[w] & 0xffffu;
-          z[h] = op == KN_ADD_OP ? (x + y) % FP_PQ : (op == KN_MUL_OP ? (x * y) % FP_PQ : fp_div_value(t, x, y));
+          z[h] = op == KN_ADD_OP ? mod_pq(x + y) : (op == KN_MUL_OP ? mod_pq(x * y) : fp_div_value(t, x, y));
         }
         c[w] = z[0] | (z[1] << 16);
       }
@@ -459,9 +558,9 @@ __global__ void fp_binary_many_kernel(BinaryMany const B, FpTables t) {
     }
     uint32_t x = in1[i1], y = in2[i2], z;
     if (op == KN_ADD_OP) {
-      z = (x + y) % FP_PQ;
+      z = mod_pq(x + y);
     } else if (op == KN_MUL_OP) {
-      z = (x * y) % FP_PQ;
+      z = mod_pq(x * y);
     } else {
       z = fp_div_value(t, x, y);
     }
@@ -516,18 +615,22 @@ __global__ void fp_reduce_rows_kernel(uint16_t const *__restrict__ in, uint16_t 
 }
 
 // ---- compare (reference src/kernel/cuda/device_tensor_kernel.cu:42-49) ---------
-__global__ void set_flag_kernel(int *flag, int v) { *flag = v; }
-
-__global__ void fp_equal_kernel(uint16_t const *__restrict__ a, uint16_t const *__restrict__ b,
-                                size_t n, int *flag) {
+__global__ void fp_differ_kernel(uint16_t const *__restrict__ a, uint16_t const *__restrict__ b,
+                                 size_t n, int *slot) {
   size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   size_t stride = (size_t)gridDim.x * blockDim.x;
   bool differ = false;
-  for (; i < n; i += stride) {
-    differ |= (a[i] != b[i]);
+  size_t const n8 = (((uintptr_t)a | (uintptr_t)b) & 15) == 0 ? n / 8 : 0;
+  for (size_t j = i; j < n8; j += stride) {
+    uint4v x = reinterpret_cast<uint4v const *>(a)[j];
+    uint4v y = reinterpret_cast<uint4v const *>(b)[j];
+    differ |= (x[0] != y[0]) | (x[1] != y[1]) | (x[2] != y[2]) | (x[3] != y[3]);
+  }
+  for (size_t j = n8 * 8 + i; j < n; j += stride) {
+    differ |= (a[j] != b[j]);
   }
   if (differ) {
-    *flag = 0;  // every writer stores the same value
+    *slot = 1;  // every writer stores the same value
   }
 }
 
@@ -802,20 +905,61 @@ extern "C" int mi355_fp_reduce(uint16_t const *in, uint16_t *out, size_t n_out, 
   return MI355_OK;
 }
 
+extern "C" int mi355_fp_softmax_rows(uint16_t const *X, uint16_t *E, uint16_t *R, uint16_t *P, size_t rows, int n) {
+  MI355_REQUIRE_INIT();
+  if (n <= 0) {
+    return fail(MI355_ERR_INVALID, "row length %d", n);
+  }
+  if (rows == 0) {
+    return MI355_OK;
+  }
+  // a wavefront per row while that fills the chip and its registers hold the row, else four; longer
+  // rows one operator after the other
+  bool const wave = rows >= 1024 && n <= 4096;
+  int const chunks = (n + 7) / 8, per_thread = (chunks + (wave ? 63 : 255)) / (wave ? 64 : 256);
+  size_t const blocks = wave ? (rows + 3) / 4 : rows;
+  if (per_thread <= 8 && blocks <= 2147483647u) {
+    auto *fn = wave ? (per_thread <= 1   ? fp_softmax_rows_kernel<64, 1>
+                       : per_thread <= 2 ? fp_softmax_rows_kernel<64, 2>
+                       : per_thread <= 4 ? fp_softmax_rows_kernel<64, 4>
+                                         : fp_softmax_rows_kernel<64, 8>)
+                    : (per_thread <= 1   ? fp_softmax_rows_kernel<256, 1>
+                       : per_thread <= 2 ? fp_softmax_rows_kernel<256, 2>
+                                         : fp_softmax_rows_kernel<256, 8>);
+    MI355_HIP(launch_kernel(fn, (unsigned)blocks, kThreads, 0, state().stream(), tables(), X, E, R, P, rows, n));
+    return MI355_OK;
+  }
+  if (rows > 2147483647u) {
+    return fail(MI355_ERR_UNSUPPORTED, "too many rows");
+  }
+  int const full[2] = {(int)rows, n}, one[2] = {(int)rows, 1};
+  if (int rc = mi355_fp_unary(KN_EXP_OP, X, E, rows * (size_t)n)) {
+    return rc;
+  }
+  if (int rc = mi355_fp_reduce(E, R, rows, n, n, 1)) {
+    return rc;
+  }
+  return mi355_fp_binary(KN_DIV_OP, E, full, R, one, P, full, 2);
+}
+
 extern "C" int mi355_fp_equal(uint16_t const *a, uint16_t const *b, size_t n, int *equal) {
   MI355_REQUIRE_INIT();
   State &s = state();
-  if (int rc = sync_all_queues()) {  // the operands may come from any queue
-    return rc;
+  // The operands may come from any queue: the others are waited for, this one is in order.  A
+  // mismatch is written straight to pinned host memory, so the answer needs no copy.
+  for (int q = 0; q < MI355_NUM_QUEUES; q++) {
+    if (q != tls_queue && s.queues[q] != nullptr) {
+      MI355_HIP(hipStreamSynchronize(s.queues[q]));
+    }
   }
-  set_flag_kernel<<<1, 1, 0, s.stream()>>>(s.queue_flag(), 1);
+  int volatile *flag = s.queue_flag_host();
+  *flag = 0;
   if (n > 0) {
-    fp_equal_kernel<<<grid_for(n, kThreads, 2048), kThreads, 0, s.stream()>>>(a, b, n, s.queue_flag());
+    MI355_HIP(launch_kernel(fp_differ_kernel, grid_for((n + 7) / 8, kThreads, 1024), kThreads, 0, s.stream(), a, b, n,
+                            s.queue_flag()));
   }
-  MI355_HIP(hipGetLastError());
-  MI355_HIP(hipMemcpyAsync(s.queue_flag_host(), s.queue_flag(), sizeof(int), hipMemcpyDeviceToHost, s.stream()));
   MI355_HIP(hipStreamSynchronize(s.stream()));
-  *equal = *s.queue_flag_host();
+  *equal = *flag == 0 ? 1 : 0;
   return MI355_OK;
 }
 
@@ -824,25 +968,6 @@ extern "C" int mi355_fp_equal(uint16_t const *a, uint16_t const *b, size_t n, in
 // kernels write directly (a store only where a mismatch is found), so resetting and reading
 // them needs no launch and no copy; the caller reads a range once it has waited for the
 // compares that target it.
-
-__global__ void fp_differ_kernel(uint16_t const *__restrict__ a, uint16_t const *__restrict__ b,
-                                 size_t n, int *slot) {
-  size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  size_t stride = (size_t)gridDim.x * blockDim.x;
-  bool differ = false;
-  size_t const n8 = (((uintptr_t)a | (uintptr_t)b) & 15) == 0 ? n / 8 : 0;
-  for (size_t j = i; j < n8; j += stride) {
-    uint4v x = reinterpret_cast<uint4v const *>(a)[j];
-    uint4v y = reinterpret_cast<uint4v const *>(b)[j];
-    differ |= (x[0] != y[0]) | (x[1] != y[1]) | (x[2] != y[2]) | (x[3] != y[3]);
-  }
-  for (size_t j = n8 * 8 + i; j < n; j += stride) {
-    differ |= (a[j] != b[j]);
-  }
-  if (differ) {
-    *slot = 1;  // every writer stores the same value
-  }
-}
 
 struct DifferMany {
   uint16_t const *a[MI355_MAX_COMPARE_PAIRS];

@@ -129,8 +129,8 @@ extern "C" int mi355_init(size_t arena_bytes, void **arena_base) {
   MI355_HIP(hipMemcpy(s.exp_tbl, exp_h, sizeof(exp_h), hipMemcpyHostToDevice));
   MI355_HIP(hipMemcpy(s.div_p, divp_h, sizeof(divp_h), hipMemcpyHostToDevice));
   MI355_HIP(hipMemcpy(s.div_q, divq_h, sizeof(divq_h), hipMemcpyHostToDevice));
-  MI355_HIP(hipMalloc(reinterpret_cast<void **>(&s.flag), 256));
   MI355_HIP(hipHostMalloc(reinterpret_cast<void **>(&s.flag_host), 256, hipHostMallocDefault));
+  MI355_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&s.flag), s.flag_host, 0));
   MI355_HIP(hipHostMalloc(reinterpret_cast<void **>(&s.cmp_host), sizeof(int) * MI355_COMPARE_SLOTS,
                           hipHostMallocDefault));
   memset(s.cmp_host, 0, sizeof(int) * MI355_COMPARE_SLOTS);
@@ -189,7 +189,6 @@ extern "C" int mi355_shutdown(void) {
   }
   MI355_HIP(hipFree(s.arena));
   MI355_HIP(hipFree(s.exp_tbl));
-  MI355_HIP(hipFree(s.flag));
   MI355_HIP(hipHostFree(s.flag_host));
   MI355_HIP(hipHostFree(s.cmp_host));
   for (int m = 0; m < MI355_NUM_MARKS; m++) {

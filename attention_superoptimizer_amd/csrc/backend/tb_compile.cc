@@ -570,6 +570,44 @@ static int compile_plan_padded(mi355_plan const &plan, bool f16, int pad, int ma
       }
     }
     prog.lds_bytes = peak + scratch;
+    // An exponential depends on its argument modulo 113 only, and is zero there itself; products,
+    // quotients, sums and row sums of such values stay zero.  So a product that only exponentials
+    // read needs no residue modulo 227, and one with an exponential for an operand none modulo 113.
+    std::vector<char> zero_q(prog.num_tensors, 0), only_exp(prog.num_tensors, 1), changed(prog.num_tensors, 0);
+    for (int o = 0; o < prog.num_ops; o++) {
+      DevOp const &d = prog.ops[o];
+      if (d.kind == DOP_UNARY) {  // in place: what reads the tensor before the exponential sees the argument
+        if (d.sub != TB_EXP_OP || changed[d.dst]) {
+          only_exp[d.dst] = 0;
+        }
+        changed[d.dst] = 1;
+        zero_q[d.dst] = d.sub == TB_EXP_OP;
+        continue;
+      }
+      for (int src : {d.src0, d.src1}) {
+        if (d.kind != DOP_LOAD && src >= 0 && !changed[src]) {
+          only_exp[src] = 0;
+        }
+      }
+      if (d.kind == DOP_MATMUL || (d.kind == DOP_BINARY && d.sub == TB_MUL_OP)) {
+        zero_q[d.dst] = zero_q[d.src0] || zero_q[d.src1];
+      } else if (d.kind == DOP_BINARY) {
+        zero_q[d.dst] = zero_q[d.src0] && (d.sub == TB_DIV_OP || zero_q[d.src1]);
+      } else if (d.kind == DOP_REDUCE) {
+        zero_q[d.dst] = zero_q[d.src0];
+      } else if (d.kind == DOP_CONCAT) {
+        zero_q[d.dst] = zero_q[d.src0] && zero_q[d.src1];
+      }
+      if (d.kind == DOP_MATMUL) {
+        prog.ops[o].mm_fields = zero_q[d.dst] ? 1 : 3;
+      }
+    }
+    for (int o = 0; o < prog.num_ops; o++) {
+      DevOp &d = prog.ops[o];
+      if (d.kind == DOP_MATMUL && only_exp[d.dst] && changed[d.dst]) {
+        d.mm_fields &= 2;
+      }
+    }
   }
   for (int i = 0; i < prog.num_tensors; i++) {
     prog.t[i].mcols = fast_div_magic(prog.t[i].cols);

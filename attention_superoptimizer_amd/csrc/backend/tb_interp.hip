@@ -64,16 +64,15 @@ __device__ __forceinline__ TileOrigin tile_origin(DevOp const &op, int it, int b
 // LDS table block: [0,113) exp premultiplied by the CRT lift, [128,355) div_p,
 // [384,497) div_q
 __device__ __forceinline__ uint32_t lds_exp(uint16_t const *tbl, uint32_t x) {
-  return tbl[x % FP_Q];
+  return tbl[residue_q(x)];
 }
 __device__ __forceinline__ uint32_t lds_div(uint16_t const *tbl, uint32_t x, uint32_t y) {
-  uint32_t z = (x % FP_P) * tbl[128 + y % FP_P] * FP_Q_MUL_P_MOD_1 +
-               (x % FP_Q) * tbl[384 + y % FP_Q] * FP_P_MUL_Q_MOD_1;
-  return z % FP_PQ;
+  return fp_from_residues(residue_p(__umul24(residue_p(x), tbl[128 + residue_p(y)])),
+                          __umul24(residue_q(x), tbl[384 + residue_q(y)]));
 }
 __device__ __forceinline__ uint32_t lds_silu(uint16_t const *tbl, uint32_t x) {
-  uint32_t neg = (FP_PQ - x) % FP_PQ;
-  uint32_t den = (1u + lds_exp(tbl, neg)) % FP_PQ;
+  uint32_t neg = mod_pq(FP_PQ - x);
+  uint32_t den = mod_pq(1u + lds_exp(tbl, neg));
   return lds_div(tbl, x, den);
 }
 
@@ -91,11 +90,6 @@ __device__ __forceinline__ int fdiv(int e, uint32_t magic) {
 // 25651 is fixed by its two residues, so the value equals the reference's
 // `(r + a*b) % 25651` chain (matmul.h:773-804) bit for bit.  m, n, k, kc multiples of 4.
 // scratch: Ap[2][kc/4][m + 4] then Bp[2][kc/4][n] dwords; thread tiles are 4 x 4.
-__device__ __forceinline__ uint32_t pack_residues(uint32_t v0, uint32_t v1, uint32_t v2,
-                                                  uint32_t v3, uint32_t mod) {
-  return (v0 % mod) | ((v1 % mod) << 8) | ((v2 % mod) << 16) | ((v3 % mod) << 24);
-}
-
 __device__ void fp_matmul_packed(uint16_t const *A, uint16_t const *B, uint16_t *C, int m, int n,
                                  int k, DevOp const &op, uint32_t *scratch, int tid) {
   int const kc = op.mm_kc, kq = kc / 4, lda = m + 4;
@@ -109,8 +103,8 @@ __device__ void fp_matmul_packed(uint16_t const *A, uint16_t const *B, uint16_t 
       int const row = fdiv(e, op.mg0), q = e - row * kq;
       uint2 v = *reinterpret_cast<uint2 const *>(A + row * k + k0 + 4 * q);
       uint32_t v0 = v.x & 0xffffu, v1 = v.x >> 16, v2 = v.y & 0xffffu, v3 = v.y >> 16;
-      Ap[q * lda + row] = pack_residues(v0, v1, v2, v3, FP_P);
-      Ap[(kq + q) * lda + row] = pack_residues(v0, v1, v2, v3, FP_Q);
+      Ap[q * lda + row] = residues_p4(v0, v1, v2, v3);
+      Ap[(kq + q) * lda + row] = residues_q4(v0, v1, v2, v3);
     }
     for (int e = tid; e < kq * n2; e += kInterpThreads) {
       int const q = fdiv(e, op.mg1), c2 = (e - q * n2) * 2;
@@ -120,10 +114,10 @@ __device__ void fp_matmul_packed(uint16_t const *A, uint16_t const *B, uint16_t 
       uint32_t w2 = *reinterpret_cast<uint32_t const *>(bp + 2 * n);
       uint32_t w3 = *reinterpret_cast<uint32_t const *>(bp + 3 * n);
       uint2 pp, qq;
-      pp.x = pack_residues(w0 & 0xffffu, w1 & 0xffffu, w2 & 0xffffu, w3 & 0xffffu, FP_P);
-      pp.y = pack_residues(w0 >> 16, w1 >> 16, w2 >> 16, w3 >> 16, FP_P);
-      qq.x = pack_residues(w0 & 0xffffu, w1 & 0xffffu, w2 & 0xffffu, w3 & 0xffffu, FP_Q);
-      qq.y = pack_residues(w0 >> 16, w1 >> 16, w2 >> 16, w3 >> 16, FP_Q);
+      pp.x = residues_p4(w0 & 0xffffu, w1 & 0xffffu, w2 & 0xffffu, w3 & 0xffffu);
+      pp.y = residues_p4(w0 >> 16, w1 >> 16, w2 >> 16, w3 >> 16);
+      qq.x = residues_q4(w0 & 0xffffu, w1 & 0xffffu, w2 & 0xffffu, w3 & 0xffffu);
+      qq.y = residues_q4(w0 >> 16, w1 >> 16, w2 >> 16, w3 >> 16);
       *reinterpret_cast<uint2 *>(Bp + q * n + c2) = pp;
       *reinterpret_cast<uint2 *>(Bp + (kq + q) * n + c2) = qq;
     }
@@ -160,15 +154,14 @@ __device__ void fp_matmul_packed(uint16_t const *A, uint16_t const *B, uint16_t 
         uint32_t z[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-          z[j] = ((accp[i][j] % FP_P) * FP_Q_MUL_P_MOD_1 + (accq[i][j] % FP_Q) * FP_P_MUL_Q_MOD_1) %
-                 FP_PQ;
+          z[j] = fp_from_residues(mod_p(accp[i][j]), mod_q(accq[i][j]));
         }
         if (k0 > 0) {
           uint2 old = *reinterpret_cast<uint2 const *>(cp);
-          z[0] = (z[0] + (old.x & 0xffffu)) % FP_PQ;
-          z[1] = (z[1] + (old.x >> 16)) % FP_PQ;
-          z[2] = (z[2] + (old.y & 0xffffu)) % FP_PQ;
-          z[3] = (z[3] + (old.y >> 16)) % FP_PQ;
+          z[0] = mod_pq(z[0] + (old.x & 0xffffu));
+          z[1] = mod_pq(z[1] + (old.x >> 16));
+          z[2] = mod_pq(z[2] + (old.y & 0xffffu));
+          z[3] = mod_pq(z[3] + (old.y >> 16));
         }
         uint2 out;
         out.x = z[0] | (z[1] << 16);
@@ -189,14 +182,6 @@ __device__ void fp_matmul_packed(uint16_t const *A, uint16_t const *B, uint16_t 
 // consecutive columns of one row of C.  One CRT recombination per output and k chunk.
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ uint32_t signed_residues_p(uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3) {
-  auto one = [](uint32_t x) {
-    uint32_t const r = x % FP_P;
-    return (r > 113u ? r + 29u : r) & 0xffu;  // r - 227 = r + 29 (mod 256)
-  };
-  return one(v0) | (one(v1) << 8) | (one(v2) << 16) | (one(v3) << 24);
-}
-
 __device__ void fp_matmul_mfma(uint16_t const *A, uint16_t const *B, uint16_t *C, int m, int n, int k,
                                DevOp const &op, unsigned char *scratch, int tid) {
   // A is packed `mb` rows at a time (op.mm_mb, a multiple of 16 that divides m; the whole
@@ -211,6 +196,9 @@ __device__ void fp_matmul_mfma(uint16_t const *A, uint16_t const *B, uint16_t *C
     return (((byte >> 4) ^ ((row >> key_shift) & key_mask)) << 4) | (byte & 15);
   };
   int const n2 = n / 2;
+  // residue fields this product needs (compile_plan): a field that nobody reads, or that is zero
+  // because an operand's is, is neither packed nor multiplied
+  bool const do_p = (uniform(op.mm_fields) & 1) != 0, do_q = (uniform(op.mm_fields) & 2) != 0;
   int const wave = tid / 64, lane = tid % 64, r = lane % 16, g = lane / 16;
   int const mt_n = (n + 31) / 32, mt = ((mb + 31) / 32) * mt_n;  // 32 x 32 pieces of a row block
   for (int k0 = 0; k0 < k; k0 += kc) {
@@ -225,13 +213,16 @@ __device__ void fp_matmul_mfma(uint16_t const *A, uint16_t const *B, uint16_t *C
       uint32_t w2 = *reinterpret_cast<uint32_t const *>(bp + 2 * n);
       uint32_t w3 = *reinterpret_cast<uint32_t const *>(bp + 3 * n);
       int const at0 = c2 * pitch + swz(c2, 4 * q), at1 = (c2 + 1) * pitch + swz(c2 + 1, 4 * q);
-      *reinterpret_cast<uint32_t *>(Bb + at0) =
-          signed_residues_p(w0 & 0xffffu, w1 & 0xffffu, w2 & 0xffffu, w3 & 0xffffu);
-      *reinterpret_cast<uint32_t *>(Bb + at1) = signed_residues_p(w0 >> 16, w1 >> 16, w2 >> 16, w3 >> 16);
-      *reinterpret_cast<uint32_t *>(Bb + n * pitch + at0) =
-          pack_residues(w0 & 0xffffu, w1 & 0xffffu, w2 & 0xffffu, w3 & 0xffffu, FP_Q);
-      *reinterpret_cast<uint32_t *>(Bb + n * pitch + at1) =
-          pack_residues(w0 >> 16, w1 >> 16, w2 >> 16, w3 >> 16, FP_Q);
+      if (do_p) {
+        *reinterpret_cast<uint32_t *>(Bb + at0) =
+            residues_p4_signed(w0 & 0xffffu, w1 & 0xffffu, w2 & 0xffffu, w3 & 0xffffu);
+        *reinterpret_cast<uint32_t *>(Bb + at1) = residues_p4_signed(w0 >> 16, w1 >> 16, w2 >> 16, w3 >> 16);
+      }
+      if (do_q) {
+        *reinterpret_cast<uint32_t *>(Bb + n * pitch + at0) =
+            residues_q4(w0 & 0xffffu, w1 & 0xffffu, w2 & 0xffffu, w3 & 0xffffu);
+        *reinterpret_cast<uint32_t *>(Bb + n * pitch + at1) = residues_q4(w0 >> 16, w1 >> 16, w2 >> 16, w3 >> 16);
+      }
     }
     for (int m0 = 0; m0 < m; m0 += mb) {
       if (m0 > 0) {
@@ -242,8 +233,12 @@ __device__ void fp_matmul_mfma(uint16_t const *A, uint16_t const *B, uint16_t *C
         uint2 v = *reinterpret_cast<uint2 const *>(A + (m0 + row) * k + k0 + 4 * q);
         uint32_t v0 = v.x & 0xffffu, v1 = v.x >> 16, v2 = v.y & 0xffffu, v3 = v.y >> 16;
         int const at = row * pitch + swz(row, 4 * q);
-        *reinterpret_cast<uint32_t *>(Ab + at) = signed_residues_p(v0, v1, v2, v3);
-        *reinterpret_cast<uint32_t *>(Ab + mb * pitch + at) = pack_residues(v0, v1, v2, v3, FP_Q);
+        if (do_p) {
+          *reinterpret_cast<uint32_t *>(Ab + at) = residues_p4_signed(v0, v1, v2, v3);
+        }
+        if (do_q) {
+          *reinterpret_cast<uint32_t *>(Ab + mb * pitch + at) = residues_q4(v0, v1, v2, v3);
+        }
       }
       __syncthreads();
       for (int t = wave; t < mt; t += kInterpThreads / 64) {
@@ -265,21 +260,24 @@ __device__ void fp_matmul_mfma(uint16_t const *A, uint16_t const *B, uint16_t *C
           acc[e / 4][(e / 2) % 2][e % 2] = v4i{0, 0, 0, 0};
         }
         for (int ks = 0; ks < kc; ks += 64) {
-          v4i ap[2], aq[2], bp[2], bq[2];
 #pragma unroll
-          for (int i = 0; i < 2; i++) {
-            int const ca = (((ks >> 4) + g) ^ a_key[i]) << 4, cb = (((ks >> 4) + g) ^ b_key[i]) << 4;
-            ap[i] = *reinterpret_cast<v4i const *>(a_at[i] + ca);
-            aq[i] = *reinterpret_cast<v4i const *>(a_at[i] + mb * pitch + ca);
-            bp[i] = *reinterpret_cast<v4i const *>(b_at[i] + cb);
-            bq[i] = *reinterpret_cast<v4i const *>(b_at[i] + n * pitch + cb);
-          }
+          for (int f = 0; f < 2; f++) {
+            if (f ? !do_q : !do_p) {
+              continue;
+            }
+            v4i a[2], b[2];
 #pragma unroll
-          for (int i = 0; i < 2; i++) {
+            for (int i = 0; i < 2; i++) {
+              int const ca = (((ks >> 4) + g) ^ a_key[i]) << 4, cb = (((ks >> 4) + g) ^ b_key[i]) << 4;
+              a[i] = *reinterpret_cast<v4i const *>(a_at[i] + f * mb * pitch + ca);
+              b[i] = *reinterpret_cast<v4i const *>(b_at[i] + f * n * pitch + cb);
+            }
 #pragma unroll
-            for (int jn = 0; jn < 2; jn++) {
-              acc[0][i][jn] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bp[jn], ap[i], acc[0][i][jn], 0, 0, 0);
-              acc[1][i][jn] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bq[jn], aq[i], acc[1][i][jn], 0, 0, 0);
+            for (int i = 0; i < 2; i++) {
+#pragma unroll
+              for (int jn = 0; jn < 2; jn++) {
+                acc[f][i][jn] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[jn], a[i], acc[f][i][jn], 0, 0, 0);
+              }
             }
           }
         }
@@ -298,10 +296,10 @@ __device__ void fp_matmul_mfma(uint16_t const *A, uint16_t const *B, uint16_t *C
             }
             if (k0 > 0) {
               uint2 old = *reinterpret_cast<uint2 const *>(cp);
-              z[0] = (z[0] + (old.x & 0xffffu)) % FP_PQ;
-              z[1] = (z[1] + (old.x >> 16)) % FP_PQ;
-              z[2] = (z[2] + (old.y & 0xffffu)) % FP_PQ;
-              z[3] = (z[3] + (old.y >> 16)) % FP_PQ;
+              z[0] = mod_pq(z[0] + (old.x & 0xffffu));
+              z[1] = mod_pq(z[1] + (old.x >> 16));
+              z[2] = mod_pq(z[2] + (old.y & 0xffffu));
+              z[3] = mod_pq(z[3] + (old.y >> 16));
             }
             uint2 out;
             out.x = z[0] | (z[1] << 16);
@@ -316,8 +314,8 @@ __device__ void fp_matmul_mfma(uint16_t const *A, uint16_t const *B, uint16_t *C
 
 __device__ __forceinline__ uint32_t add_mod_pair(uint32_t a, uint32_t b) {
   // two uint16 lanes: (a + b) mod 25651 in each
-  uint32_t lo = ((a & 0xffffu) + (b & 0xffffu)) % FP_PQ;
-  uint32_t hi = ((a >> 16) + (b >> 16)) % FP_PQ;
+  uint32_t lo = mod_pq((a & 0xffffu) + (b & 0xffffu));
+  uint32_t hi = mod_pq((a >> 16) + (b >> 16));
   return lo | (hi << 16);
 }
 
@@ -406,14 +404,19 @@ __device__ __forceinline__ void fp_interp_block(DevProgram const &P, unsigned ch
           DevTensor const &t = P.t[op.dst];
           uint16_t *p = reinterpret_cast<uint16_t *>(lds + t.off);
           int const n = t.rows * t.cols;
-          if (op.sub == TB_EXP_OP) {
-            for (int e = tid; e < n; e += kInterpThreads) {
-              p[e] = static_cast<uint16_t>(lds_exp(tbl, p[e]));
+          // (16 bytes at a time; every tile starts on a 16-byte boundary)
+          bool const exp = uniform(op.sub) == TB_EXP_OP;
+          for (int e = tid; e < n / 8; e += kInterpThreads) {
+            uint4v w = reinterpret_cast<uint4v const *>(p)[e];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+              uint32_t const lo = w[j] & 0xffffu, hi = w[j] >> 16;
+              w[j] = exp ? lds_exp(tbl, lo) | (lds_exp(tbl, hi) << 16) : lds_silu(tbl, lo) | (lds_silu(tbl, hi) << 16);
             }
-          } else {
-            for (int e = tid; e < n; e += kInterpThreads) {
-              p[e] = static_cast<uint16_t>(lds_silu(tbl, p[e]));
-            }
+            reinterpret_cast<uint4v *>(p)[e] = w;
+          }
+          for (int e = n / 8 * 8 + tid; e < n; e += kInterpThreads) {
+            p[e] = static_cast<uint16_t>(exp ? lds_exp(tbl, p[e]) : lds_silu(tbl, p[e]));
           }
           break;
         }
@@ -427,6 +430,33 @@ __device__ __forceinline__ void fp_interp_block(DevProgram const &P, unsigned ch
           int const n = to.rows * to.cols;
           int const r1 = t1.rows == to.rows ? t1.cols : 0, c1 = t1.cols == to.cols ? 1 : 0;
           int const r2 = t2.rows == to.rows ? t2.cols : 0, c2 = t2.cols == to.cols ? 1 : 0;
+          int const cols = uniform(to.cols);
+          if (cols % 8 == 0) {
+            // eight neighbours of a row at a time: an operand that has the row holds them in 16 bytes,
+            // one that has a single column is the same for all
+            int const cpr = cols / 8;
+            auto eight = [&](uint16_t const *x, int at, int step) {
+              if (step) {
+                return *reinterpret_cast<uint4v const *>(x + at);
+              }
+              uint32_t const y = x[at] * 0x10001u;
+              return uint4v{y, y, y, y};
+            };
+            for (int e = tid; e < n / 8; e += kInterpThreads) {
+              int const r = fdiv(e, to.mcpr), c = (e - r * cpr) * 8;
+              uint4v const a = eight(x1, r * r1 + c * c1, c1), b = eight(x2, r * r2 + c * c2, c2);
+              uint4v z;
+#pragma unroll
+              for (int j = 0; j < 4; j++) {
+                uint32_t const al = a[j] & 0xffffu, ah = a[j] >> 16, bl = b[j] & 0xffffu, bh = b[j] >> 16;
+                z[j] = op.sub == TB_DIV_OP   ? lds_div(tbl, al, bl) | (lds_div(tbl, ah, bh) << 16)
+                       : op.sub == TB_ADD_OP ? mod_pq(al + bl) | (mod_pq(ah + bh) << 16)
+                                             : mod_pq(al * bl) | (mod_pq(ah * bh) << 16);
+              }
+              *reinterpret_cast<uint4v *>(y + e * 8) = z;
+            }
+            break;
+          }
           for (int e = tid; e < n; e += kInterpThreads) {
             int const r = fdiv(e, to.mcols), c = e - r * to.cols;
             uint32_t a = x1[r * r1 + c * c1];
@@ -435,9 +465,9 @@ __device__ __forceinline__ void fp_interp_block(DevProgram const &P, unsigned ch
             if (op.sub == TB_DIV_OP) {
               z = lds_div(tbl, a, b);
             } else if (op.sub == TB_ADD_OP) {
-              z = (a + b) % FP_PQ;
+              z = mod_pq(a + b);
             } else {
-              z = (a * b) % FP_PQ;
+              z = mod_pq(a * b);
             }
             y[e] = static_cast<uint16_t>(z);
           }
@@ -455,9 +485,19 @@ __device__ __forceinline__ void fp_interp_block(DevProgram const &P, unsigned ch
             int const lane16 = tid & 15;
             for (int e = tid >> 4; e < n; e += kInterpThreads / 16) {
               uint16_t const *row = x + e * deg;
-              uint32_t r = 0;
-              for (int kk = lane16; kk < deg; kk += 16) {
-                r += row[kk];  // an LDS tile is far too small to overflow 32 bits here
+              uint32_t r = 0;  // (an LDS tile is far too small to overflow 32 bits here)
+              if (deg % 8 == 0) {
+                for (int kk = lane16; kk < deg / 8; kk += 16) {
+                  uint4v const w = reinterpret_cast<uint4v const *>(row)[kk];
+#pragma unroll
+                  for (int j = 0; j < 4; j++) {
+                    r += (w[j] & 0xffffu) + (w[j] >> 16);
+                  }
+                }
+              } else {
+                for (int kk = lane16; kk < deg; kk += 16) {
+                  r += row[kk];
+                }
               }
               r %= FP_PQ;
               r += __shfl_xor(r, 8, 16);
@@ -534,7 +574,7 @@ __device__ __forceinline__ void fp_interp_block(DevProgram const &P, unsigned ch
             for (int e = tid; e < n; e += kInterpThreads) {
               uint32_t v = x[e];
               if (!first) {
-                v = (v + acc[e]) % FP_PQ;
+                v = mod_pq(v + acc[e]);
               }
               if (last) {
                 int const r = fdiv(e, ta.mcols), c = e - r * ta_cols;
@@ -561,7 +601,7 @@ __device__ __forceinline__ void fp_load_tables(unsigned char *lds, uint16_t cons
   uint16_t *tbl = reinterpret_cast<uint16_t *>(lds);
   int const tid = threadIdx.x;
   for (int i = tid; i < (int)FP_Q; i += kInterpThreads) {
-    tbl[i] = static_cast<uint16_t>((g_exp[i] * FP_Q_MUL_P_MOD_1) % FP_PQ);
+    tbl[i] = static_cast<uint16_t>(fp_from_residues(g_exp[i], 0u));
     tbl[384 + i] = g_divq[i];
   }
   for (int i = tid; i < (int)FP_P; i += kInterpThreads) {
@@ -1168,7 +1208,7 @@ static void choose_splits(DevProgram &prog, PlanExtents const &ext, int num_outp
   prog.splits = 1;
   int const blocks = (int)fp_program_blocks(prog);
   int const F = prog.forloop_range;
-  if (F < 2 || blocks >= 192) {
+  if (F < 2 || blocks >= 192 || prog.fused == 5) {
     return;
   }
   size_t used = 0;
@@ -1202,10 +1242,33 @@ static int prepare(mi355_plan const *plan, void const *const *inputs, void *cons
     try_fused_fp = t == TB_MATMUL_OP || t == TB_EXP_OP || t == TB_SILU_OP;
   }
   try_fused_fp = try_fused_fp && matmuls == 1;
-  int rc = compile_plan(*plan, f16, (try_fused || try_fused_fp) ? (1 << 30) : state().max_lds, prog, ext,
+  // (three loaders, two matmuls, one exponential)
+  int kinds[3] = {0, 0, 0};
+  for (int o = 0; o < plan->num_operators; o++) {
+    int const t = plan->operator_types[o];
+    kinds[0] += t == TB_INPUT_OP ? 1 : 0;
+    kinds[1] += t == TB_MATMUL_OP ? 1 : 0;
+    kinds[2] += t == TB_EXP_OP ? 1 : 0;
+  }
+  bool const try_fp_attention = !f16 && !state().force_interpreter && state().fp_vector_dot_only == 0 && kinds[0] == 3 && kinds[1] == 2 && kinds[2] == 1;
+  int rc = compile_plan(*plan, f16, (try_fused || try_fused_fp || try_fp_attention) ? (1 << 30) : state().max_lds, prog, ext,
                         err, declared);
   if (rc != MI355_OK) {
     return fail(rc, "%s", err.c_str());
+  }
+  if (try_fp_attention) {
+    for (int i = 0; i < plan->num_dmem_inputs; i++) {
+      prog.in[i] = inputs[i];
+    }
+    for (int i = 0; i < plan->num_dmem_outputs; i++) {
+      prog.out[i] = outputs[i];
+    }
+    if (!fp_attn_applicable(prog)) {
+      rc = compile_plan(*plan, false, state().max_lds, prog, ext, err);
+      if (rc != MI355_OK) {
+        return fail(rc, "%s", err.c_str());
+      }
+    }
   }
   if (try_fused_fp) {
     // the fused fingerprint matmul keeps no tile in LDS either: same two-step lowering
@@ -1325,6 +1388,17 @@ static int launch(DevProgram const &prog, bool f16) {
     s.last().threads = kInterpThreads;
     s.last().lds_bytes = prog.lds_bytes;
     s.last().row_split = prog.splits;
+    return MI355_OK;
+  }
+  if (!f16 && prog.fused == 5) {
+    if (int rc = launch_fp_attn(prog, s.stream())) {
+      return rc;
+    }
+    s.last().kernel_id = MI355_KERNEL_FP_ATTENTION;
+    s.last().workgroups = (int)fp_program_blocks(prog);
+    s.last().threads = kInterpThreads;
+    s.last().lds_bytes = prog.lds_bytes;
+    s.last().row_split = 1;
     return MI355_OK;
   }
   if (prog.fused != 0) {
@@ -1616,20 +1690,22 @@ static int launch_fp_chunk(std::vector<DevProgram> &progs, std::vector<PlanExten
   int const scale = (int)std::min<long long>(64, (1024 + total - 1) / total);
   size_t used = 0;
   for (int i = 0; i < n; i++) {
-    set_splits(progs[i], exts[i], num_outputs[i], std::min(progs[i].forloop_range, scale), used);
+    if (progs[i].fused != 5) {
+      set_splits(progs[i], exts[i], num_outputs[i], std::min(progs[i].forloop_range, scale), used);
+    }
   }
   int const record = (int)sizeof(DevProgram);
   // Launch classes.  Interpreter programs by LDS need (a launch requests the largest need of
   // its members, which bounds how many workgroups share a compute unit); fused matmul
   // programs by register tiles per thread (a template argument of their kernel), those on
-  // the matrix cores in a class of their own.
-  constexpr int kClasses = 7;
+  // the matrix cores in a class of their own, and the attention family in another.
+  constexpr int kClasses = 8;
   int const bounds[3] = {24 * 1024, 64 * 1024, s.max_lds - record - 16};
   // (with fewer than three interpreter workgroups per compute unit in the whole chunk nobody's
   // occupancy is at stake, and one launch is a third of the latency of three in a row)
   long long interp_blocks = 0;
   for (DevProgram const &p : progs) {
-    if (p.fused != 4 && p.lds_bytes <= bounds[2]) {
+    if (p.fused == 0 && p.lds_bytes <= bounds[2]) {
       interp_blocks += (long long)p.grid[0] * p.splits * p.grid[1] * p.grid[2];
     }
   }
@@ -1637,6 +1713,9 @@ static int launch_fp_chunk(std::vector<DevProgram> &progs, std::vector<PlanExten
   auto class_of = [&](DevProgram const &p) {
     if (p.fused == 4) {
       return p.fg[5] ? 6 : (p.fg[3] == 1 ? 3 : (p.fg[3] == 2 ? 4 : 5));
+    }
+    if (p.fused == 5) {
+      return 7;
     }
     for (int c = 0; c < 3; c++) {
       if (p.lds_bytes <= bounds[c]) {
@@ -1732,6 +1811,14 @@ static int launch_fp_chunk(std::vector<DevProgram> &progs, std::vector<PlanExten
       int lds = 0;
       for (int k = class_begin[c]; k < class_begin[c + 1]; k++) {
         lds = std::max(lds, progs[order[k]].lds_bytes);
+      }
+      if (c == 7) {
+        int const blocks = hf[first_off[c] + first_cnt[c]];
+        if (int rc = launch_fp_attn_multi(dp + class_begin[c], df + first_off[c], first_cnt[c], blocks, lds, s.stream())) {
+          return rc;
+        }
+        launched += blocks;
+        continue;
       }
       if (c == 6) {
         int const blocks = hf[first_off[c] + first_cnt[c]];

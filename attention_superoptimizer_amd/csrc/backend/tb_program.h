@@ -59,6 +59,7 @@ struct DevOp {
   int cat_a, cat_b, cat_inner;               // CONCAT
   int mm_kc;  // MATMUL, uint16 interpreter: k chunk of the packed-residue path, 0 = scalar path
   int mm_mb;  // MATMUL, matrix-core variant (sub == 1): rows of A packed at a time
+  int mm_fields;  // MATMUL, uint16: residues worth computing, bit 0 modulo 227, bit 1 modulo 113
   // division magics.  MATMUL: kc / 4, n / 2, n / 4.  REDUCE: inner.  CONCAT: inner, a + b.
   // LOAD of a column-major tensor: the tile's rows, rows / 8.
   uint32_t mg0, mg1, mg2;
@@ -69,7 +70,7 @@ struct alignas(16) DevProgram {
   int forloop_range;
   int lds_bytes;  // dynamic LDS the interpreter requests (tables included)
   int fused;      // fp16: 1 / 2 / 3 = run by the fused attention / GEMM / combine kernel; uint16:
-                  // 4 = run by the fused fingerprint matmul kernel; 0 = the interpreter
+                  // 4 / 5 = run by the fused fingerprint matmul / attention kernel; 0 = the interpreter
   int fg[6];      // fused fingerprint matmul: loader of A, loader of B, k chunk, register tiles per
                   // thread, thread groups sharing a tile's k range (small tiles), 1 = matrix-core
                   // route (the operand tensors are read from residue planes, see pl / pl_geo)
@@ -149,12 +150,19 @@ int fp_mfma_split_programs(DevProgram const *const *progs, int n, hipStream_t st
 int launch_fp_mfma_gemm(DevProgram const &P, hipStream_t stream);
 int launch_fp_mfma_gemm_multi(DevProgram const *progs, int const *first_block, int n, int blocks,
                               hipStream_t stream);
+// Attention family of the same (fp_attn.hip): recognise (marks the program), launch one, launch many.
+bool fp_attn_applicable(DevProgram &P);
+int launch_fp_attn(DevProgram const &P, hipStream_t stream);
+int launch_fp_attn_multi(DevProgram const *progs, int const *first_block, int n, int blocks, int lds_bytes, hipStream_t stream);
 constexpr int kFpMfmaLdsBytes = 32768;  // wavefront sums of a tile whose k range is shared
 inline bool fp_needs_matrix_cores(DevProgram const &p) {
   return (p.fp_unary[0] | p.fp_unary[1] | p.fp_unary[2]) != 0;
 }
 // Workgroups a fused matmul program is launched with (grouped blocks count once).
 inline long long fp_program_blocks(DevProgram const &p) {
+  if (p.fused == 5) {
+    return (long long)p.grid[0] * p.grid[1] * p.grid[2] * p.pl_geo[0];
+  }
   long long const gx = p.fused == 4 && p.fg[5] ? p.pl_group[0] : 1, gy = p.fused == 4 && p.fg[5] ? p.pl_group[1] : 1;
   return (long long)(p.grid[0] / gx) * p.splits * (p.grid[1] / gy) * p.grid[2];
 }

@@ -645,17 +645,30 @@ static bool run_matmul_then(KNOperator const *mm, KNOperator const *next) {
   return true;
 }
 
-// exp, the sum of its rows and their division
+// exp, the sum of its rows and their division, as operators (every storage order: fingerprints are
+// row-major whatever the layout)
 static bool is_softmax_rows(KNOperator const *e, KNOperator const *r, KNOperator const *d) {
   if (e->op_type != KN_EXP_OP || d->op_type != KN_DIV_OP ||
       (r->op_type != KN_REDUCTION_0_OP && r->op_type != KN_REDUCTION_1_OP && r->op_type != KN_REDUCTION_2_OP)) {
     return false;
   }
-  DTensor const &X = e->input_tensors[0], &E = e->output_tensors[0], &R = r->output_tensors[0], &P = d->output_tensors[0];
+  DTensor const &E = e->output_tensors[0], &R = r->output_tensors[0], &P = d->output_tensors[0];
   int const last = E.num_dims - 1;
   return r->input_tensors[0].guid == E.guid && static_cast<KNReductionOp const *>(r)->reduction_dim_idx == last &&
-         R.dim[last] == 1 && d->input_tensors[0].guid == E.guid && d->input_tensors[1].guid == R.guid && same_shape(E, P) &&
-         !column_major(X) && !column_major(E) && !column_major(R) && !column_major(P);
+         R.dim[last] == 1 && d->input_tensors[0].guid == E.guid && d->input_tensors[1].guid == R.guid && same_shape(E, P);
+}
+
+// Operators i, i + 1, i + 2 of a graph as one fingerprint launch.
+bool fingerprint_softmax_rows(std::vector<KNOperator *> const &ops, size_t i) {
+  if (i + 2 >= ops.size() || !is_softmax_rows(ops[i], ops[i + 1], ops[i + 2])) {
+    return false;
+  }
+  require_device("fingerprint_softmax_rows");
+  DTensor const &E = ops[i]->output_tensors[0];
+  size_t const n = (size_t)E.dim[E.num_dims - 1];
+  MI355_CALL(mi355_fp_softmax_rows(ops[i]->input_tensors[0].fp_ptr, E.fp_ptr, ops[i + 1]->output_tensors[0].fp_ptr,
+                                   ops[i + 2]->output_tensors[0].fp_ptr, E.num_elements() / n, (int)n));
+  return true;
 }
 
 static void run_softmax_rows(KNOperator const *e, KNOperator const *r, KNOperator const *d) {
@@ -668,7 +681,11 @@ void execute_all(Graph const &graph) {
   require_device("execute_all");
   std::vector<KNOperator *> const &ops = graph.operators;
   size_t const n = ops.size();
-  auto softmax_at = [&](size_t i) { return i + 2 < n && is_softmax_rows(ops[i], ops[i + 1], ops[i + 2]); };
+  auto softmax_at = [&](size_t i) {
+    return i + 2 < n && is_softmax_rows(ops[i], ops[i + 1], ops[i + 2]) && !column_major(ops[i]->input_tensors[0]) &&
+           !column_major(ops[i]->output_tensors[0]) && !column_major(ops[i + 1]->output_tensors[0]) &&
+           !column_major(ops[i + 2]->output_tensors[0]);
+  };
   for (size_t i = 0; i < n;) {
     if (softmax_at(i)) {
       run_softmax_rows(ops[i], ops[i + 1], ops[i + 2]);

@@ -26,6 +26,7 @@ namespace kernel {
 // kernel_device.cc: the lowered program of a customized operator and its bound pointers
 void lower_customized(KNCustomizedOp const &op, bool fingerprint, mi355_plan *plan,
                       void const **inputs, void **outputs);
+bool fingerprint_softmax_rows(std::vector<KNOperator *> const &ops, size_t i);
 }  // namespace kernel
 
 namespace search {
@@ -122,8 +123,12 @@ void fingerprint_graph(kernel::Graph const &g, uint64_t input_seed, VerifyStats 
   fill_inputs({&g}, input_seed);
   for (KNOperator *op : g.operators) {
     account(op, stats);
-    if (op->op_type != KN_INPUT_OP) {
-      op->fingerprint();
+  }
+  for (size_t i = 0; i < g.operators.size(); i++) {
+    if (kernel::fingerprint_softmax_rows(g.operators, i)) {
+      i += 2;
+    } else if (g.operators[i]->op_type != KN_INPUT_OP) {
+      g.operators[i]->fingerprint();
     }
   }
 }
@@ -206,6 +211,10 @@ static void fingerprint_graphs(std::vector<kernel::Graph *> const &graphs, uint6
           continue;
         }
         any = true;
+        if (kernel::fingerprint_softmax_rows(ops, cursor[k] - 1)) {
+          cursor[k] += 2;
+          continue;
+        }
         if (op->op_type == KN_MATMUL_OP) {
           DTensor const &a = op->input_tensors[0], &b = op->input_tensors[1];
           int const nd = a.num_dims;

@@ -86,6 +86,7 @@ typedef struct mi355_launch_info {
 #define MI355_KERNEL_F16_GEMM 4      /* fused skinny-GEMM family (split for-loop, ordered fix-up) */
 #define MI355_KERNEL_F16_COMBINE 5   /* fused fold-partials-and-divide family */
 #define MI355_KERNEL_FP_GEMM 6       /* fused fingerprint tiled-matmul family (uint16) */
+#define MI355_KERNEL_FP_ATTENTION 7  /* fused fingerprint attention family (uint16) */
 
 /* Backend options (mi355_set_option).  FORCE_INTERPRETER = 1 sends every customized op,
  * fp16 or fingerprint, through the generic LDS interpreter instead of a fused kernel
@@ -258,6 +259,9 @@ int mi355_fp_binary_many(int const *ops, uint16_t const *const *in1, int const *
 /* compute_reduction_fingerprint, src/kernel/cuda/reduction_kernel.cu:80-133 */
 int mi355_fp_reduce(uint16_t const *in, uint16_t *out, size_t n_out, int factor,
                     int in_stride, int out_stride);
+/* E = exp(X), R[row] = sum of a row of E, P = E / R for `rows` rows of n elements: what mi355_fp_unary,
+ * mi355_fp_reduce and mi355_fp_binary one after the other leave. */
+int mi355_fp_softmax_rows(uint16_t const *X, uint16_t *E, uint16_t *R, uint16_t *P, size_t rows, int n);
 /* DTensor::has_same_fingerprint's element loop, src/kernel/cuda/device_tensor_kernel.cu:36-52,
  * done on the device; writes 1/0 to *equal (blocking: 4 bytes come back, not 2 tensors) */
 int mi355_fp_equal(uint16_t const *a, uint16_t const *b, size_t n, int *equal);
