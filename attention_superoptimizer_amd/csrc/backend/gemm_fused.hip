@@ -8,10 +8,13 @@
 //                                                                 cpp_examples/lora.cc:45-67)
 //
 // These are HBM-bound: what matters is how many bytes of weights are in flight, not
-// the MFMAs.  Two kernels.  gemm_lanes_kernel (further down) runs a plan in ONE launch with
+// the MFMAs.  Three kernels.  gemm_lanes_kernel (further down) runs a plan in ONE launch with
 // the output tile cut into 16 x 16 pieces, one workgroup each, whose wavefronts take the
-// for-loop's iterations side by side; it serves the launch-bound members.  gemm_fused_kernel
-// cuts the for-loop instead and needs a second launch to add the ranges.  Its design:
+// for-loop's iterations side by side; it serves the launch-bound members.  gemm_stream_kernel
+// (gemm_stream.h) takes the ones whose weights' bytes cost: iterations of whole 64 k.
+// gemm_fused_kernel takes the rest (iterations of 96 or 160 k, more rows than half of them);
+// like the streaming kernel it cuts the for-loop and needs a second launch to add the ranges.
+// Its design:
 //  * the plan's grid is a lower bound on parallelism.  Each logical block's for-loop
 //    is cut into `ksplit` contiguous ranges handled by different workgroups, sized so
 //    that a few workgroups sit on every compute unit; a workgroup issues every load
@@ -46,7 +49,7 @@
 #include <string>
 
 #include "gemm_tiles.h"
-#include "mi355_kernels/gemm.h"
+#include "mi355_kernels/gemm_stream.h"
 
 namespace mi355 {
 
@@ -331,13 +334,12 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // plan (measured on the LoRA plan: 202 MB of requests for 34 MB), which is what bounds a plan
   // of tens of MB; the range-splitting kernel moves whole lines once.
   // With column-major weights a piece's columns are whole lines of its own, read straight into
-  // registers, so the first cost is gone; measured on the configurations of the benchmark the one
-  // launch then also wins for the two-weight plan (gated MLP, first half, 235 MB: 45.8 against
-  // 49.0 us) but not for the others (LoRA, 34 MB: 14.0 against 12.4 us; gated MLP, second half,
-  // 117 MB: 36.2 against 24.7 us), where each wavefront's loads of its activation rows and of the
-  // lora A tile outnumber its weight loads.
+  // registers, so the first cost is gone; the one launch then also wins for a two-weight plan of up to
+  // 64 MB (16 x 2560 x 6400, 65 MB: 16.2 us against 17.1 of the streaming kernel and its fold; 235 MB:
+  // 54.6 against 48.4) but not for the others, where each wavefront's loads of its activation rows
+  // and of the lora A tile outnumber its weight loads.
   long long const weight_bytes = blocks * F * (long long)(G.nb * G.KT * 64 + (G.lora ? G.KT * 16 : 0)) * 2;
-  bool const two_weights_cm = G.wcm && G.nb == 2 && blocks * S <= 4096;
+  bool const two_weights_cm = G.wcm && G.nb == 2 && blocks * S <= 4096 && (weight_bytes <= (68LL << 20) || emit_sink() != nullptr);
   if (s.gemm_mode == 0 && !two_weights_cm && (blocks * S > 1024 || weight_bytes > (8LL << 20))) {
     return 0;
   }
@@ -386,6 +388,101 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   return rc;
 }
 
+// the fold of a split for-loop: the launch, or its source text
+int launch_combine(GemmParams const &A, int nb, dim3 blocks) {
+  if (EmitSink *sink = emit_sink()) {
+    emit_launch(*sink, "gemm_combine_kernel", emit_fmt("%d", nb), blocks, 256, 0, literal(A, "P"));
+    return 1;
+  }
+  State &s = state();
+  int const lds = A.forloop_range * 1024;
+  if (lds > s.max_lds) {
+    MI355_HIP(launch_kernel(nb == 1 ? gemm_combine_kernel<1> : gemm_combine_kernel<2>, blocks, 256, 0, s.stream(), A));
+    return 1;
+  }
+  auto *fn = nb == 1 ? gemm_fold_kernel<1> : gemm_fold_kernel<2>;
+  MI355_GRANT_LDS(fn, lds);
+  MI355_HIP(launch_kernel(fn, dim3(blocks.x * nb * ((A.M + 7) / 8), blocks.y, blocks.z), 256, lds, s.stream(), A));
+  return 1;
+}
+
+template <int NB, int PRO, bool LORA, bool WCM, int MT>
+int launch_stream_one(StreamParams const &L, dim3 grid, int lds) {
+  auto *fn = gemm_stream_kernel<NB, PRO, LORA, WCM, MT>;
+  MI355_GRANT_LDS(fn, lds);
+  MI355_HIP(launch_kernel(fn, grid, 256, lds, state().stream(), L));
+  return 1;
+}
+
+// gemm_stream_kernel for this plan (see include/mi355_kernels/gemm_stream.h), or 0.
+int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A) {
+  State &s = state();
+  int const mt = G.M <= 16 ? 1 : (G.M <= 32 ? 2 : 4), F = P.forloop_range;
+  // (with more rows than half an iteration's k the product slots rival the weights: the kernel that
+  // keeps its sums in registers where a block is not split stays ahead there)
+  if (s.any_size_kernels || !G.whole || G.KT % 64 != 0 || 2 * G.M > G.KT || emit_sink() != nullptr) {
+    return 0;  // (a printed program takes gemm_fused_kernel, which prints)
+  }
+  long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
+  int const ring = 4 * kStreamRing * stream_slot_bytes(G.pro, G.lora, mt);
+  int const results = F * G.nb * G.M * 128;
+  size_t const slab = (size_t)blocks * results;
+  // One range per block where the blocks alone occupy the chip and a wavefront has a few steps to
+  // make: no slab and no second launch (4 x 8192 x 2048 in 64-k iterations: 8.9 us against 12).
+  // Otherwise four iterations, one per wavefront, to a range, as far as that many workgroups are
+  // resident at a time: a slot of 10 KB leaves room for two on a compute unit, which then also gain
+  // from taking turns; a larger one for one, where a second round would start late (32 x 3840 x 5120:
+  // 13.8 us in 240 workgroups, 16.0 in 300).
+  int const steps = (F + 3) / 4 * (G.KT / 64) * G.nb;
+  bool const fits = ring + results <= s.max_lds;
+  int ks = 1;
+  if (!(fits && blocks >= 96 && steps <= 8) && slab <= s.scratch_bytes) {
+    long long const most = (ring <= 80 * 1024 ? 1024 : 256) / blocks;
+    ks = (int)std::max<long long>(1, std::min<long long>((F + 3) / 4, most));
+  }
+  if (ks == 1 && !fits) {
+    return 0;
+  }
+  int const per = (F + ks - 1) / ks;
+  ks = (F + per - 1) / per;  // (no empty range)
+  StreamParams L{};
+  L.g = A;
+  L.g.ksplit = ks;
+  L.g.scratch = static_cast<_Float16 *>(s.scratch());
+  L.results = ring;
+  int const lds = ring + (ks == 1 ? results : 0);
+  if ((long long)P.grid[0] * ks > 2147483647LL) {
+    return 0;
+  }
+  dim3 const grid(P.grid[0] * ks, P.grid[1], P.grid[2]);
+  int rc = 0;
+#define MI355_STREAM_CASE(NBV, PROV, LORAV, MTV)                                            \
+  if (G.nb == NBV && G.pro == PROV && G.lora == LORAV && mt == MTV) {                       \
+    rc = G.wcm ? launch_stream_one<NBV, PROV, LORAV, true, MTV>(L, grid, lds)               \
+               : launch_stream_one<NBV, PROV, LORAV, false, MTV>(L, grid, lds);             \
+  }
+  MI355_STREAM_CASE(1, PRO_NONE, false, 1)
+  MI355_STREAM_CASE(1, PRO_NONE, false, 2)
+  MI355_STREAM_CASE(1, PRO_NONE, false, 4)
+  MI355_STREAM_CASE(1, PRO_EXP, false, 1)
+  MI355_STREAM_CASE(1, PRO_SILU, false, 1)
+  MI355_STREAM_CASE(2, PRO_NONE, false, 1)
+  MI355_STREAM_CASE(1, PRO_SILU_MUL, false, 1)
+  MI355_STREAM_CASE(1, PRO_NONE, true, 1)
+#undef MI355_STREAM_CASE
+  if (rc == 1 && ks > 1) {
+    rc = launch_combine(L.g, G.nb, dim3(P.grid[0], P.grid[1], P.grid[2]));
+  }
+  if (rc == 1) {
+    s.last().kernel_id = MI355_KERNEL_F16_GEMM;
+    s.last().workgroups = grid.x * grid.y * grid.z;
+    s.last().threads = 256;
+    s.last().lds_bytes = lds;
+    s.last().row_split = ks;
+  }
+  return rc;
+}
+
 }  // namespace
 
 std::string gemm_params_literal(GemmParams const &A, char const *var) { return literal(A, var); }
@@ -420,6 +517,9 @@ int try_launch_gemm(DevProgram const &P) {
   A.KT = G.KT;
   A.forloop_range = P.forloop_range;
   if (int const rc = try_launch_lanes(P, G, A)) {
+    return rc;
+  }
+  if (int const rc = try_launch_stream(P, G, A)) {
     return rc;
   }
   if (!G.whole || s.any_size_kernels) {
@@ -481,12 +581,8 @@ int try_launch_gemm(DevProgram const &P) {
   MI355_GEMM_CASE(1, 1, PRO_SILU_MUL, false)
   MI355_GEMM_CASE(1, 1, PRO_NONE, true)
 #undef MI355_GEMM_CASE
-  if (rc == 1 && ksplit > 1 && sink) {
-    emit_launch(*sink, "gemm_combine_kernel", emit_fmt("%d", G.nb), dim3(P.grid[0], P.grid[1], P.grid[2]), 256, 0,
-                literal(A, "P"));
-  } else if (rc == 1 && ksplit > 1) {
-    dim3 cgrid(P.grid[0], P.grid[1], P.grid[2]);
-    MI355_HIP(launch_kernel(G.nb == 1 ? gemm_combine_kernel<1> : gemm_combine_kernel<2>, cgrid, 256, 0, s.stream(), A));
+  if (rc == 1 && ksplit > 1) {
+    rc = launch_combine(A, G.nb, dim3(P.grid[0], P.grid[1], P.grid[2]));
   }
   if (rc == 1) {
     s.last().kernel_id = MI355_KERNEL_F16_GEMM;

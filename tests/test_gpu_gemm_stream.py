@@ -1,0 +1,42 @@
+"""The streaming skinny-GEMM kernel against the fp16 oracle: rows around the edges of a 16-row group,
+for-loops of one range and of many (ranges that do not divide by the wavefronts), every member of the
+family, both storage orders.  (Option 7 = 1 keeps small plans off the one-launch kernel.)"""
+import pytest
+
+from test_gpu_gemm_tiles import COL, ROW, _run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def ranges(abi):
+    assert abi.mi355_set_option(7, 1) == 0
+    yield
+    assert abi.mi355_set_option(7, 0) == 0
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("m,blocks,kt,loop", [
+    (1, 100, 64, 7), (16, 3, 64, 1), (17, 5, 64, 9), (15, 2, 512, 6), (33, 4, 128, 30), (64, 3, 128, 5), (4, 300, 64, 20),
+    (2, 1, 64, 200)])
+def test_plain(rt, ranges, m, blocks, kt, loop, order):
+    from attention_superoptimizer_amd import workloads as W
+    spec, _ = W.tiled_matmul(m, 64 * blocks, kt * loop, (blocks, 1, 1), loop, (-1, -1, -1), (1, -1, -1), (1, -1, -1))
+    _run(rt, spec, order, f"{m} x {blocks}, {kt} x {loop} {order}")
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("m", [1, 9, 16])
+def test_gated_mlp_prologues_and_lora(rt, ranges, m, order):
+    from attention_superoptimizer_amd import workloads as W
+    spec, _ = W.config5_gated_mlp(m=m, d=192, h=640, grid1=10, F1=3, grid2=3, F2=5)
+    _run(rt, spec, order, f"gated mlp {m} {order}", std=0.05)
+    for op in ("tb_exp_op", "tb_silu_op"):
+        spec = [W._inp([m, 320]), W._inp([320, 128], COL),
+                {"op": "customized", "in": [[0, 0], [1, 0]],
+                 "plan": W._plan((2, 1, 1), 5, [(-1, -1, -1), (1, -1, -1)], (1, 0), (1, -1, -1),
+                                 [(op, [(0, 0)]), ("tb_matmul_op", [(2, 0), (1, 0)])])}]
+        _run(rt, spec, order, f"{op} {m} {order}")
+    spec, _ = W.config4_lora(m=m, d=128 * 6, r=16, grid=3, F=6)
+    spec[1], spec[3] = W._inp([128 * 6, 192], COL), W._inp([16, 192], COL)
+    _run(rt, spec, order, f"lora {m} {order}")
