@@ -111,6 +111,7 @@ ABI = {
     "mi355_customized_fp": (_ci, [_pplan, _pvp, _pvp]),
     "mi355_customized_fp_static": (_ci, [_pplan, _pvp, _pvp]),
     "mi355_customized_fp_batch": (_ci, [_pplan, _ci, _pvp, _pvp]),
+    "mi355_customized_fp_batch_within": (_ci, [_pplan, _ci, _pvp, _pvp, _vp, _vp]),
     "mi355_plan_extents": (_ci, [_pplan, _pll, _pll, _pi, _pi]),
     "mi355_customized_run": (_ci, [_pplan, _pvp, _pvp]),
     "mi355_prepare": (_ci, [_pplan, _pvp, _pvp, _ci, _pvp]),

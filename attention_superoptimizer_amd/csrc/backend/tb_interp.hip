@@ -1879,6 +1879,12 @@ static int launch_fp_chunk(std::vector<DevProgram> &progs, std::vector<PlanExten
 
 extern "C" int mi355_customized_fp_batch(mi355_plan const *plans, int n,
                                          void const *const *inputs, void *const *outputs) {
+  return mi355_customized_fp_batch_within(plans, n, inputs, outputs, nullptr, nullptr);
+}
+
+extern "C" int mi355_customized_fp_batch_within(mi355_plan const *plans, int n, void const *const *inputs,
+                                                void *const *outputs, long long const *in_elems,
+                                                long long const *out_elems) {
   MI355_REQUIRE_INIT();
   if (n < 0 || (n > 0 && (plans == nullptr || inputs == nullptr || outputs == nullptr))) {
     return fail(MI355_ERR_INVALID, "bad batch (n = %d)", n);
@@ -1908,6 +1914,16 @@ extern "C" int mi355_customized_fp_batch(mi355_plan const *plans, int n,
                      outputs + (size_t)i * MI355_MAX_DMEM_OUTPUTS, false, prog, &ext);
     if (rc != MI355_OK) {
       return rc;
+    }
+    for (int j = 0; in_elems != nullptr && j < plans[i].num_dmem_inputs; j++) {
+      if (ext.in_elems[j] > in_elems[(size_t)i * MI355_MAX_DMEM_INPUTS + j]) {
+        return fail(MI355_ERR_INVALID, "operator %d: input loader would read past its tensor", i);
+      }
+    }
+    for (int j = 0; out_elems != nullptr && j < plans[i].num_dmem_outputs; j++) {
+      if (ext.out_elems[j] > out_elems[(size_t)i * MI355_MAX_DMEM_OUTPUTS + j]) {
+        return fail(MI355_ERR_INVALID, "operator %d: output saver would write past its tensor", i);
+      }
     }
     size_t need = 0;
     if (prog.fused == 4 && fp_mfma_gemm_fits(prog, ext, &need)) {

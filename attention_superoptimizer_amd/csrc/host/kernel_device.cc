@@ -362,13 +362,22 @@ static LoweredOp lower(KNCustomizedOp const &op, bool fingerprint) {
   return l;
 }
 
-// for batched submission (verify.cc): the lowered program and its bound pointers
+// for batched submission (verify.cc): the lowered program, its bound pointers and how many elements the
+// tensors behind them hold (the batch call checks the program against these: it lowers it anyway)
 void lower_customized(KNCustomizedOp const &op, bool fingerprint, mi355_plan *plan,
-                      void const **inputs, void **outputs) {
-  LoweredOp l = lower(op, fingerprint);
+                      void const **inputs, void **outputs, long long *in_elems, long long *out_elems) {
+  LoweredOp l = lower_unchecked(op, fingerprint);
   *plan = l.plan;
   std::memcpy(inputs, l.inputs, sizeof(l.inputs));
   std::memcpy(outputs, l.outputs, sizeof(l.outputs));
+  int ii = 0, oo = 0;
+  for (mirage::threadblock::TBOperator *t : op.bgraph.operators) {
+    if (t->op_type == TB_INPUT_OP) {
+      in_elems[ii++] = (long long)static_cast<mirage::threadblock::TBInputOp *>(t)->dtensor.num_elements();
+    } else if (t->op_type == TB_OUTPUT_OP) {
+      out_elems[oo++] = (long long)static_cast<mirage::threadblock::TBOutputOp *>(t)->dtensor.num_elements();
+    }
+  }
 }
 
 // A run of the operator repeats the launches the backend prepared for it the first time, as long

@@ -19,14 +19,14 @@
 #include <numeric>
 #include <thread>
 #include <unordered_map>
-#include <unordered_set>
 
 namespace mirage {
 namespace kernel {
 // kernel_device.cc: the lowered program of a customized operator and its bound pointers
 void lower_customized(KNCustomizedOp const &op, bool fingerprint, mi355_plan *plan,
-                      void const **inputs, void **outputs);
+                      void const **inputs, void **outputs, long long *in_elems, long long *out_elems);
 bool fingerprint_softmax_rows(std::vector<KNOperator *> const &ops, size_t i);
+void prefetch_graph(Graph const &g, int level, bool write);
 }  // namespace kernel
 
 namespace search {
@@ -38,16 +38,20 @@ using namespace mirage::type;
 #define MI355_CALL(expr) MIRAGE_CHECK((expr) == MI355_OK, mi355_last_error())
 
 std::vector<DTensor> graph_outputs(kernel::Graph const &g) {
-  std::unordered_set<size_t> consumed;
-  for (KNOperator const *op : g.operators) {
-    for (DTensor const &t : op->input_tensors) {
-      consumed.insert(t.guid);
+  auto consumed = [&g](size_t guid, size_t producer) {
+    for (size_t i = producer + 1; i < g.operators.size(); i++) {  // (a consumer comes after its producer)
+      for (DTensor const &t : g.operators[i]->input_tensors) {
+        if (t.guid == guid) {
+          return true;
+        }
+      }
     }
-  }
+    return false;
+  };
   std::vector<DTensor> outs;
-  for (KNOperator const *op : g.operators) {
-    for (DTensor const &t : op->output_tensors) {
-      if (consumed.count(t.guid) == 0) {
+  for (size_t i = 0; i < g.operators.size(); i++) {
+    for (DTensor const &t : g.operators[i]->output_tensors) {
+      if (!consumed(t.guid, i)) {
         outs.push_back(t);
       }
     }
@@ -143,6 +147,11 @@ static void fingerprint_graphs(std::vector<kernel::Graph *> const &graphs, uint6
                                VerifyStats *stats) {
   size_t const n = graphs.size();
   std::vector<size_t> cursor(n, 0);
+  for (int level = 0; level < 4; level++) {
+    for (kernel::Graph *g : graphs) {
+      kernel::prefetch_graph(*g, level, false);
+    }
+  }
   fill_inputs(std::vector<kernel::Graph const *>(graphs.begin(), graphs.end()), input_seed);
   // Input number j of every graph is filled from (input_seed, j), so inputs j of two graphs
   // with the same element count hold the same values (candidates of one problem: all of them).
@@ -177,6 +186,7 @@ static void fingerprint_graphs(std::vector<kernel::Graph *> const &graphs, uint6
   std::vector<mi355_plan> plans;
   std::vector<void const *> ins;
   std::vector<void *> outs;
+  std::vector<long long> in_elems, out_elems;
   int b_op[MI355_MAX_BINARY_OPS], b_nd[MI355_MAX_BINARY_OPS];
   uint16_t const *b_in1[MI355_MAX_BINARY_OPS], *b_in2[MI355_MAX_BINARY_OPS];
   uint16_t *b_out[MI355_MAX_BINARY_OPS];
@@ -202,6 +212,8 @@ static void fingerprint_graphs(std::vector<kernel::Graph *> const &graphs, uint6
     plans.clear();
     ins.clear();
     outs.clear();
+    in_elems.clear();
+    out_elems.clear();
     bool any = false;
     for (size_t k = 0; k < n; k++) {
       std::vector<KNOperator *> const &ops = graphs[k]->operators;
@@ -267,9 +279,12 @@ static void fingerprint_graphs(std::vector<kernel::Graph *> const &graphs, uint6
         plans.emplace_back();
         ins.resize(ins.size() + MI355_MAX_DMEM_INPUTS, nullptr);
         outs.resize(outs.size() + MI355_MAX_DMEM_OUTPUTS, nullptr);
+        in_elems.resize(ins.size(), 0);
+        out_elems.resize(outs.size(), 0);
         kernel::lower_customized(*static_cast<kernel::KNCustomizedOp *>(op), true, &plans.back(),
-                                 &ins[ins.size() - MI355_MAX_DMEM_INPUTS],
-                                 &outs[outs.size() - MI355_MAX_DMEM_OUTPUTS]);
+                                 &ins[ins.size() - MI355_MAX_DMEM_INPUTS], &outs[outs.size() - MI355_MAX_DMEM_OUTPUTS],
+                                 &in_elems[ins.size() - MI355_MAX_DMEM_INPUTS],
+                                 &out_elems[outs.size() - MI355_MAX_DMEM_OUTPUTS]);
         for (size_t i = ins.size() - MI355_MAX_DMEM_INPUTS; i < ins.size(); i++) {
           if (ins[i] != nullptr) {
             ins[i] = shared_input(static_cast<uint16_t *>(const_cast<void *>(ins[i])));
@@ -281,7 +296,8 @@ static void fingerprint_graphs(std::vector<kernel::Graph *> const &graphs, uint6
     flush_matmuls();
     flush_binaries();
     if (!plans.empty()) {
-      MI355_CALL(mi355_customized_fp_batch(plans.data(), (int)plans.size(), ins.data(), outs.data()));
+      MI355_CALL(mi355_customized_fp_batch_within(plans.data(), (int)plans.size(), ins.data(), outs.data(), in_elems.data(),
+                                                  out_elems.data()));
     }
     if (!any) {
       break;

@@ -317,6 +317,10 @@ int mi355_customized_fp_static(mi355_plan const *plan, void const *const *inputs
  * device memory), plus one launch that folds the partial sums of every split for-loop. */
 int mi355_customized_fp_batch(mi355_plan const *plans, int n, void const *const *inputs,
                               void *const *outputs);
+/* The same for a caller that knows how many elements each tensor holds (in_elems, out_elems laid out
+ * like inputs and outputs; null: not checked): a plan that would reach past one is refused. */
+int mi355_customized_fp_batch_within(mi355_plan const *plans, int n, void const *const *inputs, void *const *outputs,
+                                     long long const *in_elems, long long const *out_elems);
 
 /* Host-only check of a plan (no device needed): 1 + the largest element index the
  * plan reads from each input / writes to each output, and the LDS the two
