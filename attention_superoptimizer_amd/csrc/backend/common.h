@@ -159,24 +159,36 @@ int fail(int code, char const *fmt, ...);
     }                                                                               \
   } while (0)
 
+// a b + c with 24-bit a and b: an instruction of full rate, spelled out because the compiler, which sees
+// that only the low bits of a residue are asked for, puts a 64-bit multiply-add at a quarter of it in
+// its place.  Bits of `a` beyond 24 cost the result its bits beyond 24.
+__device__ __forceinline__ uint32_t mad24(uint32_t a, int b, uint32_t c) {
+  uint32_t r;
+  asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
+  return r;
+}
 // Residues of a 16-bit value.  The compiler lowers `%` by a constant to 32-bit multiply-highs, which
 // run at a quarter of the rate of a 24-bit multiply; for values below 2^16 a 24-bit reciprocal is exact
 // (37118 = ceil(2^22 / 113); 36954 = floor(2^23 / 227), so the value is taken one higher).
-__device__ __forceinline__ uint32_t residue_q(uint32_t x) { return x - __umul24(__umul24(x, 37118u) >> 22, FP_Q); }
-__device__ __forceinline__ uint32_t residue_p(uint32_t x) { return x - __umul24((__umul24(x, 36954u) + 36954u) >> 23, FP_P); }
+__device__ __forceinline__ uint32_t residue_q(uint32_t x) {
+  return mad24((uint32_t)__umul24(x, 37118u) >> 22, -(int)FP_Q, x);
+}
+__device__ __forceinline__ uint32_t residue_p(uint32_t x) {
+  return mad24(((uint32_t)__umul24(x, 36954u) + 36954u) >> 23, -(int)FP_P, x);
+}
 // the residue modulo 227 in [-113, 113]: what a signed byte holds
 __device__ __forceinline__ int residue_p_signed(uint32_t x) {
-  return (int)(x - __umul24((__umul24(x, 36954u) + 36954u * 114u) >> 23, FP_P));
+  return (int)mad24(((uint32_t)__umul24(x, 36954u) + 36954u * 114u) >> 23, -(int)FP_P, x);
 }
 // Residues of any 32-bit value: one multiply-high; the quotient times the modulus by a 24-bit multiply,
 // of which only the low bits matter (a residue is below 2^8 / 2^15).
-__device__ __forceinline__ uint32_t mod_p(uint32_t x) { return (x - __umul24(x / FP_P, FP_P)) & 0xffu; }
-__device__ __forceinline__ uint32_t mod_q(uint32_t x) { return (x - __umul24(x / FP_Q, FP_Q)) & 0xffu; }
-__device__ __forceinline__ uint32_t mod_pq(uint32_t x) { return x - __umul24(x / FP_PQ, FP_PQ); }
+__device__ __forceinline__ uint32_t mod_p(uint32_t x) { return mad24(x / FP_P, -(int)FP_P, x) & 0xffu; }
+__device__ __forceinline__ uint32_t mod_q(uint32_t x) { return mad24(x / FP_Q, -(int)FP_Q, x) & 0xffu; }
+__device__ __forceinline__ uint32_t mod_pq(uint32_t x) { return mad24(x / FP_PQ, -(int)FP_PQ, x); }
 // The ring value with residues p modulo 227 (p < 227) and q modulo 113 (any 16-bit q).  227 is 1
 // modulo 113, so p + 227 t has residue p + t there: t = q - p.
 __device__ __forceinline__ uint32_t fp_from_residues(uint32_t p, uint32_t q) {
-  return p + __umul24(residue_q(q + 2 * FP_Q - p), FP_P);
+  return mad24(residue_q(q + 2 * FP_Q - p), FP_P, p);
 }
 // four of them as bytes
 __device__ __forceinline__ uint32_t pack_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
@@ -194,22 +206,84 @@ __device__ __forceinline__ uint32_t residues_p4_signed(uint32_t a, uint32_t b, u
                     (uint32_t)residue_p_signed(d));
 }
 
+// Residues of two fingerprint values (16 bits each) as signed bytes, the low bytes of the halves of p and
+// q: what the int8 matrix products want, at three instructions a value for both fields (ten through
+// residue_p_signed and residue_q).  The quotient is estimated in packed fp16: added to 1536 it is rounded
+// to an integer, whose low byte is the quotient's.  An estimate one off where the value lies close to the
+// middle between two multiples leaves a remainder that still fits: over all of [0, 25651) they are in
+// [-125, 117] modulo 227 and in [-66, 63] modulo 113.
+typedef _Float16 fp_half2 __attribute__((ext_vector_type(2)));
+typedef unsigned short fp_ushort2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void residue_pairs(uint32_t v, uint32_t &p, uint32_t &q) {
+  fp_ushort2 const x = __builtin_bit_cast(fp_ushort2, v);
+  fp_half2 const h = __builtin_convertvector(x, fp_half2), one_and_half_k = {(_Float16)1536.0f, (_Float16)1536.0f};
+  fp_half2 const by_p = __builtin_bit_cast(fp_half2, 0x1c831c83u), by_q = __builtin_bit_cast(fp_half2, 0x20882088u);
+  fp_ushort2 const tp = __builtin_bit_cast(fp_ushort2, __builtin_elementwise_fma(h, by_p, one_and_half_k));
+  fp_ushort2 const tq = __builtin_bit_cast(fp_ushort2, __builtin_elementwise_fma(h, by_q, one_and_half_k));
+  p = __builtin_bit_cast(uint32_t, (fp_ushort2)(x - tp * (unsigned short)FP_P));
+  q = __builtin_bit_cast(uint32_t, (fp_ushort2)(x - tq * (unsigned short)FP_Q));
+}
+// of four values in a row
+__device__ __forceinline__ void residues_row(uint2 v, uint32_t &p, uint32_t &q) {
+  uint32_t p0, q0, p1, q1;
+  residue_pairs(v.x, p0, q0);
+  residue_pairs(v.y, p1, q1);
+  p = __builtin_amdgcn_perm(p1, p0, 0x06040200u);
+  q = __builtin_amdgcn_perm(q1, q0, 0x06040200u);
+}
+// of the columns of four rows of four
+__device__ __forceinline__ void residues_patch(uint2 const *rows, uint32_t *p, uint32_t *q) {
+  auto turn = [](uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t *out) {
+    uint32_t const ab = __builtin_amdgcn_perm(b, a, 0x06020400u), cd = __builtin_amdgcn_perm(d, c, 0x06020400u);
+    out[0] = __builtin_amdgcn_perm(cd, ab, 0x05040100u);
+    out[1] = __builtin_amdgcn_perm(cd, ab, 0x07060302u);
+  };
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    uint32_t pp[4], qq[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      residue_pairs(h == 0 ? rows[i].x : rows[i].y, pp[i], qq[i]);
+    }
+    turn(pp[0], pp[1], pp[2], pp[3], p + 2 * h);
+    turn(qq[0], qq[1], qq[2], qq[3], q + 2 * h);
+  }
+}
+
+// Fingerprint value from sums of products of such residues over k <= FEW ? 128 : 32768, the sums started
+// from multiples of the moduli that keep them above zero: a negative sum would need a fix-up.  FEW: the
+// sums are below 2^22, where 2^30 / 227 and 2^30 / 113 rounded up give exact quotients by 24-bit
+// multiply-highs, which run at four times the rate of 32-bit ones.
+constexpr int kSumBaseFewP = 227 * 9000, kSumBaseFewQ = 113 * 5000;
+constexpr int kSumBaseP = 227 * 2256000, kSumBaseQ = 113 * 1270000;
+template <bool FEW>
+__device__ __forceinline__ uint32_t fp_from_based_sums(uint32_t sum_p, uint32_t sum_q) {
+  auto hi24 = [](uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_mul_hi_u32_u24 %0, %1, %2" : "=v"(r) : "v"(a), "s"(b));
+    return r;
+  };
+  uint32_t const p = mad24(FEW ? hi24(sum_p << 2, 4730141u) : __umulhi(sum_p, 605457945u) >> 5, -(int)FP_P, sum_p);
+  uint32_t const y = sum_q - p;
+  return mad24(mad24(FEW ? hi24(y << 2, 9502141u) : __umulhi(y, 1216273925u) >> 5, -(int)FP_Q, y), FP_P, p);
+}
+
 // A sum of residue products, |x| < 2^31, modulo 227: one signed multiply-high (605457945 =
-// ceil(2^37 / 227) is exact below 2^31), the quotient times 227 by a 24-bit multiply of which the low
-// byte is right.  A negative multiple of 227 leaves 227.
+// ceil(2^37 / 227) is exact below 2^31); of the quotient times 227, by a 24-bit multiply, the low byte is
+// right.  A negative multiple of 227 leaves 227.
 __device__ __forceinline__ uint32_t reduce_p(int x) {
-  uint32_t const r = (static_cast<uint32_t>(x) - __umul24(static_cast<uint32_t>(__mulhi(x, 605457945) >> 5), FP_P)) & 0xffu;
+  uint32_t const r = mad24(static_cast<uint32_t>(__mulhi(x, 605457945) >> 5), -(int)FP_P, static_cast<uint32_t>(x)) & 0xffu;
   return r < r - FP_P ? r : r - FP_P;
 }
 // 0 <= x < 2^31 modulo 113 (1216273925 = ceil(2^37 / 113)); the general mod_q takes a fix-up more
 __device__ __forceinline__ uint32_t reduce_q(uint32_t x) {
-  return (x - __umul24(__umulhi(x, 1216273925u) >> 5, FP_Q)) & 0xffu;
+  return mad24(__umulhi(x, 1216273925u) >> 5, -(int)FP_Q, x) & 0xffu;
 }
 // Fingerprint value of a matmul output from its two residue sums (matrix-core kernels): |sum_p| <
 // 2^31 (operands recentred to [-113, 113]), 0 <= sum_q < 2^31 - 226.
 __device__ __forceinline__ uint32_t fp_from_residue_sums(int sum_p, int sum_q) {
   uint32_t const p = reduce_p(sum_p);
-  return p + __umul24(reduce_q(static_cast<uint32_t>(sum_q) + 2 * FP_Q - p), FP_P);
+  return mad24(reduce_q(static_cast<uint32_t>(sum_q) + 2 * FP_Q - p), FP_P, p);
 }
 
 // The fingerprint lookup tables in device memory and the ring operations built on them

@@ -12,11 +12,12 @@
 // chunk of K and V goes from memory (the next chunk is in flight while this one is multiplied) through
 // registers, where 4 x 4 patches are reduced to bytes and turned, into LDS as MFMA operands; K^T is the
 // first operand, so a lane ends up with 16 scores of one query, looks their exponentials up and has the
-// second product's operand without exchanging anything (V's rows are stored in the order that gives).
+// second product's operand without exchanging anything (V's keys are stored in the order that gives).
 //
 // What bounds it: the vector instructions that reduce and look up (the matrix products are a tenth).
 // The interpreter ran these plans operator by operator on 16-bit tiles in LDS: 32 x 16 blocks of
-// 64 x 64 tiles, 4 iterations: 64 us there.
+// 64 x 64 tiles, 4 iterations: 64 us there; 14.5 with residues one value at a time and staging writes
+// that met in the banks, 12.9 here.
 #include "common.h"
 #include "tb_program.h"
 
@@ -105,14 +106,20 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
       if (at < d) {
         x = *reinterpret_cast<uint2 const *>(q + at);
       }
-      uint32_t const a = x.x & 0xffffu, b = x.x >> 16, e = x.y & 0xffffu, f = x.y >> 16;
-      qf[w] = (int)residues_q4(a, b, e, f);
-      qp[w] = SCORES ? (int)residues_p4_signed(a, b, e, f) : 0;
+      uint32_t rp, rq;
+      residues_row(x, rp, rq);
+      qf[w] = (int)rq;
+      qp[w] = (int)rp;
     }
   }
 
-  // ---- staging: patch (hi, lo) of a chunk is 4 rows from 4 hi, 4 columns from 4 lo
+  // ---- staging: patch (hi, lo) of a chunk of K is 4 rows from 4 hi, 4 columns from 4 lo; of V, 4 columns
+  // from 4 lo of the keys 16 (hi / 4) + 4 i + hi % 4.  Column 4 lo + u becomes row lo of matrix tile u: the
+  // lanes of a write differ in their banks, and a lane's scores are those of keys 16 g + 4 r + j, which is
+  // the order V's keys then have.
   int const hi = tid / 16, lo = tid % 16;
+  // (past the end of a tile the last patch stands in: elements of K past d meet zeros of Q, keys past n
+  // are masked, elements of V past dv are not stored)
   uint2 kr[KW][4], vr[KW][4];
   auto fetch = [&](int it, int group) {
     uint16_t const *const k = tile_at(P.k, bx, by, bz, it);
@@ -120,16 +127,12 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
 #pragma unroll
     for (int w = 0; w < KW; w++) {
       int const key0 = (group * KW + w) * kChunk;
-      bool const k_in = key0 + 4 * lo < n && 4 * hi < d, v_in = key0 + 4 * hi < n && 4 * lo < dv;
+      int const kk = min(4 * hi, d - 4), kc = min(key0 + 4 * lo, n - 4), vc = min(4 * lo, dv - 4);
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        kr[w][i] = vr[w][i] = uint2{0, 0};
-        if (k_in) {
-          kr[w][i] = *reinterpret_cast<uint2 const *>(k + (long long)(4 * hi + i) * ld_k + key0 + 4 * lo);
-        }
-        if (v_in) {
-          vr[w][i] = *reinterpret_cast<uint2 const *>(v + (long long)(key0 + 4 * hi + i) * ld_v + 4 * lo);
-        }
+        kr[w][i] = *reinterpret_cast<uint2 const *>(k + (long long)(kk + i) * ld_k + kc);
+        int const vk = min(key0 + 16 * (hi / 4) + 4 * i + hi % 4, n - 1);
+        vr[w][i] = *reinterpret_cast<uint2 const *>(v + (long long)vk * ld_v + vc);
       }
     }
   };
@@ -137,18 +140,17 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
 #pragma unroll
     for (int w = 0; w < KW; w++) {
       unsigned char *const kq = tiles + w * PLANES * kPlane, *const vp = kq + kPlane, *const kp = vp + kPlane;
-      auto half = [](uint2 x, int u) { return (u < 2 ? x.x : x.y) >> (16 * (u & 1)) & 0xffffu; };
+      uint32_t p[4], q[4], v[4], unused[4];
+      residues_patch(kr[w], p, q);
+      residues_patch(vr[w], v, unused);
 #pragma unroll
       for (int u = 0; u < 4; u++) {
-        uint32_t const a = half(kr[w][0], u), b = half(kr[w][1], u), e = half(kr[w][2], u), f = half(kr[w][3], u);
-        int const at = (4 * lo + u) * kPitch + 4 * hi;  // key 4 lo + u, elements 4 hi .. + 3
-        *reinterpret_cast<uint32_t *>(kq + at) = residues_q4(a, b, e, f);
+        int const at = (16 * u + lo) * kPitch + 4 * hi;
+        *reinterpret_cast<uint32_t *>(kq + at) = q[u];
         if (SCORES) {
-          *reinterpret_cast<uint32_t *>(kp + at) = residues_p4_signed(a, b, e, f);
+          *reinterpret_cast<uint32_t *>(kp + at) = p[u];
         }
-        // key 16 j + 4 g + r of the chunk sits at byte 16 g + 4 j + r of a row of V^T
-        *reinterpret_cast<uint32_t *>(vp + (4 * lo + u) * kPitch + 16 * (hi % 4) + 4 * (hi / 4)) =
-            residues_p4_signed(half(vr[w][0], u), half(vr[w][1], u), half(vr[w][2], u), half(vr[w][3], u));
+        *reinterpret_cast<uint32_t *>(vp + at) = v[u];
       }
     }
   };
@@ -159,7 +161,9 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
   for (int x = 0; x < 4; x++) {
     o[x] = total[x] = v4i{0, 0, 0, 0};
   }
-  v4i const zero = {0, 0, 0, 0};
+  // scores modulo 113 start from a multiple of 113 that keeps them above zero
+  constexpr int kBase = 113 * 2500;
+  v4i const zero = {0, 0, 0, 0}, base = {kBase, kBase, kBase, kBase};
   // (sums of bytes: a chunk adds less than 2^20 to an element of O, so they are folded long before
   // they could reach 2^31)
   int folded = 0;
@@ -178,27 +182,30 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
     int const key0 = (this_group * KW + kw) * kChunk;
     if (key0 < n) {
       unsigned char const *const kq = tiles + kw * PLANES * kPlane, *const vp = kq + kPlane, *const kp = vp + kPlane;
+      // keys past the tile (exp(0) is not zero): the first `inside` bytes of every e[j] count
+      int const inside = (n - key0 - 16 * g) / 4;
+      uint32_t const mask = inside >= 4 ? ~0u : inside <= 0 ? 0u : (1u << (8 * inside)) - 1;
       v4i e;
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         v4i const k = *reinterpret_cast<v4i const *>(kq + (16 * j + c) * kPitch + 16 * g);
-        v4i const x = __builtin_amdgcn_mfma_i32_16x16x64_i8(k, qf, zero, 0, 0, 0);
+        v4i const x = __builtin_amdgcn_mfma_i32_16x16x64_i8(k, qf, base, 0, 0, 0);
         if (SCORES) {
           v4i const y = __builtin_amdgcn_mfma_i32_16x16x64_i8(*reinterpret_cast<v4i const *>(kp + (16 * j + c) * kPitch + 16 * g),
                                                               qp, zero, 0, 0, 0);
-          rs += y[0] + y[1] + y[2] + y[3];  // (keys past the tile are zero)
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            rs += r < inside ? y[r] : 0;
+          }
         }
-        // A score is below 64 * 112^2 < 2^20.  2320 = ceil(2^18 / 113) gives its quotient or one more:
+        // A score is within 64 * 66^2 of the base: in (0, 2^20).  2320 = ceil(2^18 / 113) gives its quotient or one more:
         // the remainder is in [-49, 112], and the table starts below zero.
         int b[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-          b[r] = exps[x[r] - (int)__umul24(__umul24((uint32_t)x[r], 2320u) >> 18, FP_Q)];
+          b[r] = exps[(int)mad24((uint32_t)__umul24((uint32_t)x[r], 2320u) >> 18, -(int)FP_Q, (uint32_t)x[r])];
         }
-        e[j] = (int)pack_bytes((uint32_t)b[0], (uint32_t)b[1], (uint32_t)b[2], (uint32_t)b[3]);
-        if (key0 + 16 * j + 4 * g >= n) {
-          e[j] = 0;  // exp(0) is not zero
-        }
+        e[j] = (int)(pack_bytes((uint32_t)b[0], (uint32_t)b[1], (uint32_t)b[2], (uint32_t)b[3]) & mask);
         if (!SCORES) {
           rs = __builtin_amdgcn_sdot4(e[j], 0x01010101, rs, false);
         }
@@ -297,14 +304,14 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
   }
   uint16_t *const og = tile_at(P.o, bx, by, bz, 0) + (long long)row * P.o.ld;
 #pragma unroll
-  for (int x = 0; x < 4; x++) {
-    if (16 * x + 4 * g < dv) {
+  for (int e = 0; e < 4; e++) {  // a lane's columns are 16 g .. + 15: 4 e + x from tile x
+    if (16 * g + 4 * e < dv) {
       uint32_t z[4];
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        z[r] = fp_from_residues(reduce_p(total[x][r]), 0u);
+      for (int x = 0; x < 4; x++) {
+        z[x] = fp_from_residues(reduce_p(total[x][e]), 0u);
       }
-      *reinterpret_cast<uint2 *>(og + 16 * x + 4 * g) = uint2{z[0] | (z[1] << 16), z[2] | (z[3] << 16)};
+      *reinterpret_cast<uint2 *>(og + 16 * g + 4 * e) = uint2{z[0] | (z[1] << 16), z[2] | (z[3] << 16)};
     }
   }
   if (P.r.ptr != nullptr && g == 0) {

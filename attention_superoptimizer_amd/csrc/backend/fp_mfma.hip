@@ -24,6 +24,7 @@
 // launch and every logical block reads its tiles from the planes through the plan's own
 // strides; see fp_mfma_gemm_block.
 #include "common.h"
+#include "fp_direct.h"
 #include "tb_program.h"
 
 // fp_mfma_matmul_big_kernel loads registers by inline assembly and waits for them later: code
@@ -1233,6 +1234,18 @@ extern "C" int mi355_fp_matmul_many(uint16_t const *const *A, uint16_t const *co
   // cannot take this path at all (no k, planes too large) goes through the single entry point
   int begin = 0;
   while (begin < count) {
+    int direct = begin;
+    while (direct < count && fp_direct_pays(batch[direct], m[direct], n[direct], k[direct])) {
+      direct++;
+    }
+    if (direct > begin) {
+      if (int rc = launch_fp_direct(A + begin, B + begin, C + begin, batch + begin, m + begin, n + begin, k + begin,
+                                    direct - begin)) {
+        return rc;
+      }
+      begin = direct;
+      continue;
+    }
     size_t need = 0;
     if (state().fp_vector_dot_only ||
         !mfma_matmul_fits(batch[begin], m[begin], n[begin], k[begin], &need) ||
@@ -1247,7 +1260,8 @@ extern "C" int mi355_fp_matmul_many(uint16_t const *const *A, uint16_t const *co
     size_t total = need;
     while (end < count && end - begin < kMaxJobs) {
       size_t more = 0;
-      if (!mfma_matmul_fits(batch[end], m[end], n[end], k[end], &more) ||
+      if (fp_direct_pays(batch[end], m[end], n[end], k[end]) ||
+          !mfma_matmul_fits(batch[end], m[end], n[end], k[end], &more) ||
           total + more > state().planes_bytes) {
         break;
       }

@@ -9,6 +9,7 @@
 // multipliers.  (sum a*b) mod 25651 is fixed by its two residues, so the result
 // is bit-identical for operands < 25651.
 #include "common.h"
+#include "fp_direct.h"
 
 #include <algorithm>
 #include <cstring>
@@ -736,6 +737,9 @@ extern "C" int mi355_fp_matmul(uint16_t const *A, uint16_t const *B, uint16_t *C
   }
   if (batch > 65535) {
     return fail(MI355_ERR_UNSUPPORTED, "batch %d exceeds grid.z", batch);
+  }
+  if (fp_direct_pays(batch, m, n, k)) {
+    return launch_fp_direct(&A, &B, &C, &batch, &m, &n, &k, 1);
   }
   if (mfma_matmul_pays(batch, m, n, k)) {
     return launch_mfma_matmul(A, B, C, batch, m, n, k);
