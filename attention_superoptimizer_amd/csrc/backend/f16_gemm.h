@@ -169,6 +169,102 @@ struct OperandStage {
   }
 };
 
+// Which tile, batch and k range: an XCD (one L2) gets consecutive ids; the k ranges of a tile sit next to
+// each other, and tiles go down four tile rows before they move to the next columns.
+__device__ __forceinline__ void gemm_tile(AnyGemm const &G, int bm, int bn, int &split, int &batch, int &row0, int &col0) {
+  unsigned const xcd = blockIdx.x % 8, each = G.total / 8, more = G.total % 8;
+  unsigned id = xcd * each + (xcd < more ? xcd : more) + blockIdx.x / 8;
+  split = (int)(id % (unsigned)G.ksplit);
+  id /= (unsigned)G.ksplit;
+  batch = (int)(id / (unsigned)G.tiles_per_batch);
+  int const t0 = (int)(id % (unsigned)G.tiles_per_batch);
+  int const per_group = 4 * G.tiles_n, first_m = 4 * (t0 / per_group);
+  int const gsz = (G.tiles_m - first_m) < 4 ? (G.tiles_m - first_m) : 4;
+  row0 = (first_m + (t0 % per_group) % gsz) * bm;
+  col0 = (t0 % per_group) / gsz * bn;
+}
+
+// The way out of a workgroup's sums: fp16 rows and the consumer's result, or a k range's fp32 sums.  `tile`
+// is LDS nothing else uses any more; `owner`: wavefronts that hold sums.
+template <int BM, int BN, int TM, int TN, int NT>
+__device__ __forceinline__ void gemm_store(AnyGemm const &G, float4v const (&acc)[TM][TN], _Float16 *tile, bool owner, int lane,
+                                           int split, int batch, int row0, int col0, int wm0, int wn0) {
+  // acc[i][j][e] = C[wm0 + 16 i + lane % 16][wn0 + 16 j + 4 (lane / 16) + e]
+  int const g = lane / 16, c = lane % 16;
+  if (G.ksplit > 1) {
+    if (owner) {
+      int const batches = (int)(G.total / (unsigned)(G.ksplit * G.tiles_per_batch));
+      float *const P = G.partial + ((size_t)split * batches + batch) * (size_t)G.m * G.n;
+#pragma unroll
+      for (int i = 0; i < TM; i++) {
+        int const row = row0 + wm0 + 16 * i + c;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+          int const col = col0 + wn0 + 16 * j + 4 * g;
+          if (row < G.m && col + 4 <= G.n) {
+            *reinterpret_cast<float4_any *>(P + (size_t)row * G.n + col) = acc[i][j];
+          } else if (row < G.m) {
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+              if (col + e < G.n) {
+                P[(size_t)row * G.n + col + e] = acc[i][j][e];
+              }
+            }
+          }
+        }
+      }
+    }
+    return;
+  }
+  // ---- out through LDS: rows of 16-byte chunks
+  constexpr int LDC = BN + 8;
+  if (owner) {
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        *reinterpret_cast<half4 *>(tile + (wm0 + 16 * i + c) * LDC + wn0 + 16 * j + 4 * g) =
+            __builtin_convertvector(acc[i][j], half4);
+      }
+    }
+  }
+  __syncthreads();
+  size_t const matrix = (size_t)batch * G.m * G.n;
+  for (int e = threadIdx.x; e < BM * (BN / 8); e += NT) {
+    int const r = e / (BN / 8), c8 = 8 * (e % (BN / 8)), row = row0 + r, col = col0 + c8;
+    if (row < G.m && col < G.n) {
+      half8 const v = *reinterpret_cast<half8 const *>(tile + r * LDC + c8);
+      size_t const at = matrix + (size_t)row * G.n + col;
+      if (col + 8 <= G.n) {
+        *reinterpret_cast<half8_any *>(G.C + at) = v;
+        if (G.epilogue != EPI_NONE) {
+          half8 x = v;
+          if (G.epilogue >= EPI_ADD) {
+            x = *reinterpret_cast<half8_any const *>(G.X + at);
+          }
+          half8 y;
+#pragma unroll
+          for (int u = 0; u < 8; u++) {
+            y[u] = static_cast<_Float16>(epilogue_value(G.epilogue, static_cast<float>(v[u]), static_cast<float>(x[u])));
+          }
+          *reinterpret_cast<half8_any *>(G.E + at) = y;
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < 7; u++) {
+          if (col + u < G.n) {
+            G.C[at + u] = v[u];
+            if (G.epilogue != EPI_NONE) {
+              float const x = G.epilogue >= EPI_ADD ? static_cast<float>(G.X[at + u]) : 0.0f;
+              G.E[at + u] = static_cast<_Float16>(epilogue_value(G.epilogue, static_cast<float>(v[u]), x));
+            }
+          }
+        }
+      }
+    }
+  }
+}
+
 // A workgroup owns a BM x BN tile of C and a range of k.  Its KG groups of wavefronts (WM x WN of the
 // tile per wavefront) take a part of the range each and add their sums up in LDS at the end: with few
 // tiles that is what keeps a compute unit busy.  A stage of 64 k goes global -> registers (two stages
@@ -195,16 +291,8 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG) void f16_gemm_any_
   int const tid = threadIdx.x % NTG, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   _Float16 *const bufs = reinterpret_cast<_Float16 *>(lds) + kg * 2 * BUF;
 
-  // Which tile: an XCD (one L2) gets consecutive ids; the k ranges of a tile sit next to each
-  // other, and tiles go down four tile rows before they move to the next columns.
-  unsigned const xcd = blockIdx.x % 8, each = G.total / 8, more = G.total % 8;
-  unsigned id = xcd * each + (xcd < more ? xcd : more) + blockIdx.x / 8;
-  int const split = (int)(id % (unsigned)G.ksplit);
-  id /= (unsigned)G.ksplit;
-  int const batch = (int)(id / (unsigned)G.tiles_per_batch), t0 = (int)(id % (unsigned)G.tiles_per_batch);
-  int const per_group = 4 * G.tiles_n, first_m = 4 * (t0 / per_group);
-  int const gsz = (G.tiles_m - first_m) < 4 ? (G.tiles_m - first_m) : 4;
-  int const row0 = (first_m + (t0 % per_group) % gsz) * BM, col0 = (t0 % per_group) / gsz * BN;
+  int split, batch, row0, col0;
+  gemm_tile(G, BM, BN, split, batch, row0, col0);
 
   SA sa;
   SB sb;
@@ -347,81 +435,8 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG) void f16_gemm_any_
       }
     }
   }
-  // acc[i][j][e] = C[wm0 + 16 i + lane % 16][wn0 + 16 j + 4 (lane / 16) + e]
-  int const g = lane / 16, c = lane % 16;
-  if (G.ksplit > 1) {
-    if (kg == 0) {
-      int const batches = (int)(G.total / (unsigned)(G.ksplit * G.tiles_per_batch));
-      float *const P = G.partial + ((size_t)split * batches + batch) * (size_t)G.m * G.n;
-#pragma unroll
-      for (int i = 0; i < TM; i++) {
-        int const row = row0 + wm0 + 16 * i + c;
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-          int const col = col0 + wn0 + 16 * j + 4 * g;
-          if (row < G.m && col + 4 <= G.n) {
-            *reinterpret_cast<float4_any *>(P + (size_t)row * G.n + col) = acc[i][j];
-          } else if (row < G.m) {
-#pragma unroll
-            for (int e = 0; e < 3; e++) {
-              if (col + e < G.n) {
-                P[(size_t)row * G.n + col + e] = acc[i][j][e];
-              }
-            }
-          }
-        }
-      }
-    }
-    return;
-  }
-  // ---- out through LDS: rows of 16-byte chunks
-  constexpr int LDC = BN + 8;
-  _Float16 *const tile = reinterpret_cast<_Float16 *>(lds) + (KG - 1) * TM * TN * NTG * 8;
-  if (kg == 0) {
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-#pragma unroll
-      for (int j = 0; j < TN; j++) {
-        *reinterpret_cast<half4 *>(tile + (wm0 + 16 * i + c) * LDC + wn0 + 16 * j + 4 * g) =
-            __builtin_convertvector(acc[i][j], half4);
-      }
-    }
-  }
-  __syncthreads();
-  size_t const matrix = (size_t)batch * G.m * G.n;
-  for (int e = threadIdx.x; e < BM * (BN / 8); e += NT) {
-    int const r = e / (BN / 8), c8 = 8 * (e % (BN / 8)), row = row0 + r, col = col0 + c8;
-    if (row < G.m && col < G.n) {
-      half8 const v = *reinterpret_cast<half8 const *>(tile + r * LDC + c8);
-      size_t const at = matrix + (size_t)row * G.n + col;
-      if (col + 8 <= G.n) {
-        *reinterpret_cast<half8_any *>(G.C + at) = v;
-        if (G.epilogue != EPI_NONE) {
-          half8 x = v;
-          if (G.epilogue >= EPI_ADD) {
-            x = *reinterpret_cast<half8_any const *>(G.X + at);
-          }
-          half8 y;
-#pragma unroll
-          for (int u = 0; u < 8; u++) {
-            y[u] = static_cast<_Float16>(epilogue_value(G.epilogue, static_cast<float>(v[u]), static_cast<float>(x[u])));
-          }
-          *reinterpret_cast<half8_any *>(G.E + at) = y;
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < 7; u++) {
-          if (col + u < G.n) {
-            G.C[at + u] = v[u];
-            if (G.epilogue != EPI_NONE) {
-              float const x = G.epilogue >= EPI_ADD ? static_cast<float>(G.X[at + u]) : 0.0f;
-              G.E[at + u] = static_cast<_Float16>(epilogue_value(G.epilogue, static_cast<float>(v[u]), x));
-            }
-          }
-        }
-      }
-    }
-  }
+  gemm_store<BM, BN, TM, TN, NT>(G, acc, reinterpret_cast<_Float16 *>(lds) + (KG - 1) * TM * TN * NTG * 8, kg == 0, lane, split, batch,
+                                 row0, col0, wm0, wn0);
 }
 
 template <int BM, int BN, int WM, int WN, int KG, bool A_KC, bool B_KC>
@@ -430,6 +445,402 @@ constexpr int any_gemm_lds() {
   constexpr int stages = KG * 2 * (OperandStage<BM, NTG, A_KC>::HALFS + OperandStage<BN, NTG, B_KC>::HALFS) * 2;
   constexpr int out = (KG - 1) * (WM / 16) * (WN / 16) * NTG * 16 + BM * (BN + 8) * 2;
   return stages > out ? stages : out;
+}
+
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ uint32_t gemm_lds_address(void const *p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void const *)p;
+}
+__device__ __forceinline__ void gemm_dma16(_Float16 const *gbase, uint32_t lane_byte_offset, uint32_t lds_wave_base) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(lds_wave_base)), "v"(lane_byte_offset), "s"(gbase)
+               : "m0", "memory");
+}
+template <int N>
+__device__ __forceinline__ void gemm_wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
+#pragma clang diagnostic pop
+
+// Products whose rows are whole 16-byte chunks and whose k is whole stages of 64: f16_gemm_any_kernel's
+// tiles and k ranges, but a stage goes to LDS directly (global_load_lds_dwordx4), without the registers and
+// the LDS stores of the way through them; a ring of three stages, two in flight.  A direct load writes its
+// 64 chunks in lane order, so the LDS rows are not padded: chunk q of row r sits at position q ^ (r / 2 % 8)
+// where k is contiguous, at q ^ 2 (r % 8) (64 columns: ^ 2 (r / 2 % 4)) where a row is one k; both spread an
+// operand read over all banks.
+//
+// What bounds it: the 35 bytes a cycle that a compute unit gets from its caches (64 x 64 x 64: 470 cycles,
+// of matrix instructions 128), whatever the number of stages in flight; so a wide tile where there are
+// tiles enough.  f16_gemm_any_kernel and here: [300, 2048] . [2048, 5504] row-major 20.1 and 16.2 us,
+// [1024, 2048] . [2048, 5504] 39.6 and 35.4, [2048, 2048] . [2048, 2048] 28.9 and 24.4 (704 TFLOP/s).
+template <int R, int NT, bool KC>
+struct DirectStage {
+  static constexpr int BK = 64, CH = R * BK / 8 / NT, LD = KC ? BK : R, HALFS = R * BK;
+  static_assert(R * BK / 8 % NT == 0, "a stage splits evenly over the threads");
+  _Float16 const *base;
+  size_t step;       // elements from a stage to the next
+  uint32_t off[CH];  // bytes from the stage's first element
+
+  __device__ __forceinline__ static int turned(int r, int q) { return KC ? q ^ (r / 2 % 8) : R == 64 ? q ^ (2 * (r / 2 % 4)) : q ^ (2 * (r % 8)); }
+
+  // (rows and chunks past the matrix re-read its last ones)
+  __device__ __forceinline__ void init(_Float16 const *matrix, int rows, int row0, int k, int tid) {
+    base = matrix + (KC ? (size_t)row0 * k : (size_t)row0);
+    step = KC ? (size_t)BK : (size_t)BK * rows;
+#pragma unroll
+    for (int i = 0; i < CH; i++) {
+      int const p = i * NT + tid;
+      if (KC) {
+        int const r = p / 8, rr = row0 + r < rows ? r : rows - 1 - row0;
+        off[i] = 2u * (uint32_t)(rr * k + 8 * turned(r, p % 8));
+      } else {
+        int const r = p / (R / 8), q = 8 * turned(r, p % (R / 8));
+        off[i] = 2u * (uint32_t)(r * rows + (row0 + q + 8 <= rows ? q : rows - 8 - row0));
+      }
+    }
+  }
+  __device__ __forceinline__ void issue(int stage, uint32_t lds, int wave) const {
+    _Float16 const *const p = base + (size_t)stage * step;
+#pragma unroll
+    for (int i = 0; i < CH; i++) {
+      gemm_dma16(p, off[i], lds + 16u * (uint32_t)(i * NT + wave * 64));
+    }
+  }
+  // operand of rows r0 .. r0 + 15, k step s of 32: lane (g, c) holds [r0 + c][32 s + 8 g .. + 7]
+  __device__ __forceinline__ static half8 operand(_Float16 const *tile, int r0, int s, int lane) {
+    int const g = lane / 16, c = lane % 16;
+    if (KC) {
+      return *reinterpret_cast<half8 const *>(tile + (r0 + c) * LD + 8 * turned(r0 + c, 4 * s + g));
+    }
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    typedef short4v __attribute__((address_space(3))) *lds_p;
+    int const r = 32 * s + 8 * g + (c >> 2), q = r0 / 8 + ((c & 3) >> 1), in = 4 * (c & 1);
+    _Float16 const *const p = tile + r * LD + 8 * turned(r, q) + in, *const p4 = tile + (r + 4) * LD + 8 * turned(r + 4, q) + in;
+    half4 const lo = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                   (lds_p)(__attribute__((address_space(3))) void *)p));
+    half4 const hi = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                   (lds_p)(__attribute__((address_space(3))) void *)p4));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+};
+
+constexpr int kDirectRing = 3;
+
+template <int BM, int BN, int WM, int WN, bool B_KC>
+__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void f16_gemm_direct_kernel(AnyGemm const G) {
+  constexpr int NT = 64 * (BM / WM) * (BN / WN), TM = WM / 16, TN = WN / 16;
+  using SA = DirectStage<BM, NT, true>;
+  using SB = DirectStage<BN, NT, B_KC>;
+  constexpr int STAGE = SA::HALFS + SB::HALFS, LPS = SA::CH + SB::CH;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  _Float16 *const ring = reinterpret_cast<_Float16 *>(lds);
+  int const tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+
+  int split, batch, row0, col0;
+  gemm_tile(G, BM, BN, split, batch, row0, col0);
+  SA sa;
+  SB sb;
+  sa.init(G.A + (size_t)batch * G.m * G.k, G.m, row0, G.k, tid);
+  sb.init(G.B + (size_t)batch * G.k * G.n, G.n, col0, G.k, tid);
+  int const whole = G.k / 64, first = split * G.steps_per_range < whole ? split * G.steps_per_range : whole;
+  int const T = (whole - first) < G.steps_per_range ? (whole - first) : G.steps_per_range;
+  int const wm0 = (wave / (BN / WN)) * WM, wn0 = (wave % (BN / WN)) * WN;
+
+  float4v acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  }
+  uint32_t const ring_at = gemm_lds_address(ring);
+  auto issue = [&](int t, int slot) {
+    uint32_t const at = ring_at + 2u * (uint32_t)(slot * STAGE);
+    sa.issue(first + t, at, wave);
+    sb.issue(first + t, at + 2u * (uint32_t)SA::HALFS, wave);
+  };
+  struct Operands {
+    half8 a[TM], b[TN];
+  };
+  auto read = [&](Operands &x, int slot, int s) {
+    _Float16 const *const buf = ring + slot * STAGE;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      x.a[i] = SA::operand(buf, wm0 + 16 * i, s, lane);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      x.b[j] = SB::operand(buf + SA::HALFS, wn0 + 16 * j, s, lane);
+    }
+  };
+  auto multiply = [&](Operands const &x) {
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.b[j], x.a[i], acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  // stage t has landed (this wavefront's share) when at most stage t + 1 is outstanding
+  auto landed = [&](int t) {
+    if (t + 1 < T) {
+      gemm_wait_vm<LPS>();
+    } else {
+      gemm_wait_vm<0>();
+    }
+  };
+  // Skewed by half a stage: every batch of operand reads is followed by the multiplications of the batch
+  // before it.
+  if (T > 0) {
+    issue(0, 0);
+    if (T > 1) {
+      issue(1, 1);
+    }
+    landed(0);
+    __syncthreads();
+    if (T > 2) {
+      issue(2, 2);
+    }
+    Operands x0, x1;
+    read(x0, 0, 0);
+    for (int t = 0, slot = 0; t < T; t++) {
+      int const next = slot + 1 < kDirectRing ? slot + 1 : 0;
+      read(x1, slot, 1);
+      multiply(x0);
+      if (t + 1 < T) {
+        landed(t + 1);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wavefront's reads of stage t are in registers
+        __syncthreads();                                    // stage t + 1 is there, stage t is free
+        if (t + 3 < T) {
+          issue(t + 3, slot);
+        }
+        read(x0, next, 0);
+      }
+      multiply(x1);
+      slot = next;
+    }
+    __syncthreads();
+  }
+  gemm_store<BM, BN, TM, TN, NT>(G, acc, ring, true, lane, split, batch, row0, col0, wm0, wn0);
+}
+
+template <int BM, int BN>
+constexpr int direct_gemm_lds() {
+  constexpr int ring = kDirectRing * (BM + BN) * 128, out = BM * (BN + 8) * 2;
+  return ring > out ? ring : out;
+}
+
+// Products whose rows are whole 16-byte chunks and whose k is whole steps of 32.  A workgroup's tile is as
+// before, but each of its four wavefronts has ALL of the tile and every fourth step of k: an element of an
+// operand then leaves LDS once per workgroup rather than once per wavefront that shares its row, and a
+// wavefront needs no barrier until the four sums are added up.  A step goes to the wavefront's own ring in
+// LDS by direct loads (global_load_lds_dwordx4), RING - 1 of them in flight while one is multiplied from
+// registers.  A direct load writes its 64 chunks in lane order, so LDS rows are not padded: chunk q of row r
+// sits at position q ^ (r / 4 % 4) where k is contiguous, at q ^ 2 (r % 8) (64 columns: ^ 2 (r / 2 % 4))
+// where a row is one k; both spread an operand read over all banks.
+//
+// What bounds it: as above; the operand reads and barriers it saves count where the tile is small and the
+// steps of a workgroup are a chain: 0.14 us for 64 k of a 16 x 64 tile (f16_gemm_any_kernel: 0.24).
+// [16, 2048] . [2048, 5504] 10.2 -> 7.5 us, [96, 512] . [512, 1024] 5.5 -> 4.7, [512, 4096] . [4096, 512]
+// 13.0 -> 12.1.
+template <int R, bool KC>
+struct WaveStage {
+  static constexpr int BK = 32, CH = R * BK / 8 / 64, LD = KC ? BK : R, HALFS = R * BK;
+  _Float16 const *base;
+  size_t step;       // elements from a step of k to the next
+  uint32_t off[CH];  // bytes from the step's first element
+
+  __device__ __forceinline__ static int turned(int r, int q) { return KC ? q ^ (r / 4 % 4) : R == 64 ? q ^ (2 * (r / 2 % 4)) : q ^ (2 * (r % 8)); }
+
+  // (rows and chunks past the matrix re-read its last ones)
+  __device__ __forceinline__ void init(_Float16 const *matrix, int rows, int row0, int k, int lane) {
+    base = matrix + (KC ? (size_t)row0 * k : (size_t)row0);
+    step = KC ? (size_t)BK : (size_t)BK * rows;
+#pragma unroll
+    for (int i = 0; i < CH; i++) {
+      int const p = i * 64 + lane;
+      if (KC) {
+        int const r = p / 4, rr = row0 + r < rows ? r : rows - 1 - row0;
+        off[i] = 2u * (uint32_t)(rr * k + 8 * turned(r, p % 4));
+      } else {
+        int const r = p / (R / 8), q = 8 * turned(r, p % (R / 8));
+        off[i] = 2u * (uint32_t)(r * rows + (row0 + q + 8 <= rows ? q : rows - 8 - row0));
+      }
+    }
+  }
+  __device__ __forceinline__ void issue(int t, uint32_t lds) const {
+    _Float16 const *const p = base + (size_t)t * step;
+#pragma unroll
+    for (int i = 0; i < CH; i++) {
+      gemm_dma16(p, off[i], lds + 1024u * (uint32_t)i);
+    }
+  }
+  // operand of rows r0 .. r0 + 15: lane (g, c) holds [r0 + c][8 g .. + 7]
+  __device__ __forceinline__ static half8 operand(_Float16 const *tile, int r0, int lane) {
+    int const g = lane / 16, c = lane % 16;
+    if (KC) {
+      return *reinterpret_cast<half8 const *>(tile + (r0 + c) * LD + 8 * turned(r0 + c, g));
+    }
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    typedef short4v __attribute__((address_space(3))) *lds_p;
+    int const r = 8 * g + (c >> 2), q = r0 / 8 + ((c & 3) >> 1), in = 4 * (c & 1);
+    _Float16 const *const p = tile + r * LD + 8 * turned(r, q) + in, *const p4 = tile + (r + 4) * LD + 8 * turned(r + 4, q) + in;
+    half4 const lo = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                   (lds_p)(__attribute__((address_space(3))) void *)p));
+    half4 const hi = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                   (lds_p)(__attribute__((address_space(3))) void *)p4));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+};
+
+template <int BM, int BN, int RING, bool B_KC>
+__global__ __launch_bounds__(256) void f16_gemm_waves_kernel(AnyGemm const G) {
+  constexpr int TM = BM / 16, TN = BN / 16, TQ = TN / 4;
+  using SA = WaveStage<BM, true>;
+  using SB = WaveStage<BN, B_KC>;
+  constexpr int STEP = SA::HALFS + SB::HALFS, LPS = SA::CH + SB::CH;
+  static_assert(RING >= 3 && RING <= 4 && (RING - 1) * LPS < 64, "waits for two or three steps");
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  int const lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  _Float16 *const ring = reinterpret_cast<_Float16 *>(lds) + wave * RING * STEP;
+
+  int split, batch, row0, col0;
+  gemm_tile(G, BM, BN, split, batch, row0, col0);
+  SA sa;
+  SB sb;
+  sa.init(G.A + (size_t)batch * G.m * G.k, G.m, row0, G.k, lane);
+  sb.init(G.B + (size_t)batch * G.k * G.n, G.n, col0, G.k, lane);
+  // this range's steps [first, last); the wavefront's are first + wave, + 4, ..
+  int const all = G.k / 32, first = split * G.steps_per_range < all ? split * G.steps_per_range : all;
+  int const last = all - first < G.steps_per_range ? all : first + G.steps_per_range;
+  int const T = (last - first - wave + 3) / 4;
+
+  float4v acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  }
+  uint32_t const ring_at = gemm_lds_address(ring);
+  auto issue = [&](int t, int slot) {
+    uint32_t const at = ring_at + 2u * (uint32_t)(slot * STEP);
+    sa.issue(first + wave + 4 * t, at);
+    sb.issue(first + wave + 4 * t, at + 2u * (uint32_t)SA::HALFS);
+  };
+  struct Operands {
+    half8 a[TM], b[TN];
+  };
+  auto read = [&](Operands &x, int slot) {
+    _Float16 const *const buf = ring + slot * STEP;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      x.a[i] = SA::operand(buf, 16 * i, lane);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      x.b[j] = SB::operand(buf + SA::HALFS, 16 * j, lane);
+    }
+  };
+  auto multiply = [&](Operands const &x) {
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.b[j], x.a[i], acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  // step t has landed when at most the RING - 1 steps after it are outstanding
+  auto landed = [&](int t) {
+    int const later = T - 1 - t;
+    if (later >= RING - 1) {
+      gemm_wait_vm<(RING - 1) * LPS>();
+    } else if (RING > 3 && later >= 2) {
+      gemm_wait_vm<2 * LPS>();
+    } else if (later >= 1) {
+      gemm_wait_vm<LPS>();
+    } else {
+      gemm_wait_vm<0>();
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < RING; t++) {
+    if (t < T) {
+      issue(t, t);
+    }
+  }
+  // one step: its operands are in registers; the next one's are read and its slot filled again
+  int slot = 0;
+  auto advance = [&](Operands &next, Operands const &now, int t) {
+    slot = slot + 1 < RING ? slot + 1 : 0;
+    if (t + 1 < T) {
+      landed(t + 1);
+      read(next, slot);
+    }
+    multiply(now);
+    if (t + 1 + RING < T) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the reads have left the slot)
+      issue(t + 1 + RING, slot);
+    }
+  };
+  if (T > 0) {
+    Operands x0, x1;
+    landed(0);
+    read(x0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (RING < T) {
+      issue(RING, 0);
+    }
+    for (int t = 0; t < T; t += 2) {
+      advance(x1, x0, t);
+      if (t + 1 < T) {
+        advance(x0, x1, t + 1);
+      }
+    }
+  }
+  // ---- the wavefronts' sums, in wavefront order: each adds up a quarter of the columns
+  float4v *const sums = reinterpret_cast<float4v *>(lds);  // [4 wavefronts][TM][TN][64]
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      sums[((wave * TM + i) * TN + j) * 64 + lane] = acc[i][j];
+    }
+  }
+  __syncthreads();
+  float4v quarter[TM][TQ];
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+#pragma unroll
+    for (int j = 0; j < TQ; j++) {
+      float4v v = sums[(i * TN + wave * TQ + j) * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < 4; w++) {
+        float4v const x = sums[((w * TM + i) * TN + wave * TQ + j) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          v[e] += x[e];
+        }
+      }
+      quarter[i][j] = v;
+    }
+  }
+  __syncthreads();
+  gemm_store<BM, BN, TM, TQ, 256>(G, quarter, reinterpret_cast<_Float16 *>(lds), true, lane, split, batch, row0, col0, 0,
+                                  wave * TQ * 16);
+}
+
+template <int BM, int BN, int RING>
+constexpr int waves_gemm_lds() {
+  constexpr int ring = 4 * RING * (BM + BN) * 64, sums = 4 * BM * BN * 4;
+  return ring > sums ? ring : sums;
 }
 
 }  // namespace mi355

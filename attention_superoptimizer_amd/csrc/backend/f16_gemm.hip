@@ -6,6 +6,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 namespace mi355 {
@@ -101,23 +102,6 @@ __global__ __launch_bounds__(kThreads) void f16_matmul_kernel(_Float16 const *__
 //    clamped on load and masked on store (m and n are arbitrary, k a multiple of 32);
 //  * workgroup ids are renumbered so that an XCD (whose 32 compute units share one L2) works on
 //    a compact block of tiles: 4 tile rows deep, walked column by column.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ uint32_t gemm_lds_address(void const *p) {
-  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void const *)p;
-}
-__device__ __forceinline__ void gemm_dma16(_Float16 const *gbase, uint32_t lane_byte_offset, uint32_t lds_wave_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane(lds_wave_base)), "v"(lane_byte_offset), "s"(gbase)
-               : "m0", "memory");
-}
-template <int N>
-__device__ __forceinline__ void gemm_wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
-}
-#pragma clang diagnostic pop
-
 struct GemmArgs {
   _Float16 const *A, *Bt;  // [batch][m][k], [batch][n][k]
   _Float16 *C;             // [batch][m][n]
@@ -393,14 +377,25 @@ static int launch_gemm_nt(GemmArgs &G, int batch) {
 // ---- f16_gemm_any_kernel: instantiations and the choice between them -------------------------
 namespace {
 
+// f16_gemm_any_kernel, f16_gemm_direct_kernel, f16_gemm_waves_kernel
+enum TileKind { STAGED, DIRECT, WAVES };
 struct AnyTile {
   int bm, bn, wm, wn, kg, lds;
+  TileKind kind;
   void (*fn)(AnyGemm);
   int threads() const { return 64 * (bm / wm) * (bn / wn) * kg; }
 };
 template <int BM, int BN, int WM, int WN, int KG, bool A_KC, bool B_KC>
 AnyTile any_tile() {
-  return {BM, BN, WM, WN, KG, any_gemm_lds<BM, BN, WM, WN, KG, A_KC, B_KC>(), f16_gemm_any_kernel<BM, BN, WM, WN, KG, A_KC, B_KC>};
+  return {BM, BN, WM, WN, KG, any_gemm_lds<BM, BN, WM, WN, KG, A_KC, B_KC>(), STAGED, f16_gemm_any_kernel<BM, BN, WM, WN, KG, A_KC, B_KC>};
+}
+template <int BM, int BN, int WM, int WN, bool B_KC>
+AnyTile direct_tile() {
+  return {BM, BN, WM, WN, 1, direct_gemm_lds<BM, BN>(), DIRECT, f16_gemm_direct_kernel<BM, BN, WM, WN, B_KC>};
+}
+template <int BM, int BN, int RING, bool B_KC>
+AnyTile waves_tile() {
+  return {BM, BN, BM, BN, 4, waves_gemm_lds<BM, BN, RING>(), WAVES, f16_gemm_waves_kernel<BM, BN, RING, B_KC>};
 }
 // [A k-contiguous][B k-contiguous]; a column-major A is rare (a layout search may ask for one), so
 // it gets the middle tiles only
@@ -410,7 +405,9 @@ std::vector<AnyTile> any_tiles_row_major_a() {
           any_tile<32, 64, 32, 16, 1, true, B_KC>(),  any_tile<32, 64, 32, 16, 2, true, B_KC>(),
           any_tile<64, 64, 32, 32, 1, true, B_KC>(),  any_tile<64, 64, 32, 32, 2, true, B_KC>(),
           any_tile<64, 128, 32, 64, 1, true, B_KC>(), any_tile<64, 128, 32, 64, 2, true, B_KC>(),
-          any_tile<128, 128, 64, 64, 1, true, B_KC>()};
+          any_tile<128, 128, 64, 64, 1, true, B_KC>(), direct_tile<64, 64, 32, 32, B_KC>(),
+          direct_tile<64, 128, 32, 64, B_KC>(),        direct_tile<128, 64, 64, 32, B_KC>(),
+          waves_tile<16, 64, 4, B_KC>(),               waves_tile<32, 64, 4, B_KC>()};
 }
 std::vector<AnyTile> const &any_tiles(bool a_kc, bool b_kc) {
   static std::vector<AnyTile> const row[2] = {any_tiles_row_major_a<false>(), any_tiles_row_major_a<true>()};
@@ -425,7 +422,18 @@ std::vector<AnyTile> const &any_tiles(bool a_kc, bool b_kc) {
 // average).  A launch, then either the latency of its k stages one after another (0.24 us each) or,
 // with the compute units full, what they have to move: 128-byte rows through the vector cache, into
 // LDS and from there to the operands, and the matrix instructions.  k ranges need a second launch.
+// (The kernels that load LDS directly: 3.2 us, and 35 bytes a cycle per compute unit; a lone workgroup
+// waits 1.4 times as long for a stage, but not where wavefronts go their own ways.  15 shapes, within 15 %.)
 double any_gemm_cost(AnyTile const &t, int batch, int m, int n, int k, int ksplit) {
+  if (t.kind != STAGED) {
+    double const stages = (k / 32 + 2 * ksplit - 1) / (2 * ksplit), stage = (t.bm + t.bn) * 128.0 / 35.0 / 2400.0;
+    double per_cu = (double)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch * ksplit / 256.0;
+    if (t.kind == WAVES || per_cu < 3.0) {
+      per_cu = std::ceil(per_cu);  // (the compute unit with the most workgroups is the last to finish)
+    }
+    double const us = 3.2 + stages * stage * std::max(per_cu, t.kind == DIRECT ? 1.4 : 1.0) + per_cu * 0.9e-4 * t.bm * t.bn;
+    return us + (ksplit > 1 ? 2.0 + 0.3 * ksplit + 1.4e-6 * batch * (double)m * n * ksplit : 0.0);
+  }
   int const stages = (k / 64 + ksplit * t.kg - 1) / (ksplit * t.kg) + (k % 64 != 0 ? 1 : 0);
   double const tiles = (double)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch * ksplit;
   double const rows = 3.0 * (t.bm + t.bn) + (t.bm / t.wm) * (t.bn / t.wn) * (t.wm + t.wn);
@@ -446,10 +454,15 @@ int launch_gemm_any(AnyGemm &G, int batch, bool a_kc, bool b_kc) {
   double least = 0.0;
   int ksplit = 1;
   size_t const range_bytes = (size_t)batch * G.m * G.n * sizeof(float);
+  bool const chunks = a_kc && (b_kc || G.n % 8 == 0) &&
+                      ((reinterpret_cast<uintptr_t>(G.A) | reinterpret_cast<uintptr_t>(G.B)) & 15) == 0;
   for (AnyTile const &t : any_tiles(a_kc, b_kc)) {
+    if (t.kind != STAGED && (!chunks || G.k % (t.kind == DIRECT ? 64 : 32) != 0)) {
+      continue;
+    }
     for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
       // (a range is a stage per group at least, and the ranges' sums fit this queue's scratch)
-      if (s > 1 && (G.k / 64 < s * t.kg || state().scratch() == nullptr || range_bytes * s > state().scratch_bytes)) {
+      if (s > 1 && (G.k / 64 < s * (t.kind == WAVES ? 1 : t.kg) || state().scratch() == nullptr || range_bytes * s > state().scratch_bytes)) {
         break;
       }
       double const us = any_gemm_cost(t, batch, G.m, G.n, G.k, s);
@@ -464,7 +477,8 @@ int launch_gemm_any(AnyGemm &G, int batch, bool a_kc, bool b_kc) {
   G.tiles_n = (G.n + best->bn - 1) / best->bn;
   G.tiles_per_batch = G.tiles_m * G.tiles_n;
   G.ksplit = ksplit;
-  G.steps_per_range = (G.k / 64 + ksplit * best->kg - 1) / (ksplit * best->kg);
+  G.steps_per_range = best->kind == WAVES ? (G.k / 32 + ksplit - 1) / ksplit
+                                          : (G.k / 64 + ksplit * best->kg - 1) / (ksplit * best->kg);
   G.partial = static_cast<float *>(state().scratch());
   long long const total = (long long)G.tiles_per_batch * batch * ksplit;
   if (total > 2147483647LL) {
