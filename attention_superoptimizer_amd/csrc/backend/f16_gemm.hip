@@ -4,10 +4,11 @@
 // straight into LDS, f16_matmul_kernel takes rows of fewer than eight elements.
 #include "f16_gemm.h"
 #include "common.h"
+#include "f16_gemm_choice.h"
 
 #include <algorithm>
-#include <cmath>
-#include <vector>
+#include <array>
+#include <utility>
 
 namespace mi355 {
 
@@ -272,14 +273,13 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void f16_gemm_nt_kernel
   __builtin_amdgcn_wave_barrier();
   _Float16 *const Cb = G.C + (size_t)batch * G.m * G.n;
   constexpr int CPR = WN / 8;  // 16-byte chunks per row of the piece
-  bool const vec = G.n % 8 == 0;
   for (int e = lane; e < WM * CPR; e += 64) {
     int const r = e / CPR, c8 = (e % CPR) * 8;
     int const row = row0 + wm0 + r, col = col0 + wn0 + c8;
     if (row < G.m && col < G.n) {
       half8 const v = *reinterpret_cast<half8 const *>(piece + r * LDW + c8);
-      if (vec && col + 8 <= G.n) {
-        *reinterpret_cast<half8 *>(Cb + (size_t)row * G.n + col) = v;
+      if (col + 8 <= G.n) {
+        *reinterpret_cast<half8_any *>(Cb + (size_t)row * G.n + col) = v;
       } else {
         for (int x = 0; x < 8 && col + x < G.n; x++) {
           Cb[(size_t)row * G.n + col + x] = v[x];
@@ -374,120 +374,60 @@ static int launch_gemm_nt(GemmArgs &G, int batch) {
   return MI355_OK;
 }
 
-// ---- f16_gemm_any_kernel: instantiations and the choice between them -------------------------
+// ---- the tiles of f16_gemm_choice.h: instantiations and launches ----------------------------------
 namespace {
 
-// f16_gemm_any_kernel, f16_gemm_direct_kernel, f16_gemm_waves_kernel
-enum TileKind { STAGED, DIRECT, WAVES };
-struct AnyTile {
-  int bm, bn, wm, wn, kg, lds;
-  TileKind kind;
+struct TileKernel {
   void (*fn)(AnyGemm);
-  int threads() const { return 64 * (bm / wm) * (bn / wn) * kg; }
+  int lds;
 };
-template <int BM, int BN, int WM, int WN, int KG, bool A_KC, bool B_KC>
-AnyTile any_tile() {
-  return {BM, BN, WM, WN, KG, any_gemm_lds<BM, BN, WM, WN, KG, A_KC, B_KC>(), STAGED, f16_gemm_any_kernel<BM, BN, WM, WN, KG, A_KC, B_KC>};
+template <bool A_KC, int I>
+constexpr GemmTile kTile = kGemmTiles[I];
+template <int I>
+constexpr GemmTile kTile<false, I> = kGemmTilesColumnMajorA[I];
+
+template <int I, bool A_KC, bool B_KC>
+constexpr TileKernel tile_kernel() {
+  constexpr GemmTile t = kTile<A_KC, I>;
+  if constexpr (t.kind == STAGED) {
+    return {f16_gemm_any_kernel<t.bm, t.bn, t.wm, t.wn, t.kg, A_KC, B_KC>, any_gemm_lds<t.bm, t.bn, t.wm, t.wn, t.kg, A_KC, B_KC>()};
+  } else if constexpr (t.kind == DIRECT) {
+    return {f16_gemm_direct_kernel<t.bm, t.bn, t.wm, t.wn, B_KC>, direct_gemm_lds<t.bm, t.bn>()};
+  } else {
+    return {f16_gemm_waves_kernel<t.bm, t.bn, kWavesRing, B_KC>, waves_gemm_lds<t.bm, t.bn, kWavesRing>()};
+  }
 }
-template <int BM, int BN, int WM, int WN, bool B_KC>
-AnyTile direct_tile() {
-  return {BM, BN, WM, WN, 1, direct_gemm_lds<BM, BN>(), DIRECT, f16_gemm_direct_kernel<BM, BN, WM, WN, B_KC>};
+template <bool A_KC, bool B_KC, size_t... I>
+TileKernel tile_kernel_at(int i, std::index_sequence<I...>) {
+  static constexpr std::array<TileKernel, sizeof...(I)> all = {tile_kernel<(int)I, A_KC, B_KC>()...};
+  return all[i];
 }
-template <int BM, int BN, int RING, bool B_KC>
-AnyTile waves_tile() {
-  return {BM, BN, BM, BN, 4, waves_gemm_lds<BM, BN, RING>(), WAVES, f16_gemm_waves_kernel<BM, BN, RING, B_KC>};
-}
-// [A k-contiguous][B k-contiguous]; a column-major A is rare (a layout search may ask for one), so
-// it gets the middle tiles only
-template <bool B_KC>
-std::vector<AnyTile> any_tiles_row_major_a() {
-  return {any_tile<16, 64, 16, 16, 1, true, B_KC>(),  any_tile<16, 64, 16, 16, 2, true, B_KC>(),
-          any_tile<32, 64, 32, 16, 1, true, B_KC>(),  any_tile<32, 64, 32, 16, 2, true, B_KC>(),
-          any_tile<64, 64, 32, 32, 1, true, B_KC>(),  any_tile<64, 64, 32, 32, 2, true, B_KC>(),
-          any_tile<64, 128, 32, 64, 1, true, B_KC>(), any_tile<64, 128, 32, 64, 2, true, B_KC>(),
-          any_tile<128, 128, 64, 64, 1, true, B_KC>(), direct_tile<64, 64, 32, 32, B_KC>(),
-          direct_tile<64, 128, 32, 64, B_KC>(),        direct_tile<128, 64, 64, 32, B_KC>(),
-          waves_tile<16, 64, 4, B_KC>(),               waves_tile<32, 64, 4, B_KC>()};
-}
-std::vector<AnyTile> const &any_tiles(bool a_kc, bool b_kc) {
-  static std::vector<AnyTile> const row[2] = {any_tiles_row_major_a<false>(), any_tiles_row_major_a<true>()};
-  static std::vector<AnyTile> const col[2] = {
-      {any_tile<64, 64, 32, 32, 1, false, false>(), any_tile<64, 64, 32, 32, 2, false, false>()},
-      {any_tile<64, 64, 32, 32, 1, false, true>(), any_tile<64, 64, 32, 32, 2, false, true>()}};
-  return (a_kc ? row : col)[b_kc ? 1 : 0];
+TileKernel tile_kernel_of(int i, bool a_kc, bool b_kc) {
+  using Row = std::make_index_sequence<sizeof(kGemmTiles) / sizeof(GemmTile)>;
+  using Col = std::make_index_sequence<sizeof(kGemmTilesColumnMajorA) / sizeof(GemmTile)>;
+  if (a_kc) {
+    return b_kc ? tile_kernel_at<true, true>(i, Row{}) : tile_kernel_at<true, false>(i, Row{});
+  }
+  return b_kc ? tile_kernel_at<false, true>(i, Col{}) : tile_kernel_at<false, false>(i, Col{});
 }
 
-// Microseconds a tile shape is expected to take: a line fitted to 27,000 timed launches (114 shapes,
-// m from 1 to 2048, n and k from 64 to 5504; the choice it makes is 2.6 % above the best on
-// average).  A launch, then either the latency of its k stages one after another (0.24 us each) or,
-// with the compute units full, what they have to move: 128-byte rows through the vector cache, into
-// LDS and from there to the operands, and the matrix instructions.  k ranges need a second launch.
-// (The kernels that load LDS directly: 3.2 us, and 35 bytes a cycle per compute unit; a lone workgroup
-// waits 1.4 times as long for a stage, but not where wavefronts go their own ways.  15 shapes, within 15 %.)
-double any_gemm_cost(AnyTile const &t, int batch, int m, int n, int k, int ksplit) {
-  if (t.kind != STAGED) {
-    double const stages = (k / 32 + 2 * ksplit - 1) / (2 * ksplit), stage = (t.bm + t.bn) * 128.0 / 35.0 / 2400.0;
-    double per_cu = (double)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch * ksplit / 256.0;
-    if (t.kind == WAVES || per_cu < 3.0) {
-      per_cu = std::ceil(per_cu);  // (the compute unit with the most workgroups is the last to finish)
-    }
-    double const us = 3.2 + stages * stage * std::max(per_cu, t.kind == DIRECT ? 1.4 : 1.0) + per_cu * 0.9e-4 * t.bm * t.bn;
-    return us + (ksplit > 1 ? 2.0 + 0.3 * ksplit + 1.4e-6 * batch * (double)m * n * ksplit : 0.0);
-  }
-  int const stages = (k / 64 + ksplit * t.kg - 1) / (ksplit * t.kg) + (k % 64 != 0 ? 1 : 0);
-  double const tiles = (double)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch * ksplit;
-  double const rows = 3.0 * (t.bm + t.bn) + (t.bm / t.wm) * (t.bn / t.wn) * (t.wm + t.wn);
-  double const stage = t.kg * (1.2 * rows + 0.2 * t.bm * t.bn / 32.0) / 2400.0;
-  double per_cu = tiles / 256.0;
-  if (per_cu <= 2.0) {
-    per_cu = per_cu <= 1.0 ? 1.0 : 2.0;
-  }
-  double us = 2.4 + 0.4 * (t.kg - 1) + std::max(0.24 * stages, per_cu * stages * stage) + per_cu * 0.9e-4 * t.bm * t.bn;
-  if (ksplit > 1) {
-    us += 2.0 + 0.3 * ksplit + 1.4e-6 * batch * (double)m * n * ksplit;
-  }
-  return us;
-}
-
-int launch_gemm_any(AnyGemm &G, int batch, bool a_kc, bool b_kc) {
-  AnyTile const *best = nullptr;
-  double least = 0.0;
-  int ksplit = 1;
-  size_t const range_bytes = (size_t)batch * G.m * G.n * sizeof(float);
-  bool const chunks = a_kc && (b_kc || G.n % 8 == 0) &&
-                      ((reinterpret_cast<uintptr_t>(G.A) | reinterpret_cast<uintptr_t>(G.B)) & 15) == 0;
-  for (AnyTile const &t : any_tiles(a_kc, b_kc)) {
-    if (t.kind != STAGED && (!chunks || G.k % (t.kind == DIRECT ? 64 : 32) != 0)) {
-      continue;
-    }
-    for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
-      // (a range is a stage per group at least, and the ranges' sums fit this queue's scratch)
-      if (s > 1 && (G.k / 64 < s * (t.kind == WAVES ? 1 : t.kg) || state().scratch() == nullptr || range_bytes * s > state().scratch_bytes)) {
-        break;
-      }
-      double const us = any_gemm_cost(t, batch, G.m, G.n, G.k, s);
-      if (best == nullptr || us < least) {
-        best = &t;
-        least = us;
-        ksplit = s;
-      }
-    }
-  }
-  G.tiles_m = (G.m + best->bm - 1) / best->bm;
-  G.tiles_n = (G.n + best->bn - 1) / best->bn;
+int launch_gemm_tiles(AnyGemm &G, int batch, bool a_kc, bool b_kc, GemmChoice const &choice) {
+  GemmTile const &t = (a_kc ? kGemmTiles : kGemmTilesColumnMajorA)[choice.tile];
+  TileKernel const kernel = tile_kernel_of(choice.tile, a_kc, b_kc);
+  G.tiles_m = (G.m + t.bm - 1) / t.bm;
+  G.tiles_n = (G.n + t.bn - 1) / t.bn;
   G.tiles_per_batch = G.tiles_m * G.tiles_n;
-  G.ksplit = ksplit;
-  G.steps_per_range = best->kind == WAVES ? (G.k / 32 + ksplit - 1) / ksplit
-                                          : (G.k / 64 + ksplit * best->kg - 1) / (ksplit * best->kg);
+  G.ksplit = choice.ksplit;
+  G.steps_per_range = t.kind == WAVES ? (G.k / 32 + G.ksplit - 1) / G.ksplit : (G.k / 64 + G.ksplit * t.kg - 1) / (G.ksplit * t.kg);
   G.partial = static_cast<float *>(state().scratch());
-  long long const total = (long long)G.tiles_per_batch * batch * ksplit;
+  long long const total = (long long)G.tiles_per_batch * batch * G.ksplit;
   if (total > 2147483647LL) {
     return fail(MI355_ERR_UNSUPPORTED, "matmul has too many output tiles");
   }
   G.total = (unsigned)total;
-  MI355_GRANT_LDS(best->fn, best->lds);
-  MI355_HIP(launch_kernel(best->fn, G.total, best->threads(), best->lds, state().stream(), G));
-  if (ksplit > 1) {
+  MI355_GRANT_LDS(kernel.fn, kernel.lds);
+  MI355_HIP(launch_kernel(kernel.fn, G.total, t.threads(), kernel.lds, state().stream(), G));
+  if (G.ksplit > 1) {
     size_t const n = (size_t)batch * G.m * G.n, blocks = (n / 4 + kThreads) / kThreads;
     MI355_HIP(launch_kernel(f16_gemm_fold_kernel, (unsigned)std::min<size_t>(blocks, 4096), kThreads, 0, state().stream(), G, n));
   }
@@ -510,40 +450,35 @@ int run_matmul(AnyGemm G, int batch, int a_column_major, int b_column_major, boo
   if (state().f16_matmul_route == 1 && k > 0) {  // an empty sum is zeros from the kernel below
     return vendor_gemm(G.A, G.B, G.C, batch, m, n, k, a_column_major, b_column_major);
   }
-  // 256 x 256 tiles once they alone fill the chip.  That kernel wants k contiguous in both operands,
-  // k in whole steps of 32 and 16-byte aligned rows; an operand stored the other way round is first
-  // copied transposed into this queue's plane memory (the fingerprint matmuls' workspace: work of
-  // one queue is ordered, so the two never overlap).
-  long long const big_tiles = (long long)((m + 255) / 256) * ((n + 255) / 256) * batch;
   bool const aligned = ((reinterpret_cast<uintptr_t>(G.A) | reinterpret_cast<uintptr_t>(G.B)) & 15) == 0;
-  size_t const a_bytes = a_column_major ? (size_t)batch * m * k * 2 : 0;
-  size_t const b_bytes = b_column_major ? 0 : (size_t)batch * k * n * 2;
-  size_t const a_room = (a_bytes + 255) & ~(size_t)255;
-  bool const fits = state().planes() != nullptr && a_room + b_bytes <= state().planes_bytes;
-  if (big_tiles >= 192 && k >= 256 && k % kGemmBK == 0 && aligned && fits && (size_t)std::max(m, n) * (size_t)k < ((size_t)1 << 30)) {
+  GemmChoice const choice =
+      choose_gemm({batch, m, n, k, a_column_major != 0, b_column_major != 0, aligned, state().scratch() == nullptr ? 0 : state().scratch_bytes,
+                   state().planes() == nullptr ? 0 : state().planes_bytes});
+  // Transposed copies go into this queue's plane memory (the fingerprint matmuls' workspace: work of one
+  // queue is ordered, so the two never overlap).
+  char *room = state().planes();
+  if (choice.copy_a) {  // the buffer is [k][m] per matrix
+    auto *at = reinterpret_cast<_Float16 *>(room);
+    if (int rc = launch_transpose(G.A, at, batch, k, m)) {
+      return rc;
+    }
+    G.A = at;
+    room += ((size_t)batch * m * k * 2 + 255) & ~(size_t)255;
+  }
+  if (choice.copy_b) {  // the buffer is [k][n] per matrix
+    auto *bt = reinterpret_cast<_Float16 *>(room);
+    if (int rc = launch_transpose(G.B, bt, batch, k, n)) {
+      return rc;
+    }
+    G.B = bt;
+  }
+  if (choice.route == GEMM_BIG) {
     GemmArgs N{G.A, G.B, G.C, m, n, k, 0, 0, 0, 0};
-    if (a_column_major) {  // the buffer is [k][m] per matrix
-      auto *at = reinterpret_cast<_Float16 *>(state().planes());
-      if (int rc = launch_transpose(G.A, at, batch, k, m)) {
-        return rc;
-      }
-      N.A = at;
-    }
-    if (!b_column_major) {  // the buffer is [k][n] per matrix
-      auto *bt = reinterpret_cast<_Float16 *>(state().planes() + a_room);
-      if (int rc = launch_transpose(G.B, bt, batch, k, n)) {
-        return rc;
-      }
-      N.Bt = bt;
-    }
     return launch_gemm_nt<256, 256, 128, 64>(N, batch);
   }
-  // Byte offsets inside a tile are 31-bit numbers; a contiguous direction shorter than a chunk of
-  // eight goes element by element.
-  int const a_row = a_column_major ? m : k, b_row = b_column_major ? k : n;
-  if (std::min(a_row, b_row) >= 8 && std::max(a_row, b_row) < (1 << 22)) {
+  if (choice.route == GEMM_TILES) {
     *applied = true;
-    return launch_gemm_any(G, batch, !a_column_major, b_column_major != 0);
+    return launch_gemm_tiles(G, batch, !a_column_major || choice.copy_a, b_column_major != 0, choice);
   }
   dim3 grid((n + 63) / 64, (m + 63) / 64, batch);
   MI355_HIP(launch_kernel(f16_matmul_kernel, grid, kThreads, 0, state().stream(), G.A, G.B, G.C, m, n, k, a_column_major ? 1 : k,

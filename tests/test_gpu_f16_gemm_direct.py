@@ -32,3 +32,37 @@ def test_direct_matmuls_match_float(rt, abi, batch, m, n, k, b_kc):
     Bf = B.float().transpose(1, 2).contiguous() if b_kc else B.float()
     want = torch.bmm(A.float(), Bf)
     assert (C.float() - want).abs().max().item() <= 2e-3 * want.abs().max().item()
+
+
+def _matmul(abi, A, B, batch, m, n, k, a_cm, b_cm):
+    """C on the device, between guard rows that must stay as they are; and the product in float."""
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    C = torch.full((batch * m * n + 128,), -7.0, device="cuda", dtype=torch.float16)
+    C[64:-64] = float("nan")
+    torch.cuda.synchronize()
+    assert abi.mi355_f16_matmul_layout(p(A), p(B), p(C[64:]), batch, m, n, k, a_cm, b_cm) == 0
+    assert abi.mi355_sync() == 0
+    assert (C[:64] == -7).all() and (C[-64:] == -7).all()
+    Af = A.float().transpose(1, 2).contiguous() if a_cm else A.float()
+    Bf = B.float().transpose(1, 2).contiguous() if b_cm else B.float()
+    return C[64:-64].view(batch, m, n).float(), torch.bmm(Af, Bf)
+
+
+@pytest.mark.parametrize("batch,m,n,k,a_cm,b_cm", [
+    (32, 500, 1000, 32, 0, 1),    # one step of the 256 x 256 kernel, ragged tiles
+    (1, 4090, 4096, 64, 0, 1),    # two
+    (1, 4096, 4093, 96, 0, 1),    # three, rows of C on no boundary
+    (8, 2048, 2040, 160, 0, 1),   # five: one more than its ring has slots
+    (1, 3071, 4099, 224, 0, 1),
+    (4, 2048, 2048, 128, 1, 1),   # copies of the operands stored the other way round
+    (1, 4096, 4096, 1024, 0, 0),
+    (200, 130, 130, 96, 0, 1),    # many ragged tiles, a step left over
+    (12, 1040, 1040, 128, 0, 1),
+])
+def test_products_of_many_large_tiles(rt, abi, batch, m, n, k, a_cm, b_cm):
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A = torch.randn((batch, k, m) if a_cm else (batch, m, k), device="cuda", generator=gen).half()
+    B = torch.randn((batch, n, k) if b_cm else (batch, k, n), device="cuda", generator=gen).half()
+    got, want = _matmul(abi, A, B, batch, m, n, k, a_cm, b_cm)
+    # half an fp16 place of the result, and k fp32 additions in another order
+    assert ((got - want).abs() <= 2.0 ** -11 * want.abs() + 1e-6 * k ** 0.5 * want.abs().max() + 1e-6).all()
