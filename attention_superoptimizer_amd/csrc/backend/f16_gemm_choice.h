@@ -96,14 +96,27 @@ inline double gemm_copy_cost(size_t bytes) { return 6.7 + 0.44e-6 * bytes; }
 // The kernel of least expected time among those that take the product.
 inline GemmChoice choose_gemm(GemmShape const &s) {
   GemmChoice best{GEMM_ELEMENTS, false, false, 0, 1, 0.0};
-  // Byte offsets inside a tile are 31-bit numbers; a contiguous direction shorter than a chunk of
-  // eight goes element by element.
-  int const a_row = s.a_column_major ? s.m : s.k, b_row = s.b_column_major ? s.k : s.n;
-  if (std::min(a_row, b_row) >= 8 && std::max(a_row, b_row) < (1 << 22)) {
-    bool const chunks = !s.a_column_major && (s.b_column_major || s.n % 8 == 0) && s.aligned;
+  size_t const a_bytes = s.a_column_major ? (size_t)s.batch * s.m * s.k * 2 : 0, a_room = (a_bytes + 255) & ~(size_t)255;
+  size_t const b_bytes = s.b_column_major ? 0 : (size_t)s.batch * s.k * s.n * 2;
+  // The tiles, on A as it is stored or on a copy of a column-major one: that has all the tiles, and pays
+  // where a product is large and k long: [563, 3520] . [3520, 6177] 64 us as stored, 51 with the copy,
+  // [2048, 4096] . [4096, 4096] 114 and 89, [2048, 2048] . [2048, 2048] 32 and 32, [1024, 1024] . [1024, 1024]
+  // 7.5 and 13.
+  for (bool const copy_a : {false, true}) {
+    if (copy_a && (!s.a_column_major || best.route == GEMM_ELEMENTS || a_room > s.copy_bytes)) {
+      continue;
+    }
+    bool const a_kc = !s.a_column_major || copy_a;
+    // Byte offsets inside a tile are 31-bit numbers; a contiguous direction shorter than a chunk of
+    // eight goes element by element.
+    int const a_row = a_kc ? s.k : s.m, b_row = s.b_column_major ? s.k : s.n;
+    if (std::min(a_row, b_row) < 8 || std::max(a_row, b_row) >= (1 << 22)) {
+      continue;
+    }
+    bool const chunks = a_kc && (s.b_column_major || s.n % 8 == 0) && s.aligned;
     size_t const range_bytes = (size_t)s.batch * s.m * s.n * sizeof(float);
-    GemmTile const *const tiles = s.a_column_major ? kGemmTilesColumnMajorA : kGemmTiles;
-    int const count = s.a_column_major ? (int)(sizeof(kGemmTilesColumnMajorA) / sizeof(GemmTile)) : (int)(sizeof(kGemmTiles) / sizeof(GemmTile));
+    GemmTile const *const tiles = a_kc ? kGemmTiles : kGemmTilesColumnMajorA;
+    int const count = (int)((a_kc ? sizeof(kGemmTiles) : sizeof(kGemmTilesColumnMajorA)) / sizeof(GemmTile));
     for (int i = 0; i < count; i++) {
       GemmTile const &t = tiles[i];
       if (t.kind != STAGED && (!chunks || s.k % (t.kind == DIRECT ? 64 : 32) != 0)) {
@@ -115,9 +128,9 @@ inline GemmChoice choose_gemm(GemmShape const &s) {
           break;
         }
         // (with A column-major the 64 x 64 tiles take 0.8 of the line, 560 of the products below)
-        double const us = gemm_tile_cost(t, s.batch, s.m, s.n, s.k, ranges) * (s.a_column_major ? 0.8 : 1.0);
+        double const us = gemm_tile_cost(t, s.batch, s.m, s.n, s.k, ranges) * (a_kc ? 1.0 : 0.8) + (copy_a ? gemm_copy_cost(a_bytes) : 0.0);
         if (best.route == GEMM_ELEMENTS || us < best.us) {
-          best = {GEMM_TILES, false, false, i, ranges, us};
+          best = {GEMM_TILES, copy_a, false, i, ranges, us};
         }
       }
     }
@@ -126,8 +139,6 @@ inline GemmChoice choose_gemm(GemmShape const &s) {
   // an operand stored the other way round is first copied transposed.  (Its consumer stays a launch of its
   // own: applied in the store, exp on [32, 2048, 2048] made the two 210 us instead of 209, a product by a
   // tensor 296 instead of 271.)
-  size_t const a_bytes = s.a_column_major ? (size_t)s.batch * s.m * s.k * 2 : 0, a_room = (a_bytes + 255) & ~(size_t)255;
-  size_t const b_bytes = s.b_column_major ? 0 : (size_t)s.batch * s.k * s.n * 2;
   bool const fits = a_room + b_bytes <= s.copy_bytes;
   if (s.k >= 32 && s.k % 32 == 0 && s.aligned && fits && (size_t)std::max(s.m, s.n) * (size_t)s.k < ((size_t)1 << 30)) {
     double const us = gemm_big_cost(s.batch, s.m, s.n, s.k) + (s.a_column_major ? gemm_copy_cost(a_bytes) : 0.0) +

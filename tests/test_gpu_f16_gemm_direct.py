@@ -58,6 +58,10 @@ def _matmul(abi, A, B, batch, m, n, k, a_cm, b_cm):
     (1, 4096, 4096, 1024, 0, 0),
     (200, 130, 130, 96, 0, 1),    # many ragged tiles, a step left over
     (12, 1040, 1040, 128, 0, 1),
+    (1, 563, 6177, 3520, 1, 0),   # a copy of A alone
+    (1, 1024, 4104, 4096, 1, 1),
+    (7, 964, 1679, 448, 1, 0),
+    (2, 4, 512, 64, 1, 1),        # rows of A shorter than a chunk
 ])
 def test_products_of_many_large_tiles(rt, abi, batch, m, n, k, a_cm, b_cm):
     gen = torch.Generator(device="cuda").manual_seed(m + n + k)
