@@ -9,6 +9,7 @@ device work without an MI355X aborts inside the runtime.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -239,13 +240,19 @@ def runtime():
 
 
 def spec():
-    """The extension that builds graph specs (linked against the runtime)."""
+    """The extension that builds graph specs (linked against the runtime); None where the package was
+    built without it.  One that is there and does not load is an error."""
     global _spec
     if _spec is None:
         runtime()
-        from . import _spec as module
-        _spec = module
-    return _spec
+        name = __package__ + "._spec"
+        try:
+            _spec = importlib.import_module(name)
+        except ModuleNotFoundError as e:
+            if e.name != name:
+                raise
+            _spec = False
+    return _spec or None
 
 
 def last_error() -> str:

@@ -2,7 +2,8 @@
 
   libmi355_backend.so   HIP kernels + the C ABI of include/mi355_abi.h
   libmirage_runtime.so  the mirage:: host API (C++) + its C facade for ctypes
-  _spec.so              CPython extension: graph specs built without a ctypes call per operator
+  _spec.<ABI>.so        CPython extension: graph specs built without a ctypes call per operator
+                        (left out where Python's headers are missing)
   mirage_profile        the reference's cpp_examples/profile.cc over that API
   generated/            HIP programs written by Graph::generate_hip_program for the example
                         graphs of codegen.py, compiled as libraries and executables
@@ -23,7 +24,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 BACKEND_LIB = os.path.join(HERE, "libmi355_backend.so")
 RUNTIME_LIB = os.path.join(HERE, "libmirage_runtime.so")
-SPEC_LIB = os.path.join(HERE, "_spec.so")
+SPEC_LIB = os.path.join(HERE, "_spec" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops off: packed FP32 forms have produced silent wrong results on these boxes
@@ -122,7 +123,11 @@ def build_runtime():
 
 def build_spec_reader():
     """_spec: the CPython extension that reads graph specs (graph.build_from_spec)."""
-    _run(["g++", "-O2", "-fPIC", "-std=c++17", "-shared", "-I", INCLUDE, "-I", sysconfig.get_paths()["include"], "-o", SPEC_LIB,
+    headers = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(headers, "Python.h")):
+        print(f"no Python.h in {headers}: graph specs are built through ctypes", flush=True)
+        return
+    _run(["g++", "-O2", "-fPIC", "-std=c++17", "-shared", "-I", INCLUDE, "-I", headers, "-o", SPEC_LIB,
           os.path.join(CSRC, "python", "spec.cc"), "-L" + HERE, "-lmirage_runtime", "-lmi355_backend", "-Wl,-rpath,$ORIGIN"])
 
 

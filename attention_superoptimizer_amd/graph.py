@@ -414,9 +414,38 @@ def verify_batch_end(ticket):
     return [bool(eq[i]) for i in range(n)], _stats(st)
 
 
+def _build_in_python(g: KNGraph, spec: List[dict]) -> List[List[DTensor]]:
+    """What _spec.build does, a ctypes call per operator."""
+    vals: List[List[DTensor]] = []
+
+    def get(ref):
+        return vals[ref[0]][ref[1]]
+
+    for op in spec:
+        k = op["op"]
+        if k == "input":
+            vals.append([g.new_input(op["dims"], DT_FLOAT16, op.get("layout", "DmemRowMajor"))])
+        elif k == "matmul":
+            vals.append([g.matmul(get(op["in"][0]), get(op["in"][1]))])
+        elif k in ("exp", "silu"):
+            vals.append([g._unary(k, get(op["in"][0]))])
+        elif k in ("add", "mul", "div"):
+            vals.append([g._binary(k, get(op["in"][0]), get(op["in"][1]))])
+        elif k == "reduction":
+            vals.append([g.reduction(get(op["in"][0]), op["dim"], op.get("size", 1))])
+        elif k == "customized":
+            vals.append(g.customized([get(r) for r in op["in"]], op["plan"]))
+        else:
+            raise ValueError(k)
+    return vals
+
+
 def build_from_spec(spec: List[dict], graph: Optional[KNGraph] = None):
     """Builds a graph spec (see workloads.py) through the host API.
     Returns (graph, per-operator lists of output tensors)."""
     g = graph or KNGraph()
-    return g, N.spec().build(g._g.value, spec if isinstance(spec, list) else list(spec), DTensor, DMEM_LAYOUT, SMEM_LAYOUT,
+    native = N.spec()
+    if native is None:
+        return g, _build_in_python(g, spec)
+    return g, native.build(g._g.value, spec if isinstance(spec, list) else list(spec), DTensor, DMEM_LAYOUT, SMEM_LAYOUT,
                              KN_OP, TB_OP, InfeasibleOperator)

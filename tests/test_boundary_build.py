@@ -8,6 +8,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 import pytest
 
@@ -85,6 +86,19 @@ def test_cmake_configures_and_builds_for_gfx950(tmp_path):
     env = dict(os.environ, MIRAGE_HOST_ONLY="1")
     out = subprocess.check_output([sys.executable, "-c", probe], env=env).decode()
     assert out.strip() == "ok"
+    # the Python package runs on what CMake builds, its reader of graph specs included
+    pkg = tmp_path / "attention_superoptimizer_amd"
+    shutil.copytree(PKG, pkg, ignore=shutil.ignore_patterns("*.so", "*.o", "csrc", "generated", "__pycache__", "mirage_profile"))
+    extensions = list(build.glob("_spec*.so"))
+    assert [e.name for e in extensions] == ["_spec" + sysconfig.get_config_var("EXT_SUFFIX")]
+    for lib in [backend, runtime] + extensions:
+        shutil.copy(lib, pkg)
+    probe = ("from attention_superoptimizer_amd import _native as N, graph as G, workloads as W\n"
+             "G.set_smem_budget(1 << 20)\n"
+             "g, vals = G.build_from_spec(W.config2_gqa_decode()[0])\n"
+             "print(N.spec().__file__, N.BACKEND_PATH, len(vals))\n")
+    out = subprocess.check_output([sys.executable, "-c", probe], env=env, cwd=tmp_path).decode().split()
+    assert out == [str(pkg / extensions[0].name), str(pkg / "libmi355_backend.so"), "4"]
 
 
 def test_reference_json_call_sites_compile_and_run(tmp_path):
