@@ -81,6 +81,15 @@ bool ints(PyObject *seq, int n, int *out) {
   return ok;
 }
 
+// a list or tuple of exactly two, as unpacking it wants
+bool is_pair(PyObject *o) {
+  Py_ssize_t const n = PySequence_Size(o);
+  if (n >= 0 && n != 2) {
+    PyErr_SetString(PyExc_ValueError, "two values are expected");
+  }
+  return n == 2;
+}
+
 // a code given by name, or as a number where `number_too`
 bool code(PyObject *table, PyObject *o, bool number_too, int *v) {
   if (number_too && !PyUnicode_Check(o)) {
@@ -146,7 +155,7 @@ bool read_plan(PyObject *plan, Tables const &t, mirage_c_plan *p) {
   }
   for (int i = 0; i < (int)n_ops; i++) {
     PyObject *op = PySequence_GetItem(ops, i);
-    PyObject *name = op == nullptr ? nullptr : PySequence_GetItem(op, 0);
+    PyObject *name = op == nullptr || !is_pair(op) ? nullptr : PySequence_GetItem(op, 0);
     PyObject *operands = name == nullptr ? nullptr : PySequence_GetItem(op, 1);
     bool ok = operands != nullptr && code(t.tb_op, name, true, &p->op_type[i]);
     Py_ssize_t const n = ok ? PySequence_Size(operands) : -1;
@@ -158,7 +167,7 @@ bool read_plan(PyObject *plan, Tables const &t, mirage_c_plan *p) {
     p->op_num_operands[i] = (int)n;
     for (int j = 0; ok && j < (int)n; j++) {
       PyObject *pair = PySequence_GetItem(operands, j);
-      ok = pair != nullptr && ints(pair, 2, p->op_operands[i][j]);
+      ok = pair != nullptr && is_pair(pair) && ints(pair, 2, p->op_operands[i][j]);
       Py_XDECREF(pair);
     }
     Py_XDECREF(operands);

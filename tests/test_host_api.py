@@ -260,6 +260,14 @@ def test_verify_ring_never_hands_out_what_a_live_batch_owns():
         rt.mirage_verify_ring_destroy(ring)
 
 
+# ---- the two readers of a graph spec: the extension, and the ctypes calls it stands in for ----------
+def _readers():
+    if N.spec() is None:
+        pytest.skip("built without the extension")
+    return [lambda g, s: N.spec().build(g._g.value, s, G.DTensor, G.DMEM_LAYOUT, G.SMEM_LAYOUT, G.KN_OP, G.TB_OP,
+                                        G.InfeasibleOperator), G._build_in_python]
+
+
 def _outcome(read, spec):
     """The graph a reader builds, as JSON and tensors without their ids, or the error it raises."""
     g = G.KNGraph()
@@ -271,6 +279,65 @@ def _outcome(read, spec):
         return type(e)
     finally:
         g.close()
+
+
+def _all_specs():
+    for name in sorted(W.REFERENCE_EXAMPLES):
+        yield from W.REFERENCE_EXAMPLES[name]
+    for name in sorted(W.BASELINE_CONFIGS):
+        yield from (s for s in W.BASELINE_CONFIGS[name]() if s is not None)
+    yield from load_gqa_fixture()["generated_graphs"]
+
+
+def test_readers_build_the_same_graphs():
+    native, python = _readers()
+    n = 0
+    for spec in _all_specs():
+        want = _outcome(python, spec)
+        assert not isinstance(want, type), want
+        assert _outcome(native, spec) == want
+        n += 1
+    assert n > 60
+
+
+@pytest.mark.parametrize("change", [
+    {}, {"block_dim": [64, 2, 1]}, {"reduction_dimx": 16}, {"input_smem_layouts": []}, {"input_smem_layouts": None},
+    {"input_smem_layouts": ["SmemColumnMajor", "SmemRowMajor"]}, {"input_smem_layouts": [201, 299]},
+    {"grid_dim": (4, 1, 1)}, {"input_map": ((-1, -1, -1), (1, -1, -1))},      # tuples as well as lists
+    {"grid_dim": [4, 1]}, {"input_map": [[-1, -1], [1, -1, -1]]}, {"input_map": [[-1, -1, -1]] * 5}, {"forloop_dim": [1]},
+    {"forloop_range": None}, {"forloop_range": "4"}, {"forloop_range": 8}, {"ops": [["tb_nothing_op", [[0, 0]]]]},
+    {"ops": [["tb_matmul_op", [[0, 0], [1, 0], [0, 0]]]]}, {"ops": [["tb_exp_op", [[0, 0]]]] * 17}, {"ops": [[2003, [[0, 0], [1, 0]]]]},
+    {"ops": [["tb_matmul_op"]]}, {"ops": [["tb_matmul_op", [[0, 0], [1, 0]], 0]]}, {"ops": [["tb_matmul_op", [[0, 0, 0], [1, 0]]]]},
+    {"ops": [["tb_matmul_op", [[0], [1, 0]]]]}, {"ops": [[]]}, {"input_smem_layouts": ["SmemNothing", "SmemRowMajor"]}, {"output_map": 1},
+])
+def test_readers_take_the_same_plans(change):
+    native, python = _readers()
+    spec, _ = W.tiled_matmul(16, 256, 256, (4, 1, 1), 4, (-1, -1, -1), (1, -1, -1), (1, -1, -1))
+    spec = [dict(op) for op in spec]
+    spec[2]["plan"] = {**spec[2]["plan"], **change}
+    assert _outcome(native, spec) == _outcome(python, spec)
+
+
+@pytest.mark.parametrize("key", ["grid_dim", "output_map", "forloop_range", "input_map", "forloop_dim", "ops"])
+def test_readers_miss_the_same_keys(key):
+    native, python = _readers()
+    spec, _ = W.tiled_matmul(16, 256, 256, (4, 1, 1), 4, (-1, -1, -1), (1, -1, -1), (1, -1, -1))
+    spec = [dict(op) for op in spec]
+    spec[2]["plan"] = {k: v for k, v in spec[2]["plan"].items() if k != key}
+    assert _outcome(native, spec) == _outcome(python, spec) == KeyError
+
+
+@pytest.mark.parametrize("op", [
+    {"op": "exp", "in": [[0, 0]]}, {"op": "exp", "in": [[-1, -1]]}, {"op": "mul", "in": [[0, 0], [0, 0]]},
+    {"op": "reduction", "in": [[0, 0]], "dim": 1}, {"op": "reduction", "in": [[0, 0]], "dim": 1, "size": 64},
+    {"op": "reduction", "in": [[0, 0]]}, {"op": "exp", "in": [[1, 0]]}, {"op": "exp", "in": [[0, 1]]}, {"op": "exp"},
+    {"op": "matmul", "in": [[0, 0]]}, {"op": "matmul", "in": [[0, 0], [0, 0]]}, {"op": "nothing", "in": [[0, 0]]},
+    {"op": "input", "dims": [4, 4], "layout": "DmemNothing"}, {"op": "input", "dims": [2.5]}, {},
+])
+def test_readers_take_the_same_operators(op):
+    native, python = _readers()
+    spec = [{"op": "input", "dims": [64, 256]}, op]
+    assert _outcome(native, spec) == _outcome(python, spec)
 
 
 def test_a_package_without_the_extension_builds_graphs(monkeypatch):
