@@ -59,9 +59,10 @@ __device__ __forceinline__ float prologue(int pro, float x) {
   if (pro == PRO_EXP) {
     return __expf(x);
   }
-  // (a reciprocal is within one unit of the last fp32 place; the full division is ten instructions
-  // more, and the gate's activations are what its kernels spend their vector time on)
-  return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x));
+  // x / (1 + exp(-x)): the quotient by a reciprocal, one correction, infinities and NaN as a division has
+  // them.  Half the instructions of the full division, and for every fp16 x its result.
+  float const d = 1.0f + __expf(-x), r = __builtin_amdgcn_rcpf(d), q = x * r;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, x), r, q), d, x);
 }
 
 // Transposing stage of a [R][C] tile (C contiguous, row stride ld) into dst[C][R]
