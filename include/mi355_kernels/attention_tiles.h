@@ -220,15 +220,25 @@ __global__ __launch_bounds__(attn_tiles_lanes(D, RPW, CHB) * 64) void attn_tiles
           for (int rp = 0; rp < RPW; rp++) {
             rs[rp] = sum_lane_groups(rs[rp]);
             if (HAS_DIV) {
-              float const inv = __builtin_amdgcn_rcpf(static_cast<float>(static_cast<_Float16>(rs[rp])));
+              // E / sum, rounded to fp32 and then to fp16 as the division is: the reciprocal's product with one
+              // correction is the nearest fp32 number.  (Without it quotients below 2^-14 came out one unit
+              // off where they lie next to the middle of two fp16 numbers.  An infinite sum: 0, or no number
+              // where E is infinite too; E is finite under a finite sum.)
+              float const sum = static_cast<float>(static_cast<_Float16>(rs[rp])), inv = __builtin_amdgcn_rcpf(sum);
+              float const by = __builtin_isinf(sum) ? 0.0f : -sum;
+              auto quotient = [&](_Float16 e) {
+                float q = __builtin_fmaf(static_cast<float>(e), inv, 0.0f);
+                q = __builtin_fmaf(__builtin_fmaf(by, q, static_cast<float>(e)), inv, q);
+                asm volatile("" : "+v"(q));  // (fused with the conversion the last step would round once)
+                return static_cast<_Float16>(q);
+              };
 #pragma unroll
               for (int p = 0; p < PAIRS; p++) {
 #pragma unroll
                 for (int w = 0; w < 4; w++) {
                   // (slots of blocks that do not exist hold anything and are never multiplied)
                   half2v const e2 = __builtin_bit_cast(half2v, pk[rp][p][w]);
-                  half2v const p2 = {static_cast<_Float16>(__builtin_fmaf(static_cast<float>(e2[0]), inv, 0.0f)),
-                                     static_cast<_Float16>(__builtin_fmaf(static_cast<float>(e2[1]), inv, 0.0f))};
+                  half2v const p2 = {quotient(e2[0]), quotient(e2[1])};
                   pk[rp][p][w] = __builtin_bit_cast(uint32_t, p2);
                 }
               }

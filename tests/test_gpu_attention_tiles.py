@@ -2,6 +2,7 @@
 of a 16-row group and of a wavefront's row groups, key tiles of an odd and an even number of
 16-key blocks (one block, a lone last block, more than one chunk of registers), fewer and more
 iterations than lanes, both forms, both storage orders, row tiles that join into one tall tile."""
+import numpy as np
 import pytest
 
 from helpers import assert_f16_close, normal_f16
@@ -56,3 +57,70 @@ def test_prefill_row_tiles_join(rt, hd, row_tile, blocks, keys, loop, order):
              "plan": W._plan((heads, 1, blocks), loop, [(0, -1, 1), (0, 2, -1), (0, 1, -1)], (-1, 2, 1), (0, 2, 1),
                              W.ATT_OPS, dimx=hd)}]
     _run(rt, spec, f"prefill {hd} {row_tile} x {blocks}, {keys} x {loop} {order}")
+
+
+def _tile_values(rt, make, groups, keys, order, scores, v):
+    """A plan's first results for one iteration of `keys` keys: rows of one-hot queries, so that the scores
+    are the keys' values themselves."""
+    spec, _ = make(groups=groups, rows=64, seq=keys, kv_blocks=1, F=1)
+    for i in (1, 2):
+        spec[i]["layout"] = order
+    q = np.broadcast_to(np.eye(64, dtype=np.float16), (groups, 64, 64))
+    got = _graph_f16(rt, spec, {0: q, 1: scores, 2: v})
+    assert _last_kernels[0] == KERNEL_ATTENTION
+    return got[3]
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("keys", [16, 48])
+@pytest.mark.parametrize("peaked", [False, True], ids=["even", "peaked"])
+def test_division_is_the_quotient(rt, keys, order, peaked):
+    """P = E / sum to the bit, with E of a few units, and with sums of 6 and 12 next to which the other keys
+    vanish: their quotients are subnormal numbers, many in the middle of two.  E and the sums come from the
+    form without the division, the values of V show P one by one; E is of a range in which any order of
+    adding gives the same fp16 sum."""
+    from attention_superoptimizer_amd import workloads as W
+    groups = 64
+    rng = np.random.default_rng(keys)
+    scores = rng.uniform(*((-16.6, -10.4) if peaked else (-2.7, 2.0)), (groups, 64, keys)).astype(np.float16)
+    if peaked:
+        scores[::2, :, :6] = scores[1::2, :, :12] = 0
+    v = np.zeros((groups, keys, 64), np.float16)
+    v[:, np.arange(keys), np.arange(keys)] = 1
+    e, sums = _tile_values(rt, W.gqa_inc_decode, groups, keys, order, scores, v)
+    p = _tile_values(rt, W.config2_gqa_decode, groups, keys, order, scores, v)[0]
+    e, sums = e.reshape(groups, 64, 64)[:, :, :keys].astype(np.float32), sums.reshape(groups, 64, -1)[:, :, :1].astype(np.float32)
+    assert np.array_equal(e.astype(np.float64).sum(2, keepdims=True).astype(np.float16).astype(np.float32), sums)
+    assert not peaked or set(sums.ravel()) == {6, 12}
+    np.testing.assert_array_equal(p.reshape(groups, 64, 64)[:, :, :keys], (e / sums).astype(np.float16))
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+def test_division_of_sums_out_of_range(rt, abi, order):
+    """Scores whose exponentials overflow or vanish, infinities and NaN: what the interpreter's statements
+    give, number for number."""
+    from attention_superoptimizer_amd import workloads as W
+    groups, keys = 3, 48
+    rng = np.random.default_rng(9)
+    scores = rng.uniform(-1, 1, (groups, 64, keys)).astype(np.float16)
+    scores[0, 0] = -30          # every exponential and the sum are zero: no number
+    scores[0, 1] = 9            # the sum is infinite, no exponential is: zeros
+    scores[0, 2, 5] = 12        # one exponential and the sum are infinite
+    scores[0, 3] = -16          # the smallest numbers
+    scores[1, 0, 7] = 11.09     # close to the largest
+    v = np.broadcast_to(np.eye(keys, 64, dtype=np.float16), (groups, keys, 64))
+    for make in (W.gqa_inc_decode, W.config2_gqa_decode):
+        fused = _tile_values(rt, make, groups, keys, order, scores, v)
+        assert abi.mi355_set_option(1, 1) == 0
+        try:
+            _last_kernels[:] = []
+            spec, _ = make(groups=groups, rows=64, seq=keys, kv_blocks=1, F=1)
+            for i in (1, 2):
+                spec[i]["layout"] = order
+            want = _graph_f16(rt, spec, {0: np.broadcast_to(np.eye(64, dtype=np.float16), (groups, 64, 64)), 1: scores, 2: v})[3]
+        finally:
+            assert abi.mi355_set_option(1, 0) == 0
+        for f, w in zip(fused, want):
+            assert np.array_equal(np.isnan(f), np.isnan(w)) and np.array_equal(np.isposinf(f), np.isposinf(w))
+            ok = np.isfinite(w)
+            assert_f16_close(f[ok], w[ok], what=make.__name__)
