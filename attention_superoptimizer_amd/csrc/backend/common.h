@@ -206,11 +206,11 @@ __device__ __forceinline__ uint32_t residues_p4_signed(uint32_t a, uint32_t b, u
                     (uint32_t)residue_p_signed(d));
 }
 
-// Residues of two fingerprint values (16 bits each) as signed bytes, the low bytes of the halves of p and
+// Residues of two values below 2^15 (16 bits each) as signed bytes, the low bytes of the halves of p and
 // q: what the int8 matrix products want, at three instructions a value for both fields (ten through
 // residue_p_signed and residue_q).  The quotient is estimated in packed fp16: added to 1536 it is rounded
 // to an integer, whose low byte is the quotient's.  An estimate one off where the value lies close to the
-// middle between two multiples leaves a remainder that still fits: over all of [0, 25651) they are in
+// middle between two multiples leaves a remainder that still fits: over all of [0, 32768) they are in
 // [-125, 117] modulo 227 and in [-66, 63] modulo 113.
 typedef _Float16 fp_half2 __attribute__((ext_vector_type(2)));
 typedef unsigned short fp_ushort2 __attribute__((ext_vector_type(2)));
@@ -222,6 +222,39 @@ __device__ __forceinline__ void residue_pairs(uint32_t v, uint32_t &p, uint32_t 
   fp_ushort2 const tq = __builtin_bit_cast(fp_ushort2, __builtin_elementwise_fma(h, by_q, one_and_half_k));
   p = __builtin_bit_cast(uint32_t, (fp_ushort2)(x - tp * (unsigned short)FP_P));
   q = __builtin_bit_cast(uint32_t, (fp_ushort2)(x - tq * (unsigned short)FP_Q));
+}
+// A caller may write any 16-bit value: those of 2^15 and up are brought into the ring first, by at most two
+// subtractions of 227 * 113 (below it x - 25651 wraps to more than x).  That would be two instructions a
+// value (82.9 -> 87.6 us of a verification); so a wavefront looks at the top bits of what it stages, a
+// quarter of one, and only does it where it finds one set.
+template <int A, int B>
+__device__ __forceinline__ uint32_t fp_bits(uint2 const (&x)[A][B]) {
+  uint32_t seen = 0;
+#pragma unroll
+  for (int a = 0; a < A; a++) {
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      seen |= x[a][b].x | x[a][b].y;
+    }
+  }
+  return seen;
+}
+__device__ __forceinline__ bool fp_past_residues(uint32_t seen) { return __any((int)(seen & 0x80008000u)) != 0; }
+template <int A, int B>
+__device__ __forceinline__ void fp_into_ring(uint2 (&x)[A][B]) {
+  fp_ushort2 const ring = {(unsigned short)FP_PQ, (unsigned short)FP_PQ};
+  auto pair = [&](uint32_t v) {
+    fp_ushort2 r = __builtin_bit_cast(fp_ushort2, v);
+    r = __builtin_elementwise_min(r, (fp_ushort2)(r - ring));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(r, (fp_ushort2)(r - ring)));
+  };
+#pragma unroll
+  for (int a = 0; a < A; a++) {
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      x[a][b] = uint2{pair(x[a][b].x), pair(x[a][b].y)};
+    }
+  }
 }
 // of four values in a row
 __device__ __forceinline__ void residues_row(uint2 v, uint32_t &p, uint32_t &q) {

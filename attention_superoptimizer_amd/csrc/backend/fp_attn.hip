@@ -99,15 +99,22 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
   v4i qf, qp;
   {
     uint16_t const *q = tile_at(P.q, bx, by, bz, 0) + (long long)(row < m ? row : m - 1) * ld_q;
+    uint2 x[1][4];
 #pragma unroll
     for (int w = 0; w < 4; w++) {
       int const at = 16 * g + 4 * w;
-      uint2 x = {0, 0};
+      x[0][w] = uint2{0, 0};
       if (at < d) {
-        x = *reinterpret_cast<uint2 const *>(q + at);
+        x[0][w] = *reinterpret_cast<uint2 const *>(q + at);
       }
+    }
+    if (fp_past_residues(fp_bits(x))) {
+      fp_into_ring(x);
+    }
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
       uint32_t rp, rq;
-      residues_row(x, rp, rq);
+      residues_row(x[0][w], rp, rq);
       qf[w] = (int)rq;
       qp[w] = (int)rp;
     }
@@ -137,6 +144,10 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
     }
   };
   auto stage = [&]() {
+    if (fp_past_residues(fp_bits(kr) | fp_bits(vr))) {
+      fp_into_ring(kr);
+      fp_into_ring(vr);
+    }
 #pragma unroll
     for (int w = 0; w < KW; w++) {
       unsigned char *const kq = tiles + w * PLANES * kPlane, *const vp = kq + kPlane, *const kp = vp + kPlane;

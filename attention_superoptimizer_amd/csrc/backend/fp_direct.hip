@@ -97,6 +97,10 @@ __global__ __launch_bounds__(kThreads) void fp_direct_kernel(DirectMany const D)
     }
   };
   auto stage = [&](int step) {
+    if (fp_past_residues(fp_bits(ra) | fp_bits(rb))) {
+      fp_into_ring(ra);
+      fp_into_ring(rb);
+    }
 #pragma unroll
     for (int u = 0; u < KW; u++) {
       unsigned char *const ap = lds + u * CHUNK, *const aq = ap + A_BYTES, *const bp = aq + A_BYTES, *const bq = bp + B_BYTES;

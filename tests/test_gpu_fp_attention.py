@@ -59,6 +59,23 @@ def test_fused_fingerprint_attention(rt, abi, form, b, m, row_blocks, n, F, kv_b
 
 
 @pytest.mark.parametrize("form", ["sums", "divided", "scores"])
+def test_fused_fingerprint_attention_of_any_16_bit_values(rt, form):
+    spec = _spec(form, 4, 64, 2, 64, 2, 2, 64, 64)
+    ins = {i: np.random.default_rng(i).permutation(np.resize(np.arange(65536, dtype=np.uint16), int(np.prod(spec[i]["dims"]))))
+           .reshape(spec[i]["dims"]) for i in range(3)}
+    g, vals = rt.build_from_spec(spec)
+    try:
+        for i, a in ins.items():
+            vals[i][0].write_fingerprint(a)
+        g.fingerprint(3)
+        got = [t.read_fingerprint() for t in vals[3]]
+    finally:
+        g.close()
+    for x, y in zip(got, orc.eval_graph(spec, "fp", {i: a % FP_PQ for i, a in ins.items()})[3]):
+        np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("form", ["sums", "divided", "scores"])
 def test_fused_fingerprint_attention_in_a_batch(rt, abi, form):
     specs = [_spec(form, 2, 16, 2, 64, 2, 2, 64, 64), _spec(form, 2, 32, 1, 128, 1, 2, 64, 64)]
     graphs = [rt.build_from_spec(s) for s in specs]

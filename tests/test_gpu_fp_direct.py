@@ -40,3 +40,19 @@ def test_direct_matmul_of_every_ring_value_with_itself(rt, abi, k):
         for i, C in enumerate(got):
             v = vals[(lo + i) * per:][:C.shape[0], None, None]
             np.testing.assert_array_equal(C, np.broadcast_to(k * v * v % FP_PQ, C.shape))
+
+
+@pytest.mark.parametrize("n", [4, 64, 6])  # whole groups of four, whole tiles, odd rows
+def test_direct_matmul_of_every_16_bit_value(rt, abi, n):
+    """Operands hold any 16-bit value, in the ring or past it, as in the other fingerprint kernels."""
+    every = np.arange(65536, dtype=np.uint16)
+    shapes = [(16, 64, n, 64), (18, 64, n, 60)]
+    for flip in (False, True):  # every value as an element of A, and of B
+        def fill(i, d, flip=flip):
+            if (i >= 100) == flip:
+                return np.resize(every, int(np.prod(d))).reshape(d)
+            return uniform_fp(d, 3 + i)
+
+        ins, got = _matmul_many(abi, rt, shapes, fill)
+        for (A, B), C, s in zip(ins, got, shapes):
+            np.testing.assert_array_equal(C, orc.fp_matmul(A % FP_PQ, B % FP_PQ), err_msg=str(s))
