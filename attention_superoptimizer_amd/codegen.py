@@ -33,6 +33,9 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=on",
 # with INTERPRETER_SUFFIX, every customized operator as the specialised interpreter
 EXAMPLES = ["C1_fused_matmul", "C2_gqa_decode", "C3_mha_prefill", "C4_lora", "C5a_gated_mlp", "mlp"]
 INTERPRETER_SUFFIX = "_interp"
+# plans of tile sizes that the kernels of whole tiles are not built for: generated in the first form
+# only, as libraries
+ODD_TILES = ["attention_keys_of_48", "attention_keys_of_48_divided", "prefill_rows_of_80", "gated_mlp_columns_of_48", "lora_rank_8"]
 OPT_FORCE_INTERPRETER = 1
 
 
@@ -40,6 +43,16 @@ def example_spec(name: str) -> List[dict]:
     from . import workloads as W
     if name.endswith(INTERPRETER_SUFFIX):
         name = name[:-len(INTERPRETER_SUFFIX)]
+    if name == "attention_keys_of_48":
+        return W.gqa_inc_decode(groups=5, rows=12, seq=48 * 6 * 5, kv_blocks=6, F=5)[0]
+    if name == "attention_keys_of_48_divided":
+        return W.config2_gqa_decode(groups=3, rows=33, seq=48 * 4 * 3, kv_blocks=4, F=3)[0]
+    if name == "prefill_rows_of_80":
+        return W.config3_mha_prefill(heads=3, seq=80 * 6, hd=64, q_split=6, F=6, rows2=16)[0]
+    if name == "gated_mlp_columns_of_48":
+        return W.config5_gated_mlp(m=13, d=192, h=480, grid1=10, F1=2, grid2=3, F2=5)[0]
+    if name == "lora_rank_8":
+        return W.config4_lora(m=9, d=160 * 4, r=8, grid=10, F=4)[0]
     if name in W.BASELINE_CONFIGS:
         return W.BASELINE_CONFIGS[name]()[0]
     return W.REFERENCE_EXAMPLES[name][0]
@@ -93,6 +106,10 @@ def build_examples() -> None:
         src = generate(name)
         compile_library(src, library_path(name))
         compile_program(src, program_path(name))
+        print("generated and compiled", src, flush=True)
+    for name in ODD_TILES:
+        src = generate(name)
+        compile_library(src, library_path(name))
         print("generated and compiled", src, flush=True)
 
 

@@ -115,6 +115,9 @@ std::string literal(LaneParams const &L) {
                 L.m_pieces, L.m_gx, L.m_gy);
   return t;
 }
+std::string literal(StreamParams const &L) {
+  return literal(L.g, "G") + "    mi355::StreamParams P{};\n    P.g = G;\n" + emit_fmt("    P.results = %d;\n", L.results);
+}
 char const *tf(bool b) { return b ? "true" : "false"; }
 
 struct GMatch {
@@ -339,7 +342,7 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // 54.6 against 48.4) but not for the others, where each wavefront's loads of its activation rows
   // and of the lora A tile outnumber its weight loads.
   long long const weight_bytes = blocks * F * (long long)(G.nb * G.KT * 64 + (G.lora ? G.KT * 16 : 0)) * 2;
-  bool const two_weights_cm = G.wcm && G.nb == 2 && blocks * S <= 4096 && (weight_bytes <= (68LL << 20) || emit_sink() != nullptr);
+  bool const two_weights_cm = G.wcm && G.nb == 2 && blocks * S <= 4096 && weight_bytes <= (68LL << 20);
   if (s.gemm_mode == 0 && !two_weights_cm && (blocks * S > 1024 || weight_bytes > (8LL << 20))) {
     return 0;
   }
@@ -390,24 +393,32 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
 
 // the fold of a split for-loop: the launch, or its source text
 int launch_combine(GemmParams const &A, int nb, dim3 blocks) {
-  if (EmitSink *sink = emit_sink()) {
-    emit_launch(*sink, "gemm_combine_kernel", emit_fmt("%d", nb), blocks, 256, 0, literal(A, "P"));
-    return 1;
-  }
   State &s = state();
   int const lds = A.forloop_range * 1024;
+  dim3 const fold_grid(blocks.x * nb * ((A.M + 7) / 8), blocks.y, blocks.z);
+  if (EmitSink *sink = emit_sink()) {
+    bool const fold = lds <= s.max_lds;
+    emit_launch(*sink, fold ? "gemm_fold_kernel" : "gemm_combine_kernel", emit_fmt("%d", nb), fold ? fold_grid : blocks, 256,
+                fold ? lds : 0, literal(A, "P"));
+    return 1;
+  }
   if (lds > s.max_lds) {
     MI355_HIP(launch_kernel(nb == 1 ? gemm_combine_kernel<1> : gemm_combine_kernel<2>, blocks, 256, 0, s.stream(), A));
     return 1;
   }
   auto *fn = nb == 1 ? gemm_fold_kernel<1> : gemm_fold_kernel<2>;
   MI355_GRANT_LDS(fn, lds);
-  MI355_HIP(launch_kernel(fn, dim3(blocks.x * nb * ((A.M + 7) / 8), blocks.y, blocks.z), 256, lds, s.stream(), A));
+  MI355_HIP(launch_kernel(fn, fold_grid, 256, lds, s.stream(), A));
   return 1;
 }
 
 template <int NB, int PRO, bool LORA, bool WCM, int MT>
 int launch_stream_one(StreamParams const &L, dim3 grid, int lds) {
+  if (EmitSink *sink = emit_sink()) {
+    sink->headers |= 32u;
+    emit_launch(*sink, "gemm_stream_kernel", emit_fmt("%d, %d, %s, %s, %d", NB, PRO, tf(LORA), tf(WCM), MT), grid, 256, lds, literal(L));
+    return 1;
+  }
   auto *fn = gemm_stream_kernel<NB, PRO, LORA, WCM, MT>;
   MI355_GRANT_LDS(fn, lds);
   MI355_HIP(launch_kernel(fn, grid, 256, lds, state().stream(), L));
@@ -420,8 +431,8 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A)
   int const mt = G.M <= 16 ? 1 : (G.M <= 32 ? 2 : 4), F = P.forloop_range;
   // (with more rows than half an iteration's k the product slots rival the weights: the kernel that
   // keeps its sums in registers where a block is not split stays ahead there)
-  if (s.any_size_kernels || !G.whole || G.KT % 64 != 0 || 2 * G.M > G.KT || emit_sink() != nullptr) {
-    return 0;  // (a printed program takes gemm_fused_kernel, which prints)
+  if (s.any_size_kernels || !G.whole || G.KT % 64 != 0 || 2 * G.M > G.KT) {
+    return 0;
   }
   long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
   int const ring = 4 * kStreamRing * stream_slot_bytes(G.pro, G.lora, mt);
@@ -436,7 +447,8 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A)
   int const steps = (F + 3) / 4 * (G.KT / 64) * G.nb;
   bool const fits = ring + results <= s.max_lds;
   int ks = 1;
-  if (!(fits && blocks >= 96 && steps <= 8) && slab <= s.scratch_bytes) {
+  EmitSink *const sink = emit_sink();
+  if (!(fits && blocks >= 96 && steps <= 8) && slab <= (sink ? kEmitScratchBytes : s.scratch_bytes)) {
     long long const most = (ring <= 80 * 1024 ? 1024 : 256) / blocks;
     ks = (int)std::max<long long>(1, std::min<long long>((F + 3) / 4, most));
   }
@@ -449,6 +461,9 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A)
   L.g = A;
   L.g.ksplit = ks;
   L.g.scratch = static_cast<_Float16 *>(s.scratch());
+  if (sink) {  // a printed program allocates the workspace itself
+    L.g.scratch = ks > 1 ? reinterpret_cast<_Float16 *>(kEmitScratch) : nullptr;
+  }
   L.results = ring;
   int const lds = ring + (ks == 1 ? results : 0);
   if ((long long)P.grid[0] * ks > 2147483647LL) {
@@ -471,6 +486,9 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A)
   MI355_STREAM_CASE(1, PRO_NONE, true, 1)
 #undef MI355_STREAM_CASE
   if (rc == 1 && ks > 1) {
+    if (sink) {
+      sink->scratch_bytes = std::max(sink->scratch_bytes, slab);
+    }
     rc = launch_combine(L.g, G.nb, dim3(P.grid[0], P.grid[1], P.grid[2]));
   }
   if (rc == 1) {

@@ -188,7 +188,7 @@ inline bool has_column_major_saver(DevProgram const &P) {
 struct EmitSink {
   std::string text;          // statements of the launcher body
   unsigned headers = 0;      // bit 0: attention.h, bit 1: gemm.h, bit 2: combine.h, bit 3: attention_tiles.h,
-                             // bit 4: gemm_tiles.h
+                             // bit 4: gemm_tiles.h, bit 5: gemm_stream.h
   size_t scratch_bytes = 0;  // workspace the printed launches share (0: none)
 };
 EmitSink *&emit_sink();

@@ -50,16 +50,35 @@ def test_fused_families_are_emitted_as_their_kernels(tmp_path):
     assert text.count("__global__") == 0
     assert "mi355::attn_stream_kernel<128, 64, 128, false, 4, 2, true, 1><<<dim3(32, 1, 16), 256, 65536, stream>>>(P);" in text
     assert '#include "mi355_kernels/combine.h"' in text and "mi355::combine_fused_kernel<8, 0, 4><<<dim3(32, 64, 1), 256, 0, stream>>>(P);" in text
-    # C4: the range kernel and its fold share a workspace the program allocates once
+    # C4: the streaming kernel and its fold share a workspace the program allocates once
     spec, _ = W.config4_lora()
     text = _emit(spec, tmp_path / "c4.hip")
-    assert "mi355::gemm_fused_kernel<1, 1, 0, true, 256, true><<<" in text
-    assert "mi355::gemm_combine_kernel<1><<<dim3(64, 1, 1), 256, 0, stream>>>(P);" in text
+    assert '#include "mi355_kernels/gemm_stream.h"' in text
+    assert "mi355::gemm_stream_kernel<1, 0, true, true, 1><<<" in text
+    assert "mi355::gemm_fold_kernel<1><<<dim3(128, 1, 1), 256, 16384, stream>>>(P);" in text
     assert "static void *scratch = nullptr;" in text and "P.scratch = static_cast<_Float16 *>(scratch);" in text
     # C1: the one-launch kernel
     spec, _ = W.config1_fused_matmul()
     text = _emit(spec, tmp_path / "c1.hip")
     assert "mi355::gemm_lanes_kernel<64, 1, 0, false, true><<<dim3(256, 1, 1), 1024," in text
+
+
+def test_gated_mlp_prints_the_streaming_kernel(tmp_path):
+    """235 MB of two weights: the kernel the backend runs, not the one-launch kernel for small ones."""
+    spec, _ = W.config5_gated_mlp()
+    text = _emit(spec, tmp_path / "c5.hip")
+    assert text.count("__global__") == 0 and "gemm_lanes_kernel" not in text
+    assert "mi355::gemm_stream_kernel<2, 0, false, true, 1><<<" in text and "mi355::gemm_stream_kernel<1, 3, false, true, 1><<<" in text
+    assert "mi355::gemm_fold_kernel<1><<<" in text
+
+
+@pytest.mark.parametrize("name,kernel", [
+    ("attention_keys_of_48", "attn_tiles_kernel<64, false, true, "), ("attention_keys_of_48_divided", "attn_tiles_kernel<64, true, true, "),
+    ("prefill_rows_of_80", "attn_tiles_kernel<64, false, true, "), ("gated_mlp_columns_of_48", "gemm_tiles_kernel<"),
+    ("lora_rank_8", "gemm_tiles_kernel<")])
+def test_plans_of_odd_tiles_are_printed_as_their_kernels(tmp_path, name, kernel):
+    text = _emit(CG.example_spec(name), tmp_path / "odd.hip")
+    assert text.count("__global__") == 0 and "mi355::" + kernel in text, text
 
 
 def test_program_structure_of_the_decode_attention_graph(tmp_path):

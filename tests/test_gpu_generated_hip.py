@@ -22,11 +22,13 @@ OPT_FORCE_INTERPRETER = 1
 # standard deviations of the normal inputs, by graph and input position
 STD = {"C1_fused_matmul": 0.1, "C2_gqa_decode": 0.125, "C3_mha_prefill": 128 ** -0.5,
        "C4_lora": {0: 0.25, 1: 0.02, 2: 0.02, 3: 0.02},
-       "C5a_gated_mlp": {0: 0.25, 1: 0.02, 2: 0.02, 3: 0.02}, "mlp": 0.05}
+       "C5a_gated_mlp": {0: 0.25, 1: 0.02, 2: 0.02, 3: 0.02}, "mlp": 0.05,
+       "attention_keys_of_48": 0.125, "attention_keys_of_48_divided": 0.125, "prefill_rows_of_80": 0.125,
+       "gated_mlp_columns_of_48": 0.05, "lora_rank_8": 0.05}
 # |V| for the prefill attention graph: with V of both signs the fp16 for-loop accumulators pass
 # through values far above the final one, and two correct evaluations that order a tile product's
 # fp32 additions differently end one accumulator ulp apart, above the plain tolerance
-NON_NEGATIVE = {"C3_mha_prefill": (2,)}
+NON_NEGATIVE = {"C3_mha_prefill": (2,), "attention_keys_of_48": (2,), "attention_keys_of_48_divided": (2,), "prefill_rows_of_80": (2,)}
 
 _oracle_cache = {}
 
@@ -94,6 +96,12 @@ def test_generated_program_matches_the_backend(rt, abi, name, interpreter):
     finally:
         g.close()
         assert abi.mi355_set_option(OPT_FORCE_INTERPRETER, 0) == 0
+
+
+@pytest.mark.parametrize("name", ["attention_keys_of_48", "attention_keys_of_48_divided", "prefill_rows_of_80",
+                                  "gated_mlp_columns_of_48", "lora_rank_8"])
+def test_generated_program_of_odd_tiles_matches_the_backend(rt, abi, name):
+    test_generated_program_matches_the_backend(rt, abi, name, False)
 
 
 def test_generated_decode_attention_runs_at_the_backends_speed(rt, abi):
