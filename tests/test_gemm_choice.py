@@ -73,6 +73,11 @@ def test_choice_for_a_column_major_a(choose, shape, b_cm, big, tiles, copied):
     assert c["route"] == "tiles" and not c["copy_a"] and not c["copy_b"]
 
 
+def test_consumers_of_the_large_kernel_are_covered(choose):
+    """The sizes the consumer test means the 256 x 256 kernel with."""
+    assert choose(1, 4090, 4096, 128)["route"] == "big"
+
+
 def test_small_tiles_do_not_queue_for_lds(choose):
     """[200, 130, 96] . [200, 96, 130]: 3000 tiles of 32 x 64, one ring to a compute unit, take 23.8 us; 64 x 64 take 9."""
     c = choose(200, 130, 130, 96)

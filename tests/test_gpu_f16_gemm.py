@@ -44,12 +44,10 @@ def _execute(build, inputs, whole):
         g.close()
 
 
-@pytest.mark.parametrize("b,m,n,k", [(1, 1, 8, 16), (2, 33, 77, 65), (1, 40, 130, 3001), (1, 3, 6, 20), (1, 3600, 3700, 256)])
+@pytest.mark.parametrize("b,m,n,k", [(1, 1, 8, 16), (2, 33, 77, 65), (1, 40, 130, 3001), (1, 3, 6, 20), (1, 3600, 3700, 256),
+                                     (1, 4090, 4096, 128)])
 @pytest.mark.parametrize("op", ["exp", "silu", "add", "mul", "div", "rdiv"])
 def test_consumer_in_the_matmul(rt, abi, op, b, m, n, k):
-    if m > 1000 and op not in ("silu", "mul"):
-        pytest.skip("the large tiles once per kind")
-
     def build(g):
         A, B, X = g.new_input((b, m, k)), g.new_input((b, k, n), layout="DmemColumnMajor"), g.new_input((b, m, n))
         C = g.matmul(A, B)
@@ -74,3 +72,73 @@ def test_softmax_rows(rt, abi, b, m, n):
     np.testing.assert_array_equal(whole[1], single[1])
     for w, s in zip(whole[2:], single[2:]):  # (another order of the row sum)
         assert_f16_close(w, s, rtol=2e-3, atol=1e-6, what="row sum or quotient")
+
+
+def _odd_numbers(a, seed):
+    """A few infinities and NaN at the edges and inside, and values whose products overflow fp16."""
+    rng = np.random.default_rng(seed)
+    a = a.copy()
+    flat = a.reshape(-1)
+    flat[-1], flat[0] = np.inf, -np.inf
+    flat[rng.integers(0, flat.size, 3)] = np.nan
+    flat[rng.integers(0, flat.size, 3)] = 60000
+    return a
+
+
+@pytest.mark.parametrize("batch,m,n,k", [
+    (2, 33, 77, 65), (1, 3, 333, 3001), (1, 130, 200, 320), (2, 100, 136, 96), (1, 17, 4096, 512), (1, 2100, 4100, 64)])
+def test_infinities_and_nan_stay_where_they_belong(rt, abi, monkeypatch, batch, m, n, k):
+    """An infinity or NaN reaches the products it is part of and no other: padding of tiles, repeated rows and
+    shifted chunks of k multiply nothing with it."""
+    import test_gpu_f16
+    monkeypatch.setattr(test_gpu_f16, "normal_f16", lambda d, std, seed: _odd_numbers(normal_f16(d, std, seed), seed))
+    for a_cm, b_cm in ((0, 1), (0, 0), (1, 1), (1, 0)):
+        a, b, got = _abi_matmul(rt, abi, batch, m, n, k, a_cm, b_cm, 5)
+        with np.errstate(all="ignore"):
+            want = np.matmul(a.astype(np.float32), b.astype(np.float32)).astype(np.float16)
+        what = f"A cm {a_cm}, B cm {b_cm}"
+        assert np.array_equal(np.isnan(got), np.isnan(want)), what
+        assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want)), what
+        ok = np.isfinite(want)
+        assert ok.any()
+        assert_f16_close(got[ok], want[ok], what=what)
+
+
+@pytest.mark.parametrize("b,m,n,k", [(2, 33, 77, 65), (1, 40, 136, 320), (1, 16, 512, 512), (1, 40, 130, 3001)])
+@pytest.mark.parametrize("op", ["exp", "silu", "add", "mul", "div", "rdiv"])
+def test_consumer_of_numbers_out_of_range(rt, abi, op, b, m, n, k):
+    def build(g):
+        A, B, X = g.new_input((b, m, k)), g.new_input((b, k, n), layout="DmemColumnMajor"), g.new_input((b, m, n))
+        C = g.matmul(A, B)
+        return A, B, X, C, g._unary(op, C) if op in ("exp", "silu") else g.div(X, C) if op == "rdiv" else g._binary(op, C, X)
+
+    ins = [_odd_numbers(normal_f16([b, m, k], 1.0, 1), 1), _odd_numbers(normal_f16([b, k, n], 1.0, 2), 2),
+           _odd_numbers(normal_f16([b, m, n], 1.0, 3), 3)]
+    ins[0][:, 0] = 0   # (a row of zeros: x / 0 and 0 / 0)
+    ins[2][:, 0, ::2] = 0
+    for whole, single in zip(_execute(build, ins, True), _execute(build, ins, False)):
+        np.testing.assert_array_equal(whole, single)
+
+
+@pytest.mark.parametrize("m,n", [(1, 7), (600, 513), (1024, 65), (1030, 4096), (5, 4097), (2, 20001)])
+def test_softmax_rows_out_of_range(rt, abi, m, n):
+    """Rows of -inf, rows with +inf or NaN, rows whose exponentials or whose sum overflow, rows that vanish."""
+    def build(g):
+        X = g.new_input((1, m, n))
+        E = g.exp(X)
+        R = g.reduction(E, 2)
+        return X, E, R, g.div(E, R)
+
+    x = normal_f16([1, m, n], 0.5, 4)
+    kinds = [lambda r: r.fill(-np.inf), lambda r: r.__setitem__(n // 2, np.inf), lambda r: r.__setitem__(n - 1, np.nan),
+             lambda r: r.__setitem__(0, 12), lambda r: r.fill(11), lambda r: r.fill(-20), lambda r: r.__setitem__(0, -np.inf)]
+    for i in range(m):
+        if m <= 5 or i % 3 == 0:
+            kinds[(i + n) % len(kinds)](x[0, i])
+    whole, single = _execute(build, [x], True), _execute(build, [x], False)
+    np.testing.assert_array_equal(whole[1], single[1])
+    for w, s in zip(whole[2:], single[2:]):
+        assert np.array_equal(np.isnan(w), np.isnan(s)) and np.array_equal(np.isinf(w), np.isinf(s))
+        ok = np.isfinite(s)
+        # (one order of the fp32 row sum against another: two fp16 places, where they are normal numbers)
+        assert_f16_close(w[ok], s[ok], rtol=2e-3, atol=1e-6, what="row sum or quotient")

@@ -70,3 +70,27 @@ def test_products_of_many_large_tiles(rt, abi, batch, m, n, k, a_cm, b_cm):
     got, want = _matmul(abi, A, B, batch, m, n, k, a_cm, b_cm)
     # half an fp16 place of the result, and k fp32 additions in another order
     assert ((got - want).abs() <= 2.0 ** -11 * want.abs() + 1e-6 * k ** 0.5 * want.abs().max() + 1e-6).all()
+
+
+@pytest.mark.parametrize("a_cm,b_cm", [(0, 1), (0, 0), (1, 1), (1, 0)])
+@pytest.mark.parametrize("batch,m,n,k", [
+    (1, 16, 64, 64), (2, 33, 72, 128), (1, 300, 520, 512), (1, 64, 256, 4096), (1, 3000, 4096, 64), (2, 9, 7, 40)])
+@pytest.mark.parametrize("off", [(1, 0, 0), (0, 3, 0), (0, 0, 1), (5, 7, 3)])
+def test_operands_on_no_boundary(rt, abi, batch, m, n, k, a_cm, b_cm, off):
+    """Bases that are whole elements and nothing more: the kernels of 16-byte chunks leave these to others."""
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    make = lambda count, o: torch.randn(count + 8, device="cuda", generator=gen).half()[o:o + count]  # noqa: E731
+    A, B = make(batch * m * k, off[0]), make(batch * n * k, off[1])
+    C = torch.full((batch * m * n + 64,), -7.0, device="cuda", dtype=torch.float16)
+    out = C[32 + off[2]:32 + off[2] + batch * m * n]
+    out.fill_(float("nan"))
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    torch.cuda.synchronize()
+    assert abi.mi355_f16_matmul_layout(p(A), p(B), p(out), batch, m, n, k, a_cm, b_cm) == 0
+    assert abi.mi355_sync() == 0
+    assert (C[:32 + off[2]] == -7).all() and (C[32 + off[2] + batch * m * n:] == -7).all()
+    Af = A.view(batch, k, m).float().transpose(1, 2).contiguous() if a_cm else A.view(batch, m, k).float()
+    Bf = B.view(batch, n, k).float().transpose(1, 2).contiguous() if b_cm else B.view(batch, k, n).float()
+    want = torch.bmm(Af, Bf)
+    # half an fp16 place of the result, and k fp32 additions in another order
+    assert ((out.view(batch, m, n).float() - want).abs() <= 2.0 ** -11 * want.abs() + 1e-6 * k ** 0.5 * want.abs().max() + 1e-6).all()

@@ -40,3 +40,44 @@ def test_gated_mlp_prologues_and_lora(rt, ranges, m, order):
     spec, _ = W.config4_lora(m=m, d=128 * 6, r=16, grid=3, F=6)
     spec[1], spec[3] = W._inp([128 * 6, 192], COL), W._inp([16, 192], COL)
     _run(rt, spec, order, f"lora {m} {order}")
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("option,value", [(7, 1), (7, 2), (9, 1)], ids=["stream", "lanes", "tiles"])
+@pytest.mark.parametrize("family", ["plain", "silu", "exp", "gated", "lora"])
+def test_infinities_and_nan(rt, abi, family, option, value, order):
+    """Infinities, NaN, prologues that overflow and sums that do, in the first and last rows, columns and
+    iterations: the interpreter's pattern, and its numbers where they are finite."""
+    import numpy as np
+    from attention_superoptimizer_amd import workloads as W
+    from helpers import assert_f16_close, normal_f16
+    from test_gpu_f16 import _graph_f16
+    m = 9
+    if family == "gated":
+        spec, _ = W.config5_gated_mlp(m=m, d=192, h=640, grid1=10, F1=3, grid2=3, F2=5)
+    elif family == "lora":
+        spec, _ = W.config4_lora(m=m, d=128 * 6, r=16, grid=3, F=6)
+        spec[1], spec[3] = W._inp([128 * 6, 192], COL), W._inp([16, 192], COL)
+    else:
+        ops = [("tb_matmul_op", [(0, 0), (1, 0)])] if family == "plain" else [
+            (f"tb_{family}_op", [(0, 0)]), ("tb_matmul_op", [(2, 0), (1, 0)])]
+        spec = [W._inp([m, 320]), W._inp([320, 128], COL),
+                {"op": "customized", "in": [[0, 0], [1, 0]],
+                 "plan": W._plan((2, 1, 1), 5, [(-1, -1, -1), (1, -1, -1)], (1, 0), (1, -1, -1), ops)}]
+    spec = [dict(op, layout=order) if op["op"] == "input" and i > 0 else op for i, op in enumerate(spec)]
+    ins = {i: normal_f16(op["dims"], 0.1, 5 + i) for i, op in enumerate(spec) if op["op"] == "input"}
+    x, w = ins[0], ins[1]
+    x[0, 0], x[2, 5], x[3, 7], x[m - 1, -1] = np.inf, np.nan, 60000, -np.inf
+    w[3, 1], w[-1, -1], w[0, 4] = np.inf, np.nan, 50000
+    got = {}
+    for name, (o, v) in {"fused": (option, value), "interpreter": (1, 1)}.items():
+        assert abi.mi355_set_option(o, v) == 0
+        try:
+            got[name] = [t for i, r in enumerate(_graph_f16(rt, spec, ins)) if spec[i]["op"] == "customized" for t in r]
+        finally:
+            assert abi.mi355_set_option(o, 0) == 0
+    for i, (f, want) in enumerate(zip(got["fused"], got["interpreter"])):
+        assert np.array_equal(np.isnan(f), np.isnan(want)) and np.array_equal(np.isposinf(f), np.isposinf(want))
+        ok = np.isfinite(want)
+        assert not ok.all() and (ok.any() or i > 0)  # (a NaN column of the first operator is in all sums of a second)
+        assert_f16_close(f[ok], want[ok], what=family)
