@@ -225,8 +225,8 @@ __device__ __forceinline__ void residue_pairs(uint32_t v, uint32_t &p, uint32_t 
 }
 // A caller may write any 16-bit value: those of 2^15 and up are brought into the ring first, by at most two
 // subtractions of 227 * 113 (below it x - 25651 wraps to more than x).  That would be two instructions a
-// value (82.9 -> 87.6 us of a verification); so a wavefront looks at the top bits of what it stages, a
-// quarter of one, and only does it where it finds one set.
+// value (82.9 -> 87.6 us of a verification); so a wavefront looks at the top bits of what it has staged, a
+// quarter of one, and only where it finds one set does it stage again (no difference in the kernels' times).
 template <int A, int B>
 __device__ __forceinline__ uint32_t fp_bits(uint2 const (&x)[A][B]) {
   uint32_t seen = 0;

@@ -143,11 +143,7 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
       }
     }
   };
-  auto stage = [&]() {
-    if (fp_past_residues(fp_bits(kr) | fp_bits(vr))) {
-      fp_into_ring(kr);
-      fp_into_ring(vr);
-    }
+  auto put = [&]() {
 #pragma unroll
     for (int w = 0; w < KW; w++) {
       unsigned char *const kq = tiles + w * PLANES * kPlane, *const vp = kq + kPlane, *const kp = vp + kPlane;
@@ -163,6 +159,14 @@ __device__ __forceinline__ void fp_attn_block(FpAttn const &P, FpTables const t,
         }
         *reinterpret_cast<uint32_t *>(vp + at) = v[u];
       }
+    }
+  };
+  auto stage = [&]() {
+    put();
+    if (fp_past_residues(fp_bits(kr) | fp_bits(vr))) {  // (looked at last: the first values are not kept waiting)
+      fp_into_ring(kr);
+      fp_into_ring(vr);
+      put();
     }
   };
 

@@ -96,11 +96,7 @@ __global__ __launch_bounds__(kThreads) void fp_direct_kernel(DirectMany const D)
       }
     }
   };
-  auto stage = [&](int step) {
-    if (fp_past_residues(fp_bits(ra) | fp_bits(rb))) {
-      fp_into_ring(ra);
-      fp_into_ring(rb);
-    }
+  auto put = [&](int step) {
 #pragma unroll
     for (int u = 0; u < KW; u++) {
       unsigned char *const ap = lds + u * CHUNK, *const aq = ap + A_BYTES, *const bp = aq + A_BYTES, *const bq = bp + B_BYTES;
@@ -122,6 +118,14 @@ __global__ __launch_bounds__(kThreads) void fp_direct_kernel(DirectMany const D)
         *reinterpret_cast<uint32_t *>(bp + at) = p[v];
         *reinterpret_cast<uint32_t *>(bq + at) = q[v];
       }
+    }
+  };
+  auto stage = [&](int step) {
+    put(step);
+    if (fp_past_residues(fp_bits(ra) | fp_bits(rb))) {  // (looked at last: the first values are not kept waiting)
+      fp_into_ring(ra);
+      fp_into_ring(rb);
+      put(step);
     }
   };
 
