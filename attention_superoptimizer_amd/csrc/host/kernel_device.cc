@@ -686,6 +686,48 @@ static void run_softmax_rows(KNOperator const *e, KNOperator const *r, KNOperato
   MI355_CALL(mi355_f16_softmax_rows(X.data_ptr, E.data_ptr, R.data_ptr, P.data_ptr, E.num_elements() / n, (int)n));
 }
 
+// A matmul, the softmax of its rows and the matmul of that, operators i .. i + 4: the un-fused attention
+// graph.  Nothing else in it may be read by a later of these operators.
+static bool is_attention_rows(std::vector<KNOperator *> const &ops, size_t i) {
+  if (i + 4 >= ops.size() || ops[i]->op_type != KN_MATMUL_OP || ops[i + 4]->op_type != KN_MATMUL_OP ||
+      !is_softmax_rows(ops[i + 1], ops[i + 2], ops[i + 3])) {
+    return false;
+  }
+  DTensor const &S = ops[i]->output_tensors[0], &P = ops[i + 3]->output_tensors[0], &V = ops[i + 4]->input_tensors[1];
+  if (ops[i + 1]->input_tensors[0].guid != S.guid || ops[i + 4]->input_tensors[0].guid != P.guid) {
+    return false;
+  }
+  for (size_t j = i; j < i + 4; j++) {
+    if (V.guid == ops[j]->output_tensors[0].guid) {
+      return false;
+    }
+  }
+  return true;
+}
+
+static bool run_attention_rows(std::vector<KNOperator *> const &ops, size_t i) {
+  if (!is_attention_rows(ops, i)) {
+    return false;
+  }
+  DTensor const &Q = ops[i]->input_tensors[0], &K = ops[i]->input_tensors[1], &V = ops[i + 4]->input_tensors[1];
+  bool row_major = !column_major(Q);
+  for (size_t j = i; j < i + 5; j++) {
+    row_major = row_major && !column_major(ops[j]->output_tensors[0]);
+  }
+  if (!row_major || column_major(K) != column_major(V)) {
+    return false;
+  }
+  int batch, m, n, k, batch2, m2, dv, n2;
+  matmul_extents(Q, K, batch, m, n, k);
+  matmul_extents(ops[i + 4]->input_tensors[0], V, batch2, m2, dv, n2);
+  int taken = 0;
+  MI355_CALL(mi355_f16_attention_rows(Q.data_ptr, K.data_ptr, V.data_ptr, ops[i]->output_tensors[0].data_ptr,
+                                      ops[i + 1]->output_tensors[0].data_ptr, ops[i + 2]->output_tensors[0].data_ptr,
+                                      ops[i + 3]->output_tensors[0].data_ptr, ops[i + 4]->output_tensors[0].data_ptr, batch, m, n, k,
+                                      dv, column_major(K) ? 1 : 0, &taken));
+  return taken != 0;
+}
+
 void execute_all(Graph const &graph) {
   require_device("execute_all");
   std::vector<KNOperator *> const &ops = graph.operators;
@@ -696,7 +738,9 @@ void execute_all(Graph const &graph) {
            !column_major(ops[i + 2]->output_tensors[0]);
   };
   for (size_t i = 0; i < n;) {
-    if (softmax_at(i)) {
+    if (run_attention_rows(ops, i)) {
+      i += 5;
+    } else if (softmax_at(i)) {
       run_softmax_rows(ops[i], ops[i + 1], ops[i + 2]);
       i += 3;
     } else if (i + 1 < n && !softmax_at(i + 1) && run_matmul_then(ops[i], ops[i + 1])) {

@@ -386,6 +386,12 @@ int mi355_f16_matmul_then(void const *A, void const *B, void *C, int batch, int 
 /* E = exp(X), R[row] = sum of a row of E, P = E / R for `rows` rows of n elements: what
  * mi355_f16_unary, mi355_f16_reduce and mi355_f16_binary one after the other leave. */
 int mi355_f16_softmax_rows(void const *X, void *E, void *R, void *P, size_t rows, int n);
+/* The un-fused attention graph: S = Q . K, E, R and P of S as above, O = P . V for `batch` matrices of m
+ * query rows, n keys and head sizes d and dv: what the operators one after the other leave (fp32 sums may
+ * be added in another order).  Q and the results are row-major, K and V in the storage order named.
+ * *taken = 0 and nothing enqueued where one launch does not take these sizes, or does not pay. */
+int mi355_f16_attention_rows(void const *Q, void const *K, void const *V, void *S, void *E, void *R, void *P,
+                             void *O, int batch, int m, int n, int d, int dv, int kv_column_major, int *taken);
 /* out[b][c][r] = in[b][r][c] for `batch` [rows, cols] matrices: the row-major copy of a
  * DmemColumnMajor tensor (call it with rows = the tensor's columns and cols = its rows) for
  * the element-wise operators and reductions, which index their inputs flat as
