@@ -10,7 +10,7 @@
 namespace mi355 {
 
 struct TilesShape {
-  int rpw = 1, chb = 4, ip = 1, split = 1, lds = 0;
+  int rpw = 1, pairs = 0, ip = 1, split = 1, lds = 0;
 };
 // Whether attn_tiles_kernel takes query tiles of `m` rows against key tiles of NK keys, and in
 // which shape; `blocks` = logical thread blocks, F = for-loop range.

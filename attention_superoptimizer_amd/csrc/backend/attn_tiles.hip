@@ -12,40 +12,44 @@ namespace mi355 {
 
 namespace {
 
-template <int D, bool HAS_DIV, bool CM, int RPW, int CHB>
+template <int D, bool HAS_DIV, bool CM, int RPW, int PAIRS>
 int launch_tiles_one(AttnParams const &A, dim3 grid, int ip, int lds) {
   if (EmitSink *sink = emit_sink()) {
     sink->headers |= 8u;
     emit_launch(*sink, "attn_tiles_kernel",
-                emit_fmt("%d, %s, %s, %d, %d", D, HAS_DIV ? "true" : "false", CM ? "true" : "false", RPW, CHB), grid, 64 * ip, lds,
+                emit_fmt("%d, %s, %s, %d, %d", D, HAS_DIV ? "true" : "false", CM ? "true" : "false", RPW, PAIRS), grid, 64 * ip, lds,
                 attn_params_literal(A));
     return 1;
   }
-  auto *fn = attn_tiles_kernel<D, HAS_DIV, CM, RPW, CHB>;
+  auto *fn = attn_tiles_kernel<D, HAS_DIV, CM, RPW, PAIRS>;
   MI355_GRANT_LDS(fn, lds);
   MI355_HIP(launch_kernel(fn, grid, 64 * ip, lds, state().stream(), A));
   return 1;
 }
 
 template <int D, bool HAS_DIV, bool CM>
-int launch_tiles_shape(AttnParams const &A, dim3 grid, int rpw, int chb, int ip, int lds) {
-  switch (rpw * 10 + chb) {
-    case 12: return launch_tiles_one<D, HAS_DIV, CM, 1, 2>(A, grid, ip, lds);
-    case 14: return launch_tiles_one<D, HAS_DIV, CM, 1, 4>(A, grid, ip, lds);
-    case 22: return launch_tiles_one<D, HAS_DIV, CM, 2, 2>(A, grid, ip, lds);
-    case 24: return launch_tiles_one<D, HAS_DIV, CM, 2, 4>(A, grid, ip, lds);
-    default: break;
-  }
-  if constexpr (D == 64 && HAS_DIV) {
-    switch (rpw * 10 + chb) {
-      case 16: return launch_tiles_one<D, HAS_DIV, CM, 1, 6>(A, grid, ip, lds);
-      case 18: return launch_tiles_one<D, HAS_DIV, CM, 1, 8>(A, grid, ip, lds);
-      case 26: return launch_tiles_one<D, HAS_DIV, CM, 2, 6>(A, grid, ip, lds);
-      case 28: return launch_tiles_one<D, HAS_DIV, CM, 2, 8>(A, grid, ip, lds);
+int launch_tiles_shape(AttnParams const &A, dim3 grid, int rpw, int pairs, int ip, int lds) {
+  if constexpr (!HAS_DIV) {
+    return rpw == 1 ? launch_tiles_one<D, false, CM, 1, 0>(A, grid, ip, lds) : launch_tiles_one<D, false, CM, 2, 0>(A, grid, ip, lds);
+  } else {
+    switch (rpw * 10 + pairs) {
+      case 11: return launch_tiles_one<D, true, CM, 1, 1>(A, grid, ip, lds);
+      case 12: return launch_tiles_one<D, true, CM, 1, 2>(A, grid, ip, lds);
+      case 21: return launch_tiles_one<D, true, CM, 2, 1>(A, grid, ip, lds);
+      case 22: return launch_tiles_one<D, true, CM, 2, 2>(A, grid, ip, lds);
       default: break;
     }
+    if constexpr (D == 64) {
+      switch (rpw * 10 + pairs) {
+        case 13: return launch_tiles_one<D, true, CM, 1, 3>(A, grid, ip, lds);
+        case 14: return launch_tiles_one<D, true, CM, 1, 4>(A, grid, ip, lds);
+        case 23: return launch_tiles_one<D, true, CM, 2, 3>(A, grid, ip, lds);
+        case 24: return launch_tiles_one<D, true, CM, 2, 4>(A, grid, ip, lds);
+        default: break;
+      }
+    }
+    return 0;
   }
-  return 0;
 }
 
 }  // namespace
@@ -55,16 +59,10 @@ bool choose_attn_tiles(int D, int DV, int NK, int m, bool has_div, bool cm, long
   if (D != DV || (D != 64 && D != 128) || NK % 16 != 0 || NK < 16 || m < 1) {
     return false;
   }
-  int const nb = NK / 16;
-  // Blocks of keys in registers at a time: the fewest that hold the tile, four at most (two or three
-  // wavefronts per SIMD; with eight there is one: prefill in 80-key tiles 74 us against 51).  The
-  // division needs the row sum of the whole tile before P.V, so there the tile is one chunk.
-  t.chb = nb <= 2 ? 2 : 4;
-  if (has_div && nb > 4) {
-    t.chb = nb <= 6 ? 6 : 8;
-    if (D != 64 || nb > 8) {
-      return false;
-    }
+  // The division needs the row sum of the whole tile before P.V: its exponentials stay in registers.
+  t.pairs = has_div ? (NK / 16 + 1) / 2 : 0;
+  if (t.pairs > (D == 64 ? 4 : 2)) {
+    return false;
   }
   // Two row groups per wavefront (each K / V operand then feeds two matrix instructions) where that
   // leaves a workgroup for almost every compute unit, unless rounding the row groups up to whole
@@ -74,12 +72,11 @@ bool choose_attn_tiles(int D, int DV, int NK, int m, bool has_div, bool cm, long
   t.split = (groups + t.rpw - 1) / t.rpw;
   // Iteration lanes: one wavefront per iteration up to what the instantiation allows, evened out
   // over the rounds.
-  int const most = attn_tiles_lanes(D, t.rpw, t.chb);
-  int const slot = (16 * t.rpw * (DV + 8) + 16 * t.rpw) * 2, strips = cm ? 0 : (D * 40 + 32 * (DV + 8)) * 2;
+  int const most = attn_tiles_lanes(D, t.pairs);
   for (int cap = most; cap >= 1; cap--) {
     int const rounds = (F + cap - 1) / cap;
     t.ip = (F + rounds - 1) / rounds;
-    t.lds = (rounds > 1 ? 2 : 1) * t.ip * slot + t.ip * strips;
+    t.lds = attn_tiles_lds(D, t.rpw, t.ip, rounds);
     if (t.lds <= max_lds) {
       return true;
     }
@@ -90,18 +87,18 @@ bool choose_attn_tiles(int D, int DV, int NK, int m, bool has_div, bool cm, long
 int launch_attn_tiles(AttnParams const &A, dim3 grid, int D, bool has_div, bool cm, TilesShape const &t) {
   if (D == 64) {
     if (has_div) {
-      return cm ? launch_tiles_shape<64, true, true>(A, grid, t.rpw, t.chb, t.ip, t.lds)
-                : launch_tiles_shape<64, true, false>(A, grid, t.rpw, t.chb, t.ip, t.lds);
+      return cm ? launch_tiles_shape<64, true, true>(A, grid, t.rpw, t.pairs, t.ip, t.lds)
+                : launch_tiles_shape<64, true, false>(A, grid, t.rpw, t.pairs, t.ip, t.lds);
     }
-    return cm ? launch_tiles_shape<64, false, true>(A, grid, t.rpw, t.chb, t.ip, t.lds)
-              : launch_tiles_shape<64, false, false>(A, grid, t.rpw, t.chb, t.ip, t.lds);
+    return cm ? launch_tiles_shape<64, false, true>(A, grid, t.rpw, t.pairs, t.ip, t.lds)
+              : launch_tiles_shape<64, false, false>(A, grid, t.rpw, t.pairs, t.ip, t.lds);
   }
   if (has_div) {
-    return cm ? launch_tiles_shape<128, true, true>(A, grid, t.rpw, t.chb, t.ip, t.lds)
-              : launch_tiles_shape<128, true, false>(A, grid, t.rpw, t.chb, t.ip, t.lds);
+    return cm ? launch_tiles_shape<128, true, true>(A, grid, t.rpw, t.pairs, t.ip, t.lds)
+              : launch_tiles_shape<128, true, false>(A, grid, t.rpw, t.pairs, t.ip, t.lds);
   }
-  return cm ? launch_tiles_shape<128, false, true>(A, grid, t.rpw, t.chb, t.ip, t.lds)
-            : launch_tiles_shape<128, false, false>(A, grid, t.rpw, t.chb, t.ip, t.lds);
+  return cm ? launch_tiles_shape<128, false, true>(A, grid, t.rpw, t.pairs, t.ip, t.lds)
+            : launch_tiles_shape<128, false, false>(A, grid, t.rpw, t.pairs, t.ip, t.lds);
 }
 
 }  // namespace mi355

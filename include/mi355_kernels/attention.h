@@ -185,9 +185,9 @@ __device__ __forceinline__ void decode_block(AttnParams const &P, int &bx, int &
   unsigned const ext[3] = {gridDim.x, gridDim.y, gridDim.z};
   unsigned const total = ext[0] * ext[1] * ext[2];
   unsigned id = blockIdx.x + ext[0] * (blockIdx.y + ext[1] * blockIdx.z);
-  if (total % 8 == 0) {
-    id = (id % 8) * (total / 8) + id / 8;
-  }
+  // an XCD (one L2) gets consecutive ids, also where they do not divide by eight
+  unsigned const xcd = id % 8, more = total % 8;
+  id = xcd * (total / 8) + (xcd < more ? xcd : more) + id / 8;
   // divisions by the extents are multiply-highs with magics the host computed (exact while
   // id * extent < 2^32, which the host checks): this runs before the first load can go out
   unsigned digit[3];  // digit i of the id belongs to grid dim perm[i]

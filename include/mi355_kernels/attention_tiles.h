@@ -5,43 +5,59 @@
 // statement in the generic LDS interpreter.
 //
 // A workgroup owns 16 RPW query rows and walks the for-loop in rounds: wavefront ip of IP takes
-// iteration r0 + ip by itself, K and V operands going from global memory into its registers (an
-// MFMA operand of a column-major tile IS sixteen contiguous bytes per lane; a row-major tile takes
-// one trip through a private strip of LDS and a transposing read), and leaves the iteration's fp16
-// result in an LDS slot of its own.  After one barrier all threads add the round's slots to
-// their registers in ITERATION order with one fp16 rounding per add, the sequence of roundings of
-// the sequential loop (reference src/kernel/triton_code_gen.cc:223-232).  Slots are double
-// buffered, so a round costs one barrier.
+// iteration r0 + ip by itself and leaves its fp16 result in LDS.  After one barrier all threads add the
+// round's results up in ITERATION order with one fp16 rounding per add, the sequence of roundings of the
+// sequential loop (reference src/kernel/triton_code_gen.cc:223-232); after another the next round may write.
 //
-// What bounds it: the trip to memory at decode sizes (a wavefront issues all of an iteration's
-// loads before it waits for the first), the conversions and exponentials beside the matrix
-// instructions at prefill sizes.  Two row groups share every K and V operand where there are enough
-// of them, which halves the L2 -> register traffic of a prefill.
-// Keys of a pair of 16-key blocks are permuted as in attention.h (see cm_swizzle_key) so that a
-// lane's eight values of P are consecutive keys; a lone last block keeps the plain order and takes
-// the 16 x 16 x 16 instruction.
+// K and V go pair by pair of 16-key blocks from memory into registers, in the order they have in memory, and
+// from there through a strip of LDS of the wavefront's own (with a transposing read where the reduction index
+// is not the contiguous one); the strip is also where the iteration's result ends.  An operand of a
+// column-major tile IS sixteen contiguous bytes per lane, but sixteen lanes in a row are then sixteen rows,
+// and a compute unit gets 15.7 bytes a cycle that way against 58 in memory order.
+//
+// What bounds it: the trip to memory at decode sizes, at prefill sizes latency and the conversions and
+// exponentials beside the matrix instructions (so: four wavefronts of a SIMD have registers, which is why
+// sums between rounds wait in LDS).  Two row groups share every K and V operand where there are enough of
+// them, which halves the L2 -> register traffic of a prefill.  With operands straight from memory, a tile's keys
+// in registers at once and workgroups of an XCD from anywhere, both launches of [12, 1040, 1040] in tiles
+// of 80 took 24.6 us column-major and 35.5 row-major, now 19.6 and 19.7; head size 128, [16, 1024, 1008] in
+// tiles of 128 x 48, 59.5 and 41.3; [64, 1, 16384] in tiles of 64 65.9 and 57.3.
 #pragma once
+
+#include <type_traits>
 
 #include "attention.h"
 
 namespace mi355 {
 
-// CHB: 16-key blocks of K and V held in registers at a time.  A longer key tile is walked in chunks
-// of CHB blocks; the form with the division needs the whole tile's row sum first, so its tile is
-// one chunk (the host checks).  AttnParams as used here: rows = query rows of a block, stages =
-// keys of a tile, lds_stage_bytes unused.
-// Most iteration lanes of a workgroup: eight where 256 registers hold a wavefront's operands.
-constexpr int attn_tiles_lanes(int D, int RPW, int CHB) { return RPW == 1 && CHB <= 4 && D == 64 ? 8 : 4; }
+// Keys of a pair of 16-key blocks are permuted as in attention.h (see cm_swizzle_key) so that a lane's
+// eight values of P are consecutive keys; a lone last block is a pair whose second half counts for nothing.
+// AttnParams as used here: rows = query rows of a block, stages = keys of a tile, lds_stage_bytes unused.
+// PAIRS: with the division, which needs the whole tile's row sum before P . V, the pairs of a tile, whose
+// exponentials stay in registers (the host checks); 0 without it, the pairs then go through one by one.
+// Most iteration lanes of a workgroup: eight where four wavefronts of a SIMD have registers.
+constexpr int attn_tiles_lanes(int D, int PAIRS) { return D == 64 && PAIRS <= 2 ? 8 : 4; }
+// Halfs of a wavefront's strip: 32 keys of K or V as rows of D elements (pitch D + 8) or of 32 keys (pitch
+// 40), or an iteration's result: 16 RPW rows of the same pitch and their sums.
+constexpr int attn_tiles_strip(int D, int RPW) {
+  int const keys = D * 40 > 32 * (D + 8) ? D * 40 : 32 * (D + 8), result = 16 * RPW * (D + 8) + 16 * RPW;
+  return keys > result ? keys : result;
+}
 
-template <int D, bool HAS_DIV, bool CM, int RPW, int CHB>
-__global__ __launch_bounds__(attn_tiles_lanes(D, RPW, CHB) * 64) void attn_tiles_kernel(AttnParams const) {
+// Bytes of LDS of a workgroup: the strips, and the sums between rounds.
+constexpr int attn_tiles_lds(int D, int RPW, int ip, int rounds) {
+  return 2 * (ip * attn_tiles_strip(D, RPW) + (rounds > 1 ? 16 * RPW * (D + 8) + 16 * RPW : 0));
+}
+
+template <int D, bool HAS_DIV, bool CM, int RPW, int PAIRS>
+__global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
+    __attribute__((amdgpu_waves_per_eu(attn_tiles_lanes(D, PAIRS) == 8 ? 4 : 1))) void attn_tiles_kernel(AttnParams const) {
   AttnParams const P = load_kernel_arguments<AttnParams, 4>();  // (blockDim.x is read)
-  constexpr int DV = D, DB = DV / 16, DK = D / 32, PAIRS = CHB / 2;
-  constexpr int ROWS = 16 * RPW, LDO = DV + 8, SLOT = ROWS * LDO + ROWS;
-  constexpr int CPR = DV / 8;                // 16-byte chunks of a result row
-  constexpr int OWN = ROWS * CPR / 64;       // most chunks a thread adds up (one wavefront)
-  constexpr int KLD = 40, VLD = DV + 8;      // row strides of the row-major staging strips
-  static_assert(CHB % 2 == 0 && (D == 64 || D == 128), "pairs of key blocks, head size 64 or 128");
+  constexpr int DB = D / 16, DK = D / 32, ROWS = 16 * RPW, LD = D + 8, KLD = 40;  // pitches of rows of D and of keys
+  constexpr int CPR = D / 8;                // 16-byte chunks of a row
+  constexpr int CHUNKS = D / 16, KEYS = 64 / CPR;  // chunks a lane holds of a pair; keys per chunk of a wavefront
+  constexpr int STRIP = attn_tiles_strip(D, RPW);
+  static_assert((D == 64 || D == 128) && HAS_DIV == (PAIRS > 0), "head size 64 or 128");
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   int const tid = threadIdx.x, NT = blockDim.x, IP = NT / 64;
   int const lane = tid % 64, ip = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -49,313 +65,362 @@ __global__ __launch_bounds__(attn_tiles_lanes(D, RPW, CHB) * 64) void attn_tiles
   int bx, by, bz, slice;
   decode_block(P, bx, by, bz, slice);
   int const row_base = slice * ROWS, m = P.rows, nb = P.stages / 16, F = P.forloop_range;
-  int const nchunks = HAS_DIV ? 1 : (nb + CHB - 1) / CHB;
-  _Float16 *const slots = reinterpret_cast<_Float16 *>(lds);  // [1 or 2][IP][SLOT]
-  _Float16 *const k_strip = slots + (F > IP ? 2 : 1) * IP * SLOT + ip * (D * KLD + 32 * VLD);
-  _Float16 *const v_strip = k_strip + D * KLD;
+  int const pairs = HAS_DIV ? PAIRS : (nb + 1) / 2;
+  bool const odd = nb % 2 != 0;  // the last pair is a lone block
+  // a wavefront's LDS: its strip, and the result of its iteration once the strip is done with
+  _Float16 *const all = reinterpret_cast<_Float16 *>(lds), *const strip = all + ip * STRIP;
+  _Float16 *const sums = all + IP * STRIP;  // [ROWS][LD], the row sums: with more than one round
 
-  // ---- loads -------------------------------------------------------------------------------
-  // K of chunk `ch` of iteration `it`.  Column-major: the operands of S^T.  Row-major: the pair's
-  // [D][32 keys] strip as 16-byte chunks, lane by lane (a lone block: [D][16 keys]).
-  uint4v kr[CHB][DK];
-  auto load_k = [&](int it, int ch) {
-    int const ld = P.k.d_cols, nbc = (nb - ch * CHB) < CHB ? (nb - ch * CHB) : CHB;
-    _Float16 const *kg = static_cast<_Float16 const *>(P.k.ptr) + tile_offset(P.k, bx, by, bz, it) +
-                         (CM ? (long long)(16 * CHB * ch) * ld : (long long)(16 * CHB * ch));
+  // ---- loads and their way into the strip ----------------------------------------------------
+  // 32 keys of K or V lie in memory as rows of D elements (`by_key`: K column-major, V row-major) or as D
+  // rows of 32 keys; lane l takes the 16-byte chunk l of what follows each other.  Of a lone block the first
+  // half is read twice: the loads are always the same number.
+  // Of the operand that has 32 keys in a row two pairs are loaded together where registers allow (DEPTH): the
+  // 64 bytes of a row that a pair is are half a line, and a line fetched in two halves at different times
+  // costs memory twice ([64 groups, 16384 keys] 86 us instead of 61).
+  constexpr int DEPTH = !HAS_DIV && RPW == 1 ? 2 : 1, KS = CM ? 1 : DEPTH, VS = CM ? DEPTH : 1;
+  uint4v kr[KS][CHUNKS], vr[VS][CHUNKS];
+  auto load = [&](bool by_key, _Float16 const *from, int ld, bool lone, uint4v (&to)[CHUNKS]) {
+    char const *const at = reinterpret_cast<char const *>(from);
+    int const row = by_key ? lane / CPR : lone ? lane / 2 : lane / 4, pos = by_key ? lane % CPR : lone ? lane % 2 : lane % 4;
+    uint32_t const off = 2u * (uint32_t)(row * ld + 8 * pos);
+    long long const step = 2LL * (by_key ? KEYS : lone ? 32 : 16) * ld;
 #pragma unroll
-    for (int p = 0; p < PAIRS; p++) {
-      // (one path for pairs and lone blocks, offsets selected: the registers keep fixed places)
-      bool const lone = 2 * p + 1 >= nbc;
-      int const k_row = CM ? (lone ? c : 8 * a4 + b4) : (lone ? lane / 2 : lane / 4);
-      int const k_pos = CM ? 8 * g : 8 * (lone ? lane % 2 : lane % 4);
+    for (int i = 0; i < CHUNKS; i++) {
+      to[i] = *reinterpret_cast<uint4v const *>(at + (i < CHUNKS / 2 ? i : lone ? i - CHUNKS / 2 : i) * step + off);
+    }
+  };
+  auto load_k = [&](int slot, int it, int p) {
+    _Float16 const *const tile = static_cast<_Float16 const *>(P.k.ptr) + tile_offset(P.k, bx, by, bz, it);
+    load(CM, tile + (CM ? (long long)(32 * p) * P.k.d_cols : 32 * p), P.k.d_cols, odd && p == pairs - 1, kr[slot]);
+  };
+  auto load_v = [&](int slot, int it, int p) {
+    _Float16 const *const tile = static_cast<_Float16 const *>(P.v.ptr) + tile_offset(P.v, bx, by, bz, it);
+    load(!CM, tile + (CM ? 32 * p : (long long)(32 * p) * P.v.d_cols), P.v.d_cols, odd && p == pairs - 1, vr[slot]);
+  };
+  // (Places in the strip are one number per lane plus constants.)  K by keys: key 8 a + 4 j + b at row
+  // 16 j + 4 a + b, which makes a lane's eight scores consecutive keys.
+  _Float16 *const key_at = strip + lane / CPR * LD + 8 * (lane % CPR);
+  _Float16 *const turned_at = D == 64 ? strip + (16 * (lane / 32) + lane / 8 % 4) * LD + 8 * (lane % 8) : key_at;
+  _Float16 *const pair_at = strip + lane / 4 * KLD + 8 * (lane % 4), *const lone_at = strip + lane / 2 * KLD + 8 * (lane % 2);
+  auto stage_k = [&](int slot, bool lone) {
 #pragma unroll
-      for (int i = 0; i < 2 * DK; i++) {
-        if (2 * p + (i < DK ? 0 : 1) < nbc) {
-          int const off = CM ? (32 * p + 4 * (i / DK) + k_row) * ld + 32 * (i % DK) + k_pos
-                             : ((lone ? 32 * i : 16 * i) + k_row) * ld + 32 * p + k_pos;
-          kr[2 * p + i / DK][i % DK] = *reinterpret_cast<uint4v const *>(kg + off);
-        }
+    for (int i = 0; i < CHUNKS; i++) {
+      if (CM) {
+        *reinterpret_cast<uint4v *>(turned_at + (D == 64 ? 4 * i : 16 * (i % 2) + 4 * (i / 2)) * LD) = kr[slot][i];
+      } else if (!lone) {
+        *reinterpret_cast<uint4v *>(pair_at + 16 * i * KLD) = kr[slot][i];
+      } else if (i < CHUNKS / 2) {
+        *reinterpret_cast<uint4v *>(lone_at + 32 * i * KLD) = kr[slot][i];
+      }
+    }
+    asm volatile("" ::: "memory");  // (a wavefront's LDS operations complete in order)
+  };
+  auto stage_v = [&](int slot, bool lone) {  // (the half that a lone block does not have: zeros)
+    uint4v const zero = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < CHUNKS; i++) {
+      if (!CM) {
+        *reinterpret_cast<uint4v *>(key_at + KEYS * i * LD) = lone && i >= CHUNKS / 2 ? zero : vr[slot][i];
+      } else if (!lone) {
+        *reinterpret_cast<uint4v *>(pair_at + 16 * i * KLD) = vr[slot][i];
+      } else {
+        *reinterpret_cast<uint4v *>(lone_at + 32 * (i % (CHUNKS / 2)) * KLD + (i < CHUNKS / 2 ? 0 : 16)) = i < CHUNKS / 2 ? vr[slot][i] : zero;
+      }
+    }
+    asm volatile("" ::: "memory");
+  };
+
+  // The next DEPTH pairs of K or V: past an iteration's last one the wavefront's next iteration, past its last
+  // iteration (or the for-loop's, which is read again and counts for nothing) that one once more.
+  int const steps = (F + IP - 1) / IP * pairs;  // of every wavefront, the same number
+  int k_it = ip < F ? ip : F - 1, k_pair = 0, v_it = k_it, v_pair = 0;
+  auto advance = [&](int &it, int &pair) {
+    pair++;
+    if (pair == pairs) {
+      pair = 0;
+      it = it + IP < F ? it + IP : F - 1;
+    }
+  };
+  auto load_ks = [&](int slots) {
+#pragma unroll
+    for (int slot = 0; slot < KS; slot++) {
+      if (slot < slots) {
+        load_k(slot, k_it, k_pair);
+        advance(k_it, k_pair);
       }
     }
   };
-  // V likewise: column-major V^T[16t + c][32p + 8g ..] (a lone block: keys 8 (g / 2) .., of which the
-  // lane uses the half 4 (g % 2) ..), row-major the [32 keys][DV] strip
-  uint4v vr[PAIRS][DB];
-  auto load_v = [&](int it, int ch) {
-    int const ld = P.v.d_cols, nbc = (nb - ch * CHB) < CHB ? (nb - ch * CHB) : CHB;
-    _Float16 const *vg = static_cast<_Float16 const *>(P.v.ptr) + tile_offset(P.v, bx, by, bz, it) +
-                         (CM ? (long long)(16 * CHB * ch) : (long long)(16 * CHB * ch) * ld);
+  auto load_vs = [&](int slots) {
 #pragma unroll
-    for (int p = 0; p < PAIRS; p++) {
-      bool const lone = 2 * p + 1 >= nbc;
-      int const v_pos = 8 * (lone ? g / 2 : g);
-#pragma unroll
-      for (int t = 0; t < DB; t++) {
-        if (2 * p + (CM || t < DB / 2 ? 0 : 1) < nbc) {
-          int const q = 64 * t + lane;
-          int const off = CM ? (16 * t + c) * ld + 32 * p + v_pos : (32 * p + q / CPR) * ld + 8 * (q % CPR);
-          vr[p][t] = *reinterpret_cast<uint4v const *>(vg + off);
-        }
+    for (int slot = 0; slot < VS; slot++) {
+      if (slot < slots) {
+        load_v(slot, v_it, v_pair);
+        advance(v_it, v_pair);
       }
     }
   };
 
   // Q fragments: Q[row c][32kk + 8g .. +7] (rows past the tile re-read its last one: every row is
-  // worked on by itself and theirs are not stored)
+  // worked on by itself and theirs are not stored), through the strip as well
   half8 qf[RPW][DK];
   {
     _Float16 const *q = static_cast<_Float16 const *>(P.q.ptr) + tile_offset(P.q, bx, by, bz, 0);
+    uint4v raw[RPW][CHUNKS / 2];
 #pragma unroll
     for (int rp = 0; rp < RPW; rp++) {
-      int const row = row_base + 16 * rp + c;
-      _Float16 const *qr = q + (long long)(row < m ? row : m - 1) * P.q.d_cols + 8 * g;
+#pragma unroll
+      for (int i = 0; i < CHUNKS / 2; i++) {
+        int const row = row_base + 16 * rp + KEYS * i + lane / CPR;
+        raw[rp][i] = *reinterpret_cast<uint4v const *>(q + (long long)(row < m ? row : m - 1) * P.q.d_cols + 8 * (lane % CPR));
+      }
+    }
+    load_ks(steps < DEPTH ? 1 : DEPTH);
+    load_vs(steps < DEPTH ? 1 : DEPTH);
+#pragma unroll
+    for (int rp = 0; rp < RPW; rp++) {
+#pragma unroll
+      for (int i = 0; i < CHUNKS / 2; i++) {
+        *reinterpret_cast<uint4v *>(key_at + KEYS * i * LD) = raw[rp][i];
+      }
+      asm volatile("" ::: "memory");
 #pragma unroll
       for (int kk = 0; kk < DK; kk++) {
-        qf[rp][kk] = *reinterpret_cast<half8 const *>(qr + 32 * kk);
+        qf[rp][kk] = *reinterpret_cast<half8 const *>(strip + c * LD + 32 * kk + 8 * g);
       }
+      asm volatile("" ::: "memory");
     }
   }
-  if (ip < F) {
-    load_k(ip, 0);
-  }
-  half2v acc[OWN][4];  // this thread's chunks of the result (fp16 sums)
-#pragma unroll
-  for (int i = 0; i < OWN; i++) {
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      acc[i][e] = half2v{(_Float16)0.0f, (_Float16)0.0f};
-    }
-  }
-  _Float16 racc = (_Float16)0.0f;  // row sum of row `tid`
   half2v const ones = {(_Float16)1.0f, (_Float16)1.0f};
   constexpr float LOG2E = 1.44269504088896340736f;
+  float4v o[RPW][DB];
+  float rs[RPW];
 
-  int buf = 0;
-  for (int r0 = 0; r0 < F; r0 += IP, buf ^= 1) {
-    int const it = r0 + ip;
-    _Float16 *const round = slots + buf * IP * SLOT;
-    if (it < F) {
-      float4v o[RPW][DB];
-      float rs[RPW];
+  // S^T = K^T . Q^T of a staged pair, exp, row sums: S to fp16, exp in fp32, the result to fp16; the row
+  // sum adds the rounded values in fp32.  pk: the exponentials of keys 8 g .. + 7 of row c.
+  auto scores = [&](bool lone, uint32_t (&pk)[RPW][4]) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      float4v s[RPW];
 #pragma unroll
       for (int rp = 0; rp < RPW; rp++) {
-        rs[rp] = 0.0f;
+        s[rp] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+      }
 #pragma unroll
-        for (int t = 0; t < DB; t++) {
-          o[rp][t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int kk = 0; kk < DK; kk++) {
+        half8 a;
+        if (CM) {
+          a = *reinterpret_cast<half8 const *>(strip + (16 * j + c) * LD + 32 * kk + 8 * g);
+        } else {
+          _Float16 const *ka = strip + (32 * kk + 8 * g + a4) * KLD + 8 * b4 + 4 * j;
+          half4 const lo = lds_read_tr16(ka), hi = lds_read_tr16(ka + 4 * KLD);
+          a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+#pragma unroll
+        for (int rp = 0; rp < RPW; rp++) {
+          s[rp] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qf[rp][kk], s[rp], 0, 0, 0);
         }
       }
-      for (int ch = 0; ch < nchunks; ch++) {
-        int const nbc = (nb - ch * CHB) < CHB ? (nb - ch * CHB) : CHB;
-        load_v(it, ch);
-        // ---- S^T = K^T . Q^T, exp, row sums: S to fp16, exp in fp32, the result to fp16; the
-        // row sum adds the rounded values in fp32
-        uint32_t pk[RPW][PAIRS][4];
-#pragma unroll
-        for (int p = 0; p < PAIRS; p++) {
-          if (2 * p < nbc) {
-            bool const lone = 2 * p + 1 >= nbc;
-            if (!CM) {
-              if (!lone) {
-#pragma unroll
-                for (int i = 0; i < 2 * DK; i++) {
-                  *reinterpret_cast<uint4v *>(k_strip + (16 * i + lane / 4) * KLD + 8 * (lane % 4)) = kr[2 * p + i / DK][i % DK];
-                }
-              } else {
-#pragma unroll
-                for (int i = 0; i < DK; i++) {
-                  *reinterpret_cast<uint4v *>(k_strip + (32 * i + lane / 2) * KLD + 8 * (lane % 2)) = kr[2 * p][i];
-                }
-              }
-              asm volatile("" ::: "memory");  // (a wavefront's LDS operations complete in order)
-            }
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-              if (j == 0 || !lone) {
-                float4v s[RPW];
-#pragma unroll
-                for (int rp = 0; rp < RPW; rp++) {
-                  s[rp] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-                }
-#pragma unroll
-                for (int kk = 0; kk < DK; kk++) {
-                  half8 a;
-                  if (CM) {
-                    a = __builtin_bit_cast(half8, kr[2 * p + j][kk]);
-                  } else {
-                    _Float16 const *ka = k_strip + (32 * kk + 8 * g + a4) * KLD + 16 * j + 4 * b4;
-                    half4 const lo = lds_read_tr16(ka), hi = lds_read_tr16(ka + 4 * KLD);
-                    a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                  }
-#pragma unroll
-                  for (int rp = 0; rp < RPW; rp++) {
-                    s[rp] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qf[rp][kk], s[rp], 0, 0, 0);
-                  }
-                }
-#pragma unroll
-                for (int rp = 0; rp < RPW; rp++) {
-#pragma unroll
-                  for (int h = 0; h < 2; h++) {
-                    half2v const s2 = __builtin_convertvector(float2v{s[rp][2 * h], s[rp][2 * h + 1]}, half2v);
-                    float2v const x2 = {__builtin_amdgcn_exp2f(__builtin_fmaf(static_cast<float>(s2[0]), LOG2E, 0.0f)),
-                                        __builtin_amdgcn_exp2f(__builtin_fmaf(static_cast<float>(s2[1]), LOG2E, 0.0f))};
-                    half2v const e2 = __builtin_convertvector(x2, half2v);
-                    rs[rp] = __builtin_amdgcn_fdot2(e2, ones, rs[rp], false);
-                    pk[rp][p][2 * j + h] = __builtin_bit_cast(uint32_t, e2);
-                  }
-                }
-              }
-            }
-            asm volatile("" ::: "memory");
-          }
-        }
-        // the next chunk's K (this iteration's or the next round's) flies under the rest
-        if (ch + 1 < nchunks) {
-          load_k(it, ch + 1);
-        } else if (it + IP < F) {
-          load_k(it + IP, 0);
-        }
-        if (ch == nchunks - 1) {
-#pragma unroll
-          for (int rp = 0; rp < RPW; rp++) {
-            rs[rp] = sum_lane_groups(rs[rp]);
-            if (HAS_DIV) {
-              // E / sum, rounded to fp32 and then to fp16 as the division is: the reciprocal's product with one
-              // correction is the nearest fp32 number.  (Without it quotients below 2^-14 came out one unit
-              // off where they lie next to the middle of two fp16 numbers.  An infinite sum: 0, or no number
-              // where E is infinite too; E is finite under a finite sum.)
-              float const sum = static_cast<float>(static_cast<_Float16>(rs[rp])), inv = __builtin_amdgcn_rcpf(sum);
-              float const by = __builtin_isinf(sum) ? 0.0f : -sum;
-              auto quotient = [&](_Float16 e) {
-                float q = __builtin_fmaf(static_cast<float>(e), inv, 0.0f);
-                q = __builtin_fmaf(__builtin_fmaf(by, q, static_cast<float>(e)), inv, q);
-                asm volatile("" : "+v"(q));  // (fused with the conversion the last step would round once)
-                return static_cast<_Float16>(q);
-              };
-#pragma unroll
-              for (int p = 0; p < PAIRS; p++) {
-#pragma unroll
-                for (int w = 0; w < 4; w++) {
-                  // (slots of blocks that do not exist hold anything and are never multiplied)
-                  half2v const e2 = __builtin_bit_cast(half2v, pk[rp][p][w]);
-                  half2v const p2 = {quotient(e2[0]), quotient(e2[1])};
-                  pk[rp][p][w] = __builtin_bit_cast(uint32_t, p2);
-                }
-              }
-            }
-          }
-        }
-        // ---- O += P . V, V^T first: o[rp][t][r] = O[row c][16t + 4g + r]
-#pragma unroll
-        for (int p = 0; p < PAIRS; p++) {
-          if (2 * p + 1 < nbc) {
-            if (!CM) {
-#pragma unroll
-              for (int t = 0; t < DB; t++) {
-                int const q = 64 * t + lane;
-                *reinterpret_cast<uint4v *>(v_strip + (q / CPR) * VLD + 8 * (q % CPR)) = vr[p][t];
-              }
-              asm volatile("" ::: "memory");
-            }
-#pragma unroll
-            for (int t = 0; t < DB; t++) {
-              half8 b;
-              if (CM) {
-                b = __builtin_bit_cast(half8, vr[p][t]);
-              } else {
-                _Float16 const *vb = v_strip + (4 * g + a4) * VLD + 16 * t + 4 * b4;
-                half4 const lo = lds_read_tr16(vb), hi = lds_read_tr16(vb + 16 * VLD);
-                b = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-              }
-#pragma unroll
-              for (int rp = 0; rp < RPW; rp++) {
-                uint4v const a = {pk[rp][p][0], pk[rp][p][1], pk[rp][p][2], pk[rp][p][3]};
-                o[rp][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, __builtin_bit_cast(half8, a), o[rp][t], 0, 0, 0);
-              }
-            }
-            asm volatile("" ::: "memory");
-          } else if (2 * p < nbc) {
-            if (!CM) {
-#pragma unroll
-              for (int t = 0; t < DB / 2; t++) {
-                int const q = 64 * t + lane;
-                *reinterpret_cast<uint4v *>(v_strip + (q / CPR) * VLD + 8 * (q % CPR)) = vr[p][t];
-              }
-              asm volatile("" ::: "memory");
-            }
-#pragma unroll
-            for (int t = 0; t < DB; t++) {
-              half4 b;
-              if (CM) {
-                b = __builtin_bit_cast(half4, (g & 1) ? uint2v{vr[p][t].z, vr[p][t].w} : uint2v{vr[p][t].x, vr[p][t].y});
-              } else {
-                b = lds_read_tr16(v_strip + (4 * g + a4) * VLD + 16 * t + 4 * b4);
-              }
-#pragma unroll
-              for (int rp = 0; rp < RPW; rp++) {
-                uint2v const a = {pk[rp][p][0], pk[rp][p][1]};
-                o[rp][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(b, __builtin_bit_cast(half4, a), o[rp][t], 0, 0, 0);
-              }
-            }
-            asm volatile("" ::: "memory");
-          }
-        }
-      }
-      // ---- this iteration's result, fp16, to its slot
-      _Float16 *const slot = round + ip * SLOT;
 #pragma unroll
       for (int rp = 0; rp < RPW; rp++) {
 #pragma unroll
-        for (int t = 0; t < DB; t++) {
-          half2v const lo = __builtin_convertvector(float2v{o[rp][t][0], o[rp][t][1]}, half2v);
-          half2v const hi = __builtin_convertvector(float2v{o[rp][t][2], o[rp][t][3]}, half2v);
-          uint2v const w = {__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
-          *reinterpret_cast<uint2v *>(slot + (16 * rp + c) * LDO + 16 * t + 4 * g) = w;
+        for (int h = 0; h < 2; h++) {
+          half2v const s2 = __builtin_convertvector(float2v{s[rp][2 * h], s[rp][2 * h + 1]}, half2v);
+          float2v const x2 = {__builtin_amdgcn_exp2f(__builtin_fmaf(static_cast<float>(s2[0]), LOG2E, 0.0f)),
+                              __builtin_amdgcn_exp2f(__builtin_fmaf(static_cast<float>(s2[1]), LOG2E, 0.0f))};
+          pk[rp][2 * j + h] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x2, half2v));
         }
-        if (!HAS_DIV && g == 0) {
-          slot[ROWS * LDO + 16 * rp + c] = static_cast<_Float16>(rs[rp]);
-        }
+      }
+    }
+#pragma unroll
+    for (int rp = 0; rp < RPW; rp++) {
+#pragma unroll
+      for (int w = 0; w < 4; w++) {
+        pk[rp][w] = lone && g >= 2 ? 0u : pk[rp][w];
+        rs[rp] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, pk[rp][w]), ones, rs[rp], false);
+      }
+    }
+    asm volatile("" ::: "memory");
+  };
+  // O += P . V of a staged pair, V^T first: o[rp][t][r] = O[row c][16t + 4g + r]
+  auto values = [&](uint32_t const (&pk)[RPW][4]) {
+#pragma unroll
+    for (int t = 0; t < DB; t++) {
+      half8 b;
+      if (CM) {
+        b = *reinterpret_cast<half8 const *>(strip + (16 * t + c) * KLD + 8 * g);
+      } else {
+        _Float16 const *vb = strip + (8 * g + a4) * LD + 16 * t + 4 * b4;
+        half4 const lo = lds_read_tr16(vb), hi = lds_read_tr16(vb + 4 * LD);
+        b = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+#pragma unroll
+      for (int rp = 0; rp < RPW; rp++) {
+        uint4v const a = {pk[rp][0], pk[rp][1], pk[rp][2], pk[rp][3]};
+        o[rp][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, __builtin_bit_cast(half8, a), o[rp][t], 0, 0, 0);
+      }
+    }
+    asm volatile("" ::: "memory");
+  };
+
+  auto start = [&]() {
+#pragma unroll
+    for (int rp = 0; rp < RPW; rp++) {
+      rs[rp] = 0.0f;
+#pragma unroll
+      for (int t = 0; t < DB; t++) {
+        o[rp][t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    }
+  };
+  // ---- the end of an iteration, of the wavefronts' iterations r0 .. r0 + IP - 1
+  auto finish = [&](int r0) {
+    // ---- this iteration's result, fp16, where the strip was
+#pragma unroll
+    for (int rp = 0; rp < RPW; rp++) {
+#pragma unroll
+      for (int t = 0; t < DB; t++) {
+        half2v const lo = __builtin_convertvector(float2v{o[rp][t][0], o[rp][t][1]}, half2v);
+        half2v const hi = __builtin_convertvector(float2v{o[rp][t][2], o[rp][t][3]}, half2v);
+        uint2v const w = {__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
+        *reinterpret_cast<uint2v *>(strip + (16 * rp + c) * LD + 16 * t + 4 * g) = w;
+      }
+      if (!HAS_DIV && g == 0) {
+        strip[ROWS * LD + 16 * rp + c] = static_cast<_Float16>(rs[rp]);
       }
     }
     __syncthreads();
     // ---- the round's results in iteration order, one fp16 rounding per add (a packed fp16 add
-    // is the exact sum rounded once)
+    // is the exact sum rounded once).  Between rounds the sums wait in LDS, not in registers.
     int const n = (F - r0) < IP ? (F - r0) : IP;
+    bool const first = r0 == 0, done = r0 + IP >= F;
+    _Float16 *const og = static_cast<_Float16 *>(const_cast<void *>(P.o.ptr)) + tile_offset(P.o, bx, by, bz, 0);
+    for (int e = tid; e < ROWS * CPR; e += NT) {
+      int const r = e / CPR, at = r * LD + 8 * (e % CPR), row = row_base + r;
+      uint4v sum = {0, 0, 0, 0};
+      if (!first) {
+        sum = *reinterpret_cast<uint4v const *>(sums + at);
+      }
+      for (int u = 0; u < n; u++) {
+        uint4v const v = *reinterpret_cast<uint4v const *>(all + u * STRIP + at);
 #pragma unroll
-    for (int i = 0; i < OWN; i++) {
-      int const e = tid + i * NT;
-      if (e < ROWS * CPR) {
-        _Float16 const *src = round + (e / CPR) * LDO + 8 * (e % CPR);
-        for (int u = 0; u < n; u++) {
-          uint4v const v = *reinterpret_cast<uint4v const *>(src + u * SLOT);
-#pragma unroll
-          for (int w = 0; w < 4; w++) {
-            uint32_t const x = v[w];  // (a bit cast of a vector element itself would read element 0)
-            acc[i][w] = acc[i][w] + __builtin_bit_cast(half2v, x);
-          }
+        for (int w = 0; w < 4; w++) {
+          uint32_t const x = v[w], y = sum[w];  // (a bit cast of a vector element itself would read element 0)
+          sum[w] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, y) + __builtin_bit_cast(half2v, x));
         }
+      }
+      if (!done) {
+        *reinterpret_cast<uint4v *>(sums + at) = sum;
+      } else if (row < m) {
+        *reinterpret_cast<uint4v *>(og + (long long)row * P.o.d_cols + 8 * (e % CPR)) = sum;
       }
     }
     if (!HAS_DIV && tid < ROWS) {
+      _Float16 sum = first ? (_Float16)0.0f : sums[ROWS * LD + tid];
       for (int u = 0; u < n; u++) {
-        racc = racc + round[u * SLOT + ROWS * LDO + tid];
+        sum = sum + all[u * STRIP + ROWS * LD + tid];
+      }
+      if (!done) {
+        sums[ROWS * LD + tid] = sum;
+      } else if (row_base + tid < m) {
+        _Float16 *const rg = static_cast<_Float16 *>(const_cast<void *>(P.r.ptr)) + tile_offset(P.r, bx, by, bz, 0);
+        rg[(long long)(row_base + tid) * P.r.d_cols] = sum;
       }
     }
-  }
-
-  _Float16 *const og = static_cast<_Float16 *>(const_cast<void *>(P.o.ptr)) + tile_offset(P.o, bx, by, bz, 0);
-#pragma unroll
-  for (int i = 0; i < OWN; i++) {
-    int const e = tid + i * NT, row = row_base + e / CPR;
-    if (e < ROWS * CPR && row < m) {
-      uint4v const w = {__builtin_bit_cast(uint32_t, acc[i][0]), __builtin_bit_cast(uint32_t, acc[i][1]),
-                        __builtin_bit_cast(uint32_t, acc[i][2]), __builtin_bit_cast(uint32_t, acc[i][3])};
-      *reinterpret_cast<uint4v *>(og + (long long)row * P.o.d_cols + 8 * (e % CPR)) = w;
+    if (!done) {
+      __syncthreads();  // (the results are read: their place is a strip again)
     }
-  }
-  if (!HAS_DIV && tid < ROWS && row_base + tid < m) {
-    _Float16 *const rg = static_cast<_Float16 *>(const_cast<void *>(P.r.ptr)) + tile_offset(P.r, bx, by, bz, 0);
-    rg[(long long)(row_base + tid) * P.r.d_cols] = racc;
+  };
+
+  if constexpr (HAS_DIV) {
+    for (int r0 = 0; r0 < F; r0 += IP) {
+      int const it = r0 + ip < F ? r0 + ip : F - 1, next = it + IP < F ? it + IP : F - 1;
+      start();
+      uint32_t pk[PAIRS][RPW][4];
+#pragma unroll
+      for (int p = 0; p < PAIRS; p++) {
+        bool const lone = odd && p == PAIRS - 1;
+        stage_k(0, lone);
+        load_k(0, p == PAIRS - 1 ? next : it, p == PAIRS - 1 ? 0 : p + 1);
+        scores(lone, pk[p]);
+      }
+#pragma unroll
+      for (int rp = 0; rp < RPW; rp++) {
+        // E / sum, rounded to fp32 and then to fp16 as the division is: the reciprocal's product with one
+        // correction is the nearest fp32 number.  (Without it quotients below 2^-14 came out one unit
+        // off where they lie next to the middle of two fp16 numbers.  An infinite sum: 0, or no number
+        // where E is infinite too; E is finite under a finite sum.)
+        float const sum = static_cast<float>(static_cast<_Float16>(sum_lane_groups(rs[rp]))), inv = __builtin_amdgcn_rcpf(sum);
+        float const by = __builtin_isinf(sum) ? 0.0f : -sum;
+        auto quotient = [&](_Float16 e) {
+          float q = __builtin_fmaf(static_cast<float>(e), inv, 0.0f);
+          q = __builtin_fmaf(__builtin_fmaf(by, q, static_cast<float>(e)), inv, q);
+          asm volatile("" : "+v"(q));  // (fused with the conversion the last step would round once)
+          return static_cast<_Float16>(q);
+        };
+#pragma unroll
+        for (int p = 0; p < PAIRS; p++) {
+#pragma unroll
+          for (int w = 0; w < 4; w++) {
+            half2v const e2 = __builtin_bit_cast(half2v, pk[p][rp][w]);
+            uint32_t const q2 = __builtin_bit_cast(uint32_t, half2v{quotient(e2[0]), quotient(e2[1])});
+            // (a lone block's missing half stays zero, whatever the sum is)
+            pk[p][rp][w] = odd && p == PAIRS - 1 && g >= 2 ? 0u : q2;
+          }
+        }
+      }
+#pragma unroll
+      for (int p = 0; p < PAIRS; p++) {
+        stage_v(0, odd && p == PAIRS - 1);
+        load_v(0, p == PAIRS - 1 ? next : it, p == PAIRS - 1 ? 0 : p + 1);
+        values(pk[p]);
+      }
+      finish(r0);
+    }
+  } else {
+    int r0 = 0, p = 0;
+    // more: another group of DEPTH steps follows.  An operand of one slot is loaded for the next step, one of
+    // DEPTH in the last step of a group for the next group.
+    auto step = [&](int slot, bool next, auto more) {
+      bool const lone = odd && p == pairs - 1, group = decltype(more)::value && slot == DEPTH - 1;
+      uint32_t pk[RPW][4];
+      stage_k(slot % KS, lone);
+      if (KS == 1 ? next : group) {
+        load_ks(DEPTH);
+      }
+      scores(lone, pk);
+      stage_v(slot % VS, lone);
+      if (VS == 1 ? next : group) {
+        load_vs(DEPTH);
+      }
+      values(pk);
+      p++;
+      if (p == pairs) {
+#pragma unroll
+        for (int rp = 0; rp < RPW; rp++) {
+          rs[rp] = sum_lane_groups(rs[rp]);
+        }
+        finish(r0);
+        start();
+        p = 0;
+        r0 += IP;
+      }
+    };
+    start();
+    int s = 0;
+    // (RPW 2: the last step loads once more what it has; a copy of the loop's body without loads costs registers)
+    for (; s + (RPW == 1 ? DEPTH : 0) < steps; s += DEPTH) {
+#pragma unroll
+      for (int slot = 0; slot < DEPTH; slot++) {
+        step(slot, true, std::true_type{});
+      }
+    }
+#pragma unroll
+    for (int slot = 0; slot < (RPW == 1 ? DEPTH : 0); slot++) {
+      if (slot == 0 || s + slot < steps) {
+        step(slot, slot + 1 < DEPTH && s + slot + 1 < steps, std::false_type{});
+      }
+    }
   }
 }
 

@@ -31,7 +31,8 @@ def _run(rt, spec, what, std=0.125):
 
 
 # rows, key tile, for-loop
-SHAPES = [(1, 48, 5), (15, 16, 1), (17, 80, 3), (33, 64, 9), (64, 48, 2), (65, 112, 4), (130, 32, 13)]
+SHAPES = [(1, 48, 5), (15, 16, 1), (17, 80, 3), (33, 64, 9), (64, 48, 2), (65, 112, 4), (130, 32, 13),
+          (7, 80, 1), (5, 32, 9), (12, 16, 17), (3, 112, 9)]  # one to six pairs of key blocks a wavefront, odd and even
 
 
 @pytest.mark.parametrize("order", [COL, ROW])
@@ -57,6 +58,33 @@ def test_prefill_row_tiles_join(rt, hd, row_tile, blocks, keys, loop, order):
              "plan": W._plan((heads, 1, blocks), loop, [(0, -1, 1), (0, 2, -1), (0, 1, -1)], (-1, 2, 1), (0, 2, 1),
                              W.ATT_OPS, dimx=hd)}]
     _run(rt, spec, f"prefill {hd} {row_tile} x {blocks}, {keys} x {loop} {order}")
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("rows,keys,loop", [(5, 16, 1), (5, 48, 3), (40, 80, 2), (33, 112, 9)])
+def test_keys_of_other_tiles_do_not_matter(rt, rows, keys, loop, order):
+    """The keys around a thread block's own are infinities and NaN: a lone last block of a tile is read as
+    half of a pair, and a block of a wavefront ahead of its turn."""
+    from attention_superoptimizer_amd import workloads as W
+    for make in (W.config2_gqa_decode, W.gqa_inc_decode):
+        spec, _ = make(groups=2, rows=rows, seq=keys * loop * 3, kv_blocks=3, F=loop)
+        for i in (1, 2):
+            spec[i]["layout"] = order
+        ins = _inputs(spec, 0.125)
+        clean = _graph_f16(rt, spec, ins)[3]
+        mine = slice(keys * loop, 2 * keys * loop)  # the second of the three thread blocks that share a query tile
+        for i, axis in ((1, 2), (2, 1)):
+            odd = np.full_like(ins[i], np.nan)
+            odd[::2] = np.inf
+            at = [slice(None)] * 3
+            at[axis] = mine
+            odd[tuple(at)] = ins[i][tuple(at)]
+            ins[i] = odd
+        got = _graph_f16(rt, spec, ins)[3]
+        assert _last_kernels[0] == KERNEL_ATTENTION
+        for g, w in zip(got, clean):
+            third = g.shape[-1] // 3
+            np.testing.assert_array_equal(g[..., third:2 * third], w[..., third:2 * third])
 
 
 def _tile_values(rt, make, groups, keys, order, scores, v):
