@@ -83,6 +83,7 @@ struct AttnParams {
   unsigned perm_ext[3], perm_magic[3], split_magic;
   int rows;     // query rows of the last row group that exist (16, or 8 for an 8-row tile: the
                 // missing rows are zeros in the Q fragment and are never stored)
+  int in_order; // 1: workgroups take blocks in launch order, not in a run of them per XCD
   unsigned long long *trace;  // per-wavefront phase timestamps (attn_direct_kernel<.., TRACE>)
   // attn_direct_kernel: the row sums are stored r_copies times, r_copy_stride elements apart
   // (a plan whose blocks each take a few value columns and all store the same row sums runs
@@ -187,7 +188,8 @@ __device__ __forceinline__ void decode_block(AttnParams const &P, int &bx, int &
   unsigned id = blockIdx.x + ext[0] * (blockIdx.y + ext[1] * blockIdx.z);
   // an XCD (one L2) gets consecutive ids, also where they do not divide by eight
   unsigned const xcd = id % 8, more = total % 8;
-  id = xcd * (total / 8) + (xcd < more ? xcd : more) + id / 8;
+  unsigned const run = xcd * (total / 8) + (xcd < more ? xcd : more) + id / 8;
+  id = P.in_order ? id : run;
   // divisions by the extents are multiply-highs with magics the host computed (exact while
   // id * extent < 2^32, which the host checks): this runs before the first load can go out
   unsigned digit[3];  // digit i of the id belongs to grid dim perm[i]

@@ -152,3 +152,28 @@ def test_division_of_sums_out_of_range(rt, abi, order):
             assert np.array_equal(np.isnan(f), np.isnan(w)) and np.array_equal(np.isposinf(f), np.isposinf(w))
             ok = np.isfinite(w)
             assert_f16_close(f[ok], w[ok], what=make.__name__)
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("rows,keys", [(8, 64), (3, 48)])
+def test_every_block_of_a_long_cache_runs_once(rt, rows, keys, order):
+    """More than 128 MB of keys and values: blocks then run in launch order, key blocks before groups.  Every
+    score is zero and every value of a block one number of its own, so that sums are exact up to the fp16
+    additions of the iterations, which numpy does as well."""
+    from attention_superoptimizer_amd import workloads as W
+    groups, kv_blocks = 16, 64
+    loop = 1 + (128 << 20) // (groups * kv_blocks * keys * 64 * 4)
+    seq = keys * loop * kv_blocks
+    spec, _ = W.gqa_inc_decode(groups=groups, rows=rows, seq=seq, kv_blocks=kv_blocks, F=loop)
+    for i in (1, 2):
+        spec[i]["layout"] = order
+    ids = (1 + np.arange(groups * kv_blocks).reshape(groups, kv_blocks) / 1024).astype(np.float16)
+    v = np.broadcast_to(np.repeat(ids, keys * loop, 1)[:, :, None], (groups, seq, 64))
+    o, r = _graph_f16(rt, spec[:4], {0: np.zeros((groups, rows, 64), np.float16), 1: normal_f16([groups, 64, seq], 1.0, 3), 2: v})[3]
+    assert _last_kernels[0] == KERNEL_ATTENTION
+    tile = (ids.astype(np.float64) * keys).astype(np.float16)
+    want, sums = np.zeros_like(tile), np.float16(0)
+    for _ in range(loop):
+        want, sums = want + tile, sums + np.float16(keys)
+    np.testing.assert_array_equal(r, np.full_like(r, sums))
+    np.testing.assert_array_equal(o.reshape(groups, rows, kv_blocks, 64), np.broadcast_to(want[:, None, :, None], (groups, rows, kv_blocks, 64)))
