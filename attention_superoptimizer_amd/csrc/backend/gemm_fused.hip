@@ -331,25 +331,35 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   if (groups * 8 * S * widest >= (1LL << 32)) {
     return 0;
   }
-  // By itself only where the launch, not the traffic, sets the time (weights of a few MB): a
-  // 16-column strip uses 32 bytes of every 128-byte line it pulls into a compute unit's L1, and
-  // every piece re-reads the activation rows, so the L2 -> L1 traffic is 4-5 x the bytes of the
-  // plan (measured on the LoRA plan: 202 MB of requests for 34 MB), which is what bounds a plan
-  // of tens of MB; the range-splitting kernel moves whole lines once.
-  // With column-major weights a piece's columns are whole lines of its own, read straight into
-  // registers, so the first cost is gone; the one launch then also wins for a two-weight plan of up to
-  // 64 MB (16 x 2560 x 6400, 65 MB: 16.2 us against 17.1 of the streaming kernel and its fold; 235 MB:
-  // 54.6 against 48.4) but not for the others, where each wavefront's loads of its activation rows
-  // and of the lora A tile outnumber its weight loads.
+  // One launch, whose pieces of 16 columns each read the activation rows, against whole lines moved once by the
+  // range-splitting kernel and a second launch that adds its ranges.
+  // Row-major weights: a 16-column strip uses 32 bytes of every line it pulls into a compute unit's vector cache,
+  // so only where the launch sets the time (16 rows, in us, here / there: 3840 columns in 128-k iterations, 16 MB,
+  // 6.7 / 8.3; 6400, 26 MB, 9.8 / 9.1; 64-column blocks of 256 k fill LDS with fewer wavefronts: 1280 columns,
+  // 10 MB, 9.6 / 7.6).
+  // Column-major weights: a piece's columns are whole lines of its own, and the line lies far out, where the
+  // activation rows that the pieces read outnumber what the second launch costs.  One weight (64 rows x 12800 x 4096
+  // 45 / 62, 8 x 28672 x 4096, 235 MB of weights, 39.6 / 53, but 64 x 28672 x 1024, 7168 pieces, 22.2 / 19.6);
+  // a LoRA tile or a second activation makes it three operand rows a column (lora 16 x 4096 x 4096 10.1 / 11.1,
+  // x 8192 17.3 / 17.1); two weights 16 x 2560 x 6400, 65 MB, 16.2 / 17.1, 235 MB 54.6 / 48.4.
   long long const weight_bytes = blocks * F * (long long)(G.nb * G.KT * 64 + (G.lora ? G.KT * 16 : 0)) * 2;
-  bool const two_weights_cm = G.wcm && G.nb == 2 && blocks * S <= 4096 && weight_bytes <= (68LL << 20);
-  if (s.gemm_mode == 0 && !two_weights_cm && (blocks * S > 1024 || weight_bytes > (8LL << 20))) {
+  bool const three = G.lora || G.pro == PRO_SILU_MUL;
+  // SiLU(a) * u is done again by each of a block's pieces, so a long k of it is worth the other kernel's second
+  // launch (the two products of a gated MLP, 3 rows: 1920 x 6400 25.7 / 23.0, 1280 x 3840 15.4 / 14.3, but 2560 x 1920
+  // 13.1 / 16.0, and 16 x 2944 x 4032, whose 64-k iterations leave that kernel four times the slab, 20.6 / 25.0).
+  bool const wide = G.pro == PRO_SILU_MUL ? G.KT > 64 && (!G.wcm || F * G.KT > 2048) : G.KT == 256 && !G.wcm;
+  long long const most_bytes = (wide ? 8LL : (!G.wcm ? 17LL : (three ? 48LL : (G.nb == 2 ? 68LL : 256LL)))) << 20;
+  if (s.gemm_mode == 0 && (blocks * S > (G.wcm ? 4096 : 1024) || weight_bytes > most_bytes)) {
     return 0;
   }
-  int const strips = G.nb + (G.lora ? 1 : 0);
-  int const wave_bytes = G.wcm ? 0 : strips * G.KT * 32 + (G.lora ? 512 : 0);
+  int const wave_bytes = lanes_wave_bytes(G.KT, G.nb, G.lora, G.wcm, G.pro);
   int const slot_bytes = F * G.nb * 512;
-  int ip = F < 16 ? F : 16;
+  // Workgroups of 16 wavefronts while about one round of them covers the grid; half that where two share a compute
+  // unit and one's loads can run under the other's products (64 rows x 6400 x 4096 in 256-k iterations: 25.5 -> 19.7
+  // us; 16 rows x 1280, 80 workgroups: 5.2 against 5.7 the other way).  With three operand rows a column the
+  // registers of 16 wavefronts fill the unit either way (a gated MLP of 16 x 1920 x 6400: 26.4 against 27.7).
+  int const waves = G.nb == 1 && !three && (long long)blocks * S * G.KT > 98304 ? 8 : 16;
+  int ip = F < waves ? F : waves;
   while (ip > 1 && ip * wave_bytes + slot_bytes > s.max_lds) {
     ip = (ip + 1) / 2;
   }

@@ -631,11 +631,18 @@ __device__ __forceinline__ half4 lane_tr16(_Float16 const *p) {
   return __builtin_bit_cast(half4, v);
 }
 
-// Column-major weights (WCM): column n of a weight tile is KT contiguous halfs, so a lane's
-// operand -- eight consecutive k of one column -- is 16 contiguous bytes of global memory, like
-// its activation rows: every operand goes straight into registers, the strips and the
-// transposing reads disappear, LDS holds the product slots only, and a piece's sixteen columns
-// are sixteen streams of whole cache lines that no other workgroup touches.
+// Activations, and column-major weights (WCM: column n of a weight tile is KT contiguous halfs, so a piece's
+// sixteen columns are sixteen streams of whole cache lines that no other workgroup touches), are
+// [16][KT] tiles whose operands are 16 contiguous bytes.  They come in units of 64 k, a line of each row, into
+// registers in the order they have in memory and become operands through 2 KB of LDS each: read as operands,
+// sixteen lanes in a row would be sixteen rows, and a compute unit then gets 15.7 bytes a cycle from its
+// vector cache against 58 (32 rows x 2240 x 1856 in 64-k iterations: 9.0 -> 5.5 us).
+constexpr int kUnitBytes = 2048;  // [16][64 k]
+// bytes of a wavefront's strips: the units being turned; row-major weights, the [16][16] piece of lora B
+constexpr int lanes_wave_bytes(int KT, int nb, bool lora, bool wcm, int pro) {
+  int const units = 1 + (pro == PRO_SILU_MUL ? 1 : 0) + (wcm ? nb + (lora ? 1 : 0) : 0);
+  return units * kUnitBytes + (wcm ? 0 : (nb + (lora ? 1 : 0)) * KT * 32 + (lora ? 512 : 0));
+}
 template <int KT, int NB, int PRO, bool LORA, bool WCM>
 __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
   fetch_kernel_arguments<sizeof(LaneParams), 4>();  // every line of the block, one trip (blockDim.x is read)
@@ -643,8 +650,8 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   constexpr int KS = KT / 32;                                // MFMA steps (and 1 KB loads) per strip
   constexpr int STRIPS = NB + (LORA ? 1 : 0);
-  // (row-major weights: the strips, + the [16][16] piece of lora B)
-  constexpr int WAVE_BYTES = WCM ? 0 : STRIPS * KT * 32 + (LORA ? 512 : 0);
+  constexpr int KU = KT / 64;                                // units
+  constexpr int WAVE_BYTES = lanes_wave_bytes(KT, NB, LORA, WCM, PRO), UNITS = 1 + (PRO == PRO_SILU_MUL) + (WCM ? STRIPS : 0);
   int const tid = threadIdx.x, lane = tid % 64, IP = blockDim.x / 64;
   int const ip = __builtin_amdgcn_readfirstlane(tid / 64);  // (wave-uniform: addresses stay scalar)
   int const g = lane / 16, c = lane % 16;
@@ -667,7 +674,7 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
   int const bx = (int)((unsigned)blk - q1 * (unsigned)L.gx), by = (int)(q1 - q2 * (unsigned)L.gy), bz = (int)q2;
   int const n0 = 16 * piece;
 
-  unsigned char *mine = lds + ip * WAVE_BYTES;
+  unsigned char *const units = lds + ip * WAVE_BYTES, *const mine = units + UNITS * kUnitBytes;
   _Float16 const *strip[STRIPS];
 #pragma unroll
   for (int b = 0; b < STRIPS; b++) {
@@ -680,9 +687,25 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
   // transposing reads
   int const ld_row = lane / 2, ld_half = lane % 2;
   int const tr_off = (c / 4) * 16 + 4 * (c % 4);
-  int const row = 16 * mt + c;                 // activation row of this lane's fragments
-  bool const row_ok = row < M;
-  int const row_ld = row_ok ? row : M - 1;
+  bool const row_ok = 16 * mt + c < M;         // activation row of this lane's fragments
+  // units: lane l has chunk l % 8 of rows l / 8 and 8 + l / 8; chunk q of row r lies at q ^ (r / 2 % 8)
+  int const l8 = lane / 8, ch8 = lane % 8;
+  int const x_row[2] = {16 * mt + l8 < M ? 16 * mt + l8 : M - 1, 16 * mt + 8 + l8 < M ? 16 * mt + 8 + l8 : M - 1};
+  auto load_rows = [&](_Float16 const *tile, int ld, int r0, int r1, uint4v (&to)[KU][2]) {
+#pragma unroll
+    for (int u = 0; u < KU; u++) {
+      to[u][0] = *reinterpret_cast<uint4v const *>(tile + (long long)r0 * ld + 64 * u + 8 * ch8);
+      to[u][1] = *reinterpret_cast<uint4v const *>(tile + (long long)r1 * ld + 64 * u + 8 * ch8);
+    }
+  };
+  auto put_unit = [&](int which, uint4v const (&from)[2]) {
+    unsigned char *const to = units + which * kUnitBytes + 128 * l8;
+    *reinterpret_cast<uint4v *>(to + 16 * (ch8 ^ (l8 / 2))) = from[0];
+    *reinterpret_cast<uint4v *>(to + 1024 + 16 * (ch8 ^ (l8 / 2 + 4))) = from[1];
+  };
+  auto operand = [&](int which, int s) {  // row c, k 32 s + 8 g ..
+    return *reinterpret_cast<half8 const *>(units + which * kUnitBytes + 128 * c + 16 * ((4 * s + g) ^ (c / 2)));
+  };
 
   half4 lb_frag = {(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
   if (LORA) {
@@ -703,19 +726,14 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     // ---- issue everything this iteration needs -------------------------------------------
-    uint4v wr[WCM ? STRIPS : 1][KS];  // column-major weights: the operands themselves
+    uint4v wr[WCM ? STRIPS : 1][KU][2], xr[KU][2], ur[KU][2];
 #pragma unroll
     for (int b = 0; b < STRIPS; b++) {
       GTile const &bt = b == NB ? P.la : (b == 0 ? P.b0 : P.b1);
       int const col0 = b == NB ? 0 : n0;  // the lora A tile is [KT][16]: whole
       if (WCM) {
-        // W^T[col0 + c][32j + 8g + 0..7]
-        _Float16 const *src = static_cast<_Float16 const *>(bt.ptr) + gtile_offset(bt, bx, by, bz, it) +
-                              (long long)(col0 + c) * bt.d_cols + 8 * g;
-#pragma unroll
-        for (int j = 0; j < KS; j++) {
-          wr[b][j] = *reinterpret_cast<uint4v const *>(src + 32 * j);
-        }
+        load_rows(static_cast<_Float16 const *>(bt.ptr) + gtile_offset(bt, bx, by, bz, it), bt.d_cols, col0 + l8, col0 + 8 + l8,
+                  wr[WCM ? b : 0]);
       } else {
         _Float16 const *src = static_cast<_Float16 const *>(bt.ptr) + gtile_offset(bt, bx, by, bz, it) + col0;
         uint32_t const off = (uint32_t)((ld_row * bt.d_cols + 8 * ld_half) * 2);
@@ -725,111 +743,103 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
         }
       }
     }
-    _Float16 const *a0 = static_cast<_Float16 const *>(P.a0.ptr) + gtile_offset(P.a0, bx, by, bz, it) +
-                         (long long)row_ld * P.a0.d_cols + 8 * g;
-    uint4v xr[KS], ur[PRO == PRO_SILU_MUL ? KS : 1];
-#pragma unroll
-    for (int j = 0; j < KS; j++) {
-      xr[j] = *reinterpret_cast<uint4v const *>(a0 + 32 * j);
-    }
+    load_rows(static_cast<_Float16 const *>(P.a0.ptr) + gtile_offset(P.a0, bx, by, bz, it), P.a0.d_cols, x_row[0], x_row[1], xr);
     if (PRO == PRO_SILU_MUL) {
-      _Float16 const *a1 = static_cast<_Float16 const *>(P.a1.ptr) + gtile_offset(P.a1, bx, by, bz, it) +
-                           (long long)row_ld * P.a1.d_cols + 8 * g;
-#pragma unroll
-      for (int j = 0; j < KS; j++) {
-        ur[j] = *reinterpret_cast<uint4v const *>(a1 + 32 * j);
-      }
+      load_rows(static_cast<_Float16 const *>(P.a1.ptr) + gtile_offset(P.a1, bx, by, bz, it), P.a1.d_cols, x_row[0], x_row[1], ur);
     }
-    // ---- one wait for all of it (direct-to-LDS loads and register loads do not complete in
-    // one order, so nothing short of "all" says that a particular one has landed) ------------
+    if (!WCM) {
+      // ---- one wait for all of it (direct-to-LDS loads and register loads do not complete in
+      // one order, so nothing short of "all" says that a particular one has landed)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+      asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
 #pragma unroll
-    for (int j = 0; j < KS; j++) {
-      asm volatile("" : "+v"(xr[j]));  // (no use of a fragment moves above the wait)
+      for (int u = 0; u < KU; u++) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          asm volatile("" : "+v"(xr[u][h]));  // (no use moves above the wait)
+          if (PRO == PRO_SILU_MUL) {
+            asm volatile("" : "+v"(ur[u][h]));
+          }
+        }
+      }
+#pragma clang diagnostic pop
+    }
+    float4v o[NB], d = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      o[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int u = 0; u < KU; u++) {
+      put_unit(0, xr[u]);
       if (PRO == PRO_SILU_MUL) {
-        asm volatile("" : "+v"(ur[j]));
+        put_unit(1, ur[u]);
       }
       if (WCM) {
 #pragma unroll
         for (int b = 0; b < STRIPS; b++) {
-          asm volatile("" : "+v"(wr[b][j]));
+          put_unit(UNITS - STRIPS + b, wr[WCM ? b : 0][u]);
         }
       }
+      asm volatile("" ::: "memory");  // (a wavefront's LDS operations complete in order)
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        int const j = 2 * u + h;
+        // ---- activation fragments: rows past M are zero, prologue in registers
+        half8 x = operand(0, h);
+        if (PRO == PRO_EXP || PRO == PRO_SILU) {
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            x[e] = static_cast<_Float16>(prologue(PRO, static_cast<float>(x[e])));
+          }
+        } else if (PRO == PRO_SILU_MUL) {
+          half8 const um = operand(1, h);
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            _Float16 const sg = static_cast<_Float16>(prologue(PRO_SILU, static_cast<float>(x[e])));
+            x[e] = static_cast<_Float16>(static_cast<float>(sg) * static_cast<float>(um[e]));
+          }
+        }
+        if (!row_ok) {
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            x[e] = (_Float16)0.0f;
+          }
+        }
+        // ---- products: o[r] = O[m = c][n = n0 + 4g + r]; lora's inner one, transposed:
+        // d[r] = (X.A)[m = c][n = 4g + r]
+#pragma unroll
+        for (int b = 0; b < STRIPS; b++) {
+          half8 w;
+          if (WCM) {
+            w = operand(UNITS - STRIPS + b, h);
+          } else {
+            _Float16 const *wp = strip[b] + (32 * j + 8 * g) * 16 + tr_off;
+            half4 const lo = lane_tr16(wp), hi = lane_tr16(wp + 64);
+            w = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+          }
+          float4v &to = b == NB ? d : o[b < NB ? b : 0];
+          to = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, to, 0, 0, 0);
+        }
+      }
+      asm volatile("" ::: "memory");
     }
-#pragma clang diagnostic pop
-    // ---- activation fragments: rows past M are zero, prologue in registers -----------------
-    half8 x[KS];
+    half4 dfrag;
 #pragma unroll
-    for (int j = 0; j < KS; j++) {
-      half8 v = __builtin_bit_cast(half8, xr[j]);
-      if (PRO == PRO_EXP || PRO == PRO_SILU) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          v[e] = static_cast<_Float16>(prologue(PRO, static_cast<float>(v[e])));
-        }
-      } else if (PRO == PRO_SILU_MUL) {
-        half8 const u = __builtin_bit_cast(half8, ur[j]);
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          _Float16 const sg = static_cast<_Float16>(prologue(PRO_SILU, static_cast<float>(v[e])));
-          v[e] = static_cast<_Float16>(static_cast<float>(sg) * static_cast<float>(u[e]));
-        }
-      }
-      if (!row_ok) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          v[e] = (_Float16)0.0f;
-        }
-      }
-      x[j] = v;
+    for (int r = 0; r < 4; r++) {
+      dfrag[r] = static_cast<_Float16>(d[r]);
     }
-    // ---- lora inner product, transposed: d[r] = (X.A)[m = c][n = 4g + r] -------------------
-    half4 dfrag = {(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
-    if (LORA) {
-      float4v d = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int j = 0; j < KS; j++) {
-        half8 a;
-        if (WCM) {
-          a = __builtin_bit_cast(half8, wr[WCM ? NB : 0][j]);
-        } else {
-          _Float16 const *ap = strip[NB] + (32 * j + 8 * g) * 16 + tr_off;
-          half4 const lo = lane_tr16(ap), hi = lane_tr16(ap + 64);
-          a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        }
-        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, x[j], d, 0, 0, 0);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        dfrag[r] = static_cast<_Float16>(d[r]);
-      }
-    }
-    // ---- products: o[r] = O[m = c][n = n0 + 4g + r] ----------------------------------------
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-      float4v o = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int j = 0; j < KS; j++) {
-        half8 w;
-        if (WCM) {
-          w = __builtin_bit_cast(half8, wr[WCM ? b : 0][j]);
-        } else {
-          _Float16 const *wp = strip[b] + (32 * j + 8 * g) * 16 + tr_off;
-          half4 const lo = lane_tr16(wp), hi = lane_tr16(wp + 64);
-          w = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        }
-        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x[j], o, 0, 0, 0);
-      }
       if (LORA) {
         half4 const w = WCM ? lb_frag : lane_tr16(lb_piece + (4 * g) * 16 + tr_off);  // B[k = 4g ..][n = c]
-        o = __builtin_amdgcn_mfma_f32_16x16x16f16(w, dfrag, o, 0, 0, 0);
+        o[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(w, dfrag, o[b], 0, 0, 0);
       }
       half4 p16;
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        p16[r] = static_cast<_Float16>(o[r]);
+        p16[r] = static_cast<_Float16>(o[b][r]);
       }
       *reinterpret_cast<half4 *>(slots + ((it * NB + b) * 16 + c) * 16 + 4 * g) = p16;
     }

@@ -81,3 +81,18 @@ def test_infinities_and_nan(rt, abi, family, option, value, order):
         ok = np.isfinite(want)
         assert not ok.all() and (ok.any() or i > 0)  # (a NaN column of the first operator is in all sums of a second)
         assert_f16_close(f[ok], want[ok], what=family)
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("m,blocks,kt,loop", [
+    (64, 25, 256, 3), (49, 97, 128, 9), (33, 25, 64, 17), (1, 97, 256, 9), (17, 9, 256, 16), (7, 385, 64, 2)])
+def test_one_launch_of_many_pieces(rt, abi, m, blocks, kt, loop, order):
+    """The one-launch kernel around its line between 16 and 8 wavefronts a workgroup (pieces x k = 98304),
+    with loops that its wavefronts do not divide and rows around the edges of 16."""
+    from attention_superoptimizer_amd import workloads as W
+    spec, _ = W.tiled_matmul(m, 64 * blocks, kt * loop, (blocks, 1, 1), loop, (-1, -1, -1), (1, -1, -1), (1, -1, -1))
+    assert abi.mi355_set_option(7, 2) == 0
+    try:
+        _run(rt, spec, order, f"pieces {m} x {blocks}, {kt} x {loop} {order}")
+    finally:
+        assert abi.mi355_set_option(7, 0) == 0
