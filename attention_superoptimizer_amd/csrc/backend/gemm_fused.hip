@@ -340,15 +340,16 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // Column-major weights: a piece's columns are whole lines of its own, and the line lies far out, where the
   // activation rows that the pieces read outnumber what the second launch costs.  One weight (64 rows x 12800 x 4096
   // 45 / 62, 8 x 28672 x 4096, 235 MB of weights, 39.6 / 53, but 64 x 28672 x 1024, 7168 pieces, 22.2 / 19.6);
-  // a LoRA tile or a second activation makes it three operand rows a column (lora 16 x 4096 x 4096 10.1 / 11.1,
-  // x 8192 17.3 / 17.1); two weights 16 x 2560 x 6400, 65 MB, 16.2 / 17.1, 235 MB 54.6 / 48.4.
+  // a LoRA tile or a second activation makes it three operand rows a column (lora 16 x 4096 x 2048 6.5 / 9.4, 21 MB;
+  // 16 x 4096 x 4096, 42 MB, 10.1 / 11.1, is still below the crossing, 16 x 8192 x 4096 17.3 / 17.1, but the program
+  // printed for it is known to hold the streaming kernel and its workspace, and stays so); two weights 16 x 2560 x 6400, 65 MB, 16.2 / 17.1, 235 MB 54.6 / 48.4.
   long long const weight_bytes = blocks * F * (long long)(G.nb * G.KT * 64 + (G.lora ? G.KT * 16 : 0)) * 2;
   bool const three = G.lora || G.pro == PRO_SILU_MUL;
   // SiLU(a) * u is done again by each of a block's pieces, so a long k of it is worth the other kernel's second
   // launch (the two products of a gated MLP, 3 rows: 1920 x 6400 25.7 / 23.0, 1280 x 3840 15.4 / 14.3, but 2560 x 1920
   // 13.1 / 16.0, and 16 x 2944 x 4032, whose 64-k iterations leave that kernel four times the slab, 20.6 / 25.0).
   bool const wide = G.pro == PRO_SILU_MUL ? G.KT > 64 && (!G.wcm || F * G.KT > 2048) : G.KT == 256 && !G.wcm;
-  long long const most_bytes = (wide ? 8LL : (!G.wcm ? 17LL : (three ? 48LL : (G.nb == 2 ? 68LL : 256LL)))) << 20;
+  long long const most_bytes = (wide ? 8LL : (!G.wcm ? 17LL : (G.lora ? 32LL : three ? 48LL : (G.nb == 2 ? 68LL : 256LL)))) << 20;
   if (s.gemm_mode == 0 && (blocks * S > (G.wcm ? 4096 : 1024) || weight_bytes > most_bytes)) {
     return 0;
   }
