@@ -116,7 +116,7 @@ std::string literal(LaneParams const &L) {
   return t;
 }
 std::string literal(StreamParams const &L) {
-  return literal(L.g, "G") + "    mi355::StreamParams P{};\n    P.g = G;\n" + emit_fmt("    P.results = %d;\n", L.results);
+  return literal(L.g, "G") + "    mi355::StreamParams P{};\n    P.g = G;\n" + emit_fmt("    P.results = %d;\n    P.strips = %d;\n", L.results, L.strips);
 }
 char const *tf(bool b) { return b ? "true" : "false"; }
 
@@ -446,24 +446,30 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A)
     return 0;
   }
   long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
-  int const ring = 4 * kStreamRing * stream_slot_bytes(G.pro, G.lora, mt);
-  int const results = F * G.nb * G.M * 128;
-  size_t const slab = (size_t)blocks * results;
+  int const ring = 4 * kStreamRing * stream_slot_bytes(G.pro, G.lora, G.M <= 8 ? 0 : mt);
+  int const results = F * G.M * 128;  // of one weight
+  size_t const slab = (size_t)blocks * G.nb * results;
+  // Strips of 16 columns where they fill most of the chip and two workgroups fit on a compute unit (4 rows, us, strips
+  // / ranges: 3840 columns x 4096, 240 workgroups, 7.6 / 10.7; 28672 39.9 / 51.6; two weights of 3072 x 8192
+  // with a gated MLP's second product 37.9 / 40.1).
+  int const eights = G.M <= 8 ? 1 : 2, strip_ring = 4 * columns_ring(eights) * columns_slot_bytes(eights);
+  int const strip_lds = strip_ring + F * G.M * 32;
+  bool const strips = G.wcm && G.pro == PRO_NONE && !G.lora && G.M <= 16 && 4 * G.nb * blocks >= 192 && 2 * strip_lds <= s.max_lds;
   // One range per block where the blocks alone occupy the chip and a wavefront has a few steps to
   // make: no slab and no second launch (4 x 8192 x 2048 in 64-k iterations: 8.9 us against 12).
   // Otherwise four iterations, one per wavefront, to a range, as far as that many workgroups are
   // resident at a time: a slot of 10 KB leaves room for two on a compute unit, which then also gain
   // from taking turns; a larger one for one, where a second round would start late (32 x 3840 x 5120:
   // 13.8 us in 240 workgroups, 16.0 in 300).
-  int const steps = (F + 3) / 4 * (G.KT / 64) * G.nb;
+  int const steps = (F + 3) / 4 * (G.KT / 64);
   bool const fits = ring + results <= s.max_lds;
   int ks = 1;
   EmitSink *const sink = emit_sink();
-  if (!(fits && blocks >= 96 && steps <= 8) && slab <= (sink ? kEmitScratchBytes : s.scratch_bytes)) {
-    long long const most = (ring <= 80 * 1024 ? 1024 : 256) / blocks;
+  if (!(fits && blocks * G.nb >= 96 && steps <= 8) && slab <= (sink ? kEmitScratchBytes : s.scratch_bytes)) {
+    long long const most = (ring <= 80 * 1024 ? 1024 : 256 / G.nb) / blocks;
     ks = (int)std::max<long long>(1, std::min<long long>((F + 3) / 4, most));
   }
-  if (ks == 1 && !fits) {
+  if (ks == 1 && !fits && !strips) {
     return 0;
   }
   int const per = (F + ks - 1) / ks;
@@ -476,11 +482,18 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A)
     L.g.scratch = ks > 1 ? reinterpret_cast<_Float16 *>(kEmitScratch) : nullptr;
   }
   L.results = ring;
-  int const lds = ring + (ks == 1 ? results : 0);
-  if ((long long)P.grid[0] * ks > 2147483647LL) {
+  int lds = ring + (ks == 1 ? results : 0);
+  L.strips = strips;
+  if (strips) {
+    ks = L.g.ksplit = 1;
+    L.g.scratch = nullptr;
+    L.results = strip_ring;
+    lds = strip_lds;
+  }
+  if ((long long)P.grid[0] * G.nb * (strips ? 4 : ks) > 2147483647LL) {
     return 0;
   }
-  dim3 const grid(P.grid[0] * ks, P.grid[1], P.grid[2]);
+  dim3 const grid(P.grid[0] * G.nb * (strips ? 4 : ks), P.grid[1], P.grid[2]);
   int rc = 0;
 #define MI355_STREAM_CASE(NBV, PROV, LORAV, MTV)                                            \
   if (G.nb == NBV && G.pro == PROV && G.lora == LORAV && mt == MTV) {                       \

@@ -15,10 +15,14 @@
 // slots are added in ITERATION order with one rounding per add: the arithmetic of the sequential loop
 // (reference src/kernel/triton_code_gen.cc:223-232).
 //
-// What bounds it is memory: 235 MB (two weights of 4096 x 14336, column-major) 57 us in the one-launch
-// kernel, 45 here (5.2 TB/s; a kernel that only reads them takes 38); 118 MB, one weight, 19 us (6.2).
-// The gate's activations (silu of 14336 x 16 values in every column block) are vector work on top:
-// 25 us for 117 MB.
+// Two weights are two sets of workgroups (for twice the activations' bytes): seven to a compute unit instead of
+// three and a half leave less of the last round empty (two weights of 4096 x 14336: 44.3 -> 42.3 us).
+//
+// What bounds it is memory: 235 MB (those two weights, column-major) 42 us (5.6 TB/s; a kernel that only reads
+// them takes 38); 118 MB, one weight, 19 us (6.2).  The gate's activations (silu of 14336 x 16 values in every
+// column block) are vector work on top: 24 us for 117 MB.  Up to 8 rows a slot holds 8, which leaves room for two
+// workgroups also beside the gate's second operand, and a silu is made by one lane instead of two (gated MLP of
+// 8 x 4096 x 14336: 78.9 -> 77.1 us).
 #pragma once
 
 #include "gemm.h"
@@ -28,6 +32,7 @@ namespace mi355 {
 struct StreamParams {
   GemmParams g;
   int results;  // byte offset of the iterations' results in LDS (one range only)
+  int strips;   // a workgroup takes 16 columns and the whole for-loop (stream_columns)
 };
 // Slots per wavefront.  A third one changes nothing (118 MB of weights: 19.0 us with either), two
 // workgroups on a compute unit, which two slots leave room for, do.
@@ -42,26 +47,28 @@ __device__ __forceinline__ void stream_wait() {
 }
 
 // Bytes of a slot: the weight tile, then activation rows (and the gate's second operand), then lora A.
+// mt counts 16-row groups; 0 is one of 8 rows.
 constexpr int stream_slot_bytes(int pro, bool lora, int mt) {
-  return 8192 + 2048 * mt * (pro == PRO_SILU_MUL ? 2 : 1) + (lora ? 2048 : 0);
+  return 8192 + (mt > 0 ? 2048 * mt : 1024) * (pro == PRO_SILU_MUL ? 2 : 1) + (lora ? 2048 : 0);
 }
 
-template <int NB, int PRO, bool LORA, bool WCM, int MT>
-__global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) {
-  fetch_kernel_arguments<sizeof(StreamParams), 2>();
+template <int NB, int PRO, bool LORA, bool WCM, int GROUPS>
+__device__ __forceinline__ void stream_block(StreamParams const &S) {
   GemmParams const &P = S.g;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  constexpr int W = 4, SLOT = stream_slot_bytes(PRO, LORA, MT);
-  constexpr int X_LOADS = 2 * MT * (PRO == PRO_SILU_MUL ? 2 : 1) + (LORA ? 2 : 0);  // besides the weights' 8
-  constexpr int X_AT = 8192, U_AT = X_AT + 2048 * MT, LA_AT = U_AT + (PRO == PRO_SILU_MUL ? 2048 * MT : 0);
+  constexpr int MT = GROUPS > 0 ? GROUPS : 1, EIGHTS = GROUPS > 0 ? 2 * GROUPS : 1;  // 16-row groups, loads of 8 rows
+  constexpr int W = 4, SLOT = stream_slot_bytes(PRO, LORA, GROUPS);
+  constexpr int X_LOADS = EIGHTS * (PRO == PRO_SILU_MUL ? 2 : 1) + (LORA ? 2 : 0);  // besides the weights' 8
+  constexpr int X_AT = 8192, U_AT = X_AT + 1024 * EIGHTS, LA_AT = U_AT + (PRO == PRO_SILU_MUL ? 1024 * EIGHTS : 0);
   int const tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   int const g = lane / 16, c = lane % 16;
   int const M = P.M, F = P.forloop_range, subs = P.KT / 64;
   constexpr int R = kStreamRing;
 
-  int const gx = gridDim.x / P.ksplit;
+  int const gx = gridDim.x / (P.ksplit * NB);
   int const ks = blockIdx.x % P.ksplit;  // (the ranges of a block next to each other)
-  int const bx = blockIdx.x / P.ksplit, by = blockIdx.y, bz = blockIdx.z;
+  int const block_weight = blockIdx.x / P.ksplit, b = NB == 2 ? block_weight % 2 : 0;
+  int const bx = block_weight / NB, by = blockIdx.y, bz = blockIdx.z;
   int const per = (F + P.ksplit - 1) / P.ksplit;
   int const it_begin = ks * per, n_it = (it_begin + per < F ? it_begin + per : F) - it_begin;
   int const block_linear = bx + gx * (by + gridDim.y * bz);
@@ -83,17 +90,14 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) 
   // the LDS tile (the chunk a lane FETCHES moves, its place is fixed).
   auto swizzle = [](int row) { return WCM ? (row >> 1) & 7 : (((row >> 1) & 1) | ((row >> 2) & 2)) << 1; };
   int const l8 = lane / 8, ch8 = lane % 8;
-  uint32_t w_off[2][NB];  // rows 8 j + l8: the swizzle of rows 8 apart differs, so even and odd j
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    int const ld = b == 0 ? P.b0.d_cols : P.b1.d_cols;
-    w_off[0][b] = 2u * (uint32_t)(l8 * ld + 8 * (ch8 ^ swizzle(l8)));
-    w_off[1][b] = 2u * (uint32_t)(l8 * ld + 8 * (ch8 ^ swizzle(8 + l8)));
-  }
+  GTile const &bt = NB == 2 && b == 1 ? P.b1 : P.b0;
+  // rows 8 j + l8: the swizzle of rows 8 apart differs, so even and odd j
+  uint32_t const w_off[2] = {2u * (uint32_t)(l8 * bt.d_cols + 8 * (ch8 ^ swizzle(l8))),
+                             2u * (uint32_t)(l8 * bt.d_cols + 8 * (ch8 ^ swizzle(8 + l8)))};
   // activation rows 8 j + l / 8 (rows past the tile re-read its last one: theirs are not stored)
-  uint32_t x_off[2 * MT], u_off[PRO == PRO_SILU_MUL ? 2 * MT : 1];
+  uint32_t x_off[EIGHTS], u_off[PRO == PRO_SILU_MUL ? EIGHTS : 1];
 #pragma unroll
-  for (int j = 0; j < 2 * MT; j++) {
+  for (int j = 0; j < EIGHTS; j++) {
     int const row = 8 * j + l8, rr = row < M ? row : M - 1;
     uint32_t const chunk = 8u * (uint32_t)(ch8 ^ ((row >> 1) & 7));
     x_off[j] = 2u * ((uint32_t)(rr * P.a0.d_cols) + chunk);
@@ -102,37 +106,34 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) 
     }
   }
   // lora A: column-major like the weights (16 columns), row-major k rows 32 j + l / 2 of 32 bytes
-  auto issue = [&](int it, int sub, int b, int slot) {
+  auto issue = [&](int it, int sub, int slot) {
     uint32_t const at = mine_at + (uint32_t)(slot * SLOT);
-    GTile const &bt = b == 0 ? P.b0 : P.b1;
     _Float16 const *w = static_cast<_Float16 const *>(bt.ptr) + gtile_offset(bt, bx, by, bz, it) +
                         (WCM ? (long long)(64 * sub) : (long long)(64 * sub) * bt.d_cols);
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-      lane_dma16(w + (long long)(8 * j) * bt.d_cols, w_off[j & 1][b], at + (uint32_t)(1024 * j));
+      lane_dma16(w + (long long)(8 * j) * bt.d_cols, w_off[j & 1], at + (uint32_t)(1024 * j));
     }
-    if (b == 0) {
-      _Float16 const *x = static_cast<_Float16 const *>(P.a0.ptr) + gtile_offset(P.a0, bx, by, bz, it) + 64 * sub;
+    _Float16 const *x = static_cast<_Float16 const *>(P.a0.ptr) + gtile_offset(P.a0, bx, by, bz, it) + 64 * sub;
 #pragma unroll
-      for (int j = 0; j < 2 * MT; j++) {
-        lane_dma16(x, x_off[j], at + (uint32_t)(X_AT + 1024 * j));
+    for (int j = 0; j < EIGHTS; j++) {
+      lane_dma16(x, x_off[j], at + (uint32_t)(X_AT + 1024 * j));
+    }
+    if (PRO == PRO_SILU_MUL) {
+      _Float16 const *u = static_cast<_Float16 const *>(P.a1.ptr) + gtile_offset(P.a1, bx, by, bz, it) + 64 * sub;
+#pragma unroll
+      for (int j = 0; j < EIGHTS; j++) {
+        lane_dma16(u, u_off[j], at + (uint32_t)(U_AT + 1024 * j));
       }
-      if (PRO == PRO_SILU_MUL) {
-        _Float16 const *u = static_cast<_Float16 const *>(P.a1.ptr) + gtile_offset(P.a1, bx, by, bz, it) + 64 * sub;
+    }
+    if (LORA) {
+      _Float16 const *la = static_cast<_Float16 const *>(P.la.ptr) + gtile_offset(P.la, bx, by, bz, it) +
+                           (WCM ? (long long)(64 * sub) : (long long)(64 * sub) * P.la.d_cols);
 #pragma unroll
-        for (int j = 0; j < 2 * MT; j++) {
-          lane_dma16(u, u_off[j], at + (uint32_t)(U_AT + 1024 * j));
-        }
-      }
-      if (LORA) {
-        _Float16 const *la = static_cast<_Float16 const *>(P.la.ptr) + gtile_offset(P.la, bx, by, bz, it) +
-                             (WCM ? (long long)(64 * sub) : (long long)(64 * sub) * P.la.d_cols);
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-          uint32_t const off = WCM ? 2u * (uint32_t)(l8 * P.la.d_cols + 8 * (ch8 ^ swizzle(8 * j + l8)))
-                                   : 2u * (uint32_t)((lane / 2) * P.la.d_cols + 8 * (lane % 2));
-          lane_dma16(la + (long long)(WCM ? 8 * j : 32 * j) * P.la.d_cols, off, at + (uint32_t)(LA_AT + 1024 * j));
-        }
+      for (int j = 0; j < 2; j++) {
+        uint32_t const off = WCM ? 2u * (uint32_t)(l8 * P.la.d_cols + 8 * (ch8 ^ swizzle(8 * j + l8)))
+                                 : 2u * (uint32_t)((lane / 2) * P.la.d_cols + 8 * (lane % 2));
+        lane_dma16(la + (long long)(WCM ? 8 * j : 32 * j) * P.la.d_cols, off, at + (uint32_t)(LA_AT + 1024 * j));
       }
     }
   };
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) 
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
   auto rows = [&](unsigned char const *x, int mt, int s) {
-    int const row = 16 * mt + c;
+    int const row = GROUPS > 0 ? 16 * mt + c : c % 8;
     return *reinterpret_cast<half8 const *>(x + 128 * row + 16 * ((4 * s + g) ^ ((row >> 1) & 7)));
   };
 
@@ -175,26 +176,17 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) 
     }
   }
 
-  // ---- the loop: step = one weight matrix's 64 k ---------------------------------------------------
-  int const total = n_mine > 0 ? n_mine * subs * NB : 0;
-  int i_it = 0, i_sub = 0, i_b = 0, i_slot = 0, issued = 0;  // the next step to issue
+  // ---- the loop: step = 64 k ----------------------------------------------------------------------
+  int const total = n_mine > 0 ? n_mine * subs : 0;
+  int i_it = 0, i_sub = 0, i_slot = 0, issued = 0;  // the next step to issue
   auto issue_next = [&]() {
-    if (NB == 1 || i_b == 0) {
-      issue(nth(i_it), i_sub, 0, i_slot);
-    } else {
-      issue(nth(i_it), i_sub, 1, i_slot);
-    }
+    issue(nth(i_it), i_sub, i_slot);
     issued++;
     i_slot = i_slot + 1 == R ? 0 : i_slot + 1;
-    if (NB == 2) {
-      i_b ^= 1;
-    }
-    if (NB == 1 || i_b == 0) {
-      i_sub++;
-      if (i_sub == subs) {
-        i_sub = 0;
-        i_it++;
-      }
+    i_sub++;
+    if (i_sub == subs) {
+      i_sub = 0;
+      i_it++;
     }
   };
   for (int s = 0; s < R && s < total; s++) {
@@ -202,97 +194,101 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) 
   }
   int slot = 0, step = 0;
   for (int i = 0; i < n_mine; i++) {
-    float4v o[NB][4][MT], d = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4v o[4][MT], d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
+    for (int t = 0; t < 4; t++) {
 #pragma unroll
-      for (int t = 0; t < 4; t++) {
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-          o[b][t][mt] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-        }
+      for (int mt = 0; mt < MT; mt++) {
+        o[t][mt] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
       }
     }
-    for (int sub = 0; sub < subs; sub++) {
-      half8 x[MT][2];
+    for (int sub = 0; sub < subs; sub++, step++) {
+      // this step has landed when only the loads of the one after it are outstanding
+      if (issued - 1 > step) {
+        stream_wait<8 + X_LOADS>();
+      } else {
+        stream_wait<0>();
+      }
+      unsigned char const *const at = mine + slot * SLOT;
+      half8 w[4][2], la[2], x[MT][2], u[PRO == PRO_SILU_MUL ? MT : 1][2];
 #pragma unroll
-      for (int b = 0; b < NB; b++, step++) {
-        // this step has landed when only the loads of the one after it are outstanding
-        if (issued - 1 > step) {
-          stream_wait<NB == 1 ? 8 + X_LOADS : 8>();
-        } else {
-          stream_wait<0>();
+      for (int s = 0; s < 2; s++) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          w[t][s] = weights(at, t, s);
         }
-        unsigned char const *const at = mine + slot * SLOT;
-        half8 w[4][2], la[2];
+      }
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+          x[mt][s] = rows(at + X_AT, mt, s);
+          if (PRO == PRO_SILU_MUL) {
+            u[mt][s] = rows(at + U_AT, mt, s);
+          }
+        }
+        if (LORA) {
+          if (WCM) {
+            la[s] = *reinterpret_cast<half8 const *>(at + LA_AT + 128 * c + 16 * ((4 * s + g) ^ swizzle(c)));
+          } else {
+            _Float16 const *ap = reinterpret_cast<_Float16 const *>(at + LA_AT) + (32 * s + 8 * g + (c >> 2)) * 16 + 4 * (c & 3);
+            half4 const lo = lane_tr16(ap), hi = lane_tr16(ap + 64);
+            la[s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+          }
+        }
+      }
+      // the slot is in registers: the step that takes it next may fly
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (issued < total) {
+        issue_next();
+      }
+      slot = slot + 1 == R ? 0 : slot + 1;
+      auto applied = [&](half8 v, half8 m) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          v[e] = static_cast<_Float16>(prologue(PRO == PRO_EXP ? PRO_EXP : PRO_SILU, static_cast<float>(v[e])));
+          if (PRO == PRO_SILU_MUL) {
+            v[e] = static_cast<_Float16>(static_cast<float>(v[e]) * static_cast<float>(m[e]));
+          }
+        }
+        return v;
+      };
+      if (PRO != PRO_NONE && GROUPS == 0) {
+        // Eight rows: lanes c and c + 8 hold the same values of both k steps.  Each makes one step's and the
+        // lower lane takes the other's from the upper (the upper lane's operands belong to rows that are not stored).
+        bool const upper = c >= 8;
+        half8 const v = applied(upper ? x[0][1] : x[0][0], upper ? u[0][PRO == PRO_SILU_MUL] : u[0][0]);
+        x[0][0] = v;
+        uint4v const bits = __builtin_bit_cast(uint4v, v);
+        uint4v from;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          from[e] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)bits[e], 0x128, 0xf, 0xf, false);  // row_ror:8
+        }
+        x[0][1] = __builtin_bit_cast(half8, from);
+      } else if (PRO != PRO_NONE) {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
 #pragma unroll
-          for (int t = 0; t < 4; t++) {
-            w[t][s] = weights(at, t, s);
+          for (int mt = 0; mt < MT; mt++) {
+            x[mt][s] = applied(x[mt][s], u[PRO == PRO_SILU_MUL ? mt : 0][PRO == PRO_SILU_MUL ? s : 0]);
           }
         }
-        half8 u[PRO == PRO_SILU_MUL ? MT : 1][2];
-        if (b == 0) {
-#pragma unroll
-          for (int s = 0; s < 2; s++) {
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-              x[mt][s] = rows(at + X_AT, mt, s);
-              if (PRO == PRO_SILU_MUL) {
-                u[mt][s] = rows(at + U_AT, mt, s);
-              }
-            }
-            if (LORA) {
-              if (WCM) {
-                la[s] = *reinterpret_cast<half8 const *>(at + LA_AT + 128 * c + 16 * ((4 * s + g) ^ swizzle(c)));
-              } else {
-                _Float16 const *ap = reinterpret_cast<_Float16 const *>(at + LA_AT) + (32 * s + 8 * g + (c >> 2)) * 16 + 4 * (c & 3);
-                half4 const lo = lane_tr16(ap), hi = lane_tr16(ap + 64);
-                la[s] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-              }
-            }
-          }
-        }
-        // the slot is in registers: the step that takes it next may fly
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (issued < total) {
-          issue_next();
-        }
-        slot = slot + 1 == R ? 0 : slot + 1;
-        if (b == 0) {
-          if (PRO != PRO_NONE) {
-#pragma unroll
-            for (int s = 0; s < 2; s++) {
-#pragma unroll
-              for (int mt = 0; mt < MT; mt++) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                  _Float16 v = static_cast<_Float16>(prologue(PRO == PRO_EXP ? PRO_EXP : PRO_SILU, static_cast<float>(x[mt][s][e])));
-                  if (PRO == PRO_SILU_MUL) {
-                    v = static_cast<_Float16>(static_cast<float>(v) * static_cast<float>(u[mt][s][e]));
-                  }
-                  x[mt][s][e] = v;
-                }
-              }
-            }
-          }
-          if (LORA) {
-#pragma unroll
-            for (int s = 0; s < 2; s++) {
-              d = __builtin_amdgcn_mfma_f32_16x16x32_f16(la[s], x[0][s], d, 0, 0, 0);
-            }
-          }
-        }
-        // weights first: o[b][t][mt][r] = O[16 mt + c][16 t + 4 g + r]
+      }
+      if (LORA) {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
+          d = __builtin_amdgcn_mfma_f32_16x16x32_f16(la[s], x[0][s], d, 0, 0, 0);
+        }
+      }
+      // weights first: o[t][mt][r] = O[16 mt + c][16 t + 4 g + r]
 #pragma unroll
-          for (int t = 0; t < 4; t++) {
+      for (int s = 0; s < 2; s++) {
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-              o[b][t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[t][s], x[mt][s], o[b][t][mt], 0, 0, 0);
-            }
+        for (int t = 0; t < 4; t++) {
+#pragma unroll
+          for (int mt = 0; mt < MT; mt++) {
+            o[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[t][s], x[mt][s], o[t][mt], 0, 0, 0);
           }
         }
       }
@@ -307,22 +303,19 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) 
       }
 #pragma unroll
       for (int t = 0; t < 4; t++) {
-        o[0][t][0] = __builtin_amdgcn_mfma_f32_16x16x16f16(lb_frag[t], df, o[0][t][0], 0, 0, 0);
+        o[t][0] = __builtin_amdgcn_mfma_f32_16x16x16f16(lb_frag[t], df, o[t][0], 0, 0, 0);
       }
     }
     // ---- this iteration's product, fp16 ----------------------------------------------------------
+    long long const tile = (long long)M * 64;
+    _Float16 *const to = P.ksplit > 1 ? P.scratch + (((long long)block_linear * F + it) * NB + b) * tile
+                                      : reinterpret_cast<_Float16 *>(lds + S.results) + it * (int)tile;
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-      long long const tile = (long long)M * 64;
-      _Float16 *const to = P.ksplit > 1 ? P.scratch + (((long long)block_linear * F + it) * NB + b) * tile
-                                        : reinterpret_cast<_Float16 *>(lds + S.results) + (it * NB + b) * (int)tile;
+    for (int mt = 0; mt < MT; mt++) {
+      if (16 * mt + c < M) {
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++) {
-        if (16 * mt + c < M) {
-#pragma unroll
-          for (int t = 0; t < 4; t++) {
-            *reinterpret_cast<half4 *>(to + (16 * mt + c) * 64 + 16 * t + 4 * g) = __builtin_convertvector(o[b][t][mt], half4);
-          }
+        for (int t = 0; t < 4; t++) {
+          *reinterpret_cast<half4 *>(to + (16 * mt + c) * 64 + 16 * t + 4 * g) = __builtin_convertvector(o[t][mt], half4);
         }
       }
     }
@@ -334,18 +327,150 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) 
   __syncthreads();
   typedef _Float16 half2v __attribute__((ext_vector_type(2)));
   _Float16 const *const all = reinterpret_cast<_Float16 const *>(lds + S.results);
-  for (int e = tid; e < NB * M * 16; e += 256) {
-    int const b = e / (M * 16), q = e % (M * 16), row = q / 16, col = 4 * (q % 16);
-    _Float16 const *src = all + b * M * 64 + row * 64 + col;
+  GTile const &ot = NB == 2 && b == 1 ? P.o1 : P.o0;
+  _Float16 *const og = static_cast<_Float16 *>(const_cast<void *>(ot.ptr)) + gtile_offset(ot, bx, by, bz, 0);
+  for (int e = tid; e < M * 16; e += 256) {
+    int const row = e / 16, col = 4 * (e % 16);
+    _Float16 const *src = all + row * 64 + col;
     half2v lo = {(_Float16)0.0f, (_Float16)0.0f}, hi = lo;
     for (int it = 0; it < F; it++) {  // (a packed fp16 add is the exact sum rounded once)
-      half4 const v = *reinterpret_cast<half4 const *>(src + it * NB * M * 64);
+      half4 const v = *reinterpret_cast<half4 const *>(src + it * M * 64);
       lo += half2v{v[0], v[1]};
       hi += half2v{v[2], v[3]};
     }
-    GTile const &ot = b == 0 ? P.o0 : P.o1;
-    _Float16 *og = static_cast<_Float16 *>(const_cast<void *>(ot.ptr)) + gtile_offset(ot, bx, by, bz, 0);
     *reinterpret_cast<half4 *>(og + (long long)row * ot.d_cols + col) = half4{lo[0], lo[1], hi[0], hi[1]};
+  }
+}
+
+// The same for column-major weights cut into strips of 16 columns, a workgroup with the whole for-loop each: no
+// ranges to add up, so no slab and no second launch, for activations read four times as often.
+// Bound by memory: two weights of 4096 x 14336 against 8 rows 42.9 us, ranges and their fold 47.2;
+// against 16 rows, and with a gated MLP's second product behind it, 79.5 against 82.5.
+constexpr int columns_ring(int eights) { return eights == 1 ? 6 : 4; }  // slots per wavefront, two workgroups a compute unit
+constexpr int columns_slot_bytes(int eights) { return 2048 + 1024 * eights; }
+
+template <int NB, int EIGHTS>
+__device__ __forceinline__ void stream_columns(StreamParams const &S) {
+  GemmParams const &P = S.g;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  constexpr int W = 4, R = columns_ring(EIGHTS), SLOT = columns_slot_bytes(EIGHTS), LOADS = 2 + EIGHTS;
+  int const tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  int const g = lane / 16, c = lane % 16, l8 = lane / 8, ch8 = lane % 8;
+  int const M = P.M, F = P.forloop_range, subs = P.KT / 64;
+  int const piece = blockIdx.x % 4, b = NB == 2 ? blockIdx.x / 4 % 2 : 0;
+  int const bx = blockIdx.x / (4 * NB), by = blockIdx.y, bz = blockIdx.z;
+  // A wavefront's iterations are neighbours, and it starts at another one in each block: wavefronts on every
+  // fourth iteration read 2 KB next to each other in columns 8 KB apart, all of them the same few memory channels
+  // (4 rows x 28672 x 4096: 50.5 us, 39.9 this way).
+  int const per = (F + W - 1) / W, first = wave * per;
+  int const n_mine = F - first < per ? (F > first ? F - first : 0) : per, total = n_mine * subs;
+  int const rot = n_mine > 1 ? (int)(blockIdx.x / (4 * NB) % (unsigned)n_mine) : 0;
+  GTile const &bt = NB == 2 && b == 1 ? P.b1 : P.b0;
+
+  unsigned char *const mine = lds + wave * R * SLOT;
+  uint32_t const mine_at = lane_lds_address(mine);
+  auto swizzle = [](int row) { return (row >> 1) & 7; };
+  uint32_t w_off[2], x_off[EIGHTS];
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    w_off[j] = 2u * (uint32_t)((8 * j + l8) * bt.d_cols + 8 * (ch8 ^ swizzle(8 * j + l8)));
+  }
+#pragma unroll
+  for (int j = 0; j < EIGHTS; j++) {
+    int const row = 8 * j + l8;
+    x_off[j] = 2u * (uint32_t)((row < M ? row : M - 1) * P.a0.d_cols + 8 * (ch8 ^ swizzle(row)));
+  }
+  int i_it = rot, i_sub = 0, i_slot = 0, issued = 0;  // the next step to issue
+  auto issue_next = [&]() {
+    int const it = first + i_it;
+    uint32_t const at = mine_at + (uint32_t)(i_slot * SLOT);
+    _Float16 const *w = static_cast<_Float16 const *>(bt.ptr) + gtile_offset(bt, bx, by, bz, it) +
+                        (long long)(16 * piece) * bt.d_cols + 64 * i_sub;
+    _Float16 const *x = static_cast<_Float16 const *>(P.a0.ptr) + gtile_offset(P.a0, bx, by, bz, it) + 64 * i_sub;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      lane_dma16(w, w_off[j], at + (uint32_t)(1024 * j));
+    }
+#pragma unroll
+    for (int j = 0; j < EIGHTS; j++) {
+      lane_dma16(x, x_off[j], at + (uint32_t)(2048 + 1024 * j));
+    }
+    issued++;
+    i_slot = i_slot + 1 == R ? 0 : i_slot + 1;
+    i_sub++;
+    if (i_sub == subs) {
+      i_sub = 0;
+      i_it = i_it + 1 == n_mine ? 0 : i_it + 1;
+    }
+  };
+  for (int s = 0; s < R && s < total; s++) {
+    issue_next();
+  }
+  _Float16 *const all = reinterpret_cast<_Float16 *>(lds + S.results);  // [F][M][16]
+  int slot = 0, step = 0;
+  for (int i = 0; i < n_mine; i++) {
+    float4v o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int sub = 0; sub < subs; sub++, step++) {
+      if (issued - step == R) {
+        stream_wait<(R - 1) * LOADS>();
+      } else {
+        stream_wait<0>();
+      }
+      unsigned char const *const at = mine + slot * SLOT;
+      int const xr = EIGHTS == 2 ? c : c % 8;
+      half8 w[2], x[2];
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        w[s] = *reinterpret_cast<half8 const *>(at + 128 * c + 16 * ((4 * s + g) ^ swizzle(c)));
+        x[s] = *reinterpret_cast<half8 const *>(at + 2048 + 128 * xr + 16 * ((4 * s + g) ^ swizzle(xr)));
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (issued < total) {
+        issue_next();
+      }
+      slot = slot + 1 == R ? 0 : slot + 1;
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[s], x[s], o, 0, 0, 0);
+      }
+    }
+    int const j = i + rot, it = first + (j >= n_mine ? j - n_mine : j);
+    if (c < M) {
+      *reinterpret_cast<half4 *>(all + (it * M + c) * 16 + 4 * g) = __builtin_convertvector(o, half4);
+    }
+  }
+  __syncthreads();
+  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+  if (tid < 8 * M) {
+    int const row = tid / 8, col = 2 * (tid % 8);
+    half2v a = {(_Float16)0.0f, (_Float16)0.0f};
+#pragma unroll 8
+    for (int it = 0; it < F; it++) {  // (a packed fp16 add is the exact sum rounded once)
+      a += *reinterpret_cast<half2v const *>(all + (it * M + row) * 16 + col);
+    }
+    GTile const &ot = NB == 2 && b == 1 ? P.o1 : P.o0;
+    _Float16 *const og = static_cast<_Float16 *>(const_cast<void *>(ot.ptr)) + gtile_offset(ot, bx, by, bz, 0);
+    *reinterpret_cast<half2v *>(og + (long long)row * ot.d_cols + 16 * piece + col) = a;
+  }
+}
+
+template <int NB, int PRO, bool LORA, bool WCM, int MT>
+__global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) {
+  fetch_kernel_arguments<sizeof(StreamParams), 2>();
+  if constexpr (PRO == PRO_NONE && !LORA && WCM && MT == 1) {
+    if (S.strips) {
+      if (S.g.M <= 8) {
+        stream_columns<NB, 1>(S);
+      } else {
+        stream_columns<NB, 2>(S);
+      }
+      return;
+    }
+  }
+  if (MT == 1 && S.g.M <= 8) {
+    stream_block<NB, PRO, LORA, WCM, 0>(S);
+  } else {
+    stream_block<NB, PRO, LORA, WCM, MT>(S);
   }
 }
 

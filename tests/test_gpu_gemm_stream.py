@@ -96,3 +96,21 @@ def test_one_launch_of_many_pieces(rt, abi, m, blocks, kt, loop, order):
         _run(rt, spec, order, f"pieces {m} x {blocks}, {kt} x {loop} {order}")
     finally:
         assert abi.mi355_set_option(7, 0) == 0
+
+
+@pytest.mark.parametrize("weights", [1, 2])
+@pytest.mark.parametrize("m,blocks,kt,loop", [
+    (1, 48, 64, 1), (8, 50, 64, 3), (9, 49, 192, 5), (16, 96, 128, 10), (7, 48, 512, 2), (4, 200, 64, 33), (16, 48, 64, 24)])
+def test_strips_of_16_columns(rt, ranges, m, blocks, kt, loop, weights):
+    """Column-major plans wide enough for a workgroup per 16 columns: rows around 8 and 16, loops that leave
+    wavefronts with no, one or fewer iterations, a first step that is also the last, up to the most results that
+    fit (16 rows, 24 iterations)."""
+    from attention_superoptimizer_amd import workloads as W
+    if weights == 1:
+        spec, _ = W.tiled_matmul(m, 64 * blocks, kt * loop, (blocks, 1, 1), loop, (-1, -1, -1), (1, -1, -1), (1, -1, -1))
+    else:
+        # (the first operator alone: the second adds up to 200 products of both signs in an fp16 accumulator that
+        # passes 4, where one rounding is 0.004, and ends near 0.3, whose plain bar is 0.004)
+        spec, _ = W.config5_gated_mlp(m=m, d=kt * loop, h=64 * blocks, grid1=blocks, F1=loop, grid2=kt * loop // 64, F2=blocks)
+        spec = [op for i, op in enumerate(spec[:5]) if i != 3]
+    _run(rt, spec, COL, f"strips {m} x {blocks}, {kt} x {loop}, {weights}", **({} if weights == 1 else {"std": 0.05}))
