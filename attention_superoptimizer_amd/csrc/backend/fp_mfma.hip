@@ -1136,10 +1136,14 @@ static int launch_mfma_group(uint16_t const *const *A, uint16_t const *const *B,
 extern "C" int mi355_fp_matmul(uint16_t const *A, uint16_t const *B, uint16_t *C, int batch, int m,
                                int n, int k);
 
+// From 2^27 multiplications on, and for every k that fp_direct.hip leaves: the vector kernels walk k with few
+// workgroups ([8, 96, 1152] . [8, 1152, 64] 97.1 us there, 12.4 here, [256, 2000] . [2000, 256] 240 and 12.4,
+// [1, 20000] . [20000, 1] 842 and 33; in whole 64s [64, 1088] . [1088, 64] 10.9 and 10.0, [128, 8064] . [8064, 128]
+// 28.5 and 21.3, [64, 32768] . [32768, 64] 55.8 and 56.0).
 bool mfma_matmul_pays(int batch, int m, int n, int k) {
   size_t need = 0;
   return !state().fp_vector_dot_only && mfma_matmul_fits(batch, m, n, k, &need) && need <= state().planes_bytes &&
-         (double)batch * m * n * k >= (double)(1 << 27);
+         ((double)batch * m * n * k >= (double)(1 << 27) || k > 1024);
 }
 
 int launch_mfma_matmul(uint16_t const *A, uint16_t const *B, uint16_t *C, int batch, int m, int n,

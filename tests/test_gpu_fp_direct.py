@@ -56,3 +56,20 @@ def test_direct_matmul_of_every_16_bit_value(rt, abi, n):
         ins, got = _matmul_many(abi, rt, shapes, fill)
         for (A, B), C, s in zip(ins, got, shapes):
             np.testing.assert_array_equal(C, orc.fp_matmul(A % FP_PQ, B % FP_PQ), err_msg=str(s))
+
+
+@pytest.mark.parametrize("b,m,n,k", [(1, 1, 1, 1025), (8, 96, 64, 1152), (1, 64, 64, 1088), (3, 7, 130, 2049), (1, 33, 5, 33000)])
+def test_small_products_of_a_long_k(rt, abi, b, m, n, k):
+    """Past the k of the one-launch kernel, as a graph's operator: on residue planes however small, for every
+    16-bit value, and the same as the vector kernels."""
+    from test_gpu_fingerprint import _graph_fp
+    every = np.arange(65536, dtype=np.uint16)
+    A, B = np.resize(every[::-1], b * m * k).reshape(b, m, k), uniform_fp((b, k, n), 8)
+    spec = [{"op": "input", "dims": [b, m, k]}, {"op": "input", "dims": [b, k, n]}, {"op": "matmul", "in": [[0, 0], [1, 0]]}]
+    got = _graph_fp(rt, spec, {0: A, 1: B})[2][0]
+    np.testing.assert_array_equal(got, orc.fp_matmul(A % FP_PQ, B))
+    assert abi.mi355_set_option(4, 1) == 0
+    try:
+        np.testing.assert_array_equal(got, _graph_fp(rt, spec, {0: A, 1: B})[2][0])
+    finally:
+        assert abi.mi355_set_option(4, 0) == 0
