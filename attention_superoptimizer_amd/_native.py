@@ -98,6 +98,7 @@ ABI = {
     "mi355_fp_binary_many": (_ci, [_pi, _pvp, _pi, _pvp, _pi, _pvp, _pi, _pi, _ci]),
     "mi355_fp_reduce": (_ci, [_vp, _vp, _sz, _ci, _ci, _ci]),
     "mi355_fp_softmax_rows": (_ci, [_vp, _vp, _vp, _vp, _sz, _ci]),
+    "mi355_fp_attention_rows": (_ci, [_vp] * 8 + [_ci] * 5 + [_vp]),
     "mi355_fp_equal": (_ci, [_vp, _vp, _sz, _pi]),
     "mi355_fp_big_tiles_check": (_ci, [_pi]),
     "mi355_fp_equal_reset": (_ci, [_ci, _ci]),

@@ -705,6 +705,22 @@ static bool is_attention_rows(std::vector<KNOperator *> const &ops, size_t i) {
   return true;
 }
 
+// Operators i .. i + 4 as one fingerprint launch (every storage order, as above).
+bool fingerprint_attention_rows(std::vector<KNOperator *> const &ops, size_t i) {
+  if (!is_attention_rows(ops, i)) {
+    return false;
+  }
+  require_device("fingerprint_attention_rows");
+  DTensor const &Q = ops[i]->input_tensors[0], &K = ops[i]->input_tensors[1], &V = ops[i + 4]->input_tensors[1];
+  int batch, m, n, k, batch2, m2, dv, n2, taken = 0;
+  matmul_extents(Q, K, batch, m, n, k);
+  matmul_extents(ops[i + 4]->input_tensors[0], V, batch2, m2, dv, n2);
+  MI355_CALL(mi355_fp_attention_rows(Q.fp_ptr, K.fp_ptr, V.fp_ptr, ops[i]->output_tensors[0].fp_ptr, ops[i + 1]->output_tensors[0].fp_ptr,
+                                     ops[i + 2]->output_tensors[0].fp_ptr, ops[i + 3]->output_tensors[0].fp_ptr,
+                                     ops[i + 4]->output_tensors[0].fp_ptr, batch, m, n, k, dv, &taken));
+  return taken != 0;
+}
+
 static bool run_attention_rows(std::vector<KNOperator *> const &ops, size_t i) {
   if (!is_attention_rows(ops, i)) {
     return false;

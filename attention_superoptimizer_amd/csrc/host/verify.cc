@@ -26,6 +26,7 @@ namespace kernel {
 void lower_customized(KNCustomizedOp const &op, bool fingerprint, mi355_plan *plan,
                       void const **inputs, void **outputs, long long *in_elems, long long *out_elems);
 bool fingerprint_softmax_rows(std::vector<KNOperator *> const &ops, size_t i);
+bool fingerprint_attention_rows(std::vector<KNOperator *> const &ops, size_t i);
 void prefetch_graph(Graph const &g, int level, bool write);
 }  // namespace kernel
 
@@ -129,7 +130,9 @@ void fingerprint_graph(kernel::Graph const &g, uint64_t input_seed, VerifyStats 
     account(op, stats);
   }
   for (size_t i = 0; i < g.operators.size(); i++) {
-    if (kernel::fingerprint_softmax_rows(g.operators, i)) {
+    if (kernel::fingerprint_attention_rows(g.operators, i)) {
+      i += 4;
+    } else if (kernel::fingerprint_softmax_rows(g.operators, i)) {
       i += 2;
     } else if (g.operators[i]->op_type != KN_INPUT_OP) {
       g.operators[i]->fingerprint();

@@ -264,6 +264,11 @@ int mi355_fp_reduce(uint16_t const *in, uint16_t *out, size_t n_out, int factor,
 /* E = exp(X), R[row] = sum of a row of E, P = E / R for `rows` rows of n elements: what mi355_fp_unary,
  * mi355_fp_reduce and mi355_fp_binary one after the other leave. */
 int mi355_fp_softmax_rows(uint16_t const *X, uint16_t *E, uint16_t *R, uint16_t *P, size_t rows, int n);
+/* The un-fused attention graph of fingerprints in one launch: S = Q . K, E = exp(S), R = the sums of E's rows,
+ * P = E / R, O = P . V, with Q [batch][m][d], K [batch][d][n], V [batch][n][dv]; the ring values the operators
+ * leave one by one.  *taken = 0 and nothing enqueued where one launch does not take these sizes. */
+int mi355_fp_attention_rows(uint16_t const *Q, uint16_t const *K, uint16_t const *V, uint16_t *S, uint16_t *E,
+                            uint16_t *R, uint16_t *P, uint16_t *O, int batch, int m, int n, int d, int dv, int *taken);
 /* DTensor::has_same_fingerprint's element loop, src/kernel/cuda/device_tensor_kernel.cu:36-52,
  * done on the device; writes 1/0 to *equal (blocking: 4 bytes come back, not 2 tensors) */
 int mi355_fp_equal(uint16_t const *a, uint16_t const *b, size_t n, int *equal);
