@@ -71,7 +71,7 @@ __device__ __forceinline__ half8 chunk_drop(half8 v, int s) {
 template <int R, int NT, bool KC>
 struct OperandStage {
   static constexpr int BK = 64, CHUNKS = R * BK / 8, CH = (CHUNKS + NT - 1) / NT;
-  static constexpr int LD = KC ? BK + 8 : R + 8;  // halfs; both strides spread a read over all banks
+  static constexpr int LD = KC ? BK + 8 : R + 8;  // halfs
   static constexpr int HALFS = (KC ? R : BK) * LD;
   _Float16 const *base;
   int ld, k, row_of[CH], pos_of[CH];
@@ -464,12 +464,22 @@ __device__ __forceinline__ void gemm_wait_vm() {
 }
 #pragma clang diagnostic pop
 
+// Where the 16-byte chunk q of row r of an LDS tile lies in its row.  LDS has 64 banks, 256 bytes a cycle, and
+// serves a 16-byte read in the lane groups {0-3, 12-15, 20-23, 24-27} and so on, an 8-byte one 32 lanes at a
+// time; with these every operand read below is free of bank conflicts (measured over 16 wavefronts: 231 - 244
+// bytes a cycle; rows of 64 bytes turned by r / 4 126; transposing reads 211, turned by r / 2 % 4 126).
+__device__ __forceinline__ int turned_k64(int r, int q) { return q ^ (r / 2 % 8); }     // rows of 64 k
+__device__ __forceinline__ int turned_k32(int r, int q) { return q ^ (-(r / 4) & 3); }  // rows of 32 k
+template <int R>  // a row is one k of R = 64 or 128 columns, read transposing
+__device__ __forceinline__ int turned_columns(int r, int q) {
+  static_assert(R == 64 || R == 128, "columns of a tile");
+  return q ^ (2 * (R == 64 ? r / 2 % 2 + 2 * (r / 8 % 2) : r % 4 + 4 * (r / 8 % 2)));
+}
+
 // Products whose rows are whole 16-byte chunks and whose k is whole stages of 64: f16_gemm_any_kernel's
 // tiles and k ranges, but a stage goes to LDS directly (global_load_lds_dwordx4), without the registers and
 // the LDS stores of the way through them; a ring of three stages, two in flight.  A direct load writes its
-// 64 chunks in lane order, so the LDS rows are not padded: chunk q of row r sits at position q ^ (r / 2 % 8)
-// where k is contiguous, at q ^ 2 (r % 8) (64 columns: ^ 2 (r / 2 % 4)) where a row is one k; both spread an
-// operand read over all banks.
+// 64 chunks in lane order: a lane fetches the chunk that belongs in its place.
 //
 // What bounds it: the 35 bytes a cycle that a compute unit gets from its caches (64 x 64 x 64: 470 cycles,
 // of matrix instructions 128), whatever the number of stages in flight; so a wide tile where there are
@@ -483,7 +493,13 @@ struct DirectStage {
   size_t step;       // elements from a stage to the next
   uint32_t off[CH];  // bytes from the stage's first element
 
-  __device__ __forceinline__ static int turned(int r, int q) { return KC ? q ^ (r / 2 % 8) : R == 64 ? q ^ (2 * (r / 2 % 4)) : q ^ (2 * (r % 8)); }
+  __device__ __forceinline__ static int turned(int r, int q) {
+    if constexpr (KC) {
+      return turned_k64(r, q);
+    } else {
+      return turned_columns<R>(r, q);
+    }
+  }
 
   // (rows and chunks past the matrix re-read its last ones)
   __device__ __forceinline__ void init(_Float16 const *matrix, int rows, int row0, int k, int tid) {
@@ -512,7 +528,7 @@ struct DirectStage {
   __device__ __forceinline__ static half8 operand(_Float16 const *tile, int r0, int s, int lane) {
     int const g = lane / 16, c = lane % 16;
     if (KC) {
-      return *reinterpret_cast<half8 const *>(tile + (r0 + c) * LD + 8 * turned(r0 + c, 4 * s + g));
+      return *reinterpret_cast<half8 const *>(tile + (r0 + c) * LD + 8 * turned(c, 4 * s + g));  // (16 divides r0)
     }
     typedef short short4v __attribute__((ext_vector_type(4)));
     typedef short4v __attribute__((address_space(3))) *lds_p;
@@ -594,7 +610,10 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void f16_gemm_direct_ke
     }
   };
   // Skewed by half a stage: every batch of operand reads is followed by the multiplications of the batch
-  // before it.
+  // before it.  The last stage stands behind the loop: with a condition around the reads of the next one, the
+  // multiplications behind it wait for those reads too (the compiler's count of LDS reads in flight is the
+  // least of the two ways there), and reading and multiplying take turns ([300, 2048] . [2048, 5504] row-major
+  // 18.5 -> 17.6 us, [1024, 2048] . [2048, 5504] 39.7 -> 38.0).
   if (T > 0) {
     issue(0, 0);
     if (T > 1) {
@@ -607,22 +626,24 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void f16_gemm_direct_ke
     }
     Operands x0, x1;
     read(x0, 0, 0);
-    for (int t = 0, slot = 0; t < T; t++) {
+    int slot = 0;
+    for (int t = 0; t + 1 < T; t++) {
       int const next = slot + 1 < kDirectRing ? slot + 1 : 0;
       read(x1, slot, 1);
       multiply(x0);
-      if (t + 1 < T) {
-        landed(t + 1);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wavefront's reads of stage t are in registers
-        __syncthreads();                                    // stage t + 1 is there, stage t is free
-        if (t + 3 < T) {
-          issue(t + 3, slot);
-        }
-        read(x0, next, 0);
+      landed(t + 1);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wavefront's reads of stage t are in registers
+      __syncthreads();                                    // stage t + 1 is there, stage t is free
+      if (t + 3 < T) {
+        issue(t + 3, slot);
       }
+      read(x0, next, 0);
       multiply(x1);
       slot = next;
     }
+    read(x1, slot, 1);
+    multiply(x0);
+    multiply(x1);
     __syncthreads();
   }
   gemm_store<BM, BN, TM, TN, NT>(G, acc, ring, true, lane, split, batch, row0, col0, wm0, wn0);
@@ -639,9 +660,7 @@ constexpr int direct_gemm_lds() {
 // operand then leaves LDS once per workgroup rather than once per wavefront that shares its row, and a
 // wavefront needs no barrier until the four sums are added up.  A step goes to the wavefront's own ring in
 // LDS by direct loads (global_load_lds_dwordx4), RING - 1 of them in flight while one is multiplied from
-// registers.  A direct load writes its 64 chunks in lane order, so LDS rows are not padded: chunk q of row r
-// sits at position q ^ (r / 4 % 4) where k is contiguous, at q ^ 2 (r % 8) (64 columns: ^ 2 (r / 2 % 4))
-// where a row is one k; both spread an operand read over all banks.
+// registers.
 //
 // What bounds it: as above; the operand reads and barriers it saves count where the tile is small and the
 // steps of a workgroup are a chain: 0.14 us for 64 k of a 16 x 64 tile (f16_gemm_any_kernel: 0.24).
@@ -654,7 +673,13 @@ struct WaveStage {
   size_t step;       // elements from a step of k to the next
   uint32_t off[CH];  // bytes from the step's first element
 
-  __device__ __forceinline__ static int turned(int r, int q) { return KC ? q ^ (r / 4 % 4) : R == 64 ? q ^ (2 * (r / 2 % 4)) : q ^ (2 * (r % 8)); }
+  __device__ __forceinline__ static int turned(int r, int q) {
+    if constexpr (KC) {
+      return turned_k32(r, q);
+    } else {
+      return turned_columns<R>(r, q);
+    }
+  }
 
   // (rows and chunks past the matrix re-read its last ones)
   __device__ __forceinline__ void init(_Float16 const *matrix, int rows, int row0, int k, int lane) {
@@ -683,7 +708,7 @@ struct WaveStage {
   __device__ __forceinline__ static half8 operand(_Float16 const *tile, int r0, int lane) {
     int const g = lane / 16, c = lane % 16;
     if (KC) {
-      return *reinterpret_cast<half8 const *>(tile + (r0 + c) * LD + 8 * turned(r0 + c, g));
+      return *reinterpret_cast<half8 const *>(tile + (r0 + c) * LD + 8 * turned(c, g));  // (16 divides r0)
     }
     typedef short short4v __attribute__((ext_vector_type(4)));
     typedef short4v __attribute__((address_space(3))) *lds_p;
@@ -779,10 +804,8 @@ __global__ __launch_bounds__(256) void f16_gemm_waves_kernel(AnyGemm const G) {
   int slot = 0;
   auto advance = [&](Operands &next, Operands const &now, int t) {
     slot = slot + 1 < RING ? slot + 1 : 0;
-    if (t + 1 < T) {
-      landed(t + 1);
-      read(next, slot);
-    }
+    landed(t + 1);
+    read(next, slot);
     multiply(now);
     if (t + 1 + RING < T) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the reads have left the slot)
@@ -797,11 +820,16 @@ __global__ __launch_bounds__(256) void f16_gemm_waves_kernel(AnyGemm const G) {
     if (RING < T) {
       issue(RING, 0);
     }
-    for (int t = 0; t < T; t += 2) {
+    int t = 0;  // (the last step or two behind the loop: see f16_gemm_direct_kernel)
+    for (; t + 2 < T; t += 2) {
       advance(x1, x0, t);
-      if (t + 1 < T) {
-        advance(x0, x1, t + 1);
-      }
+      advance(x0, x1, t + 1);
+    }
+    if (t + 1 < T) {
+      advance(x1, x0, t);
+      multiply(x1);
+    } else {
+      multiply(x0);
     }
   }
   // ---- the wavefronts' sums, in wavefront order: each adds up a quarter of the columns

@@ -236,22 +236,24 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void f16_gemm_nt_kernel
     issue(kGemmStages - 1);
   }
   read_step(0, 0, a0, b0);
-  for (int kt = 0; kt < KT; kt++) {
-    int const slot = kt % kGemmStages;
-    read_step(slot, 1, a1, b1);
+  // (The last stage stands behind the loop: the multiplications would otherwise wait for the next stage's reads,
+  // which one of the two ways there does not make.)
+  for (int kt = 0; kt + 1 < KT; kt++) {
+    read_step(kt % kGemmStages, 1, a1, b1);
     multiply(a0, b0);
-    if (kt + 1 < KT) {
-      landed(kt + 1);
-      // (this wavefront's reads of stage kt are in registers before it lets the others go on)
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __syncthreads();  // stage kt + 1 is there for everybody; stage kt is in everybody's registers
-      if (kt + kGemmStages < KT) {
-        issue(kt + kGemmStages);  // into the slot stage kt leaves
-      }
-      read_step((kt + 1) % kGemmStages, 0, a0, b0);
+    landed(kt + 1);
+    // (this wavefront's reads of stage kt are in registers before it lets the others go on)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();  // stage kt + 1 is there for everybody; stage kt is in everybody's registers
+    if (kt + kGemmStages < KT) {
+      issue(kt + kGemmStages);  // into the slot stage kt leaves
     }
+    read_step((kt + 1) % kGemmStages, 0, a0, b0);
     multiply(a1, b1);
   }
+  read_step((KT - 1) % kGemmStages, 1, a1, b1);
+  multiply(a0, b0);
+  multiply(a1, b1);
 
   // ---- the tile leaves through LDS: each wavefront its own WM x WN piece -------------------
   __syncthreads();  // the last stage's operand reads are done everywhere
