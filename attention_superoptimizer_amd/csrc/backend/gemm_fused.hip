@@ -111,8 +111,9 @@ std::string literal(LaneParams const &L) {
   std::string t = literal(L.g, "G") + "    mi355::LaneParams P{};\n    P.g = G;\n";
   t += emit_fmt("    P.gx = %d;\n    P.gy = %d;\n    P.blocks = %d;\n    P.mtiles = %d;\n    P.slot_base = %d;\n", L.gx,
                 L.gy, L.blocks, L.mtiles, L.slot_base);
-  t += emit_fmt("    P.m_group = %uu;\n    P.m_pieces = %uu;\n    P.m_gx = %uu;\n    P.m_gy = %uu;\n", L.m_group,
-                L.m_pieces, L.m_gx, L.m_gy);
+  t += emit_fmt("    P.pieces = %d;\n    P.rank = %d;\n    P.m_group = %uu;\n    P.m_pieces = %uu;\n    P.m_columns = %uu;\n", L.pieces,
+                L.rank, L.m_group, L.m_pieces, L.m_columns);
+  t += emit_fmt("    P.m_gx = %uu;\n    P.m_gy = %uu;\n", L.m_gx, L.m_gy);
   return t;
 }
 std::string literal(StreamParams const &L) {
@@ -288,15 +289,12 @@ int launch_kt(GemmParams const &A, dim3 grid, int lds) {
 }
 
 // gemm_lanes_kernel for this plan, or 0 when it is not the better choice (see the rule in
-// try_launch_lanes); k extents 64 / 128 / 256.
-template <int NB, int PRO, bool LORA, bool WCM>
+// try_launch_lanes); k extents 32 / 64 / 96 / 128 / 256.
+template <int NB, int PRO, int LORA, bool WCM>
 int launch_lanes_kt(LaneParams const &L, int grid, int threads, int lds) {
   if (EmitSink *sink = emit_sink()) {
-    if (!(L.g.KT == 64 || L.g.KT == 128 || L.g.KT == 256)) {
-      return 0;
-    }
     sink->headers |= 2u;
-    emit_launch(*sink, "gemm_lanes_kernel", emit_fmt("%d, %d, %d, %s, %s", L.g.KT, NB, PRO, tf(LORA), tf(WCM)),
+    emit_launch(*sink, "gemm_lanes_kernel", emit_fmt("%d, %d, %d, %s, %s", L.g.KT, NB, PRO, LORA == 2 ? "2" : tf(LORA == 1), tf(WCM)),
                 dim3(grid, 1, 1), threads, lds, literal(L));
     return 1;
   }
@@ -307,8 +305,12 @@ int launch_lanes_kt(LaneParams const &L, int grid, int threads, int lds) {
     return 1;
   };
   switch (L.g.KT) {
+    case 32:
+      return go(gemm_lanes_kernel<32, NB, PRO, LORA, WCM>);
     case 64:
       return go(gemm_lanes_kernel<64, NB, PRO, LORA, WCM>);
+    case 96:
+      return go(gemm_lanes_kernel<96, NB, PRO, LORA, WCM>);
     case 128:
       return go(gemm_lanes_kernel<128, NB, PRO, LORA, WCM>);
     case 256:
@@ -320,11 +322,16 @@ int launch_lanes_kt(LaneParams const &L, int grid, int threads, int lds) {
 
 int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) {
   State &s = state();
-  if (s.gemm_mode == 1 || s.any_size_kernels || !G.whole || !(G.KT == 64 || G.KT == 128 || G.KT == 256)) {
+  // lora A comes in 16-rank pieces, the last one half full where its columns are rows in memory; two weights in
+  // tiles of 64 columns and whole 64-k units only (programs printed for others are known to hold the tiles' kernel)
+  bool const takes = (G.nb == 1 || (G.NC == 64 && G.KT % 64 == 0)) && (G.KT == 32 || G.KT == 64 || G.KT == 96 || G.KT == 128 || G.KT == 256) && G.M <= 64 &&
+                     (!G.lora || G.rank % 16 == 0 || (G.wcm && G.rank == 8));
+  if (s.gemm_mode == 1 || s.any_size_kernels || !takes) {
     return 0;
   }
   long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
-  int const mtiles = (G.M + 15) / 16, S = 4 * mtiles, F = P.forloop_range;
+  int const mtiles = (G.M + 15) / 16, pieces = G.NC / 16, S = pieces * mtiles, F = P.forloop_range;
+  int const lora = G.lora ? (G.rank + 15) / 16 : 0;
   long long const groups = (blocks + 7) / 8;
   // (the kernel decodes the flat id with multiply-high magics: exact while id x divisor < 2^32)
   long long const widest = std::max<long long>(8 * S, std::max(P.grid[0], P.grid[1]));
@@ -343,24 +350,41 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // a LoRA tile or a second activation makes it three operand rows a column (lora 16 x 4096 x 2048 6.5 / 9.4, 21 MB;
   // 16 x 4096 x 4096, 42 MB, 10.1 / 11.1, is still below the crossing, 16 x 8192 x 4096 17.3 / 17.1, but the program
   // printed for it is known to hold the streaming kernel and its workspace, and stays so); two weights 16 x 2560 x 6400, 65 MB, 16.2 / 17.1, 235 MB 54.6 / 48.4.
-  long long const weight_bytes = blocks * F * (long long)(G.nb * G.KT * 64 + (G.lora ? G.KT * 16 : 0)) * 2;
+  long long const weight_bytes = blocks * F * (long long)(G.nb * G.KT * G.NC + (G.lora ? G.KT * G.rank : 0)) * 2;
   bool const three = G.lora || G.pro == PRO_SILU_MUL;
   // SiLU(a) * u is done again by each of a block's pieces, so a long k of it is worth the other kernel's second
   // launch (the two products of a gated MLP, 3 rows: 1920 x 6400 25.7 / 23.0, 1280 x 3840 15.4 / 14.3, but 2560 x 1920
   // 13.1 / 16.0, and 16 x 2944 x 4032, whose 64-k iterations leave that kernel four times the slab, 20.6 / 25.0).
   bool const wide = G.pro == PRO_SILU_MUL ? G.KT > 64 && (!G.wcm || F * G.KT > 2048) : G.KT == 256 && !G.wcm;
   long long const most_bytes = (wide ? 8LL : (!G.wcm ? 17LL : (G.lora ? 32LL : three ? 48LL : (G.nb == 2 ? 68LL : 256LL)))) << 20;
-  if (s.gemm_mode == 0 && (blocks * S > (G.wcm ? 4096 : 1024) || weight_bytes > most_bytes)) {
+  // Other tiles run on the any-size kernel or, in 96-k iterations of 64 columns, on the one with a barrier a step:
+  // both are behind but for larger row-major plans (us, here / there: 64 rows x 3008 x 5120 in blocks of 32 columns
+  // 13.6 / 30.7, a LoRA of rank 32 of 16 x 2304 x 3584 10.1 / 17.2, 64 x 1280 x 768 in 96-k iterations 4.0 / 8.9;
+  // row-major 16 x 6144 x 2048 in blocks of 48 12.2 / 19.6, 64 x 12800 x 2048 in 128-k iterations 39.7 / 50.8, but
+  // 64 x 3840 x 2048 in 256-k ones 19.4 / 15.7, 64 x 3840 x 1920 in 96-k ones 18.6 / 15.3 and, of 64 columns,
+  // 16 x 6400 x 3072 15.1 / 14.4).
+  bool there;
+  if (G.whole && G.KT % 64 == 0) {
+    there = blocks * S > (G.wcm ? 4096 : 1024) || weight_bytes > most_bytes;
+  } else if (G.wcm) {
+    there = false;
+  } else if (G.whole) {
+    there = weight_bytes > (17LL << 20);
+  } else {
+    there = G.M > 32 && (G.KT == 96 || G.KT == 256) && weight_bytes > (8LL << 20);
+  }
+  if (s.gemm_mode == 0 && there) {
     return 0;
   }
-  int const wave_bytes = lanes_wave_bytes(G.KT, G.nb, G.lora, G.wcm, G.pro);
+  int const wave_bytes = lanes_wave_bytes(G.KT, G.nb, lora, G.wcm, G.pro);
   int const slot_bytes = F * G.nb * 512;
   // Workgroups of 16 wavefronts while about one round of them covers the grid; half that where two share a compute
   // unit and one's loads can run under the other's products (64 rows x 6400 x 4096 in 256-k iterations: 25.5 -> 19.7
   // us; 16 rows x 1280, 80 workgroups: 5.2 against 5.7 the other way).  With three operand rows a column the
   // registers of 16 wavefronts fill the unit either way (a gated MLP of 16 x 1920 x 6400: 26.4 against 27.7).
   int const waves = G.nb == 1 && !three && (long long)blocks * S * G.KT > 98304 ? 8 : 16;
-  int ip = F < waves ? F : waves;
+  int const most = std::min(waves, lanes_most(G.KT, lora));
+  int ip = F < most ? F : most;
   while (ip > 1 && ip * wave_bytes + slot_bytes > s.max_lds) {
     ip = (ip + 1) / 2;
   }
@@ -373,24 +397,28 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   L.gy = P.grid[1];
   L.blocks = (int)blocks;
   L.mtiles = mtiles;
+  L.pieces = pieces;
+  L.rank = G.rank;
   L.slot_base = ip * wave_bytes;
-  L.m_group = fast_div_magic(8 * 4 * mtiles);
-  L.m_pieces = fast_div_magic(4 * mtiles);
+  L.m_group = fast_div_magic(8 * S);
+  L.m_pieces = fast_div_magic(S);
+  L.m_columns = fast_div_magic(pieces);
   L.m_gx = fast_div_magic(P.grid[0]);
   L.m_gy = fast_div_magic(P.grid[1]);
   int const lds = ip * wave_bytes + slot_bytes, grid = (int)(groups * 8 * S);
   int rc = 0;
 #define MI355_LANES_CASE(NBV, PROV, LORAV)                                  \
-  if (G.nb == NBV && G.pro == PROV && G.lora == LORAV) {                    \
+  if (G.nb == NBV && G.pro == PROV && lora == LORAV) {                      \
     rc = G.wcm ? launch_lanes_kt<NBV, PROV, LORAV, true>(L, grid, ip * 64, lds)   \
                : launch_lanes_kt<NBV, PROV, LORAV, false>(L, grid, ip * 64, lds); \
   }
-  MI355_LANES_CASE(1, PRO_NONE, false)
-  MI355_LANES_CASE(1, PRO_EXP, false)
-  MI355_LANES_CASE(1, PRO_SILU, false)
-  MI355_LANES_CASE(2, PRO_NONE, false)
-  MI355_LANES_CASE(1, PRO_SILU_MUL, false)
-  MI355_LANES_CASE(1, PRO_NONE, true)
+  MI355_LANES_CASE(1, PRO_NONE, 0)
+  MI355_LANES_CASE(1, PRO_EXP, 0)
+  MI355_LANES_CASE(1, PRO_SILU, 0)
+  MI355_LANES_CASE(2, PRO_NONE, 0)
+  MI355_LANES_CASE(1, PRO_SILU_MUL, 0)
+  MI355_LANES_CASE(1, PRO_NONE, 1)
+  MI355_LANES_CASE(1, PRO_NONE, 2)
 #undef MI355_LANES_CASE
   if (rc == 1) {
     s.last().kernel_id = MI355_KERNEL_F16_GEMM;

@@ -579,33 +579,33 @@ __global__ __launch_bounds__(256) void gemm_fold_kernel(GemmParams const P) {
 
 // ---------------------------------------------------------------------------------------
 // One launch, no scratch: the output tile of a logical block is cut into 16-row x 16-column
-// pieces and every piece is a workgroup of its own (four pieces across the 64 columns, one
-// row of pieces per 16 activation rows), so a plan with a handful of blocks still covers the
+// pieces and every piece is a workgroup of its own, so a plan with a handful of blocks still covers the
 // chip.  Inside a workgroup the wavefronts are ITERATION LANES: lane ip takes iterations ip,
 // ip + IP, ... of the for-loop and needs nobody else for them --
-//   * its activation rows arrive as MFMA operands straight from global memory (a lane's eight
-//     consecutive k of one row are 16 contiguous bytes), the element-wise prologue is applied
-//     in registers;
-//   * its 16-column strip of each weight tile ([KT][16], 32 contiguous bytes per k) is copied
-//     by direct-to-LDS loads into a buffer of its own and read back with transposing LDS
-//     reads, which hand a lane the eight consecutive k of one column;
+//   * its activation rows come as they lie in memory and are turned into MFMA operands through LDS, the
+//     element-wise prologue is applied in registers;
+//   * column-major weights come the same way; of row-major ones its 16-column strip of a tile ([KT][16], 32
+//     contiguous bytes per k) is copied by direct-to-LDS loads into a buffer of its own and read back with
+//     transposing LDS reads, which hand a lane the eight consecutive k of one column;
 //   * one wait for all of its loads, then KT / 32 MFMAs per weight matrix (weights as the
 //     first operand: a lane ends up with four consecutive columns of one row);
 // so the workgroup is IP independent streams with no barrier in the loop.  Every iteration's
 // product piece is rounded to fp16 into an LDS slot of its own; after ONE barrier the
 // pieces are added in ITERATION order, rounding to fp16 after each add -- the arithmetic of
 // the sequential loop (src/kernel/triton_code_gen.cc:223-232) -- and stored.
-// Workgroup ids put the four column pieces of a block on ids that are equal modulo 8, i.e. on
+// Workgroup ids put the column pieces of a block on ids that are equal modulo 8, i.e. on
 // one XCD: the 128-byte lines of a weight row that the pieces share are fetched into one L2.
 struct LaneParams {
   GemmParams g;
   int gx, gy;        // the plan's grid (x, y): the logical block index is decoded from a flat id
   int blocks;        // logical blocks
   int mtiles;        // 16-row pieces per block
+  int pieces;        // 16-column pieces per block
+  int rank;          // of lora A
   int slot_base;     // byte offset of the product slots in LDS (after the lanes' buffers)
-  // multiply-high division magics (fast_div_magic) of 8 * 4 * mtiles, 4 * mtiles, gx and gy:
+  // multiply-high division magics (fast_div_magic) of 8 * pieces * mtiles, pieces * mtiles, pieces, gx and gy:
   // the decode of the flat id is on the path to the first load
-  uint32_t m_group, m_pieces, m_gx, m_gy;
+  uint32_t m_group, m_pieces, m_columns, m_gx, m_gy;
 };
 
 #pragma clang diagnostic push
@@ -639,18 +639,21 @@ __device__ __forceinline__ half4 lane_tr16(_Float16 const *p) {
 // vector cache against 58 (32 rows x 2240 x 1856 in 64-k iterations: 9.0 -> 5.5 us).
 constexpr int kUnitBytes = 2048;  // [16][64 k]
 // bytes of a wavefront's strips: the units being turned; row-major weights, the [16][16] piece of lora B
-constexpr int lanes_wave_bytes(int KT, int nb, bool lora, bool wcm, int pro) {
-  int const units = 1 + (pro == PRO_SILU_MUL ? 1 : 0) + (wcm ? nb + (lora ? 1 : 0) : 0);
-  return units * kUnitBytes + (wcm ? 0 : (nb + (lora ? 1 : 0)) * KT * 32 + (lora ? 512 : 0));
+// (lora: 16-rank pieces of lora A, the last of them may hold 8)
+constexpr int lanes_wave_bytes(int KT, int nb, int lora, bool wcm, int pro) {
+  int const units = 1 + (pro == PRO_SILU_MUL ? 1 : 0) + (wcm ? nb + lora : 0);
+  return units * kUnitBytes + (wcm ? 0 : (nb + lora) * KT * 32 + lora * 512);
 }
-template <int KT, int NB, int PRO, bool LORA, bool WCM>
-__global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
+// most iteration lanes of a workgroup: what the registers of three tiles in flight leave
+constexpr int lanes_most(int KT, int lora) { return lora == 2 && KT == 256 ? 8 : 16; }
+template <int KT, int NB, int PRO, int LORA, bool WCM>
+__global__ __launch_bounds__(64 * lanes_most(KT, LORA)) void gemm_lanes_kernel(LaneParams const L) {
   fetch_kernel_arguments<sizeof(LaneParams), 4>();  // every line of the block, one trip (blockDim.x is read)
   GemmParams const &P = L.g;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   constexpr int KS = KT / 32;                                // MFMA steps (and 1 KB loads) per strip
-  constexpr int STRIPS = NB + (LORA ? 1 : 0);
-  constexpr int KU = KT / 64;                                // units
+  constexpr int STRIPS = NB + LORA;
+  constexpr int KU = (KT + 63) / 64;                         // units, the last one of 32 k where KT is an odd number of them
   constexpr int WAVE_BYTES = lanes_wave_bytes(KT, NB, LORA, WCM, PRO), UNITS = 1 + (PRO == PRO_SILU_MUL) + (WCM ? STRIPS : 0);
   int const tid = threadIdx.x, lane = tid % 64, IP = blockDim.x / 64;
   int const ip = __builtin_amdgcn_readfirstlane(tid / 64);  // (wave-uniform: addresses stay scalar)
@@ -660,7 +663,7 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
   // flat id -> (logical block, row piece, column piece): ids that differ by 8 x piece index
   // share a block
   auto div = [](unsigned v, uint32_t magic) { return magic == 0 ? v : __umulhi(v, magic); };
-  unsigned const S = 4 * L.mtiles;
+  unsigned const S = (unsigned)(L.pieces * L.mtiles);
   unsigned const id = blockIdx.x;
   unsigned const eighth = id >> 3;
   int const blk = (int)(div(id, L.m_group) * 8 + (id & 7));
@@ -668,7 +671,7 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
   if (blk >= L.blocks) {
     return;
   }
-  int const piece = sub % 4, mt = sub / 4;
+  int const mt = (int)div((unsigned)sub, L.m_columns), piece = sub - mt * L.pieces;
   unsigned const q1 = div((unsigned)blk, L.m_gx);  // blk / gx
   unsigned const q2 = div(q1, L.m_gy);             // blk / (gx * gy)
   int const bx = (int)((unsigned)blk - q1 * (unsigned)L.gx), by = (int)(q1 - q2 * (unsigned)L.gy), bz = (int)q2;
@@ -690,31 +693,49 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
   bool const row_ok = 16 * mt + c < M;         // activation row of this lane's fragments
   // units: lane l has chunk l % 8 of rows l / 8 and 8 + l / 8; chunk q of row r lies at q ^ (r / 2 % 8)
   int const l8 = lane / 8, ch8 = lane % 8;
-  int const x_row[2] = {16 * mt + l8 < M ? 16 * mt + l8 : M - 1, 16 * mt + 8 + l8 < M ? 16 * mt + 8 + l8 : M - 1};
-  auto load_rows = [&](_Float16 const *tile, int ld, int r0, int r1, uint4v (&to)[KU][2]) {
+  // (of a unit of 32 k: lane l has chunk l % 4 of row l / 4)
+  int const l4 = lane / 4, ch4 = lane % 4;
+  auto half_unit = [](int u) { return 64 * u + 32 == KT; };
+  auto load_rows = [&](_Float16 const *tile, int ld, int row0, int rows, uint4v (&to)[KU][2]) {  // rows past `rows` re-read one
+    auto at = [&](int r) { return tile + (long long)(row0 + r < rows ? row0 + r : rows - 1) * ld; };
 #pragma unroll
     for (int u = 0; u < KU; u++) {
-      to[u][0] = *reinterpret_cast<uint4v const *>(tile + (long long)r0 * ld + 64 * u + 8 * ch8);
-      to[u][1] = *reinterpret_cast<uint4v const *>(tile + (long long)r1 * ld + 64 * u + 8 * ch8);
+      if (half_unit(u)) {
+        to[u][0] = *reinterpret_cast<uint4v const *>(at(l4) + 64 * u + 8 * ch4);
+      } else {
+        to[u][0] = *reinterpret_cast<uint4v const *>(at(l8) + 64 * u + 8 * ch8);
+        to[u][1] = *reinterpret_cast<uint4v const *>(at(8 + l8) + 64 * u + 8 * ch8);
+      }
     }
   };
-  auto put_unit = [&](int which, uint4v const (&from)[2]) {
-    unsigned char *const to = units + which * kUnitBytes + 128 * l8;
-    *reinterpret_cast<uint4v *>(to + 16 * (ch8 ^ (l8 / 2))) = from[0];
-    *reinterpret_cast<uint4v *>(to + 1024 + 16 * (ch8 ^ (l8 / 2 + 4))) = from[1];
+  auto put_unit = [&](int which, int u, uint4v const (&from)[2]) {
+    unsigned char *const to = units + which * kUnitBytes;
+    if (half_unit(u)) {
+      *reinterpret_cast<uint4v *>(to + 128 * l4 + 16 * (ch4 ^ (l4 / 2))) = from[0];
+    } else {
+      *reinterpret_cast<uint4v *>(to + 128 * l8 + 16 * (ch8 ^ (l8 / 2))) = from[0];
+      *reinterpret_cast<uint4v *>(to + 128 * l8 + 1024 + 16 * (ch8 ^ (l8 / 2 + 4))) = from[1];
+    }
   };
   auto operand = [&](int which, int s) {  // row c, k 32 s + 8 g ..
     return *reinterpret_cast<half8 const *>(units + which * kUnitBytes + 128 * c + 16 * ((4 * s + g) ^ (c / 2)));
   };
 
-  half4 lb_frag = {(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
-  if (LORA) {
+  half4 lb_frag[LORA > 0 ? LORA : 1];
+  int const rank = L.rank;
+  if (LORA > 0) {
     _Float16 const *src = static_cast<_Float16 const *>(P.lb.ptr) + gtile_offset(P.lb, bx, by, bz, 0);
     if (WCM) {
-      // lora B^T[n0 + c][k = 4g .. + 3]: 8 bytes, loop invariant
-      lb_frag = *reinterpret_cast<half4 const *>(src + (long long)(n0 + c) * P.lb.d_cols + 4 * g);
-    } else if (lane < 32) {
-      // lora B [16][64], loop invariant: this piece's 16 columns, rows of 32 bytes
+      // lora B^T[n0 + c][k = 16 q + 4g .. + 3]: 8 bytes, loop invariant
+#pragma unroll
+      for (int q = 0; q < LORA; q++) {
+        lb_frag[q] = half4{(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
+        if (16 * q + 4 * g < rank) {
+          lb_frag[q] = *reinterpret_cast<half4 const *>(src + (long long)(n0 + c) * P.lb.d_cols + 16 * q + 4 * g);
+        }
+      }
+    } else if (lane < 32 * LORA) {
+      // lora B [16 LORA][64], loop invariant: this piece's 16 columns, rows of 32 bytes
       lane_dma16(src + n0, (uint32_t)((ld_row * P.lb.d_cols + 8 * ld_half) * 2), lane_lds_address(lb_piece));
     }
   }
@@ -729,11 +750,11 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
     uint4v wr[WCM ? STRIPS : 1][KU][2], xr[KU][2], ur[KU][2];
 #pragma unroll
     for (int b = 0; b < STRIPS; b++) {
-      GTile const &bt = b == NB ? P.la : (b == 0 ? P.b0 : P.b1);
-      int const col0 = b == NB ? 0 : n0;  // the lora A tile is [KT][16]: whole
+      GTile const &bt = b >= NB ? P.la : (b == 0 ? P.b0 : P.b1);
+      int const col0 = b >= NB ? 16 * (b - NB) : n0;
       if (WCM) {
-        load_rows(static_cast<_Float16 const *>(bt.ptr) + gtile_offset(bt, bx, by, bz, it), bt.d_cols, col0 + l8, col0 + 8 + l8,
-                  wr[WCM ? b : 0]);
+        load_rows(static_cast<_Float16 const *>(bt.ptr) + gtile_offset(bt, bx, by, bz, it), bt.d_cols, col0,
+                  b >= NB ? rank : col0 + 16, wr[WCM ? b : 0]);
       } else {
         _Float16 const *src = static_cast<_Float16 const *>(bt.ptr) + gtile_offset(bt, bx, by, bz, it) + col0;
         uint32_t const off = (uint32_t)((ld_row * bt.d_cols + 8 * ld_half) * 2);
@@ -743,9 +764,9 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
         }
       }
     }
-    load_rows(static_cast<_Float16 const *>(P.a0.ptr) + gtile_offset(P.a0, bx, by, bz, it), P.a0.d_cols, x_row[0], x_row[1], xr);
+    load_rows(static_cast<_Float16 const *>(P.a0.ptr) + gtile_offset(P.a0, bx, by, bz, it), P.a0.d_cols, 16 * mt, M, xr);
     if (PRO == PRO_SILU_MUL) {
-      load_rows(static_cast<_Float16 const *>(P.a1.ptr) + gtile_offset(P.a1, bx, by, bz, it), P.a1.d_cols, x_row[0], x_row[1], ur);
+      load_rows(static_cast<_Float16 const *>(P.a1.ptr) + gtile_offset(P.a1, bx, by, bz, it), P.a1.d_cols, 16 * mt, M, ur);
     }
     if (!WCM) {
       // ---- one wait for all of it (direct-to-LDS loads and register loads do not complete in
@@ -756,7 +777,7 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
 #pragma unroll
       for (int u = 0; u < KU; u++) {
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < (half_unit(u) ? 1 : 2); h++) {
           asm volatile("" : "+v"(xr[u][h]));  // (no use moves above the wait)
           if (PRO == PRO_SILU_MUL) {
             asm volatile("" : "+v"(ur[u][h]));
@@ -765,26 +786,30 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
       }
 #pragma clang diagnostic pop
     }
-    float4v o[NB], d = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4v o[NB], d[LORA > 0 ? LORA : 1];
+#pragma unroll
+    for (int q = 0; q < LORA; q++) {
+      d[q] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    }
 #pragma unroll
     for (int b = 0; b < NB; b++) {
       o[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
     }
 #pragma unroll
     for (int u = 0; u < KU; u++) {
-      put_unit(0, xr[u]);
+      put_unit(0, u, xr[u]);
       if (PRO == PRO_SILU_MUL) {
-        put_unit(1, ur[u]);
+        put_unit(1, u, ur[u]);
       }
       if (WCM) {
 #pragma unroll
         for (int b = 0; b < STRIPS; b++) {
-          put_unit(UNITS - STRIPS + b, wr[WCM ? b : 0][u]);
+          put_unit(UNITS - STRIPS + b, u, wr[WCM ? b : 0][u]);
         }
       }
       asm volatile("" ::: "memory");  // (a wavefront's LDS operations complete in order)
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
+      for (int h = 0; h < (half_unit(u) ? 1 : 2); h++) {
         int const j = 2 * u + h;
         // ---- activation fragments: rows past M are zero, prologue in registers
         half8 x = operand(0, h);
@@ -819,21 +844,22 @@ __global__ __launch_bounds__(1024) void gemm_lanes_kernel(LaneParams const L) {
             half4 const lo = lane_tr16(wp), hi = lane_tr16(wp + 64);
             w = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
           }
-          float4v &to = b == NB ? d : o[b < NB ? b : 0];
+          float4v &to = b >= NB ? d[b >= NB ? b - NB : 0] : o[b < NB ? b : 0];
           to = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, to, 0, 0, 0);
         }
       }
       asm volatile("" ::: "memory");
     }
-    half4 dfrag;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      dfrag[r] = static_cast<_Float16>(d[r]);
-    }
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-      if (LORA) {
-        half4 const w = WCM ? lb_frag : lane_tr16(lb_piece + (4 * g) * 16 + tr_off);  // B[k = 4g ..][n = c]
+#pragma unroll
+      for (int q = 0; q < LORA; q++) {
+        half4 dfrag;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          dfrag[r] = static_cast<_Float16>(16 * q + 4 * g < rank ? d[q][r] : 0.0f);
+        }
+        half4 const w = WCM ? lb_frag[q] : lane_tr16(lb_piece + 256 * q + (4 * g) * 16 + tr_off);  // B[k = 16 q + 4g ..][n = c]
         o[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(w, dfrag, o[b], 0, 0, 0);
       }
       half4 p16;

@@ -114,3 +114,24 @@ def test_strips_of_16_columns(rt, ranges, m, blocks, kt, loop, weights):
         spec, _ = W.config5_gated_mlp(m=m, d=kt * loop, h=64 * blocks, grid1=blocks, F1=loop, grid2=kt * loop // 64, F2=blocks)
         spec = [op for i, op in enumerate(spec[:5]) if i != 3]
     _run(rt, spec, COL, f"strips {m} x {blocks}, {kt} x {loop}, {weights}", **({} if weights == 1 else {"std": 0.05}))
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("m,cols,blocks,kt,loop,rank", [
+    (1, 16, 9, 64, 3, 0), (33, 48, 3, 128, 5, 0), (64, 128, 7, 256, 9, 0), (17, 80, 2, 64, 17, 0), (9, 32, 65, 256, 2, 0),
+    (1, 64, 5, 96, 4, 0), (50, 48, 3, 32, 18, 0), (16, 16, 9, 96, 1, 0), (3, 64, 4, 96, 6, 16), (20, 32, 3, 32, 5, 32),
+    (17, 64, 3, 64, 4, 16), (5, 64, 9, 256, 9, 32), (33, 32, 5, 128, 3, 32), (16, 64, 2, 64, 17, 8), (64, 16, 3, 256, 2, 8)])
+def test_one_launch_of_any_columns_and_rank(rt, abi, m, cols, blocks, kt, loop, rank, order):
+    """The one-launch kernel on blocks of one and more 16-column pieces, of several 16-row pieces, with a lora A
+    of half a piece (column-major; left to the tiles row-major) and of two."""
+    from attention_superoptimizer_amd import workloads as W
+    if rank == 0:
+        spec, _ = W.tiled_matmul(m, cols * blocks, kt * loop, (blocks, 1, 1), loop, (-1, -1, -1), (1, -1, -1), (1, -1, -1))
+    else:
+        spec, _ = W.config4_lora(m=m, d=kt * loop, r=rank, grid=blocks, F=loop)
+        spec[1], spec[3] = W._inp([kt * loop, cols * blocks], COL), W._inp([rank, cols * blocks], COL)
+    assert abi.mi355_set_option(7, 2) == 0
+    try:
+        _run(rt, spec, order, f"pieces {m} x {cols} x {blocks}, {kt} x {loop}, rank {rank} {order}")
+    finally:
+        assert abi.mi355_set_option(7, 0) == 0
