@@ -343,7 +343,7 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // Row-major weights: a 16-column strip uses 32 bytes of every line it pulls into a compute unit's vector cache,
   // so only where the launch sets the time (16 rows, in us, here / there: 3840 columns in 128-k iterations, 16 MB,
   // 6.7 / 8.3; 6400, 26 MB, 9.8 / 9.1; 64-column blocks of 256 k fill LDS with fewer wavefronts: 1280 columns,
-  // 10 MB, 9.6 / 7.6).
+  // 10 MB, 9.6 / 7.6; few pieces leave the chip idle: two weights of 1088 columns, 14 MB, 68 pieces, 0.5 us behind).
   // Column-major weights: a piece's columns are whole lines of its own, and the line lies far out, where the
   // activation rows that the pieces read outnumber what the second launch costs.  One weight (64 rows x 12800 x 4096
   // 45 / 62, 8 x 28672 x 4096, 235 MB of weights, 39.6 / 53, but 64 x 28672 x 1024, 7168 pieces, 22.2 / 19.6);
@@ -355,7 +355,7 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // SiLU(a) * u is done again by each of a block's pieces, so a long k of it is worth the other kernel's second
   // launch (the two products of a gated MLP, 3 rows: 1920 x 6400 25.7 / 23.0, 1280 x 3840 15.4 / 14.3, but 2560 x 1920
   // 13.1 / 16.0, and 16 x 2944 x 4032, whose 64-k iterations leave that kernel four times the slab, 20.6 / 25.0).
-  bool const wide = G.pro == PRO_SILU_MUL ? G.KT > 64 && (!G.wcm || F * G.KT > 2048) : G.KT == 256 && !G.wcm;
+  bool const wide = G.pro == PRO_SILU_MUL ? G.KT > 64 && (!G.wcm || F * G.KT > 2048) : !G.wcm && (G.KT == 256 || blocks * S < 128);
   long long const most_bytes = (wide ? 8LL : (!G.wcm ? 17LL : (G.lora ? 32LL : three ? 48LL : (G.nb == 2 ? 68LL : 256LL)))) << 20;
   // Other tiles run on the any-size kernel or, in 96-k iterations of 64 columns, on the one with a barrier a step:
   // both are behind but for larger row-major plans (us, here / there: 64 rows x 3008 x 5120 in blocks of 32 columns
