@@ -267,7 +267,7 @@ __device__ __forceinline__ void gemm_store(AnyGemm const &G, float4v const (&acc
 
 // A workgroup owns a BM x BN tile of C and a range of k.  Its KG groups of wavefronts (WM x WN of the
 // tile per wavefront) take a part of the range each and add their sums up in LDS at the end: with few
-// tiles that is what keeps a compute unit busy.  A stage of 64 k goes global -> registers (two stages
+// tiles that is what keeps a compute unit busy.  A stage of 64 k goes global -> registers (PF stages
 // ahead) -> LDS (two buffers, one barrier a stage) -> MFMA operands.  Registers rather than direct
 // loads to LDS in between, because that is where a chunk of an odd-length row can be shifted and
 // masked.  The partial stage at the end of k comes FIRST, so that the loop itself has no conditions
@@ -279,9 +279,9 @@ __device__ __forceinline__ void gemm_store(AnyGemm const &G, float4v const (&acc
 // row-major weights through a transposed copy: [8, 500, 1000] . [1000, 64] 67 -> 6.4 us,
 // [300, 2048] . [2048, 5504] row-major 39 -> 20 us, [100, 320] . [320, 755] 46 -> 4.2 us,
 // [1024, 2048] . [2048, 5504] 42 us (550 TFLOP/s).
-template <int BM, int BN, int WM, int WN, int KG, bool A_KC, bool B_KC>
+template <int BM, int BN, int WM, int WN, int KG, bool A_KC, bool B_KC, int PF = 2>
 __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG) void f16_gemm_any_kernel(AnyGemm const G) {
-  constexpr int NTG = 64 * (BM / WM) * (BN / WN), NT = NTG * KG, PF = 2;
+  constexpr int NTG = 64 * (BM / WM) * (BN / WN), NT = NTG * KG;
   constexpr int TM = WM / 16, TN = WN / 16;
   using SA = OperandStage<BM, NTG, A_KC>;
   using SB = OperandStage<BN, NTG, B_KC>;
@@ -359,8 +359,11 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG) void f16_gemm_any_
     } else if (whole > 0) {
       load(0, 0);
     }
-    if (steps > 1) {
-      load(1, 1);
+#pragma unroll
+    for (int u = 1; u < PF; u++) {
+      if (steps > u) {
+        load(u, u);
+      }
     }
     if (lead) {
       sa.mask_tail(ra[0], tail);
@@ -373,28 +376,28 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG) void f16_gemm_any_
     Operands x0, x1;
     read(x0, 0, 0);
     int t = 0;
-    for (; t + PF + 1 < steps; t += 2) {
+    for (; t + 2 * PF - 1 < steps; t += PF) {
 #pragma unroll
-      for (int u = 0; u < 2; u++) {
+      for (int u = 0; u < PF; u++) {
         load(u, t + u + PF);
         read(x1, t + u, 1);
         multiply(x0, t + u);
-        store(1 - u, t + u + 1);
+        store((u + 1) % PF, t + u + 1);
         __syncthreads();
         read(x0, t + u + 1, 0);
         multiply(x1, t + u);
       }
     }
 #pragma unroll
-    for (int u = 0; u < 3; u++) {  // the last one to three stages
+    for (int u = 0; u < 2 * PF - 1; u++) {  // the last stages
       if (t + u < steps) {
-        if (u == 0 && t + PF < steps) {
-          load(0, t + PF);
+        if (u < PF - 1 && t + u + PF < steps) {
+          load(u, t + u + PF);
         }
         read(x1, t + u, 1);
         multiply(x0, t + u);
         if (t + u + 1 < steps) {
-          store((u + 1) % 2, t + u + 1);
+          store((u + 1) % PF, t + u + 1);
         }
         __syncthreads();
         if (t + u + 1 < steps) {

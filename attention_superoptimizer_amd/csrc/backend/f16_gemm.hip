@@ -382,6 +382,7 @@ namespace {
 struct TileKernel {
   void (*fn)(AnyGemm);
   int lds;
+  void (*deep)(AnyGemm) = nullptr;  // four stages ahead instead of two
 };
 template <bool A_KC, int I>
 constexpr GemmTile kTile = kGemmTiles[I];
@@ -392,7 +393,12 @@ template <int I, bool A_KC, bool B_KC>
 constexpr TileKernel tile_kernel() {
   constexpr GemmTile t = kTile<A_KC, I>;
   if constexpr (t.kind == STAGED) {
-    return {f16_gemm_any_kernel<t.bm, t.bn, t.wm, t.wn, t.kg, A_KC, B_KC>, any_gemm_lds<t.bm, t.bn, t.wm, t.wn, t.kg, A_KC, B_KC>()};
+    constexpr int lds = any_gemm_lds<t.bm, t.bn, t.wm, t.wn, t.kg, A_KC, B_KC>();
+    if constexpr (t.bm <= 64 && t.bn == 64) {
+      return {f16_gemm_any_kernel<t.bm, t.bn, t.wm, t.wn, t.kg, A_KC, B_KC>, lds, f16_gemm_any_kernel<t.bm, t.bn, t.wm, t.wn, t.kg, A_KC, B_KC, 4>};
+    } else {
+      return {f16_gemm_any_kernel<t.bm, t.bn, t.wm, t.wn, t.kg, A_KC, B_KC>, lds};
+    }
   } else if constexpr (t.kind == DIRECT) {
     return {f16_gemm_direct_kernel<t.bm, t.bn, t.wm, t.wn, B_KC>, direct_gemm_lds<t.bm, t.bn>()};
   } else {
@@ -427,8 +433,12 @@ int launch_gemm_tiles(AnyGemm &G, int batch, bool a_kc, bool b_kc, GemmChoice co
     return fail(MI355_ERR_UNSUPPORTED, "matmul has too many output tiles");
   }
   G.total = (unsigned)total;
-  MI355_GRANT_LDS(kernel.fn, kernel.lds);
-  MI355_HIP(launch_kernel(kernel.fn, G.total, t.threads(), kernel.lds, state().stream(), G));
+  // Stages further ahead where a range is long (un-fused MLPs, us: 182 x 1830 x 1807 41.6 -> 33.3, 300 x 1027 x 2049 39.3
+  // -> 33.9, 500 x 1999 x 3001 78.0 -> 75.1); a short one has them all in its last stages, which load under conditions
+  // (from 6 on, 34 x 1455 x 790 27.7 -> 29.2).
+  auto *const fn = kernel.deep != nullptr && G.steps_per_range >= 16 ? kernel.deep : kernel.fn;
+  MI355_GRANT_LDS(fn, kernel.lds);
+  MI355_HIP(launch_kernel(fn, G.total, t.threads(), kernel.lds, state().stream(), G));
   if (G.ksplit > 1) {
     size_t const n = (size_t)batch * G.m * G.n, blocks = (n / 4 + kThreads) / kThreads;
     MI355_HIP(launch_kernel(f16_gemm_fold_kernel, (unsigned)std::min<size_t>(blocks, 4096), kThreads, 0, state().stream(), G, n));

@@ -142,3 +142,14 @@ def test_softmax_rows_out_of_range(rt, abi, m, n):
         ok = np.isfinite(s)
         # (one order of the fp32 row sum against another: two fp16 places, where they are normal numbers)
         assert_f16_close(w[ok], s[ok], rtol=2e-3, atol=1e-6, what="row sum or quotient")
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (40, 2105, 1087), (126, 2105, 1151), (182, 1807, 1027), (300, 1027, 1343),  # 16, 17 and 20 stages and a part of one
+    (126, 1300, 2049), (300, 2049, 1280), (603, 1220, 1408)])                   # 32; 20 and 22 whole stages
+def test_matmul_of_many_stages(rt, abi, m, n, k):
+    """Ranges long enough to be loaded four stages ahead: every remainder of their number by four, with and
+    without a partial stage."""
+    for a_cm, b_cm in ((0, 1), (0, 0), (1, 1)):
+        a, b, got = _abi_matmul(rt, abi, 1, m, n, k, a_cm, b_cm, 5)
+        assert_f16_close(got, orc.f16_matmul(a, b), what=f"[{m},{k}] . [{k},{n}], A cm {a_cm}, B cm {b_cm}")
