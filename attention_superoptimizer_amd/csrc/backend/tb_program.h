@@ -123,6 +123,7 @@ int try_launch_gemm(DevProgram const &prog);  // gemm_fused.hip, same convention
 bool gemm_applicable(DevProgram const &prog);
 int try_launch_combine(DevProgram const &prog);  // combine_fused.hip, same convention
 bool combine_applicable(DevProgram const &prog);
+int try_launch_fp_combine(DevProgram const &prog);  // the uint16 program of the family, same convention
 
 // Lowers `plan` for the uint16 interpreter (f16 == false: plain row-major tiles)
 // or the fp16 interpreter (f16 == true: padded rows, B operands k-contiguous).
