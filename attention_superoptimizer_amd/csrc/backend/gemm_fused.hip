@@ -349,14 +349,31 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // 45 / 62, 8 x 28672 x 4096, 235 MB of weights, 39.6 / 53, but 64 x 28672 x 1024, 7168 pieces, 22.2 / 19.6);
   // a LoRA tile or a second activation makes it three operand rows a column (lora 16 x 4096 x 2048 6.5 / 9.4, 21 MB;
   // 16 x 4096 x 4096, 42 MB, 10.1 / 11.1, is still below the crossing, 16 x 8192 x 4096 17.3 / 17.1, but the program
-  // printed for it is known to hold the streaming kernel and its workspace, and stays so); two weights 16 x 2560 x 6400, 65 MB, 16.2 / 17.1, 235 MB 54.6 / 48.4.
+  // printed for it is known to hold the streaming kernel and its workspace, and stays so); two weights in 64-k or
+  // 128-k iterations at any size (8 rows: 832 x 14336 10.6 / 13.1, 4096 x 6464 25.4 / 29.9, 4096 x 14336, 235 MB,
+  // 49.2 / 53.6), in 256-k ones 4096 x 8192, 134 MB, 28.2 / 25.4.
+  // Two row-major weights with almost a workgroup for every compute unit stand between (4096 x 3904 14.0 / 18.8,
+  // 1536 x 3904 7.0 / 8.0, but 256 workgroups 10.8 / 9.8, 404 13.6 / 10.8, and 128-k iterations 8.9 / 7.1).
   long long const weight_bytes = blocks * F * (long long)(G.nb * G.KT * G.NC + (G.lora ? G.KT * G.rank : 0)) * 2;
   bool const three = G.lora || G.pro == PRO_SILU_MUL;
-  // SiLU(a) * u is done again by each of a block's pieces, so a long k of it is worth the other kernel's second
-  // launch (the two products of a gated MLP, 3 rows: 1920 x 6400 25.7 / 23.0, 1280 x 3840 15.4 / 14.3, but 2560 x 1920
-  // 13.1 / 16.0, and 16 x 2944 x 4032, whose 64-k iterations leave that kernel four times the slab, 20.6 / 25.0).
-  bool const wide = G.pro == PRO_SILU_MUL ? G.KT > 64 && (!G.wcm || F * G.KT > 2048) : !G.wcm && (G.KT == 256 || blocks * S < 128);
-  long long const most_bytes = (wide ? 8LL : (!G.wcm ? 17LL : (G.lora ? 32LL : three ? 48LL : (G.nb == 2 ? 68LL : 256LL)))) << 20;
+  long long most_mb = 256;
+  if (!G.wcm) {
+    most_mb = G.KT == 256 || blocks * S < 128 ? 8 : (G.nb == 2 && G.KT == 64 && blocks * S < 256 ? 68 : 17);
+  } else if (G.lora || three) {
+    most_mb = G.lora ? 32 : 48;
+  } else if (G.nb == 2 && G.KT == 256) {
+    most_mb = 68;
+  }
+  // SiLU(a) * u is done again by each of a block's pieces, one piece's iterations take the same time however few
+  // pieces there are, and past 104 units of 64 k the result slots leave LDS for half the wavefronts.  The other
+  // kernel's time grows with the weights and with the slab between its launches.  Both in ns (8 and 16 rows, us,
+  // here / there: 64 k an iteration, column-major 4096 outputs of 3904 11.0 / 14.6, 2048 of 3904 10.2 / 11.3, 832 of
+  // 6464 14.9 / 12.2, 640 of 12224 31.5 / 12.2; row-major 4096 of 3904 13.1 / 14.6, 2048 of 3904 12.3 / 11.4; 128 k
+  // 3776 of 4992 12.5 / 14.0, 2048 of 8192 17.1 / 13.0; 28 plans of either order and 8 or 16 rows: the choice is the
+  // faster kernel but for four that it has within 1.5 us).
+  long long const units = (long long)F * G.KT / 64;
+  long long const here_ns = (1000 + (G.wcm ? 142 : 170) * units) * ((blocks * S + 255) / 256);
+  long long const there_ns = 7000 + blocks * units + blocks * F * 7 / 10 + 15 * F;
   // Other tiles run on the any-size kernel or, in 96-k iterations of 64 columns, on the one with a barrier a step:
   // both are behind but for larger row-major plans (us, here / there: 64 rows x 3008 x 5120 in blocks of 32 columns
   // 13.6 / 30.7, a LoRA of rank 32 of 16 x 2304 x 3584 10.1 / 17.2, 64 x 1280 x 768 in 96-k iterations 4.0 / 8.9;
@@ -365,7 +382,10 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // 16 x 6400 x 3072 15.1 / 14.4).
   bool there;
   if (G.whole && G.KT % 64 == 0) {
-    there = blocks * S > (G.wcm ? 4096 : 1024) || weight_bytes > most_bytes;
+    there = blocks * S > (G.wcm ? 4096 : 1024) || weight_bytes > (most_mb << 20);
+    if (G.pro == PRO_SILU_MUL && G.M <= 16) {
+      there = units > 104 || here_ns > there_ns;
+    }
   } else if (G.wcm) {
     there = false;
   } else if (G.whole) {
@@ -380,11 +400,17 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   int const slot_bytes = F * G.nb * 512;
   // Workgroups of 16 wavefronts while about one round of them covers the grid; half that where two share a compute
   // unit and one's loads can run under the other's products (64 rows x 6400 x 4096 in 256-k iterations: 25.5 -> 19.7
-  // us; 16 rows x 1280, 80 workgroups: 5.2 against 5.7 the other way).  With three operand rows a column the
-  // registers of 16 wavefronts fill the unit either way (a gated MLP of 16 x 1920 x 6400: 26.4 against 27.7).
-  int const waves = G.nb == 1 && !three && (long long)blocks * S * G.KT > 98304 ? 8 : 16;
+  // us; 16 rows x 1280, 80 workgroups: 5.2 against 5.7 the other way).  Two weights leave LDS for one workgroup of 13
+  // and more: half as many there too, evened out over the rounds (8 rows, column-major: 832 x 14336 14.0 -> 10.6 us,
+  // 1024 x 12224 12.1 -> 10.0, 4096 x 3904 in one round 12.3 either way; row-major 832 x 6464 8.8 -> 7.4).  The
+  // registers of 16 wavefronts with SiLU(a) * u or a LoRA tile fill the unit either way (13.1 us there, 15.0 here).
+  int const waves = G.nb == 2 || (!three && (long long)blocks * S * G.KT > 98304) ? 8 : 16;
   int const most = std::min(waves, lanes_most(G.KT, lora));
   int ip = F < most ? F : most;
+  if (G.nb == 2) {
+    int const rounds = (F + ip - 1) / ip;
+    ip = (F + rounds - 1) / rounds;
+  }
   while (ip > 1 && ip * wave_bytes + slot_bytes > s.max_lds) {
     ip = (ip + 1) / 2;
   }
@@ -494,8 +520,11 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A)
   int ks = 1;
   EmitSink *const sink = emit_sink();
   if (!(fits && blocks * G.nb >= 96 && steps <= 8) && slab <= (sink ? kEmitScratchBytes : s.scratch_bytes)) {
+    // (two weights have workgroups of their own: a wavefront of one takes two iterations of 64 k, so that one's loads
+    // run under the other's products; 8 rows x 4096 x 3904 20.4 -> 18.8 us, 2944 x 6464 22.1 -> 20.2)
     long long const most = (ring <= 80 * 1024 ? 1024 : 256 / G.nb) / blocks;
-    ks = (int)std::max<long long>(1, std::min<long long>((F + 3) / 4, most));
+    int const least = G.nb == 2 && G.KT == 64 ? 8 : 4;
+    ks = (int)std::max<long long>(1, std::min<long long>((F + least - 1) / least, most));
   }
   if (ks == 1 && !fits && !strips) {
     return 0;

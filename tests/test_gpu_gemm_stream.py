@@ -135,3 +135,17 @@ def test_one_launch_of_any_columns_and_rank(rt, abi, m, cols, blocks, kt, loop, 
         _run(rt, spec, order, f"pieces {m} x {cols} x {blocks}, {kt} x {loop}, rank {rank} {order}")
     finally:
         assert abi.mi355_set_option(7, 0) == 0
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("option", [0, 1, 2], ids=["rule", "stream", "lanes"])
+@pytest.mark.parametrize("m,loop1,loop2", [(1, 9, 17), (16, 13, 8), (8, 17, 41), (9, 64, 2)])
+def test_two_weights_uneven_rounds(rt, abi, m, loop1, loop2, option, order):
+    """Loops that do not divide by a workgroup's wavefronts, and ranges of 8 iterations whose last one is short."""
+    from attention_superoptimizer_amd import workloads as W
+    spec, _ = W.config5_gated_mlp(m=m, d=64 * loop1, h=64 * loop2, grid1=loop2, F1=loop1, grid2=loop1, F2=loop2)
+    assert abi.mi355_set_option(7, option) == 0
+    try:
+        _run(rt, spec, order, f"{m} x {64 * loop1} x {64 * loop2} {order}", std=0.02)
+    finally:
+        assert abi.mi355_set_option(7, 0) == 0
