@@ -286,7 +286,9 @@ int launch_rows(RowsAttention const &A) {
 }
 
 // A wavefront's blocks: as few as hold the row.  Eight wavefronts leave room for two workgroups on a compute
-// unit up to 768 keys ([28, 146, 828]: 280 workgroups, 19.6 us with sixteen wavefronts, 16.7 with eight).
+// unit up to 768 keys ([28, 146, 828]: 280 workgroups, 19.6 us with sixteen wavefronts, 16.7 with eight).  At
+// head size 128 twelve, with fewer blocks each, were slower: [1, 30, 700] 10.1 us, with eight 9.2, [16, 250, 1500]
+// 23.6 and 21.2 (and of five blocks or more their registers spill).
 template <bool KC>
 int launch_rows_of(RowsAttention const &A, int d) {
   int const blocks = (A.n + 31) / 32, eights = (blocks + 7) / 8;
@@ -318,12 +320,14 @@ int launch_rows_of(RowsAttention const &A, int d) {
 // 12.2 us, [8, 800, 1024] 23.5 and 15.8, [32, 1000, 500] 51.4 and 43.0, but [32, 512, 1024] 42.1 and 50.2;
 // [8, 640, 2000] 33.5 and 29.9, but [16, 512, 2000] 50.3 and 55.3.  Head size 128, [2, 1200, 600] 16.5 and
 // 11.7, but [8, 640, 600] 20.4 and 21.7; [8, 300, 1500] 25.0 and 20.0, but few workgroups with a long row
-// each leave most of the chip idle: [4, 300, 1500] 19.7 and 21.5, [1, 1, 2048] 11.4 and 16.3.
+// each leave most of the chip idle: [4, 300, 1500] 19.7 and 21.5, [1, 1, 2048] 11.4 and 16.3, [4, 30, 800] 10.7
+// and 11.3, [2, 19, 869] 12.8 and 13.3, but [8, 128, 800] 12.7 and 11.9, [1, 30, 700] 11.5 and 9.2.
 bool rows_pay(int d, int n, long long workgroups) {
   if (d == 64) {
     return n <= 512 || (n <= 1024 && workgroups <= 768) || (n <= 2048 && workgroups <= 400);
   }
-  return (n <= 256 && workgroups <= 400) || (n <= 1024 && workgroups <= 256) || (n <= 2048 && workgroups >= 128 && workgroups <= 256);
+  int const fewest = n <= 768 ? 1 : (n <= 1024 ? 64 : 128);
+  return (n <= 256 && workgroups <= 400) || (n <= 2048 && workgroups >= fewest && workgroups <= 256);
 }
 
 }  // namespace

@@ -56,6 +56,7 @@ def _check(ins, got):
     (9, 33, 500, 64),
     (2, 40, 767, 64),    # three blocks each
     (2, 40, 801, 128),
+    (22, 40, 801, 128),  # enough workgroups for a row of four blocks each
     (3, 40, 1024, 64),
     (1, 20, 1500, 64),
     (1, 300, 2047, 64),  # sixteen wavefronts with four blocks each
