@@ -368,11 +368,13 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // pieces there are, and past 104 units of 64 k the result slots leave LDS for half the wavefronts.  The other
   // kernel's time grows with the weights and with the slab between its launches.  Both in ns (8 and 16 rows, us,
   // here / there: 64 k an iteration, column-major 4096 outputs of 3904 11.0 / 14.6, 2048 of 3904 10.2 / 11.3, 832 of
-  // 6464 14.9 / 12.2, 640 of 12224 31.5 / 12.2; row-major 4096 of 3904 13.1 / 14.6, 2048 of 3904 12.3 / 11.4; 128 k
-  // 3776 of 4992 12.5 / 14.0, 2048 of 8192 17.1 / 13.0; 28 plans of either order and 8 or 16 rows: the choice is the
-  // faster kernel but for four that it has within 1.5 us).
+  // 6464 14.9 / 12.2, 640 of 12224 31.5 / 12.2; 128 k 3776 of 4992 12.5 / 14.0, 2048 of 8192 17.1 / 13.0.  Row-major
+  // weights that come from memory and not from the last-level cache cost the strips more, so those lines are of both
+  // products of a gated MLP in turn: 4096 of 3904 35.2 / 34.3, 3584 of 5440 48.7 / 45.6, 4096 of 2560 28.4 / 30.2.
+  // Of 28 such pairs of either order the choice is the faster one or within 1.1 us, but for row-major 2944 of 4032,
+  // 23.8 / 24.9 and, 16 rows, 23.8 / 26.4).
   long long const units = (long long)F * G.KT / 64;
-  long long const here_ns = (1000 + (G.wcm ? 142 : 170) * units) * ((blocks * S + 255) / 256);
+  long long const here_ns = (1000 + (G.wcm ? 142 : 225) * units) * ((blocks * S + 255) / 256);
   long long const there_ns = 7000 + blocks * units + blocks * F * 7 / 10 + 15 * F;
   // Other tiles run on the any-size kernel or, in 96-k iterations of 64 columns, on the one with a barrier a step:
   // both are behind but for larger row-major plans (us, here / there: 64 rows x 3008 x 5120 in blocks of 32 columns
