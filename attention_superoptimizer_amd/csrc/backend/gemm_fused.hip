@@ -353,12 +353,13 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // 128-k iterations at any size (8 rows: 832 x 14336 10.6 / 13.1, 4096 x 6464 25.4 / 29.9, 4096 x 14336, 235 MB,
   // 49.2 / 53.6), in 256-k ones 4096 x 8192, 134 MB, 28.2 / 25.4.
   // Two row-major weights with almost a workgroup for every compute unit stand between (4096 x 3904 14.0 / 18.8,
-  // 1536 x 3904 7.0 / 8.0, but 256 workgroups 10.8 / 9.8, 404 13.6 / 10.8, and 128-k iterations 8.9 / 7.1).
+  // 1536 x 3904 7.0 / 8.0, but 256 workgroups 10.8 / 9.8, 404 13.6 / 10.8, and 128-k iterations 8.9 / 7.1;
+  // with both products of a gated MLP 160 workgroups, 4096 x 2560, 28.4 / 25.0, 176 24.0 / 24.9, 200 25.9 either way).
   long long const weight_bytes = blocks * F * (long long)(G.nb * G.KT * G.NC + (G.lora ? G.KT * G.rank : 0)) * 2;
   bool const three = G.lora || G.pro == PRO_SILU_MUL;
   long long most_mb = 256;
   if (!G.wcm) {
-    most_mb = G.KT == 256 || blocks * S < 128 ? 8 : (G.nb == 2 && G.KT == 64 && blocks * S < 256 ? 68 : 17);
+    most_mb = G.KT == 256 || blocks * S < 128 ? 8 : (G.nb == 2 && G.KT == 64 && blocks * S >= 192 && blocks * S < 256 ? 68 : 17);
   } else if (G.lora || three) {
     most_mb = G.lora ? 32 : 48;
   } else if (G.nb == 2 && G.KT == 256) {
