@@ -306,7 +306,13 @@ int try_launch_fp_combine(DevProgram const &P) {
   CombineParams const A = combine_params(P, M);
   dim3 const grid(P.grid[0], P.grid[1], P.grid[2]);
   int const threads = std::min(256, (M.rows * (M.X / M.vec) + 63) / 64 * 64);
-  MI355_HIP(launch_kernel(M.vec == 8 ? fp_combine_kernel<8> : fp_combine_kernel<4>, grid, threads, 0, state().stream(), A, tables()));
+  State &s = state();
+  MI355_HIP(launch_kernel(M.vec == 8 ? fp_combine_kernel<8> : fp_combine_kernel<4>, grid, threads, 0, s.stream(), A, tables()));
+  s.last().kernel_id = MI355_KERNEL_FP_COMBINE;
+  s.last().workgroups = (int)(grid.x * grid.y * grid.z);
+  s.last().threads = threads;
+  s.last().lds_bytes = 0;
+  s.last().row_split = 1;
   return 1;
 }
 

@@ -1409,10 +1409,9 @@ static int launch(DevProgram const &prog, bool f16) {
   }
   dim3 grid(prog.grid[0] * (f16 ? 1 : prog.splits), prog.grid[1], prog.grid[2]);
   if (int const rc = f16 ? 0 : try_launch_fp_combine(prog)) {
-    if (rc < 0) {
-      return rc;
-    }
-  } else if (f16) {
+    return rc == 1 ? MI355_OK : rc;
+  }
+  if (f16) {
     MI355_GRANT_LDS(f16_interp_kernel, prog.lds_bytes);
     MI355_HIP(launch_kernel(f16_interp_kernel, grid, kInterpThreads, prog.lds_bytes, s.stream(), prog, s.phase_trace));
   } else {

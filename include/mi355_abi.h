@@ -87,6 +87,7 @@ typedef struct mi355_launch_info {
 #define MI355_KERNEL_F16_COMBINE 5   /* fused fold-partials-and-divide family */
 #define MI355_KERNEL_FP_GEMM 6       /* fused fingerprint tiled-matmul family (uint16) */
 #define MI355_KERNEL_FP_ATTENTION 7  /* fused fingerprint attention family (uint16) */
+#define MI355_KERNEL_FP_COMBINE 8    /* fused fold-partials-and-divide family (uint16) */
 
 /* Backend options (mi355_set_option).  FORCE_INTERPRETER = 1 sends every customized op,
  * fp16 or fingerprint, through the generic LDS interpreter instead of a fused kernel
