@@ -294,6 +294,9 @@ using namespace mi355;
 extern "C" int mi355_fp_attention_rows(uint16_t const *Q, uint16_t const *K, uint16_t const *V, uint16_t *S, uint16_t *E, uint16_t *R,
                                        uint16_t *P, uint16_t *O, int batch, int m, int n, int d, int dv, int *taken) {
   MI355_REQUIRE_INIT();
+  if (taken == nullptr) {
+    return fail(MI355_ERR_INVALID, "no place for the answer");
+  }
   *taken = 0;
   if (batch < 0 || m < 0 || n < 0 || d < 0 || dv < 0) {
     return fail(MI355_ERR_INVALID, "negative extent");

@@ -61,3 +61,7 @@ def test_a_graph_takes_it(rt, b, m, n, d, dv):
     finally:
         ops[0].close()  # (the arena is a stack)
         one[0].close()
+
+
+def test_no_place_for_the_answer(rt, abi):
+    assert abi.mi355_fp_attention_rows(*[None] * 8, 1, 16, 64, 64, 64, None) != 0
