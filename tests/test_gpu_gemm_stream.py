@@ -149,3 +149,58 @@ def test_two_weights_uneven_rounds(rt, abi, m, loop1, loop2, option, order):
         _run(rt, spec, order, f"{m} x {64 * loop1} x {64 * loop2} {order}", std=0.02)
     finally:
         assert abi.mi355_set_option(7, 0) == 0
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("family", ["exp", "silu", "silu_mul"])
+@pytest.mark.parametrize("m,cols,blocks,kt,loop,extremes", [
+    (17, 16, 9, 32, 5, False), (33, 48, 3, 96, 4, False), (64, 64, 2, 96, 3, False), (64, 48, 5, 32, 17, False),
+    (33, 64, 2, 64, 6, False), (17, 64, 9, 256, 2, False), (49, 16, 3, 128, 5, False),
+    (17, 48, 3, 96, 3, True), (33, 16, 5, 32, 4, True)])
+def test_one_launch_prologues(rt, abi, family, m, cols, blocks, kt, loop, extremes, order):
+    """The element-wise operators in front of the one-launch kernel: half units of k, more than one 16-row piece,
+    one and more 16-column pieces; infinities and NaN in the last rows and the last k of an iteration."""
+    import numpy as np
+    from attention_superoptimizer_amd import workloads as W
+    from helpers import assert_f16_close, normal_f16
+    from test_gpu_f16 import _graph_f16
+    from test_gpu_launch_records import _kernel as launched
+    k, n = kt * loop, cols * blocks
+    acts, rows, cols_map = [W._inp([m, k])], (-1, -1, -1), (1, -1, -1)
+    ops = [(f"tb_{family}_op", [(0, 0)]), ("tb_matmul_op", [(2, 0), (1, 0)])]
+    if family == "silu_mul":
+        acts.append(W._inp([m, k]))
+        ops = [("tb_silu_op", [(0, 0)]), ("tb_mul_op", [(3, 0), (1, 0)]), ("tb_matmul_op", [(4, 0), (2, 0)])]
+    na = len(acts)
+    spec = acts + [W._inp([k, n], order),
+                   {"op": "customized", "in": [[i, 0] for i in range(na + 1)],
+                    "plan": W._plan((blocks, 1, 1), loop, [rows] * na + [cols_map], (1,) * na + (0,), cols_map, ops)}]
+    # (one sign: no cancellation between iterations)
+    ins = {i: abs(normal_f16(spec[i]["dims"], 0.1, 5 + i)) for i in range(na + 1)}
+    if extremes:
+        x, w = ins[0], ins[na]
+        x[m - 1, kt - 1], x[m - 1, 0], x[16, -1], x[3, kt], x[0, 5] = np.inf, -np.inf, np.nan, 60000, -60000
+        w[kt - 1, 1], w[-1, -1], w[kt, 4] = np.inf, np.nan, 50000
+        if family == "silu_mul":
+            ins[1][m - 2, -1], ins[1][m - 3, kt - 1] = np.inf, np.nan
+    assert abi.mi355_set_option(7, 2) == 0
+    try:
+        got = _graph_f16(rt, spec, ins)[na + 1][0]
+        pieces = cols // 16 * ((m + 15) // 16)
+        assert launched() == (4, (blocks + 7) // 8 * 8 * pieces)  # the one-launch kernel's workgroups
+    finally:
+        assert abi.mi355_set_option(7, 0) == 0
+    if extremes:
+        assert abi.mi355_set_option(1, 1) == 0
+        try:
+            want = _graph_f16(rt, spec, ins)[na + 1][0]
+        finally:
+            assert abi.mi355_set_option(1, 0) == 0
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+        assert np.array_equal(np.isneginf(got), np.isneginf(want))
+        ok = np.isfinite(want)
+        assert ok.any() and not ok.all()
+        assert_f16_close(got[ok], want[ok], what=family)
+    else:
+        from oracle import evaluate as orc
+        assert_f16_close(got, orc.eval_graph(spec, "f16", ins, threads=8)[na + 1][0], what=family)
