@@ -292,7 +292,12 @@ __global__ __launch_bounds__(64 * RG * IP) void attn_fused_kernel(AttnParams con
   _Float16 *const o_stage = reinterpret_cast<_Float16 *>(tail);
   uint32_t *const slots = reinterpret_cast<uint32_t *>(tail + RG * 16 * LDO * 2);
 
+  // The loop's place in the 32-byte blocks that instructions are fetched in is worth up to 10 %, and would move with
+  // every instruction in front of it: its body starts 3 words into a block.  (Prefill of head size 128, column-major,
+  // us, by the words 0 - 7: 5 heads of 9 row blocks 55.0 49.6 51.0 49.6 50.1 50.2 55.7 54.8, 12 of 9 48.0 50.2 47.5 47.8
+  // 49.0 48.3 49.9 48.6, 25 of 9 93.4 - 94.8; row-major 12 of 9 68.0 69.5 69.2 68.6 67.8 68.3 67.0 68.3.)
   for (int it0 = 0; it0 < F; it0 += P.stages) {
+    asm volatile(".p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
     int const n_st = (F - it0) < P.stages ? (F - it0) : P.stages;
     if (it0 > 0) {
       __syncthreads();  // previous chunk fully consumed

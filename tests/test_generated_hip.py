@@ -137,3 +137,20 @@ def test_hipcc_compiles_the_program_for_gfx950(tmp_path):
         # backend library instantiates the same templates: each library binds its own
         dyn = subprocess.check_output(["readelf", "-d", str(tmp_path / "libc1.so")]).decode()
         assert "SYMBOLIC" in dyn
+
+
+def test_the_loop_of_the_fused_attention_kernel_starts_a_fetch_block(tmp_path):
+    """attn_fused_kernel's loop over key tiles: its time depends on its place in blocks of 32 bytes."""
+    if not os.path.exists(CG.HIPCC):
+        pytest.skip("no hipcc")
+    rows = 9 * 128
+    spec = [W._inp([5, rows, 128]), W._inp([5, 128, rows], "DmemColumnMajor"), W._inp([5, rows, 128], "DmemColumnMajor"),
+            {"op": "customized", "in": [[0, 0], [1, 0], [2, 0]],
+             "plan": W._plan((5, 1, 9), rows // 64, [(0, -1, 1), (0, 2, -1), (0, 1, -1)], (-1, 2, 1), (0, 2, 1), W.ATT_OPS, dimx=128)}]
+    text = _emit(spec, tmp_path / "prefill.hip")
+    assert "mi355::attn_fused_kernel<128, 64, 128, false, 1, 1, true><<<" in text
+    include = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(CG.__file__))), "include")
+    subprocess.check_call([CG.HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-I", include, "--cuda-device-only", "-S",
+                           str(tmp_path / "prefill.hip"), "-o", str(tmp_path / "prefill.s")])
+    body = open(tmp_path / "prefill.s").read()
+    assert re.search(r"Loop Header: Depth=1[\s\S]{0,600}\.p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n", body)
