@@ -288,6 +288,95 @@ int launch_kt(GemmParams const &A, dim3 grid, int lds) {
   return go(gemm_fused_kernel<MT, NB, PRO, LORA, 512, WCM>);
 }
 
+// How gemm_stream_kernel takes a plan (see include/mi355_kernels/gemm_stream.h).
+struct StreamPlan {
+  int ranges = 0;       // 0: not at all
+  bool strips = false;  // 16 columns a workgroup
+  bool pairs = false;   // both of two weights
+  int mt = 0;           // 16-row groups
+  int ring = 0, lds = 0, groups = 0;  // bytes of the slots, of LDS; workgroups of a block
+  size_t slab = 0;      // bytes between the two launches of more than one range
+};
+StreamPlan stream_plan(DevProgram const &P, GMatch const &G) {
+  State &s = state();
+  StreamPlan plan;
+  int const mt = G.M <= 16 ? 1 : (G.M <= 32 ? 2 : 4), F = P.forloop_range;
+  // (with more rows than half an iteration's k the product slots rival the weights: the kernel that
+  // keeps its sums in registers where a block is not split stays ahead there)
+  if (s.any_size_kernels || !G.whole || G.KT % 64 != 0 || 2 * G.M > G.KT) {
+    return plan;
+  }
+  long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
+  int const ring = 4 * kStreamRing * stream_slot_bytes(G.pro, G.lora, G.M <= 8 ? 0 : mt);
+  int const results = F * G.M * 128;  // of one weight
+  size_t const slab = (size_t)blocks * G.nb * results;
+  int const steps = (F + 3) / 4 * (G.KT / 64);  // of a wavefront that has a whole block of one weight
+  bool const fits = ring + results <= s.max_lds;
+  // Strips of 16 columns where they fill most of the chip and two workgroups fit on a compute unit (4 rows, us, strips
+  // / ranges: 3840 columns x 4096, 240 workgroups, 7.6 / 10.7; 28672 39.9 / 51.6; two weights of 3072 x 8192
+  // with a gated MLP's second product 37.9 / 40.1), but not where one weight's whole blocks fill it as well (below:
+  // 4 rows x 12416 x 1536 9.7 / 8.0, 16 x 14656 x 1792 13.6 / 11.4, but 16 x 7360 x 1280, 115 blocks, 6.1 / 6.8).
+  int const eights = G.M <= 8 ? 1 : 2, strip_ring = 4 * columns_ring(eights) * columns_slot_bytes(eights);
+  int const strip_lds = strip_ring + F * G.M * 32;
+  bool const strips = G.wcm && G.pro == PRO_NONE && !G.lora && G.M <= 16 && 4 * G.nb * blocks >= 192 && 2 * strip_lds <= s.max_lds &&
+                      !(G.nb == 1 && fits && blocks >= 192 && steps <= 8);
+  // One range per block where the blocks alone occupy the chip and a wavefront has a few steps to
+  // make: no slab and no second launch (4 x 8192 x 2048 in 64-k iterations: 8.9 us against 12).
+  // Otherwise four iterations, one per wavefront, to a range, as far as that many workgroups are
+  // resident at a time: a slot of 10 KB leaves room for two on a compute unit, which then also gain
+  // from taking turns; a larger one for one, where a second round would start late (32 x 3840 x 5120:
+  // 13.8 us in 240 workgroups, 16.0 in 300).
+  bool one = fits && blocks * G.nb >= 96 && steps <= 8;
+  // Blocks for more than half of the chip are not cut at all where the slab would be large beside the weights: with
+  // SiLU(a) * u (8 rows, us, one range / ranges: 14336 x 3712 in 64-k iterations 20.8 / 29.8, 8768 x 2944 14.5 / 16.8,
+  // but 114 blocks, 7296 x 4608, 20.4 either way, and 10240 x 4096 in 256-k ones, 16 steps, 24.2 / 21.7) ...
+  if (G.pro == PRO_SILU_MUL && G.M <= 8) {
+    one = one || (fits && blocks > 128 && blocks <= 256 && (steps <= 12 || blocks >= 192));
+  }
+  // ... and with two weights (8 rows, row-major: 4160 x 4096 in 256-k iterations 16.1 / 19.2, 6784 x 6144 30.1 / 35.0,
+  // 6400 x 4096 in 64-k ones 23.7 / 31.2, but 16 rows of these 41.5 / 36.8, and 4096 x 8192 39.1 / 34.1).
+  if (G.nb == 2 && 2 * blocks >= 128 && 2 * blocks <= 256) {
+    one = one || (fits && (steps <= 16 || (blocks >= 100 && steps <= 24)) && (G.M <= 8 || G.KT >= 128));
+  }
+  // Past that a compute unit has room for one workgroup of one weight: one of both then leaves less of the last
+  // round empty and reads the activations once (8 rows, row-major, us, both / one weight a workgroup: 10944 x 704 8.8 / 10.6,
+  // 8448 x 768 8.9 / 11.0, 14336 x 832 13.2 / 14.9, 14336 x 4096 50.4 / 53.8, 16 rows x 9216 x 2048 24.5 / 27.6; where two
+  // of one weight fit, 16384 x 512 9.1 / 8.7).
+  bool const pairs = !strips && G.nb == 2 && blocks > 128 && blocks <= 256 && 2 * (ring + results) > s.max_lds && ring + 2 * results <= s.max_lds;
+  one = one || pairs;
+  int ks = 1;
+  if (!one && slab <= (emit_sink() ? kEmitScratchBytes : s.scratch_bytes)) {
+    // (two weights have workgroups of their own: a wavefront of one takes two iterations of 64 k, so that one's loads
+    // run under the other's products; 8 rows x 4096 x 3904 20.4 -> 18.8 us, 2944 x 6464 22.1 -> 20.2)
+    // (eight rows of SiLU(a) * u leave room for two workgroups of long row-major iterations on a compute unit, but one
+    // has more of them in flight: 4096 x 6400 in 256-k iterations, 256 workgroups 17.2 us, 448 18.9, 2560 x 8192 15.4 and
+    // 17.4; column-major 4096 x 14336 29.4 and 28.6)
+    bool const single = ring > 80 * 1024 || (G.pro == PRO_SILU_MUL && G.KT == 256 && !G.wcm);
+    long long const most = (single ? 256 / G.nb : 1024) / blocks;
+    int const least = G.nb == 2 && G.KT == 64 ? 8 : 4;
+    ks = (int)std::max<long long>(1, std::min<long long>((F + least - 1) / least, most));
+    // (one round of long iterations rather than a part of a second: 8 rows x 2560 x 4096 in 256-k iterations 15.8 us in
+    // 320 workgroups, 13.3 in 240)
+    long long const wanted = blocks * G.nb * ks;
+    if (G.nb == 2 && G.KT == 256 && wanted > 256 && wanted < 512) {
+      ks = (int)std::max<long long>(1, 256 / (blocks * G.nb));
+    }
+  }
+  if (ks == 1 && !fits && !strips) {
+    return plan;
+  }
+  int const per = (F + ks - 1) / ks;
+  plan.strips = strips;
+  plan.pairs = pairs;
+  plan.mt = mt;
+  plan.ranges = strips ? 1 : (F + per - 1) / per;  // (no empty range)
+  plan.ring = strips ? strip_ring : ring;
+  plan.lds = strips ? strip_lds : ring + (plan.ranges == 1 ? results * (pairs ? 2 : 1) : 0);
+  plan.groups = (pairs ? 1 : G.nb) * (strips ? 4 : plan.ranges);
+  plan.slab = plan.ranges > 1 ? slab : 0;
+  return plan;
+}
+
 // gemm_lanes_kernel for this plan, or 0 when it is not the better choice (see the rule in
 // try_launch_lanes); k extents 32 / 64 / 96 / 128 / 256.
 template <int NB, int PRO, int LORA, bool WCM>
@@ -493,70 +582,45 @@ int launch_stream_one(StreamParams const &L, dim3 grid, int lds) {
   return 1;
 }
 
-// gemm_stream_kernel for this plan (see include/mi355_kernels/gemm_stream.h), or 0.
+template <bool WCM, int GROUPS>
+int launch_stream_pairs(StreamParams const &L, dim3 grid, int lds) {
+  if (EmitSink *sink = emit_sink()) {
+    sink->headers |= 32u;
+    emit_launch(*sink, "gemm_stream_pairs_kernel", emit_fmt("%s, %d", tf(WCM), GROUPS), grid, 256, lds, literal(L));
+    return 1;
+  }
+  auto *fn = gemm_stream_pairs_kernel<WCM, GROUPS>;
+  MI355_GRANT_LDS(fn, lds);
+  MI355_HIP(launch_kernel(fn, grid, 256, lds, state().stream(), L));
+  return 1;
+}
+
+// gemm_stream_kernel for this plan, or 0.
 int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A) {
   State &s = state();
-  int const mt = G.M <= 16 ? 1 : (G.M <= 32 ? 2 : 4), F = P.forloop_range;
-  // (with more rows than half an iteration's k the product slots rival the weights: the kernel that
-  // keeps its sums in registers where a block is not split stays ahead there)
-  if (s.any_size_kernels || !G.whole || G.KT % 64 != 0 || 2 * G.M > G.KT) {
+  StreamPlan const plan = stream_plan(P, G);
+  if (plan.ranges == 0 || (long long)P.grid[0] * plan.groups > 2147483647LL) {
     return 0;
   }
-  long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
-  int const ring = 4 * kStreamRing * stream_slot_bytes(G.pro, G.lora, G.M <= 8 ? 0 : mt);
-  int const results = F * G.M * 128;  // of one weight
-  size_t const slab = (size_t)blocks * G.nb * results;
-  // Strips of 16 columns where they fill most of the chip and two workgroups fit on a compute unit (4 rows, us, strips
-  // / ranges: 3840 columns x 4096, 240 workgroups, 7.6 / 10.7; 28672 39.9 / 51.6; two weights of 3072 x 8192
-  // with a gated MLP's second product 37.9 / 40.1).
-  int const eights = G.M <= 8 ? 1 : 2, strip_ring = 4 * columns_ring(eights) * columns_slot_bytes(eights);
-  int const strip_lds = strip_ring + F * G.M * 32;
-  bool const strips = G.wcm && G.pro == PRO_NONE && !G.lora && G.M <= 16 && 4 * G.nb * blocks >= 192 && 2 * strip_lds <= s.max_lds;
-  // One range per block where the blocks alone occupy the chip and a wavefront has a few steps to
-  // make: no slab and no second launch (4 x 8192 x 2048 in 64-k iterations: 8.9 us against 12).
-  // Otherwise four iterations, one per wavefront, to a range, as far as that many workgroups are
-  // resident at a time: a slot of 10 KB leaves room for two on a compute unit, which then also gain
-  // from taking turns; a larger one for one, where a second round would start late (32 x 3840 x 5120:
-  // 13.8 us in 240 workgroups, 16.0 in 300).
-  int const steps = (F + 3) / 4 * (G.KT / 64);
-  bool const fits = ring + results <= s.max_lds;
-  int ks = 1;
+  int const ks = plan.ranges, lds = plan.lds, mt = plan.mt;
   EmitSink *const sink = emit_sink();
-  if (!(fits && blocks * G.nb >= 96 && steps <= 8) && slab <= (sink ? kEmitScratchBytes : s.scratch_bytes)) {
-    // (two weights have workgroups of their own: a wavefront of one takes two iterations of 64 k, so that one's loads
-    // run under the other's products; 8 rows x 4096 x 3904 20.4 -> 18.8 us, 2944 x 6464 22.1 -> 20.2)
-    long long const most = (ring <= 80 * 1024 ? 1024 : 256 / G.nb) / blocks;
-    int const least = G.nb == 2 && G.KT == 64 ? 8 : 4;
-    ks = (int)std::max<long long>(1, std::min<long long>((F + least - 1) / least, most));
-  }
-  if (ks == 1 && !fits && !strips) {
-    return 0;
-  }
-  int const per = (F + ks - 1) / ks;
-  ks = (F + per - 1) / per;  // (no empty range)
   StreamParams L{};
   L.g = A;
   L.g.ksplit = ks;
-  L.g.scratch = static_cast<_Float16 *>(s.scratch());
-  if (sink) {  // a printed program allocates the workspace itself
-    L.g.scratch = ks > 1 ? reinterpret_cast<_Float16 *>(kEmitScratch) : nullptr;
+  L.g.scratch = ks > 1 ? static_cast<_Float16 *>(s.scratch()) : nullptr;
+  if (sink && ks > 1) {  // a printed program allocates the workspace itself
+    L.g.scratch = reinterpret_cast<_Float16 *>(kEmitScratch);
   }
-  L.results = ring;
-  int lds = ring + (ks == 1 ? results : 0);
-  L.strips = strips;
-  if (strips) {
-    ks = L.g.ksplit = 1;
-    L.g.scratch = nullptr;
-    L.results = strip_ring;
-    lds = strip_lds;
-  }
-  if ((long long)P.grid[0] * G.nb * (strips ? 4 : ks) > 2147483647LL) {
-    return 0;
-  }
-  dim3 const grid(P.grid[0] * G.nb * (strips ? 4 : ks), P.grid[1], P.grid[2]);
+  L.results = plan.ring;
+  L.strips = plan.strips;
+  dim3 const grid(P.grid[0] * plan.groups, P.grid[1], P.grid[2]);
   int rc = 0;
+  if (plan.pairs) {
+    rc = G.M <= 8 ? (G.wcm ? launch_stream_pairs<true, 0>(L, grid, lds) : launch_stream_pairs<false, 0>(L, grid, lds))
+                  : (G.wcm ? launch_stream_pairs<true, 1>(L, grid, lds) : launch_stream_pairs<false, 1>(L, grid, lds));
+  }
 #define MI355_STREAM_CASE(NBV, PROV, LORAV, MTV)                                            \
-  if (G.nb == NBV && G.pro == PROV && G.lora == LORAV && mt == MTV) {                       \
+  if (!plan.pairs && G.nb == NBV && G.pro == PROV && G.lora == LORAV && mt == MTV) {        \
     rc = G.wcm ? launch_stream_one<NBV, PROV, LORAV, true, MTV>(L, grid, lds)               \
                : launch_stream_one<NBV, PROV, LORAV, false, MTV>(L, grid, lds);             \
   }
@@ -571,7 +635,7 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A)
 #undef MI355_STREAM_CASE
   if (rc == 1 && ks > 1) {
     if (sink) {
-      sink->scratch_bytes = std::max(sink->scratch_bytes, slab);
+      sink->scratch_bytes = std::max(sink->scratch_bytes, plan.slab);
     }
     rc = launch_combine(L.g, G.nb, dim3(P.grid[0], P.grid[1], P.grid[2]));
   }

@@ -25,6 +25,8 @@
 // 8 x 4096 x 14336: 78.9 -> 77.1 us).
 #pragma once
 
+#include <type_traits>
+
 #include "gemm.h"
 
 namespace mi355 {
@@ -52,7 +54,9 @@ constexpr int stream_slot_bytes(int pro, bool lora, int mt) {
   return 8192 + (mt > 0 ? 2048 * mt : 1024) * (pro == PRO_SILU_MUL ? 2 : 1) + (lora ? 2048 : 0);
 }
 
-template <int NB, int PRO, bool LORA, bool WCM, int GROUPS>
+// TAKES: weights of a workgroup, 1 or both of two (the step of one, then the step of the other, on the same
+// activations).
+template <int NB, int PRO, bool LORA, bool WCM, int GROUPS, int TAKES = 1>
 __device__ __forceinline__ void stream_block(StreamParams const &S) {
   GemmParams const &P = S.g;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -65,10 +69,11 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
   int const M = P.M, F = P.forloop_range, subs = P.KT / 64;
   constexpr int R = kStreamRing;
 
-  int const gx = gridDim.x / (P.ksplit * NB);
+  constexpr int SETS = NB / TAKES;
+  int const gx = gridDim.x / (P.ksplit * SETS);
   int const ks = blockIdx.x % P.ksplit;  // (the ranges of a block next to each other)
-  int const block_weight = blockIdx.x / P.ksplit, b = NB == 2 ? block_weight % 2 : 0;
-  int const bx = block_weight / NB, by = blockIdx.y, bz = blockIdx.z;
+  int const block_weight = blockIdx.x / P.ksplit, b0 = SETS == 2 ? block_weight % 2 : 0;
+  int const bx = block_weight / SETS, by = blockIdx.y, bz = blockIdx.z;
   int const per = (F + P.ksplit - 1) / P.ksplit;
   int const it_begin = ks * per, n_it = (it_begin + per < F ? it_begin + per : F) - it_begin;
   int const block_linear = bx + gx * (by + gridDim.y * bz);
@@ -90,10 +95,14 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
   // the LDS tile (the chunk a lane FETCHES moves, its place is fixed).
   auto swizzle = [](int row) { return WCM ? (row >> 1) & 7 : (((row >> 1) & 1) | ((row >> 2) & 2)) << 1; };
   int const l8 = lane / 8, ch8 = lane % 8;
-  GTile const &bt = NB == 2 && b == 1 ? P.b1 : P.b0;
   // rows 8 j + l8: the swizzle of rows 8 apart differs, so even and odd j
-  uint32_t const w_off[2] = {2u * (uint32_t)(l8 * bt.d_cols + 8 * (ch8 ^ swizzle(l8))),
-                             2u * (uint32_t)(l8 * bt.d_cols + 8 * (ch8 ^ swizzle(8 + l8)))};
+  uint32_t w_off[TAKES][2];
+#pragma unroll
+  for (int q = 0; q < TAKES; q++) {
+    int const ld = NB == 2 && b0 + q == 1 ? P.b1.d_cols : P.b0.d_cols;
+    w_off[q][0] = 2u * (uint32_t)(l8 * ld + 8 * (ch8 ^ swizzle(l8)));
+    w_off[q][1] = 2u * (uint32_t)(l8 * ld + 8 * (ch8 ^ swizzle(8 + l8)));
+  }
   // activation rows 8 j + l / 8 (rows past the tile re-read its last one: theirs are not stored)
   uint32_t x_off[EIGHTS], u_off[PRO == PRO_SILU_MUL ? EIGHTS : 1];
 #pragma unroll
@@ -106,13 +115,17 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
     }
   }
   // lora A: column-major like the weights (16 columns), row-major k rows 32 j + l / 2 of 32 bytes
-  auto issue = [&](int it, int sub, int slot) {
+  auto issue = [&](int it, int sub, int q, int slot) {
     uint32_t const at = mine_at + (uint32_t)(slot * SLOT);
+    GTile const &bt = NB == 2 && b0 + q == 1 ? P.b1 : P.b0;
     _Float16 const *w = static_cast<_Float16 const *>(bt.ptr) + gtile_offset(bt, bx, by, bz, it) +
                         (WCM ? (long long)(64 * sub) : (long long)(64 * sub) * bt.d_cols);
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-      lane_dma16(w + (long long)(8 * j) * bt.d_cols, w_off[j & 1], at + (uint32_t)(1024 * j));
+      lane_dma16(w + (long long)(8 * j) * bt.d_cols, w_off[q][j & 1], at + (uint32_t)(1024 * j));
+    }
+    if (q > 0) {
+      return;
     }
     _Float16 const *x = static_cast<_Float16 const *>(P.a0.ptr) + gtile_offset(P.a0, bx, by, bz, it) + 64 * sub;
 #pragma unroll
@@ -177,12 +190,22 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
   }
 
   // ---- the loop: step = 64 k ----------------------------------------------------------------------
-  int const total = n_mine > 0 ? n_mine * subs : 0;
-  int i_it = 0, i_sub = 0, i_slot = 0, issued = 0;  // the next step to issue
+  int const total = n_mine > 0 ? n_mine * subs * TAKES : 0;
+  int i_it = 0, i_sub = 0, i_q = 0, i_slot = 0, issued = 0;  // the next step to issue
   auto issue_next = [&]() {
-    issue(nth(i_it), i_sub, i_slot);
+    if (TAKES == 1 || i_q == 0) {
+      issue(nth(i_it), i_sub, 0, i_slot);
+    } else {
+      issue(nth(i_it), i_sub, TAKES - 1, i_slot);
+    }
     issued++;
     i_slot = i_slot + 1 == R ? 0 : i_slot + 1;
+    if (TAKES == 2) {
+      i_q ^= 1;
+      if (i_q == 1) {
+        return;
+      }
+    }
     i_sub++;
     if (i_sub == subs) {
       i_sub = 0;
@@ -194,23 +217,25 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
   }
   int slot = 0, step = 0;
   for (int i = 0; i < n_mine; i++) {
-    float4v o[4][MT], d = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4v o[TAKES][4][MT], d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
+    for (int t = 0; t < 4 * TAKES; t++) {
 #pragma unroll
       for (int mt = 0; mt < MT; mt++) {
-        o[t][mt] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        o[t / 4][t % 4][mt] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
       }
     }
-    for (int sub = 0; sub < subs; sub++, step++) {
+    half8 x[MT][2];
+    auto work = [&](auto which) {
+      constexpr int q = decltype(which)::value;
       // this step has landed when only the loads of the one after it are outstanding
       if (issued - 1 > step) {
-        stream_wait<8 + X_LOADS>();
+        stream_wait<q + 1 < TAKES ? 8 : 8 + X_LOADS>();
       } else {
         stream_wait<0>();
       }
       unsigned char const *const at = mine + slot * SLOT;
-      half8 w[4][2], la[2], x[MT][2], u[PRO == PRO_SILU_MUL ? MT : 1][2];
+      half8 w[4][2], la[2], u[PRO == PRO_SILU_MUL ? MT : 1][2];
 #pragma unroll
       for (int s = 0; s < 2; s++) {
 #pragma unroll
@@ -220,6 +245,9 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
       }
 #pragma unroll
       for (int s = 0; s < 2; s++) {
+        if (q > 0) {
+          continue;
+        }
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
           x[mt][s] = rows(at + X_AT, mt, s);
@@ -288,9 +316,16 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
         for (int t = 0; t < 4; t++) {
 #pragma unroll
           for (int mt = 0; mt < MT; mt++) {
-            o[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[t][s], x[mt][s], o[t][mt], 0, 0, 0);
+            o[q][t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[t][s], x[mt][s], o[q][t][mt], 0, 0, 0);
           }
         }
+      }
+      step++;
+    };
+    for (int sub = 0; sub < subs; sub++) {
+      work(std::integral_constant<int, 0>{});
+      if constexpr (TAKES == 2) {
+        work(std::integral_constant<int, 1>{});
       }
     }
     int const it = nth(i);
@@ -303,19 +338,22 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
       }
 #pragma unroll
       for (int t = 0; t < 4; t++) {
-        o[t][0] = __builtin_amdgcn_mfma_f32_16x16x16f16(lb_frag[t], df, o[t][0], 0, 0, 0);
+        o[0][t][0] = __builtin_amdgcn_mfma_f32_16x16x16f16(lb_frag[t], df, o[0][t][0], 0, 0, 0);
       }
     }
     // ---- this iteration's product, fp16 ----------------------------------------------------------
     long long const tile = (long long)M * 64;
-    _Float16 *const to = P.ksplit > 1 ? P.scratch + (((long long)block_linear * F + it) * NB + b) * tile
-                                      : reinterpret_cast<_Float16 *>(lds + S.results) + it * (int)tile;
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-      if (16 * mt + c < M) {
+    for (int q = 0; q < TAKES; q++) {
+      _Float16 *const to = P.ksplit > 1 ? P.scratch + (((long long)block_linear * F + it) * NB + b0 + q) * tile
+                                        : reinterpret_cast<_Float16 *>(lds + S.results) + (q * F + it) * (int)tile;
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-          *reinterpret_cast<half4 *>(to + (16 * mt + c) * 64 + 16 * t + 4 * g) = __builtin_convertvector(o[t][mt], half4);
+      for (int mt = 0; mt < MT; mt++) {
+        if (16 * mt + c < M) {
+#pragma unroll
+          for (int t = 0; t < 4; t++) {
+            *reinterpret_cast<half4 *>(to + (16 * mt + c) * 64 + 16 * t + 4 * g) = __builtin_convertvector(o[q][t][mt], half4);
+          }
         }
       }
     }
@@ -326,18 +364,17 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
   // ---- the saver: the iterations' products in order ----------------------------------------------
   __syncthreads();
   typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-  _Float16 const *const all = reinterpret_cast<_Float16 const *>(lds + S.results);
-  GTile const &ot = NB == 2 && b == 1 ? P.o1 : P.o0;
-  _Float16 *const og = static_cast<_Float16 *>(const_cast<void *>(ot.ptr)) + gtile_offset(ot, bx, by, bz, 0);
-  for (int e = tid; e < M * 16; e += 256) {
-    int const row = e / 16, col = 4 * (e % 16);
-    _Float16 const *src = all + row * 64 + col;
+  for (int e = tid; e < TAKES * M * 16; e += 256) {
+    int const q = TAKES == 1 || e < M * 16 ? 0 : 1, of = e - q * M * 16, row = of / 16, col = 4 * (of % 16);
+    _Float16 const *src = reinterpret_cast<_Float16 const *>(lds + S.results) + q * F * M * 64 + row * 64 + col;
     half2v lo = {(_Float16)0.0f, (_Float16)0.0f}, hi = lo;
     for (int it = 0; it < F; it++) {  // (a packed fp16 add is the exact sum rounded once)
       half4 const v = *reinterpret_cast<half4 const *>(src + it * M * 64);
       lo += half2v{v[0], v[1]};
       hi += half2v{v[2], v[3]};
     }
+    GTile const &ot = NB == 2 && b0 + q == 1 ? P.o1 : P.o0;
+    _Float16 *const og = static_cast<_Float16 *>(const_cast<void *>(ot.ptr)) + gtile_offset(ot, bx, by, bz, 0);
     *reinterpret_cast<half4 *>(og + (long long)row * ot.d_cols + col) = half4{lo[0], lo[1], hi[0], hi[1]};
   }
 }
@@ -472,6 +509,14 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) 
   } else {
     stream_block<NB, PRO, LORA, WCM, MT>(S);
   }
+}
+
+// Both of two weights in a workgroup (a kernel of its own: with the forms above in one, its addresses do not fit the
+// scalar registers).
+template <bool WCM, int GROUPS>
+__global__ __launch_bounds__(256) void gemm_stream_pairs_kernel(StreamParams const S) {
+  fetch_kernel_arguments<sizeof(StreamParams), 2>();
+  stream_block<2, PRO_NONE, false, WCM, GROUPS, 2>(S);
 }
 
 }  // namespace mi355

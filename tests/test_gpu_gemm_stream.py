@@ -204,3 +204,38 @@ def test_one_launch_prologues(rt, abi, family, m, cols, blocks, kt, loop, extrem
     else:
         from oracle import evaluate as orc
         assert_f16_close(got, orc.eval_graph(spec, "f16", ins, threads=8)[na + 1][0], what=family)
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("m,blocks,kt,loop,col_groups,row_groups", [
+    (8, 129, 64, 11, 8, 1), (16, 256, 64, 4, 8, 1), (9, 150, 128, 5, 8, 1),  # both weights in a workgroup, row-major
+    (8, 130, 64, 40, 1, 1),   # and where strips leave no room for two workgroups on a compute unit
+    (16, 129, 64, 33, 10, 10),  # results of both do not fit, one's do not either: ranges
+    (8, 129, 64, 8, 8, 2), (8, 128, 64, 11, 8, 2), (16, 257, 64, 4, 8, 2),  # one weight in a workgroup
+    (8, 64, 256, 16, 8, 2), (8, 40, 256, 16, 8, 6), (8, 64, 256, 32, 8, 16)])  # whole for-loops, ranges in one round, in several
+def test_two_weights_in_a_workgroup(rt, ranges, m, blocks, kt, loop, col_groups, row_groups, order):
+    """Which of its forms the streaming kernel takes for two weights (workgroups to a block), and their sums."""
+    from attention_superoptimizer_amd import workloads as W
+    from test_gpu_launch_records import _kernel as launched
+    spec, _ = W.config5_gated_mlp(m=m, d=kt * loop, h=64 * blocks, grid1=blocks, F1=loop, grid2=kt * loop // 64, F2=blocks)
+    spec = [op for i, op in enumerate(spec[:5]) if i != 3]
+    _run(rt, spec, order, f"two weights {m} x {blocks}, {kt} x {loop}", std=0.05)
+    assert launched()[1] == blocks * (col_groups if order == COL else row_groups)
+
+
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("m,blocks,kt,loop,col_groups,row_groups", [
+    (8, 129, 64, 45, 1, 1), (5, 200, 256, 16, 1, 1), (8, 129, 256, 16, 4, 1), (9, 129, 64, 13, 1, 1), (8, 128, 64, 33, 7, 7),
+    (8, 40, 256, 32, 8, 6)])  # (row-major 256-k iterations: one round of workgroups)
+def test_a_second_product_in_one_range(rt, ranges, m, blocks, kt, loop, col_groups, row_groups, order):
+    """SiLU(a) * u in one range where its blocks are more than half of the compute units, up to 12 steps a
+    wavefront (more of them from 192 blocks on)."""
+    from attention_superoptimizer_amd import workloads as W
+    from test_gpu_launch_records import _kernel as launched
+    k, n, rows = kt * loop, 64 * blocks, (-1, -1, -1)
+    spec = [W._inp([m, k]), W._inp([k, n], COL),
+            {"op": "customized", "in": [[0, 0], [0, 0], [1, 0]],
+             "plan": W._plan((blocks, 1, 1), loop, [rows, rows, (1, -1, -1)], (1, 1, 0), (1, -1, -1),
+                             [("tb_silu_op", [(0, 0)]), ("tb_mul_op", [(3, 0), (1, 0)]), ("tb_matmul_op", [(4, 0), (2, 0)])])}]
+    _run(rt, spec, order, f"second product {m} x {blocks}, {kt} x {loop}", std=0.1)
+    assert launched()[1] == blocks * (col_groups if order == COL else row_groups)
