@@ -339,13 +339,23 @@ StreamPlan stream_plan(DevProgram const &P, GMatch const &G) {
     one = one || (fits && (steps <= 16 || (blocks >= 100 && steps <= 24)) && (G.M <= 8 || G.KT >= 128));
   }
   // Past that a compute unit has room for one workgroup of one weight: one of both then leaves less of the last
-  // round empty and reads the activations once (8 rows, row-major, us, both / one weight a workgroup: 10944 x 704 8.8 / 10.6,
-  // 8448 x 768 8.9 / 11.0, 14336 x 832 13.2 / 14.9, 14336 x 4096 50.4 / 53.8, 16 rows x 9216 x 2048 24.5 / 27.6; where two
-  // of one weight fit, 16384 x 512 9.1 / 8.7).
-  bool const pairs = !strips && G.nb == 2 && blocks > 128 && blocks <= 256 && 2 * (ring + results) > s.max_lds && ring + 2 * results <= s.max_lds;
+  // round empty and reads the activations once (8 rows, row-major, us, both / one weight a workgroup: 10944 x 704 8.1 / 10.6,
+  // 8448 x 768 8.0 / 11.0, 14336 x 832 12.2 / 14.9, 14336 x 4096 49.5 / 53.8, 16 rows x 9216 x 2048 23.9 / 27.6; where two
+  // of one weight fit, 16384 x 512 9.1 / 8.2).
+  bool pairs = !strips && G.nb == 2 && blocks > 128 && blocks <= 256 && 2 * (ring + results) > s.max_lds && ring + 2 * results <= s.max_lds;
   one = one || pairs;
+  // Row-major, also where their ranges are a workgroup for every compute unit: the two weights are read in turn, not
+  // side by side at the same offsets of a power-of-two stride (8 rows, us, both / one weight: 2048 x 8192 in 256-k iterations
+  // 20.5 / 23.9, in 64-k ones 27.0 / 28.5, 4096 x 4096 in 256-k ones 19.1 / 21.4, but in 64-k ones 24.7 / 22.7).
+  int const filling = (int)(256 / blocks);
+  bool const even = G.nb == 2 && !G.wcm && blocks >= 32 && blocks <= 64 && filling * blocks == 256 && (blocks < 64 || G.KT == 256) &&
+                    (F + 3) / 4 >= filling;
+  bool const slab_fits = slab <= (emit_sink() ? kEmitScratchBytes : s.scratch_bytes);
   int ks = 1;
-  if (!one && slab <= (emit_sink() ? kEmitScratchBytes : s.scratch_bytes)) {
+  if (even && slab_fits) {
+    pairs = true;
+    ks = filling;
+  } else if (!one && slab_fits) {
     // (two weights have workgroups of their own: a wavefront of one takes two iterations of 64 k, so that one's loads
     // run under the other's products; 8 rows x 4096 x 3904 20.4 -> 18.8 us, 2944 x 6464 22.1 -> 20.2)
     // (eight rows of SiLU(a) * u leave room for two workgroups of long row-major iterations on a compute unit, but one

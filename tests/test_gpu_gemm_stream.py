@@ -212,7 +212,8 @@ def test_one_launch_prologues(rt, abi, family, m, cols, blocks, kt, loop, extrem
     (8, 130, 64, 40, 1, 1),   # and where strips leave no room for two workgroups on a compute unit
     (16, 129, 64, 33, 10, 10),  # results of both do not fit, one's do not either: ranges
     (8, 129, 64, 8, 8, 2), (8, 128, 64, 11, 8, 2), (16, 257, 64, 4, 8, 2),  # one weight in a workgroup
-    (8, 64, 256, 16, 8, 2), (8, 40, 256, 16, 8, 6), (8, 64, 256, 32, 8, 16)])  # whole for-loops, ranges in one round, in several
+    (8, 65, 256, 16, 8, 2), (8, 40, 256, 16, 8, 6), (8, 63, 256, 32, 8, 16),  # whole for-loops, ranges in one round, in several
+    (8, 64, 256, 16, 8, 4), (16, 32, 64, 31, 8, 8), (9, 32, 128, 28, 8, 14)])  # both weights, a range for every compute unit
 def test_two_weights_in_a_workgroup(rt, ranges, m, blocks, kt, loop, col_groups, row_groups, order):
     """Which of its forms the streaming kernel takes for two weights (workgroups to a block), and their sums."""
     from attention_superoptimizer_amd import workloads as W
