@@ -419,6 +419,42 @@ int launch_lanes_kt(LaneParams const &L, int grid, int threads, int lds) {
   }
 }
 
+// What the chain of a wavefront's iterations takes in the one-launch kernel, and what the streaming one takes, in ns:
+// fitted to the column-major ones of 2160 plans of 2 - 256 blocks, k 256 - 24000 and every prologue, on weights that change
+// from pass to pass (rms 14 and 12 %; the chain stands 18 % above its fit, where the choice lost least).  A piece's
+// wavefronts walk the whole of k, so its time grows with k however few pieces there are, and past a few hundred iterations
+// their results leave LDS for one or two wavefronts (us, here / there: silu of 16 rows x 256 x 19264 in 64-k iterations
+// 139 / 24, of 8 x 320 x 20736 in 256-k ones 34.5 / 11.2, 4 rows x 256 x 18176 14.0 / 10.0, two weights of 4 x 1984 x 9536
+// 113 / 28, a LoRA of 4 x 448 x 15232 40 / 13; row-major two weights of 4 x 192 x 8832 42 / 13, silu of 8 x 320 x 7424
+// 19.0 / 9.1).  Row-major chains are longer still, so there the estimate only finds the clear cases.
+double lanes_chain_ns(GMatch const &G, long long units, int F, int ip, int lds, long long pieces) {
+  State &s = state();
+  // ns for 64 k, and for sixteen wavefronts on the compute unit instead of none
+  double const alone = G.nb == 2 ? 230 : G.lora ? 270 : G.pro == PRO_EXP ? 300 : G.pro == PRO_SILU ? 620 : G.pro == PRO_SILU_MUL ? 720 : 250;
+  double const more = G.nb == 2 ? 920 : G.lora ? 1030 : G.pro == PRO_EXP ? 740 : G.pro == PRO_SILU ? 1210 : G.pro == PRO_SILU_MUL ? 1390 : 560;
+  long long const resident = std::max<long long>(1, std::min<long long>(s.max_lds / lds, 16 / ip)), each = (pieces + 255) / 256;
+  int const turns = (F + ip - 1) / ip;
+  double waves = (double)ip * std::min(resident, each);
+  if (turns > 1) {  // (few wavefronts wait for memory instead of each other)
+    waves = std::max(waves, G.wcm && G.pro == PRO_NONE && G.nb == 1 && !G.lora ? 10.0 : 8.0);
+  }
+  double const chain = (double)turns * (double)units / F;
+  return 2000 + (double)((each + resident - 1) / resident) * (chain * (alone + more * waves / 16) + 550);
+}
+double stream_ns(DevProgram const &P, GMatch const &G, StreamPlan const &plan, long long weight_bytes) {
+  State &s = state();
+  int const F = P.forloop_range;
+  long long const groups = (long long)P.grid[0] * P.grid[1] * P.grid[2] * plan.groups, resident = std::max(1, s.max_lds / plan.lds);
+  int const per = (F + plan.ranges - 1) / plan.ranges;
+  double const steps = (double)((per + 3) / 4) * (G.KT / 64) * (plan.pairs ? 2 : 1) / (plan.strips ? 4 : 1);
+  double const step = 270 + (G.pro == PRO_SILU || G.pro == PRO_SILU_MUL ? (G.M > 8 ? 270 : 120) : 0);
+  double ns = 3700 + (double)weight_bytes / (plan.strips ? 6150 : 8400) + (double)((groups + 256 * resident - 1) / (256 * resident)) * steps * step;
+  if (plan.ranges > 1) {
+    ns += 3000 + (double)plan.slab * 0.45e-3 + F * (21 + 12 * G.M / 16.0);
+  }
+  return ns;
+}
+
 int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) {
   State &s = state();
   // lora A comes in 16-rank pieces, the last one half full where its columns are rows in memory; two weights in
@@ -435,6 +471,29 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // (the kernel decodes the flat id with multiply-high magics: exact while id x divisor < 2^32)
   long long const widest = std::max<long long>(8 * S, std::max(P.grid[0], P.grid[1]));
   if (groups * 8 * S * widest >= (1LL << 32)) {
+    return 0;
+  }
+  bool const three = G.lora || G.pro == PRO_SILU_MUL;
+  int const wave_bytes = lanes_wave_bytes(G.KT, G.nb, lora, G.wcm, G.pro);
+  int const slot_bytes = F * G.nb * 512;
+  // Workgroups of 16 wavefronts while about one round of them covers the grid; half that where two share a compute
+  // unit and one's loads can run under the other's products (64 rows x 6400 x 4096 in 256-k iterations: 25.5 -> 19.7
+  // us; 16 rows x 1280, 80 workgroups: 5.2 against 5.7 the other way).  Two weights leave LDS for one workgroup of 13
+  // and more: half as many there too, evened out over the rounds (8 rows, column-major: 832 x 14336 14.0 -> 10.6 us,
+  // 1024 x 12224 12.1 -> 10.0, 4096 x 3904 in one round 12.3 either way; row-major 832 x 6464 8.8 -> 7.4).  The
+  // registers of 16 wavefronts with SiLU(a) * u or a LoRA tile fill the unit either way (13.1 us there, 15.0 here).
+  int const waves = G.nb == 2 || (!three && (long long)blocks * S * G.KT > 98304) ? 8 : 16;
+  int const most = std::min(waves, lanes_most(G.KT, lora));
+  int ip = F < most ? F : most;
+  if (G.nb == 2) {
+    int const rounds = (F + ip - 1) / ip;
+    ip = (F + rounds - 1) / rounds;
+  }
+  while (ip > 1 && ip * wave_bytes + slot_bytes > s.max_lds) {
+    ip = (ip + 1) / 2;
+  }
+  int const lds = ip * wave_bytes + slot_bytes;
+  if (lds > s.max_lds) {
     return 0;
   }
   // One launch, whose pieces of 16 columns each read the activation rows, against whole lines moved once by the
@@ -455,7 +514,6 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // 1536 x 3904 7.0 / 8.0, but 256 workgroups 10.8 / 9.8, 404 13.6 / 10.8, and 128-k iterations 8.9 / 7.1;
   // with both products of a gated MLP 160 workgroups, 4096 x 2560, 28.4 / 25.0, 176 24.0 / 24.9, 200 25.9 either way).
   long long const weight_bytes = blocks * F * (long long)(G.nb * G.KT * G.NC + (G.lora ? G.KT * G.rank : 0)) * 2;
-  bool const three = G.lora || G.pro == PRO_SILU_MUL;
   long long most_mb = 256;
   if (!G.wcm) {
     most_mb = G.KT == 256 || blocks * S < 128 ? 8 : (G.nb == 2 && G.KT == 64 && blocks * S >= 192 && blocks * S < 256 ? 68 : 17);
@@ -474,8 +532,11 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   // Of 28 such pairs of either order the choice is the faster one or within 1.1 us, but for row-major 2944 of 4032,
   // 23.8 / 24.9 and, 16 rows, 23.8 / 26.4).
   long long const units = (long long)F * G.KT / 64;
-  long long const here_ns = (1000 + (G.wcm ? 142 : 225) * units) * ((blocks * S + 255) / 256);
-  long long const there_ns = 7000 + blocks * units + blocks * F * 7 / 10 + 15 * F;
+  // (In 256-k iterations a piece's loads are waited for together: 8 x 4096 x 4096 column-major 12.0 / 11.4.  One range
+  // of the other kernel has neither the slab nor its launch: 8 rows x 10112 x 768 9.3 / 5.8, 14336 x 832 12.7 / 6.2.)
+  StreamPlan const plan = G.whole && G.KT % 64 == 0 ? stream_plan(P, G) : StreamPlan{};
+  long long const here_ns = (1000 + (!G.wcm ? 225 : G.KT == 256 ? 185 : 142) * units) * ((blocks * S + 255) / 256);
+  long long const there_ns = plan.ranges == 1 ? 4000 + blocks * units : 7000 + blocks * units + blocks * F * 7 / 10 + 15 * F;
   // Other tiles run on the any-size kernel or, in 96-k iterations of 64 columns, on the one with a barrier a step:
   // both are behind but for larger row-major plans (us, here / there: 64 rows x 3008 x 5120 in blocks of 32 columns
   // 13.6 / 30.7, a LoRA of rank 32 of 16 x 2304 x 3584 10.1 / 17.2, 64 x 1280 x 768 in 96-k iterations 4.0 / 8.9;
@@ -488,6 +549,15 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
     if (G.pro == PRO_SILU_MUL && G.M <= 16) {
       there = units > 104 || here_ns > there_ns;
     }
+    if (plan.ranges > 0 && (G.pro != PRO_SILU_MUL || (G.wcm && plan.ranges == 1 && blocks * S > 256))) {
+      there = there || lanes_chain_ns(G, units, F, ip, lds, blocks * S) > stream_ns(P, G, plan, weight_bytes);
+    }
+    // Row-major, the other kernel's whole blocks on more than half of the chip, and a prologue that is not done again
+    // for every 16 columns (us, here / there: silu of 4 rows x 12416 x 640 7.6 / 6.5, lora 8576 x 768 7.5 / 6.4,
+    // two weights of 8 x 13824 x 256 6.7 / 5.8).
+    if (!G.wcm && plan.ranges == 1 && blocks >= 128 && (G.pro != PRO_NONE || G.lora || G.nb == 2)) {
+      there = true;
+    }
   } else if (G.wcm) {
     there = false;
   } else if (G.whole) {
@@ -496,27 +566,6 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
     there = G.M > 32 && (G.KT == 96 || G.KT == 256) && weight_bytes > (8LL << 20);
   }
   if (s.gemm_mode == 0 && there) {
-    return 0;
-  }
-  int const wave_bytes = lanes_wave_bytes(G.KT, G.nb, lora, G.wcm, G.pro);
-  int const slot_bytes = F * G.nb * 512;
-  // Workgroups of 16 wavefronts while about one round of them covers the grid; half that where two share a compute
-  // unit and one's loads can run under the other's products (64 rows x 6400 x 4096 in 256-k iterations: 25.5 -> 19.7
-  // us; 16 rows x 1280, 80 workgroups: 5.2 against 5.7 the other way).  Two weights leave LDS for one workgroup of 13
-  // and more: half as many there too, evened out over the rounds (8 rows, column-major: 832 x 14336 14.0 -> 10.6 us,
-  // 1024 x 12224 12.1 -> 10.0, 4096 x 3904 in one round 12.3 either way; row-major 832 x 6464 8.8 -> 7.4).  The
-  // registers of 16 wavefronts with SiLU(a) * u or a LoRA tile fill the unit either way (13.1 us there, 15.0 here).
-  int const waves = G.nb == 2 || (!three && (long long)blocks * S * G.KT > 98304) ? 8 : 16;
-  int const most = std::min(waves, lanes_most(G.KT, lora));
-  int ip = F < most ? F : most;
-  if (G.nb == 2) {
-    int const rounds = (F + ip - 1) / ip;
-    ip = (F + rounds - 1) / rounds;
-  }
-  while (ip > 1 && ip * wave_bytes + slot_bytes > s.max_lds) {
-    ip = (ip + 1) / 2;
-  }
-  if (ip * wave_bytes + slot_bytes > s.max_lds) {
     return 0;
   }
   LaneParams L{};
@@ -533,7 +582,7 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   L.m_columns = fast_div_magic(pieces);
   L.m_gx = fast_div_magic(P.grid[0]);
   L.m_gy = fast_div_magic(P.grid[1]);
-  int const lds = ip * wave_bytes + slot_bytes, grid = (int)(groups * 8 * S);
+  int const grid = (int)(groups * 8 * S);
   int rc = 0;
 #define MI355_LANES_CASE(NBV, PROV, LORAV)                                  \
   if (G.nb == NBV && G.pro == PROV && lora == LORAV) {                      \

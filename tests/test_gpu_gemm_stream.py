@@ -240,3 +240,28 @@ def test_a_second_product_in_one_range(rt, ranges, m, blocks, kt, loop, col_grou
                              [("tb_silu_op", [(0, 0)]), ("tb_mul_op", [(3, 0), (1, 0)]), ("tb_matmul_op", [(4, 0), (2, 0)])])}]
     _run(rt, spec, order, f"second product {m} x {blocks}, {kt} x {loop}", std=0.1)
     assert launched()[1] == blocks * (col_groups if order == COL else row_groups)
+
+
+@pytest.mark.parametrize("family,m,blocks,kt,loop,order,groups", [
+    ("silu", 8, 5, 256, 40, COL, 50), ("lora", 4, 7, 64, 238, COL, 238), ("two", 4, 31, 64, 149, COL, 1178),
+    ("plain", 4, 2, 256, 90, ROW, 46), ("plain", 4, 4, 256, 70, COL, 72),  # k for hundreds of iterations: ranges
+    ("silu", 8, 5, 64, 8, COL, 32), ("lora", 4, 7, 64, 16, COL, 32), ("two", 4, 31, 64, 20, COL, 128),
+    ("plain", 4, 2, 256, 12, ROW, 32), ("plain", 4, 4, 256, 16, COL, 32)])  # fewer: one launch
+def test_the_rule_counts_the_chain_of_iterations(rt, family, m, blocks, kt, loop, order, groups):
+    from attention_superoptimizer_amd import workloads as W
+    from test_gpu_launch_records import _kernel as launched
+    k, n, rows, cols = kt * loop, 64 * blocks, (-1, -1, -1), (1, -1, -1)
+    if family == "lora":
+        spec, _ = W.config4_lora(m=m, d=k, r=16, grid=blocks, F=loop)
+        spec[1], spec[3] = W._inp([k, n], COL), W._inp([16, n], COL)
+    elif family == "two":
+        spec = [W._inp([m, k]), W._inp([k, n], COL), W._inp([k, n], COL),
+                {"op": "customized", "in": [[0, 0], [1, 0], [2, 0]],
+                 "plan": W._plan((blocks, 1, 1), loop, [rows, cols, cols], (1, 0, 0), cols,
+                                 [("tb_matmul_op", [(0, 0), (1, 0)]), ("tb_matmul_op", [(0, 0), (2, 0)])])}]
+    else:
+        ops = [("tb_matmul_op", [(0, 0), (1, 0)])] if family == "plain" else [("tb_silu_op", [(0, 0)]), ("tb_matmul_op", [(2, 0), (1, 0)])]
+        spec = [W._inp([m, k]), W._inp([k, n], COL),
+                {"op": "customized", "in": [[0, 0], [1, 0]], "plan": W._plan((blocks, 1, 1), loop, [rows, cols], (1, 0), cols, ops)}]
+    _run(rt, spec, order, f"{family} {m} x {blocks}, {kt} x {loop}", std=0.03)
+    assert launched()[1] == groups
