@@ -49,6 +49,15 @@ constexpr int attn_tiles_lds(int D, int RPW, int ip, int rounds) {
   return 2 * (ip * attn_tiles_strip(D, RPW) + (rounds > 1 ? 16 * RPW * (D + 8) + 16 * RPW : 0));
 }
 
+// Everything in memory is named as global memory.  Addresses out of the parameter block are generic to the
+// compiler, whose flat loads count with a wavefront's LDS operations as well: every read of the strip then waited
+// for the loads ahead of their use, those after the last round too.  Us on the device, flat and global, one operator
+// with the division: 2 groups of 33 rows, 9 blocks of 8 tiles of 16 keys, row-major, 3.95 and 3.59; 8 of 40, 4 of 16,
+// 5.59 and 5.04; tiles of 80 keys, column-major, 10.87 and 9.72.  (Without strips, each
+// load straight to its operand: 3.25, 4.20 and 14.42; a lone block is worked on here as half of a pair.)
+typedef __attribute__((address_space(1))) uint4v global_chunk;
+typedef __attribute__((address_space(1))) _Float16 global_half;
+
 template <int D, bool HAS_DIV, bool CM, int RPW, int PAIRS>
 __global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
     __attribute__((amdgpu_waves_per_eu(attn_tiles_lanes(D, PAIRS) == 8 ? 4 : 1))) void attn_tiles_kernel(AttnParams const) {
@@ -87,7 +96,7 @@ __global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
     long long const step = 2LL * (by_key ? KEYS : lone ? 32 : 16) * ld;
 #pragma unroll
     for (int i = 0; i < CHUNKS; i++) {
-      to[i] = *reinterpret_cast<uint4v const *>(at + (i < CHUNKS / 2 ? i : lone ? i - CHUNKS / 2 : i) * step + off);
+      to[i] = *(global_chunk const *)(at + (i < CHUNKS / 2 ? i : lone ? i - CHUNKS / 2 : i) * step + off);
     }
   };
   auto load_k = [&](int slot, int it, int p) {
@@ -172,7 +181,7 @@ __global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
 #pragma unroll
       for (int i = 0; i < CHUNKS / 2; i++) {
         int const row = row_base + 16 * rp + KEYS * i + lane / CPR;
-        raw[rp][i] = *reinterpret_cast<uint4v const *>(q + (long long)(row < m ? row : m - 1) * P.q.d_cols + 8 * (lane % CPR));
+        raw[rp][i] = *(global_chunk const *)(q + (long long)(row < m ? row : m - 1) * P.q.d_cols + 8 * (lane % CPR));
       }
     }
     load_ks(steps < DEPTH ? 1 : DEPTH);
@@ -312,7 +321,7 @@ __global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
       if (!done) {
         *reinterpret_cast<uint4v *>(sums + at) = sum;
       } else if (row < m) {
-        *reinterpret_cast<uint4v *>(og + (long long)row * P.o.d_cols + 8 * (e % CPR)) = sum;
+        *(global_chunk *)(og + (long long)row * P.o.d_cols + 8 * (e % CPR)) = sum;
       }
     }
     if (!HAS_DIV && tid < ROWS) {
@@ -324,7 +333,7 @@ __global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
         sums[ROWS * LD + tid] = sum;
       } else if (row_base + tid < m) {
         _Float16 *const rg = static_cast<_Float16 *>(const_cast<void *>(P.r.ptr)) + tile_offset(P.r, bx, by, bz, 0);
-        rg[(long long)(row_base + tid) * P.r.d_cols] = sum;
+        *(global_half *)(rg + (long long)(row_base + tid) * P.r.d_cols) = sum;
       }
     }
     if (!done) {

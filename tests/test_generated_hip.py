@@ -154,3 +154,26 @@ def test_the_loop_of_the_fused_attention_kernel_starts_a_fetch_block(tmp_path):
                            str(tmp_path / "prefill.hip"), "-o", str(tmp_path / "prefill.s")])
     body = open(tmp_path / "prefill.s").read()
     assert re.search(r"Loop Header: Depth=1[\s\S]{0,600}\.p2align 5\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0\n", body)
+
+
+@pytest.mark.parametrize("head,key_tile,col,div", [(64, 16, False, True), (64, 48, True, True), (64, 80, True, False), (128, 48, False, False)])
+def test_attention_of_any_tile_size_names_its_memory_as_global(tmp_path, head, key_tile, col, div):
+    """A flat load counts as an LDS operation too: every read of a strip would wait for the loads ahead of their use."""
+    if not os.path.exists(CG.HIPCC):
+        pytest.skip("no hipcc")
+    keys, layout = key_tile * 8, "DmemColumnMajor" if col else "DmemRowMajor"
+    if div:
+        spec, _ = W.config2_gqa_decode(2, 33, keys, 1, 8)
+        for t in spec[1:3]:
+            t["layout"] = layout
+    else:
+        spec = [W._inp([2, 33, head]), W._inp([2, head, keys], layout), W._inp([2, keys, head], layout),
+                {"op": "customized", "in": [[0, 0], [1, 0], [2, 0]],
+                 "plan": W._plan((2, 1, 1), 8, [(0, -1, -1)] * 3, (-1, 2, 1), (0, -1, -1), W.ATT_OPS)}]
+    text = _emit(spec, tmp_path / "tiles.hip")
+    assert "mi355::attn_tiles_kernel<%d, %s, %s, " % (head, str(div).lower(), str(col).lower()) in text
+    include = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(CG.__file__))), "include")
+    subprocess.check_call([CG.HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-I", include, "--cuda-device-only", "-S",
+                           str(tmp_path / "tiles.hip"), "-o", str(tmp_path / "tiles.s")])
+    body = open(tmp_path / "tiles.s").read()
+    assert "global_load_dwordx4" in body and "flat_load" not in body and "flat_store" not in body
