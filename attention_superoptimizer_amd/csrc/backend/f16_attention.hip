@@ -80,7 +80,7 @@ __global__ __launch_bounds__(64 * W) void f16_attention_rows_kernel(RowsAttentio
   auto again = [&](int i) { return own_key(i) - first_key(i); };
   // A block goes from memory into registers in the order it has there: rows of D elements (`by_key`) or,
   // for each of D elements, 32 keys.  (Read as the operands it becomes, sixteen rows to sixteen lanes, it
-  // would come at a quarter of the rate: 15.7 bytes a cycle against 58.)
+  // would come at a quarter of the rate: 16 bytes a cycle against 59.)
   half8 raw[AHEAD][OPS];
   uint32_t column[OPS];  // bytes of row 16 x + lane / 4 of a matrix with n columns
 #pragma unroll

@@ -469,8 +469,8 @@ __device__ __forceinline__ void gemm_wait_vm() {
 
 // Where the 16-byte chunk q of row r of an LDS tile lies in its row.  LDS has 64 banks, 256 bytes a cycle, and
 // serves a 16-byte read in the lane groups {0-3, 12-15, 20-23, 24-27} and so on, an 8-byte one 32 lanes at a
-// time; with these every operand read below is free of bank conflicts (measured over 16 wavefronts: 231 - 244
-// bytes a cycle; rows of 64 bytes turned by r / 4 126; transposing reads 211, turned by r / 2 % 4 126).
+// time; with these every operand read below is free of bank conflicts (measured over 16 wavefronts: 236 - 240
+// bytes a cycle; rows of 64 bytes turned by r / 4 127; transposing reads 190, turned by r / 2 % 4 121).
 __device__ __forceinline__ int turned_k64(int r, int q) { return q ^ (r / 2 % 8); }     // rows of 64 k
 __device__ __forceinline__ int turned_k32(int r, int q) { return q ^ (-(r / 4) & 3); }  // rows of 32 k
 template <int R>  // a row is one k of R = 64 or 128 columns, read transposing

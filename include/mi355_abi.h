@@ -132,7 +132,8 @@ typedef struct mi355_launch_info {
  * launch with the output tile cut into 16 x 16 pieces for plans that would otherwise leave
  * most of the chip idle; the for-loop cut into ranges, plus a launch that adds them, for
  * plans whose traffic, not the launch, sets the time); 1 = always the range-splitting kernel (which takes a
- * column-major plan of up to 16 rows in strips of 16 columns instead where they fill the chip); 2 = the one-launch
+ * column-major plan of up to 16 rows in strips of 16 columns instead where they fill the chip,
+ * and both of two weights in a workgroup where that fills it better); 2 = the one-launch
  * kernel wherever it applies.  Both keep the accumulation order of the sequential loop;
  * results agree to the last bit.  A measurement knob that the tests use to cover both. */
 #define MI355_OPT_GEMM_MODE 7

@@ -13,15 +13,15 @@
 // from there through a strip of LDS of the wavefront's own (with a transposing read where the reduction index
 // is not the contiguous one); the strip is also where the iteration's result ends.  An operand of a
 // column-major tile IS sixteen contiguous bytes per lane, but sixteen lanes in a row are then sixteen rows,
-// and a compute unit gets 15.7 bytes a cycle that way against 58 in memory order.
+// and a compute unit gets 16 bytes a cycle that way against 59 in memory order.
 //
 // What bounds it: the trip to memory at decode sizes, at prefill sizes latency and the conversions and
 // exponentials beside the matrix instructions (so: four wavefronts of a SIMD have registers, which is why
 // sums between rounds wait in LDS).  Two row groups share every K and V operand where there are enough of
 // them, which halves the L2 -> register traffic of a prefill.  With operands straight from memory, a tile's keys
 // in registers at once and workgroups of an XCD from anywhere, both launches of [12, 1040, 1040] in tiles
-// of 80 took 24.6 us column-major and 35.5 row-major, now 19.6 and 19.7; head size 128, [16, 1024, 1008] in
-// tiles of 128 x 48, 59.5 and 41.3; [64, 1, 16384] in tiles of 64 65.9 and 57.3.
+// of 80 took 24.6 us column-major and 35.5 row-major, now 18.8 and 19.3; head size 128, [16, 1024, 1008] in
+// tiles of 128 x 48, 59.5 and 37.5; [64, 1, 16384] in tiles of 64 65.9 and 50.7.
 #pragma once
 
 #include <type_traits>

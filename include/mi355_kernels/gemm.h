@@ -37,7 +37,7 @@ struct GTile {
 struct GemmParams {
   GTile a0, a1;      // activation-side tiles [M][KT] (a1: second operand of the gate form)
   GTile b0, b1;      // weight tiles [KT][64]
-  GTile la, lb;      // lora: A tile [KT][16], B tile [16][64] (loop invariant)
+  GTile la, lb;      // lora: A tile [KT][r], B tile [r][64] (loop invariant), ranks r of 8, 16 and 32
   GTile o0, o1;      // outputs
   int M, KT;         // rows of the activation tile, k extent of one iteration
   int forloop_range;
@@ -635,8 +635,8 @@ __device__ __forceinline__ half4 lane_tr16(_Float16 const *p) {
 // sixteen columns are sixteen streams of whole cache lines that no other workgroup touches), are
 // [16][KT] tiles whose operands are 16 contiguous bytes.  They come in units of 64 k, a line of each row, into
 // registers in the order they have in memory and become operands through 2 KB of LDS each: read as operands,
-// sixteen lanes in a row would be sixteen rows, and a compute unit then gets 15.7 bytes a cycle from its
-// vector cache against 58 (32 rows x 2240 x 1856 in 64-k iterations: 9.0 -> 5.5 us).
+// sixteen lanes in a row would be sixteen rows, and a compute unit then gets 16 bytes a cycle from its
+// vector cache against 59 (32 rows x 2240 x 1856 in 64-k iterations: 9.0 -> 5.5 us).
 constexpr int kUnitBytes = 2048;  // [16][64 k]
 // bytes of a wavefront's strips: the units being turned; row-major weights, the [16][16] piece of lora B
 // (lora: 16-rank pieces of lora A, the last of them may hold 8)

@@ -5,8 +5,8 @@
 // A workgroup owns the 64 columns of a logical block and a range of the for-loop; each of its four
 // wavefronts takes every fourth iteration of the range and needs nobody else for it: a ring of LDS
 // slots of its own (64 columns x 64 k of one weight matrix, whole 128-byte lines, and the activations'
-// 64 k beside it) is filled by direct-to-LDS loads several 
-// in flight, no register waits for memory and no barrier stands in the loop.  Column-major weights are
+// 64 k beside it) is filled by direct-to-LDS loads, several
+// in flight; no register waits for memory and no barrier stands in the loop.  Column-major weights are
 // read back as they are, row-major ones with transposing reads; chunks are XOR-swizzled on the way in
 // so that both are free of bank conflicts.
 //
@@ -16,7 +16,8 @@
 // (reference src/kernel/triton_code_gen.cc:223-232).
 //
 // Two weights are two sets of workgroups (for twice the activations' bytes): seven to a compute unit instead of
-// three and a half leave less of the last round empty (two weights of 4096 x 14336: 44.3 -> 42.3 us).
+// three and a half leave less of the last round empty (two weights of 4096 x 14336: 44.3 -> 42.3 us).  Where that does not
+// hold, few blocks or one workgroup a compute unit, gemm_stream_pairs_kernel takes both in a workgroup (the host's rule).
 //
 // What bounds it is memory: 235 MB (those two weights, column-major) 42 us (5.6 TB/s; a kernel that only reads
 // them takes 38); 118 MB, one weight, 19 us (6.2).  The gate's activations (silu of 14336 x 16 values in every
