@@ -117,6 +117,7 @@ ABI = {
     "mi355_plan_extents": (_ci, [_pplan, _pll, _pll, _pi, _pi]),
     "mi355_customized_run": (_ci, [_pplan, _pvp, _pvp]),
     "mi355_prepare": (_ci, [_pplan, _pvp, _pvp, _ci, _pvp]),
+    "mi355_prepare_two": (_ci, [_pplan, _pvp, _pvp, _pplan, _pvp, _pvp, _ci, _pvp]),
     "mi355_prepared_run": (_ci, [_vp]),
     "mi355_prepared_free": (_ci, [_vp]),
     "mi355_customized_profile": (_ci, [_pplan, _pvp, _pvp, _ci, _ci, _ci, _pf]),

@@ -38,6 +38,7 @@
 // programs include as well.
 #include "common.h"
 #include "tb_program.h"
+#include "attn_launch.h"
 #include "attn_tiles.h"
 #include <algorithm>
 #include <cstdlib>
@@ -102,7 +103,6 @@ std::string literal(AttnParams const &A) {
                 "    P.r_copy_stride = %d;\n    P.in_order = %d;\n", A.split_magic, A.rows, A.r_copies, A.r_copy_stride, A.in_order);
   return t;
 }
-char const *tf(bool b) { return b ? "true" : "false"; }
 
 struct Match {
   int q, k, v;        // load op indices
@@ -314,168 +314,6 @@ bool merge_row_blocks(DevProgram const &P, Match &M, DevProgram &Q) {
   return false;
 }
 
-template <bool HAS_DIV, bool CM, int IP, int RPW, int NBUF, int NIT, int SPI, int IPS>
-int launch_direct_one(AttnParams const &A, dim3 grid, int lds, bool dry) {
-  if (dry) {
-    return 1;  // the question was only whether this shape is built
-  }
-  if (EmitSink *sink = emit_sink()) {
-    sink->headers |= 1u;
-    emit_launch(*sink, "attn_direct_kernel",
-                emit_fmt("64, 64, 64, %s, %d, %d, %d, %d, %d, %d, false, %s", tf(HAS_DIV), IP, RPW, NBUF, NIT, SPI, IPS,
-                         tf(CM)),
-                grid, 64 * IP, lds, literal(A));
-    return 1;
-  }
-  auto go = [&](auto *fn) -> int {
-    MI355_GRANT_LDS(fn, lds);
-    MI355_HIP(launch_kernel(fn, grid, 64 * IP, lds, state().stream(), A));
-    return 1;
-  };
-  if (SPI == 1 && IPS == 1 && A.trace != nullptr) {
-    return go(attn_direct_kernel<64, 64, 64, HAS_DIV, IP, RPW, NBUF, NIT, SPI, IPS, SPI == 1 && IPS == 1, CM>);
-  }
-  return go(attn_direct_kernel<64, 64, 64, HAS_DIV, IP, RPW, NBUF, NIT, SPI, IPS, false, CM>);
-}
-
-// The shape of a direct-staging launch: `ip` wavefronts of `rpw` row groups each, `nbuf` tile
-// pairs per wavefront, up to `nit` units of work per wavefront, `spi` strips per iteration or
-// `ips` iterations per strip.
-struct DirectShape {
-  int ip = 0, rpw = 1, nbuf = 1, nit = 1, spi = 1, ips = 1;
-  int code() const { return ((((ip * 10 + rpw) * 10 + nbuf) * 10 + nit) * 10 + spi) * 10 + ips; }
-};
-
-// 0: no instantiation for this shape
-template <bool HAS_DIV, bool CM>
-int launch_direct(AttnParams const &A, dim3 grid, DirectShape const &d, int lds, bool dry = false) {
-#define MI355_DIRECT(IPV, RPWV, NBUFV, NITV, SPIV, IPSV) \
-  case ((((IPV * 10 + RPWV) * 10 + NBUFV) * 10 + NITV) * 10 + SPIV) * 10 + IPSV: \
-    return launch_direct_one<HAS_DIV, CM, IPV, RPWV, NBUFV, NITV, SPIV, IPSV>(A, grid, lds, dry);
-  switch (d.code()) {
-    // one 64-key tile per iteration
-    MI355_DIRECT(2, 1, 1, 1, 1, 1)
-    MI355_DIRECT(4, 1, 1, 1, 1, 1)
-    MI355_DIRECT(8, 1, 1, 1, 1, 1)
-    MI355_DIRECT(4, 2, 1, 1, 1, 1)
-    MI355_DIRECT(4, 1, 2, 2, 1, 1)
-    MI355_DIRECT(4, 1, 2, 4, 1, 1)
-    MI355_DIRECT(4, 1, 2, 8, 1, 1)
-    MI355_DIRECT(4, 1, 1, 2, 1, 1)
-    MI355_DIRECT(4, 1, 1, 4, 1, 1)
-    MI355_DIRECT(4, 1, 1, 8, 1, 1)
-    MI355_DIRECT(8, 1, 1, 2, 1, 1)
-    MI355_DIRECT(8, 1, 1, 4, 1, 1)
-    // key tiles of 32 and 16: two / four iterations per strip
-    MI355_DIRECT(4, 1, 1, 1, 1, 2)
-    MI355_DIRECT(4, 2, 1, 1, 1, 2)
-    MI355_DIRECT(8, 1, 1, 1, 1, 2)
-    MI355_DIRECT(8, 1, 1, 2, 1, 2)
-    MI355_DIRECT(4, 1, 1, 1, 1, 4)
-    MI355_DIRECT(4, 2, 1, 1, 1, 4)
-    MI355_DIRECT(8, 1, 1, 1, 1, 4)
-    default: break;
-  }
-  if constexpr (!HAS_DIV) {
-    switch (d.code()) {
-      // key tiles of 128 and 256: two / four strips per iteration (no division inside)
-      MI355_DIRECT(4, 1, 1, 1, 2, 1)
-      MI355_DIRECT(8, 1, 1, 1, 2, 1)
-      MI355_DIRECT(8, 1, 1, 2, 2, 1)
-      MI355_DIRECT(8, 1, 1, 4, 2, 1)
-      MI355_DIRECT(4, 1, 1, 1, 4, 1)
-      MI355_DIRECT(8, 1, 1, 1, 4, 1)
-      MI355_DIRECT(8, 1, 1, 2, 4, 1)
-      MI355_DIRECT(8, 1, 1, 4, 4, 1)
-      default: break;
-    }
-  }
-#undef MI355_DIRECT
-  return 0;
-}
-
-template <int D, int NK, int DV, bool HAS_DIV, int RG, int IP, bool CM>
-int launch_one(AttnParams const &A, dim3 grid, int lds) {
-  if (EmitSink *sink = emit_sink()) {
-    sink->headers |= 1u;
-    emit_launch(*sink, "attn_fused_kernel", emit_fmt("%d, %d, %d, %s, %d, %d, %s", D, NK, DV, tf(HAS_DIV), RG, IP, tf(CM)),
-                grid, 64 * RG * IP, lds, literal(A));
-    return 1;
-  }
-  auto *fn = attn_fused_kernel<D, NK, DV, HAS_DIV, RG, IP, CM>;
-  MI355_GRANT_LDS(fn, lds);
-  MI355_HIP(launch_kernel(fn, grid, 64 * RG * IP, lds, state().stream(), A));
-  return 1;
-}
-
-template <int D, int NK, int DV, bool HAS_DIV, bool CM>
-int launch_waves(AttnParams const &A, dim3 grid, int rg, int ip, int lds) {
-  switch (rg * 16 + ip) {
-    case 1 * 16 + 1: return launch_one<D, NK, DV, HAS_DIV, 1, 1, CM>(A, grid, lds);
-    case 1 * 16 + 2: return launch_one<D, NK, DV, HAS_DIV, 1, 2, CM>(A, grid, lds);
-    case 1 * 16 + 4: return launch_one<D, NK, DV, HAS_DIV, 1, 4, CM>(A, grid, lds);
-    case 1 * 16 + 8: return launch_one<D, NK, DV, HAS_DIV, 1, 8, CM>(A, grid, lds);
-    case 2 * 16 + 1: return launch_one<D, NK, DV, HAS_DIV, 2, 1, CM>(A, grid, lds);
-    case 2 * 16 + 2: return launch_one<D, NK, DV, HAS_DIV, 2, 2, CM>(A, grid, lds);
-    case 2 * 16 + 4: return launch_one<D, NK, DV, HAS_DIV, 2, 4, CM>(A, grid, lds);
-    case 4 * 16 + 1: return launch_one<D, NK, DV, HAS_DIV, 4, 1, CM>(A, grid, lds);
-    case 4 * 16 + 2: return launch_one<D, NK, DV, HAS_DIV, 4, 2, CM>(A, grid, lds);
-    default: return 0;
-  }
-}
-
-template <int D, int NK, int DV>
-int launch_shape(AttnParams const &A, bool has_div, bool cm, dim3 grid, int rg, int ip, int lds) {
-  if (cm) {
-    return has_div ? launch_waves<D, NK, DV, true, true>(A, grid, rg, ip, lds)
-                   : launch_waves<D, NK, DV, false, true>(A, grid, rg, ip, lds);
-  }
-  return has_div ? launch_waves<D, NK, DV, true, false>(A, grid, rg, ip, lds)
-                 : launch_waves<D, NK, DV, false, false>(A, grid, rg, ip, lds);
-}
-
-template <int D, int NK, int DV, bool HAS_DIV, int RG, int RPW, bool CM, int SPI = 1>
-int launch_stream_one(AttnParams const &A, dim3 grid, int lds) {
-  if (EmitSink *sink = emit_sink()) {
-    sink->headers |= 1u;
-    emit_launch(*sink, "attn_stream_kernel",
-                emit_fmt("%d, %d, %d, %s, %d, %d, %s, %d", D, NK, DV, tf(HAS_DIV), RG, RPW, tf(CM), SPI), grid, 64 * RG,
-                lds, literal(A));
-    return 1;
-  }
-  auto *fn = attn_stream_kernel<D, NK, DV, HAS_DIV, RG, RPW, CM, SPI>;
-  MI355_GRANT_LDS(fn, lds);
-  MI355_HIP(launch_kernel(fn, grid, 64 * RG, lds, state().stream(), A));
-  return 1;
-}
-
-template <int D, int NK, int DV, bool CM>
-int launch_stream(AttnParams const &A, bool has_div, dim3 grid, int rg, int lds, bool wide = false, int spi = 1) {
-  if (spi > 1) {  // wider key tiles: four wavefronts of 32 rows, the form without the division
-    if (has_div || rg != 4 || wide) {
-      return 0;
-    }
-    switch (spi) {
-      case 2: return launch_stream_one<D, NK, DV, false, 4, 2, CM, 2>(A, grid, lds);
-      case 4: return launch_stream_one<D, NK, DV, false, 4, 2, CM, 4>(A, grid, lds);
-      case 8: return launch_stream_one<D, NK, DV, false, 4, 2, CM, 8>(A, grid, lds);
-      default: return 0;
-    }
-  }
-  if constexpr (D == 64) {
-    if (wide) {  // four wavefronts of 64 rows
-      return has_div ? launch_stream_one<D, NK, DV, true, 4, 4, CM>(A, grid, lds)
-                     : launch_stream_one<D, NK, DV, false, 4, 4, CM>(A, grid, lds);
-    }
-  }
-  if (has_div) {
-    return rg == 4 ? launch_stream_one<D, NK, DV, true, 4, 2, CM>(A, grid, lds)
-                   : launch_stream_one<D, NK, DV, true, 2, 2, CM>(A, grid, lds);
-  }
-  return rg == 4 ? launch_stream_one<D, NK, DV, false, 4, 2, CM>(A, grid, lds)
-                 : launch_stream_one<D, NK, DV, false, 2, 2, CM>(A, grid, lds);
-}
-
 }  // namespace
 
 // Fills the division magics decode_block uses for this launch grid; false when an id times an
@@ -667,7 +505,81 @@ bool attention_applicable(DevProgram const &P) {
   return merge_column_pieces(P, M, merged, copies, stride) && choose_direct(merged, M, d, lds);
 }
 
-int try_launch_attention(DevProgram const &P0) {
+// What the next operator's fold of rows is to this launch: a workgroup's rows, and the places of its
+// results in them.  False where the operator is no fold of exactly these results, row by row.
+//
+// With whole rows in a workgroup it always pays: both launches of [12, 1040, 1040] in tiles of 80 18.8 -> 16.4 us, of
+// [32, 2048, 2048] at head size 128 78.8 -> 75.5 (both tensors' stores are what is left), 86 prefill plans 0.78 of the
+// time in the mean, 0.53 - 0.99.  Where the pieces come from several workgroups the last of them pays three trips to the
+// memory that all XCDs share (its stores, its ticket, the pieces), 3 us against the 3.5 - 4.5 of a launch, and all others two while
+// they hold their place on a compute unit.  So: blocks that run in one round (64 groups of 16 blocks, two rounds, 50.8
+// us either way, folded 52.1), as many columns of threads as there are columns, and sixteen pieces, what a thread loads
+// together (7 groups of 16 rows, 20 pieces, one wavefront 8.8 us, folded 12.5).  135 split-KV plans 0.94 of the time
+// in the mean, 0.77 - 1.05; [5, 12, 64] against 12 pieces of 5 tiles of 48 keys 8.4 -> 7.7.
+static bool make_fold(AttnParams const &A, Match const &M, DevProgram const &P, int wg_rows, int threads, int lds, FoldRequest &f,
+                      AttnFold &out) {
+  RowFold const &R = f.rows;
+  int const C = R.S * R.X;
+  if (M.out_r < 0 || A.r_copies != 1 || state().phase_trace != nullptr || A.o.ptr != R.n || A.r.ptr != R.d || R.X != M.DV || A.o.d_cols != C || A.r.d_cols != R.SD ||
+      R.SD != R.S || (R.S > 1 && R.mode != SUM_THEN_DIV) || (long long)C * R.rows >= (1LL << 31)) {
+    return false;
+  }
+  // One grid dimension may cut the columns: piece after piece, row sum after row sum.  The others cut the rows.
+  long long stride[3];
+  int extent[3], row_dims = 0, pieces = 1;
+  for (int i = 0; i < 3; i++) {
+    out.lin[i] = out.ticket_lin[i] = 0;
+    if (P.grid[i] == 1) {
+      continue;
+    }
+    if (R.S > 1 && pieces == 1 && A.o.lin[i] == R.X && A.r.lin[i] == 1 && P.grid[i] == R.S) {
+      pieces = P.grid[i];
+      continue;
+    }
+    if (A.o.lin[i] % C != 0 || A.r.lin[i] % R.SD != 0 || A.o.lin[i] / C != A.r.lin[i] / R.SD || A.o.lin[i] / C % M.m != 0) {
+      return false;
+    }
+    out.lin[i] = A.o.lin[i] / C;
+    out.ticket_lin[i] = out.lin[i] / M.m * A.split;
+    stride[row_dims] = out.lin[i];
+    extent[row_dims++] = P.grid[i];
+  }
+  long long rows = 0;
+  if (pieces != R.S || !covers_rows(M.m, stride, extent, row_dims, rows) || rows != R.rows) {
+    return false;
+  }
+  // (what the fold writes is read by no other workgroup of this launch)
+  uintptr_t const o0 = reinterpret_cast<uintptr_t>(R.o), o1 = o0 + ((size_t)(R.rows - 1) * R.o_cols + R.X) * 2;
+  for (void const *p : {A.q.ptr, A.k.ptr, A.v.ptr, A.o.ptr, A.r.ptr}) {
+    if (reinterpret_cast<uintptr_t>(p) >= o0 && reinterpret_cast<uintptr_t>(p) < o1) {
+      return false;
+    }
+  }
+  out.n = static_cast<_Float16 const *>(R.n);
+  out.d = static_cast<_Float16 const *>(R.d);
+  out.o = static_cast<_Float16 *>(R.o);
+  out.arrivals = R.S;
+  out.S = R.S;
+  out.X = R.X;
+  out.o_cols = R.o_cols;
+  out.mxv = fast_div_magic(R.X / 4);
+  out.tickets = nullptr;
+  if (R.S > 1) {
+    int const per_cu = std::max(1, std::min(state().max_lds / std::max(lds, 1), 1024 / threads));
+    int const trips = (std::min(wg_rows, M.m) * R.X / 4 + threads - 1) / threads;
+    if (R.S > kFoldPieces || trips > (R.S <= 8 ? 2 : 1) || wg_rows * R.S * 2 + 16 > lds ||
+        (long long)P.grid[0] * P.grid[1] * P.grid[2] * A.split > 256 * per_cu) {
+      return false;
+    }
+    out.tickets = f.tickets(R.rows / M.m * A.split);
+    if (out.tickets == nullptr) {
+      return false;
+    }
+  }
+  return true;
+}
+
+int try_launch_attention(DevProgram const &P0, FoldRequest *fold) {
   Match M;
   DevProgram merged;
   DevProgram const *run = &P0;
@@ -766,7 +678,13 @@ int try_launch_attention(DevProgram const &P0) {
     if (!set_grid_magics(A, grid, streamed)) {
       return 0;
     }
-    int const rc = launch_attn_tiles(A, grid, M.D, M.has_div, M.kv_colmajor, tiles_shape);
+    AttnFoldParams F;
+    if (fold != nullptr && !make_fold(A, M, P, 16 * tiles_shape.rpw, 64 * tiles_shape.ip, tiles_shape.lds, *fold, F.fold)) {
+      return 0;
+    }
+    F.attn = A;
+    int const rc = fold != nullptr ? launch_attn_tiles_fold(F, grid, M.D, M.kv_colmajor, tiles_shape)
+                                   : launch_attn_tiles(A, grid, M.D, M.has_div, M.kv_colmajor, tiles_shape);
     if (rc == 1) {
       s.last().kernel_id = MI355_KERNEL_F16_ATTENTION;
       s.last().workgroups = grid.x * grid.y * grid.z;
@@ -792,14 +710,15 @@ int try_launch_attention(DevProgram const &P0) {
         if (!set_grid_magics(A, grid, streamed)) {
           return 0;
         }
-        int rc;
-        if (M.kv_colmajor) {
-          rc = M.D == 64 ? launch_stream<64, 64, 64, true>(A, M.has_div, grid, rgs, lds, st.wide, st.spi)
-                         : launch_stream<128, 64, 128, true>(A, M.has_div, grid, rgs, lds, false, st.spi);
-        } else {
-          rc = M.D == 64 ? launch_stream<64, 64, 64, false>(A, M.has_div, grid, rgs, lds, st.wide, st.spi)
-                         : launch_stream<128, 64, 128, false>(A, M.has_div, grid, rgs, lds, false, st.spi);
+        AttnShape const shape{M.D, M.NK, M.kv_colmajor, rgs, 1, lds, st.spi, st.wide};
+        AttnFoldParams F;
+        if (fold != nullptr && !make_fold(A, M, P, 32 * rgs, st.wide ? 256 : 64 * rgs, lds, *fold, F.fold)) {
+          return 0;
         }
+        F.attn = A;
+        int const rc = fold != nullptr ? launch_stream_fold(F, grid, shape)
+                       : M.has_div     ? launch_stream_shape<true>(A, grid, shape)
+                                       : launch_stream_shape<false>(A, grid, shape);
         if (rc == 1) {
           s.last().kernel_id = MI355_KERNEL_F16_ATTENTION;
           s.last().workgroups = grid.x * grid.y * grid.z;
@@ -835,7 +754,13 @@ int try_launch_attention(DevProgram const &P0) {
                                     s.phase_trace_bytes) {
         B.trace = nullptr;
       }
-      int const rc = M.kv_colmajor
+      AttnFoldParams F;
+      if (fold != nullptr && !make_fold(B, M, P, 16 * dshape.rpw, 64 * dshape.ip, direct_lds, *fold, F.fold)) {
+        return 0;
+      }
+      F.attn = B;
+      int const rc = fold != nullptr ? launch_direct_fold(F, M.kv_colmajor, direct_grid, dshape, direct_lds)
+                     : M.kv_colmajor
                          ? (M.has_div ? launch_direct<true, true>(B, direct_grid, dshape, direct_lds)
                                       : launch_direct<false, true>(B, direct_grid, dshape, direct_lds))
                          : (M.has_div ? launch_direct<true, false>(B, direct_grid, dshape, direct_lds)
@@ -901,15 +826,15 @@ int try_launch_attention(DevProgram const &P0) {
   if (!set_grid_magics(A, grid, streamed)) {
     return 0;
   }
-  if (M.D == 64 && M.NK == 64) {
-    rc = launch_shape<64, 64, 64>(A, M.has_div, M.kv_colmajor, grid, rg, ip, lds);
-  } else if (M.D == 64 && M.NK == 128) {
-    rc = launch_shape<64, 128, 64>(A, M.has_div, M.kv_colmajor, grid, rg, ip, lds);
-  } else if (M.D == 64 && M.NK == 256) {
-    rc = launch_shape<64, 256, 64>(A, M.has_div, M.kv_colmajor, grid, rg, ip, lds);
-  } else {
-    rc = launch_shape<128, 64, 128>(A, M.has_div, M.kv_colmajor, grid, rg, ip, lds);
+  AttnShape const shape{M.D, M.NK, M.kv_colmajor, rg, ip, lds};
+  AttnFoldParams F;
+  if (fold != nullptr && !make_fold(A, M, P, 16 * rg, 64 * nw, lds, *fold, F.fold)) {
+    return 0;
   }
+  F.attn = A;
+  rc = fold != nullptr ? launch_fused_fold(F, grid, shape)
+       : M.has_div     ? launch_fused_shape<true>(A, grid, shape)
+                       : launch_fused_shape<false>(A, grid, shape);
   if (rc == 1) {
     s.last().kernel_id = MI355_KERNEL_F16_ATTENTION;
     s.last().workgroups = grid.x * grid.y * grid.z;

@@ -12,23 +12,25 @@ namespace mi355 {
 
 namespace {
 
-template <int D, bool HAS_DIV, bool CM, int RPW, int PAIRS>
-int launch_tiles_one(AttnParams const &A, dim3 grid, int ip, int lds) {
-  if (EmitSink *sink = emit_sink()) {
-    sink->headers |= 8u;
-    emit_launch(*sink, "attn_tiles_kernel",
-                emit_fmt("%d, %s, %s, %d, %d", D, HAS_DIV ? "true" : "false", CM ? "true" : "false", RPW, PAIRS), grid, 64 * ip, lds,
-                attn_params_literal(A));
-    return 1;
+template <int D, bool HAS_DIV, bool CM, int RPW, int PAIRS, class Params>
+int launch_tiles_one(Params const &A, dim3 grid, int ip, int lds) {
+  if constexpr (std::is_same_v<Params, AttnParams>) {
+    if (EmitSink *sink = emit_sink()) {
+      sink->headers |= 8u;
+      emit_launch(*sink, "attn_tiles_kernel",
+                  emit_fmt("%d, %s, %s, %d, %d", D, HAS_DIV ? "true" : "false", CM ? "true" : "false", RPW, PAIRS), grid, 64 * ip, lds,
+                  attn_params_literal(A));
+      return 1;
+    }
   }
-  auto *fn = attn_tiles_kernel<D, HAS_DIV, CM, RPW, PAIRS>;
+  auto *fn = attn_tiles_kernel<D, HAS_DIV, CM, RPW, PAIRS, Params>;
   MI355_GRANT_LDS(fn, lds);
   MI355_HIP(launch_kernel(fn, grid, 64 * ip, lds, state().stream(), A));
   return 1;
 }
 
-template <int D, bool HAS_DIV, bool CM>
-int launch_tiles_shape(AttnParams const &A, dim3 grid, int rpw, int pairs, int ip, int lds) {
+template <int D, bool HAS_DIV, bool CM, class Params>
+int launch_tiles_shape(Params const &A, dim3 grid, int rpw, int pairs, int ip, int lds) {
   if constexpr (!HAS_DIV) {
     return rpw == 1 ? launch_tiles_one<D, false, CM, 1, 0>(A, grid, ip, lds) : launch_tiles_one<D, false, CM, 2, 0>(A, grid, ip, lds);
   } else {
@@ -96,6 +98,15 @@ int launch_attn_tiles(AttnParams const &A, dim3 grid, int D, bool has_div, bool 
   if (has_div) {
     return cm ? launch_tiles_shape<128, true, true>(A, grid, t.rpw, t.pairs, t.ip, t.lds)
               : launch_tiles_shape<128, true, false>(A, grid, t.rpw, t.pairs, t.ip, t.lds);
+  }
+  return cm ? launch_tiles_shape<128, false, true>(A, grid, t.rpw, t.pairs, t.ip, t.lds)
+            : launch_tiles_shape<128, false, false>(A, grid, t.rpw, t.pairs, t.ip, t.lds);
+}
+
+int launch_attn_tiles_fold(AttnFoldParams const &A, dim3 grid, int D, bool cm, TilesShape const &t) {
+  if (D == 64) {
+    return cm ? launch_tiles_shape<64, false, true>(A, grid, t.rpw, t.pairs, t.ip, t.lds)
+              : launch_tiles_shape<64, false, false>(A, grid, t.rpw, t.pairs, t.ip, t.lds);
   }
   return cm ? launch_tiles_shape<128, false, true>(A, grid, t.rpw, t.pairs, t.ip, t.lds)
             : launch_tiles_shape<128, false, false>(A, grid, t.rpw, t.pairs, t.ip, t.lds);

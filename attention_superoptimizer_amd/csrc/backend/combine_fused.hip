@@ -245,6 +245,54 @@ bool combine_applicable(DevProgram const &P) {
   return cmatch(P, M);
 }
 
+bool covers_rows(int m, long long *stride, int *extent, int dims, long long &rows) {
+  rows = m;
+  for (int taken = 0; taken < dims; taken++) {  // (in the order of their strides: each starts where the others end)
+    int at = taken;
+    while (at < dims && stride[at] != rows) {
+      at++;
+    }
+    if (at == dims) {
+      return false;
+    }
+    std::swap(stride[taken], stride[at]);
+    std::swap(extent[taken], extent[at]);
+    rows *= extent[taken];
+  }
+  return true;
+}
+
+bool combine_as_rows(DevProgram const &P, RowFold &R) {
+  CMatch M;
+  if (!cmatch(P, M) || M.vec != 8) {
+    return false;
+  }
+  CombineParams const A = combine_params(P, M);
+  int const C = A.S * A.X;
+  if (A.n.d_cols != C || A.d.d_cols != A.SD || (A.S > 1 && A.step != A.X)) {
+    return false;
+  }
+  long long stride[3];
+  int extent[3], dims = 0;
+  for (int i = 0; i < 3; i++) {
+    if (P.grid[i] == 1) {
+      continue;
+    }
+    long long const rows = A.n.lin[i] / C;
+    if (A.n.lin[i] % C != 0 || A.d.lin[i] != rows * A.SD || A.o.lin[i] != rows * A.o.d_cols) {
+      return false;
+    }
+    stride[dims] = rows;
+    extent[dims++] = P.grid[i];
+  }
+  long long rows = 0;
+  if (!covers_rows(A.rows, stride, extent, dims, rows) || rows >= (1LL << 31)) {
+    return false;
+  }
+  R = {A.n.ptr, A.d.ptr, const_cast<void *>(A.o.ptr), A.S, A.SD, A.X, A.o.d_cols, M.mode, (int)rows};
+  return true;
+}
+
 int try_launch_combine(DevProgram const &P) {
   CMatch M;
   if (!cmatch(P, M)) {

@@ -108,9 +108,18 @@ struct State {
   char *planes() const {
     return planes_base == nullptr ? nullptr : planes_base + (size_t)tls_queue * planes_bytes;
   }
+  // Tickets of launches whose last workgroup goes on with the work of all (attention_fold.h): per queue
+  // kTickets ints, zero whenever no launch that uses them runs.
+  static constexpr int kTickets = 1 << 16;
+  int *tickets = nullptr;
 };
 
 State &state();
+// `count` tickets of a queue that nobody else has until they are given back, or null: a launch that is made again
+// and again has its own, so that two of them never meet.  Given back they go to a later launch of the same queue,
+// behind the earlier one in it; `life` tells this mi355_init's from an earlier one's.
+int *take_tickets(int queue, int count, unsigned &life);
+void give_tickets(int queue, int *tickets, int count, unsigned life);
 
 // Raises the dynamic LDS limit of a kernel to what the device has, once per kernel: the call costs
 // the host several microseconds.  A launch that requests at most 64 KB needs none.

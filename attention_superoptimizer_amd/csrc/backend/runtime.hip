@@ -5,6 +5,7 @@
 // fingerprint lookup tables, and the event pairs every profile() uses.
 #include "common.h"
 #include <atomic>
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <unordered_set>
@@ -60,6 +61,50 @@ using namespace mi355;
 extern "C" char const *mi355_last_error(void) { return g_error; }
 
 extern "C" int mi355_is_initialised(void) { return state().ready ? 1 : 0; }
+
+// ---- tickets: handed out in units of 64 ints, first fit ------------------------------------------
+namespace mi355 {
+namespace {
+constexpr int kTicketUnit = 64, kTicketUnits = State::kTickets / kTicketUnit;
+std::mutex g_ticket_lock;  // (a handle may be dropped by another thread than its queue's)
+bool g_ticket_used[MI355_NUM_QUEUES][kTicketUnits];
+unsigned g_ticket_life = 0;  // counts allocations
+
+void forget_tickets() {
+  std::lock_guard<std::mutex> hold(g_ticket_lock);
+  std::memset(g_ticket_used, 0, sizeof(g_ticket_used));
+  g_ticket_life++;
+}
+}  // namespace
+
+int *take_tickets(int queue, int count, unsigned &life) {
+  int const units = (count + kTicketUnit - 1) / kTicketUnit;
+  if (count < 1 || units > kTicketUnits) {
+    return nullptr;
+  }
+  std::lock_guard<std::mutex> hold(g_ticket_lock);
+  bool *const used = g_ticket_used[queue];
+  int run = 0;
+  for (int u = 0; u < kTicketUnits; u++) {
+    run = used[u] ? 0 : run + 1;
+    if (run == units) {
+      std::fill(used + u + 1 - units, used + u + 1, true);
+      life = g_ticket_life;
+      return state().tickets + (size_t)queue * State::kTickets + (u + 1 - units) * kTicketUnit;
+    }
+  }
+  return nullptr;
+}
+
+void give_tickets(int queue, int *tickets, int count, unsigned life) {
+  std::lock_guard<std::mutex> hold(g_ticket_lock);
+  if (life == g_ticket_life) {
+    ptrdiff_t const at = tickets - (state().tickets + (size_t)queue * State::kTickets);
+    std::fill_n(g_ticket_used[queue] + at / kTicketUnit, (count + kTicketUnit - 1) / kTicketUnit, false);
+  }
+}
+}  // namespace mi355
+
 
 extern "C" int mi355_init(size_t arena_bytes, void **arena_base) {
   State &s = state();
@@ -163,6 +208,9 @@ extern "C" int mi355_init(size_t arena_bytes, void **arena_base) {
   s.planes_bytes = (size_t)128 << 20;  // per queue
   MI355_HIP(hipMalloc(reinterpret_cast<void **>(&s.planes_base),
                       s.planes_bytes * MI355_NUM_QUEUES));
+  MI355_HIP(hipMalloc(reinterpret_cast<void **>(&s.tickets), sizeof(int) * State::kTickets * MI355_NUM_QUEUES));
+  MI355_HIP(hipMemset(s.tickets, 0, sizeof(int) * State::kTickets * MI355_NUM_QUEUES));
+  forget_tickets();
   s.ready = true;
   if (arena_base != nullptr) {
     *arena_base = s.arena;
@@ -197,6 +245,8 @@ extern "C" int mi355_shutdown(void) {
     }
   }
   MI355_HIP(hipFree(s.scratch_base));
+  MI355_HIP(hipFree(s.tickets));
+  forget_tickets();
   MI355_HIP(hipFree(s.planes_base));
   s.planes_base = nullptr;
   if (s.phase_trace_store != nullptr) {

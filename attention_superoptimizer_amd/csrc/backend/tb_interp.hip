@@ -1974,26 +1974,67 @@ extern "C" int mi355_customized_run(mi355_plan const *plan, void const *const *i
 }
 
 // ---- prepared operators ------------------------------------------------------------------------
-// The kernel launches of one customized operator, recorded once and repeated: see launch.h.  They
-// hold for the queue (its scratch memory is in the arguments) and the options they were recorded
-// under; a run from another queue or after mi355_set_option records them again.
-struct mi355_prepared {
+// The kernel launches of one customized operator, or of two that follow each other, recorded once and
+// repeated: see launch.h.  They hold for the queue (its scratch memory is in the arguments) and the options
+// they were recorded under; a run from another queue or after mi355_set_option records them again.
+struct PreparedPlan {
   mi355_plan plan;
   void const *inputs[MI355_MAX_DMEM_INPUTS];
   void *outputs[MI355_MAX_DMEM_OUTPUTS];
+};
+struct mi355_prepared {
+  PreparedPlan op[2];
+  int ops;
   bool fp16;
   int queue;
   unsigned generation;
   LaunchList list;
   mi355_launch_info info;
+  int *tickets = nullptr;  // of `queue`
+  int num_tickets = 0;
+  unsigned tickets_life = 0;
+  void drop_tickets() {
+    if (tickets != nullptr) {
+      give_tickets(queue, tickets, num_tickets, tickets_life);
+      tickets = nullptr;
+    }
+  }
+  ~mi355_prepared() { drop_tickets(); }
 };
+
+// Two fp16 operators as one launch: 1 recorded, 0 not such a pair, < 0 an error.
+static int record_pair(mi355_prepared &p) {
+  DevProgram first, second;
+  FoldRequest fold;
+  if (prepare(&p.op[0].plan, p.op[0].inputs, p.op[0].outputs, true, first) != MI355_OK || first.fused != 1 ||
+      prepare(&p.op[1].plan, p.op[1].inputs, p.op[1].outputs, true, second) != MI355_OK || second.fused != 3 ||
+      !combine_as_rows(second, fold.rows)) {
+    return 0;
+  }
+  fold.tickets = [&](int count) {
+    p.drop_tickets();
+    p.tickets = take_tickets(p.queue, count, p.tickets_life);
+    p.num_tickets = count;
+    return p.tickets;
+  };
+  return try_launch_attention(first, &fold);
+}
 
 static int record_prepared(mi355_prepared &p) {
   p.list.launches.clear();
+  p.drop_tickets();
   p.queue = tls_queue;
   p.generation = options_generation();
   launch_recorder() = &p.list;
-  int const rc = run_plan(&p.plan, p.inputs, p.outputs, p.fp16);
+  int rc = p.ops == 2 && p.fp16 ? record_pair(p) : 0;
+  if (rc == 1) {
+    rc = MI355_OK;
+  } else if (rc == 0) {
+    p.drop_tickets();
+    for (int i = 0; i < p.ops && rc == MI355_OK; i++) {
+      rc = run_plan(&p.op[i].plan, p.op[i].inputs, p.op[i].outputs, p.fp16);
+    }
+  }
   launch_recorder() = nullptr;
   p.info = state().last();
   if (rc != MI355_OK) {
@@ -2002,23 +2043,44 @@ static int record_prepared(mi355_prepared &p) {
   return rc;
 }
 
-extern "C" int mi355_prepare(mi355_plan const *plan, void const *const *inputs, void *const *outputs, int fingerprint,
-                             mi355_prepared **prepared) {
-  MI355_REQUIRE_INIT();
-  if (plan == nullptr || inputs == nullptr || outputs == nullptr || prepared == nullptr ||
-      plan->num_dmem_inputs > MI355_MAX_DMEM_INPUTS || plan->num_dmem_outputs > MI355_MAX_DMEM_OUTPUTS) {
+static int prepare_operators(mi355_plan const *const *plans, void const *const *const *inputs, void *const *const *outputs, int ops,
+                             int fingerprint, mi355_prepared **prepared) {
+  if (prepared == nullptr) {
     return fail(MI355_ERR_INVALID, "bad argument");
   }
   std::unique_ptr<mi355_prepared> p(new mi355_prepared{});
-  p->plan = *plan;
-  std::copy(inputs, inputs + plan->num_dmem_inputs, p->inputs);
-  std::copy(outputs, outputs + plan->num_dmem_outputs, p->outputs);
+  p->ops = ops;
   p->fp16 = fingerprint == 0;
+  for (int i = 0; i < ops; i++) {
+    if (plans[i] == nullptr || inputs[i] == nullptr || outputs[i] == nullptr || plans[i]->num_dmem_inputs > MI355_MAX_DMEM_INPUTS ||
+        plans[i]->num_dmem_outputs > MI355_MAX_DMEM_OUTPUTS) {
+      return fail(MI355_ERR_INVALID, "bad argument");
+    }
+    p->op[i].plan = *plans[i];
+    std::copy(inputs[i], inputs[i] + plans[i]->num_dmem_inputs, p->op[i].inputs);
+    std::copy(outputs[i], outputs[i] + plans[i]->num_dmem_outputs, p->op[i].outputs);
+  }
   if (int rc = record_prepared(*p)) {
     return rc;
   }
   *prepared = p.release();
   return MI355_OK;
+}
+
+extern "C" int mi355_prepare(mi355_plan const *plan, void const *const *inputs, void *const *outputs, int fingerprint,
+                             mi355_prepared **prepared) {
+  MI355_REQUIRE_INIT();
+  return prepare_operators(&plan, &inputs, &outputs, 1, fingerprint, prepared);
+}
+
+extern "C" int mi355_prepare_two(mi355_plan const *first, void const *const *first_inputs, void *const *first_outputs,
+                                 mi355_plan const *second, void const *const *second_inputs, void *const *second_outputs,
+                                 int fingerprint, mi355_prepared **prepared) {
+  MI355_REQUIRE_INIT();
+  mi355_plan const *const plans[] = {first, second};
+  void const *const *const inputs[] = {first_inputs, second_inputs};
+  void *const *const outputs[] = {first_outputs, second_outputs};
+  return prepare_operators(plans, inputs, outputs, 2, fingerprint, prepared);
 }
 
 extern "C" int mi355_prepared_run(mi355_prepared *prepared) {

@@ -8,6 +8,7 @@
 #pragma once
 
 #include "mi355_abi.h"
+#include <functional>
 #include <hip/hip_runtime_api.h>
 #include <cstdint>
 #include <string>
@@ -117,11 +118,28 @@ struct PlanExtents {
 // Fused register-resident kernels for recognised graph shapes (attn_fused.hip).
 // Returns 1 when `prog` was recognised and launched, 0 when it is not of that
 // family, a negative error code on failure.
-int try_launch_attention(DevProgram const &prog);
+// `fold`: the next operator as a fold of this one's rows; the launch then does both, or nothing (0).
+struct FoldRequest;
+int try_launch_attention(DevProgram const &prog, FoldRequest *fold = nullptr);
 bool attention_applicable(DevProgram const &prog);
 int try_launch_gemm(DevProgram const &prog);  // gemm_fused.hip, same convention
 bool gemm_applicable(DevProgram const &prog);
 int try_launch_combine(DevProgram const &prog);  // combine_fused.hip, same convention
+// A fold-and-divide program as what it does to a row: row r of the result, o_cols after the one before, is
+// S pieces of X columns at n + r S X and SD denominators at d + r SD folded (the modes of combine.h), for
+// every r below `rows` once.
+struct RowFold {
+  void const *n, *d;
+  void *o;
+  int S, SD, X, o_cols, mode, rows;
+};
+bool combine_as_rows(DevProgram const &prog, RowFold &R);
+// Whether blocks of `m` rows, one per step of these dimensions, cover rows 0 .. rows - 1 once each.
+bool covers_rows(int m, long long *stride, int *extent, int dims, long long &rows);
+struct FoldRequest {
+  RowFold rows;
+  std::function<int *(int)> tickets;  // zeroed ints that are this launch's own, or null
+};
 bool combine_applicable(DevProgram const &prog);
 int try_launch_fp_combine(DevProgram const &prog);  // the uint16 program of the family, same convention
 

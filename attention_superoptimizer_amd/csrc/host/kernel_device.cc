@@ -385,7 +385,7 @@ void lower_customized(KNCustomizedOp const &op, bool fingerprint, mi355_plan *pl
 // changed the storage orders since): lowering is a few hundred nanoseconds, checking the extents
 // and choosing a kernel several microseconds.  One set per domain and queue: a queue is driven by one thread.
 struct KeptLaunch {
-  LoweredOp lowered;
+  LoweredOp lowered, next;  // next: of two operators
   mi355_prepared *prepared = nullptr;
   ~KeptLaunch() { mi355_prepared_free(prepared); }
 };
@@ -407,6 +407,23 @@ void KNCustomizedOp::launch(bool fingerprint) {
 void KNCustomizedOp::run() {
   require_device("KNCustomizedOp::run");
   launch(false);
+}
+
+void KNCustomizedOp::run_with(KNCustomizedOp &next) {
+  require_device("KNCustomizedOp::run_with");
+  LoweredOp const l = lower_unchecked(*this, false), n = lower_unchecked(next, false);
+  static_assert(sizeof(kept_two) / sizeof(kept_two[0]) == MI355_NUM_QUEUES, "per queue");
+  std::shared_ptr<KeptLaunch> &k = kept_two[mi355_queue_current()];
+  if (k == nullptr || std::memcmp(&k->lowered, &l, sizeof(l)) != 0 || std::memcmp(&k->next, &n, sizeof(n)) != 0) {
+    check_extents(*this, l);
+    check_extents(next, n);
+    k = std::make_shared<KeptLaunch>();
+    k->lowered = l;
+    k->next = n;
+    int const rc = mi355_prepare_two(&l.plan, l.inputs, l.outputs, &n.plan, n.inputs, n.outputs, 0, &k->prepared);
+    MIRAGE_CHECK(rc == MI355_OK, mi355_last_error());
+  }
+  MI355_CALL(mi355_prepared_run(k->prepared));
 }
 
 bool KNCustomizedOp::profile(ProfileResult &result) {
@@ -744,6 +761,22 @@ static bool run_attention_rows(std::vector<KNOperator *> const &ops, size_t i) {
   return taken != 0;
 }
 
+// Customized operators of which the second takes what the first computes, two results (partial numerators
+// and denominators): the backend runs such a pair in one launch where it can.
+static bool run_with_next(KNOperator *op, KNOperator *next) {
+  if (op->op_type != KN_CUSTOMIZED_OP || next->op_type != KN_CUSTOMIZED_OP || op->output_tensors.size() != 2 ||
+      next->input_tensors.size() != 2) {
+    return false;
+  }
+  int const a = next->input_tensors[0].guid, b = next->input_tensors[1].guid;
+  int const x = op->output_tensors[0].guid, y = op->output_tensors[1].guid;
+  if (!((a == x && b == y) || (a == y && b == x))) {
+    return false;
+  }
+  static_cast<KNCustomizedOp *>(op)->run_with(*static_cast<KNCustomizedOp *>(next));
+  return true;
+}
+
 void execute_all(Graph const &graph) {
   require_device("execute_all");
   std::vector<KNOperator *> const &ops = graph.operators;
@@ -759,6 +792,8 @@ void execute_all(Graph const &graph) {
     } else if (softmax_at(i)) {
       run_softmax_rows(ops[i], ops[i + 1], ops[i + 2]);
       i += 3;
+    } else if (i + 1 < n && run_with_next(ops[i], ops[i + 1])) {
+      i += 2;
     } else if (i + 1 < n && !softmax_at(i + 1) && run_matmul_then(ops[i], ops[i + 1])) {
       i += 2;
     } else {

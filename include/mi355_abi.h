@@ -355,6 +355,12 @@ int mi355_customized_run(mi355_plan const *plan, void const *const *inputs,
 typedef struct mi355_prepared mi355_prepared;
 int mi355_prepare(mi355_plan const *plan, void const *const *inputs, void *const *outputs,
                   int fingerprint, mi355_prepared **prepared);
+/* Two operators, the second behind the first: one handle, and one launch where the second folds what the
+ * first computes row by row (partial attention results).  Both operators' outputs are written; the second's
+ * overlap nothing of the first's. */
+int mi355_prepare_two(mi355_plan const *first, void const *const *first_inputs, void *const *first_outputs,
+                      mi355_plan const *second, void const *const *second_inputs, void *const *second_outputs,
+                      int fingerprint, mi355_prepared **prepared);
 int mi355_prepared_run(mi355_prepared *prepared);
 int mi355_prepared_free(mi355_prepared *prepared);
 /* KNCustomizedOp::profile, customized_kernel.cu:615-653: `warmup` untimed then

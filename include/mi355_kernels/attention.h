@@ -12,7 +12,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
+#include "attention_fold.h"
 #include "kernarg.h"
 
 namespace mi355 {
@@ -90,6 +92,53 @@ struct AttnParams {
   // as one block with the whole value tile)
   int r_copies, r_copy_stride;
 };
+// ... and of the kernels that fold as well (attention_fold.h)
+struct AttnFoldParams {
+  AttnParams attn;
+  AttnFold fold;
+};
+__device__ __forceinline__ AttnParams const &attn_part(AttnParams const &A) { return A; }
+__device__ __forceinline__ AttnParams const &attn_part(AttnFoldParams const &A) { return A.attn; }
+static_assert(sizeof(AttnParams) % 8 == 0 && sizeof(AttnFoldParams) == sizeof(AttnParams) + sizeof(AttnFold), "no padding");
+// The fold's parameters, where they are needed: the compiler would otherwise load them at the top and keep them
+// through the loop (16 scalar registers spilled).
+__device__ __forceinline__ AttnFold fold_arguments() {
+  typedef __attribute__((address_space(4))) uint32_t const constant_word;
+  auto *block = (constant_word *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(block));
+  uint32_t words[sizeof(AttnFold) / 4];
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(AttnFold) / 4; i++) {
+    words[i] = block[sizeof(AttnParams) / 4 + i];
+  }
+  AttnFold f;
+  __builtin_memcpy(&f, words, sizeof(f));
+  return f;
+}
+// The end of a kernel: nothing, or the next operator (`rows` rows from `row_base` on are this workgroup's).
+template <class Params>
+__device__ __forceinline__ void fold_part(int bx, int by, int bz, int slice, int row_base, int rows, void *lds) {
+  if constexpr (!std::is_same_v<Params, AttnParams>) {
+    attn_fold(fold_arguments(), bx, by, bz, slice, row_base, rows, lds);
+  }
+}
+template <class Params>
+__device__ __forceinline__ AttnFold next_fold() {
+  if constexpr (!std::is_same_v<Params, AttnParams>) {
+    return fold_arguments();
+  }
+  return AttnFold{};
+}
+// A chunk of eight results that is stored, and the sum of its row (read where it is asked for): folded where the
+// rows are the workgroup's own.
+template <class Params, class Sum>
+__device__ __forceinline__ void fold_chunk(AttnFold const &fold, int bx, int by, int bz, int row, int x, uint4v n, Sum sum) {
+  if constexpr (!std::is_same_v<Params, AttnParams>) {
+    if (fold.tickets == nullptr) {
+      fold_own_chunk(fold, fold_row(fold, bx, by, bz, row), x, n, sum());
+    }
+  }
+}
 
 __device__ __forceinline__ long long tile_offset(TileAddr const &t, int bx, int by, int bz,
                                                  int it) {
@@ -234,9 +283,10 @@ __device__ __forceinline__ constexpr int cm_swizzle_key(int r) {
 
 // RG row groups of 16 query rows, IP wavefronts per row group working on IP
 // consecutive for-loop iterations.
-template <int D, int NK, int DV, bool HAS_DIV, int RG, int IP, bool CM = false>
-__global__ __launch_bounds__(64 * RG * IP) void attn_fused_kernel(AttnParams const P) {
-  fetch_kernel_arguments<sizeof(AttnParams), 3>();  // every line of the block, one trip (decode_block reads gridDim.z)
+template <int D, int NK, int DV, bool HAS_DIV, int RG, int IP, bool CM = false, class Params = AttnParams>
+__global__ __launch_bounds__(64 * RG * IP) void attn_fused_kernel(Params const A) {
+  AttnParams const &P = attn_part(A);
+  fetch_kernel_arguments<sizeof(Params), 3>();  // every line of the block, one trip (decode_block reads gridDim.z)
   constexpr int LDO = DV + 8;
   constexpr int KB = NK / 16, DB = DV / 16, DK = D / 32;
   constexpr int NW = RG * IP, NT = 64 * NW;
@@ -493,6 +543,8 @@ __global__ __launch_bounds__(64 * RG * IP) void attn_fused_kernel(AttnParams con
   }
 
   // ---- store: through LDS so every lane writes a 16-byte row segment ----------------
+  AttnFold const next = next_fold<Params>();
+  bool const shared = next.tickets != nullptr;
   _Float16 *ow = o_stage + rg * 16 * LDO;
   if (ip == 0) {
 #pragma unroll
@@ -502,6 +554,9 @@ __global__ __launch_bounds__(64 * RG * IP) void attn_fused_kernel(AttnParams con
         ow[(4 * g + r) * LDO + 16 * t + c] = oacc[t][r];
       }
     }
+    if (!std::is_same_v<Params, AttnParams> && g == 0) {
+      ow[c * LDO + DV] = racc;  // (behind the row)
+    }
   }
   __syncthreads();
   if (ip == 0) {
@@ -510,15 +565,17 @@ __global__ __launch_bounds__(64 * RG * IP) void attn_fused_kernel(AttnParams con
     constexpr int CH = DV / 8;  // 16-byte chunks per row
     for (int e = lane; e < P.rows * CH; e += 64) {
       int rr = e / CH, cc = (e % CH) * 8;
-      *reinterpret_cast<uint4v *>(og + (long long)rr * P.o.d_cols + cc) =
-          *reinterpret_cast<uint4v const *>(ow + rr * LDO + cc);
+      uint4v const v = *reinterpret_cast<uint4v const *>(ow + rr * LDO + cc);
+      store_result_16(og + (long long)rr * P.o.d_cols + cc, v, shared);
+      fold_chunk<Params>(next, bx, by, bz, row_base + rr, cc, v, [&] { return ow[rr * LDO + DV]; });
     }
     if (!HAS_DIV && g == 0 && c < P.rows) {
       _Float16 *rgp = static_cast<_Float16 *>(const_cast<void *>(P.r.ptr)) +
                       tile_offset(P.r, bx, by, bz, 0);
-      rgp[(long long)(row_base + c) * P.r.d_cols] = racc;
+      store_result_2(rgp + (long long)(row_base + c) * P.r.d_cols, racc, shared);
     }
   }
+  fold_part<Params>(bx, by, bz, slice, slice * RG * 16, RG == 1 ? P.rows : RG * 16, lds);
 }
 
 // Throughput variant for large problems: every wavefront owns RPW row groups of 16
@@ -552,8 +609,9 @@ __device__ __forceinline__ constexpr int stream_swizzle_key(int r) {
 // MSUM (the form without the division): the row sums are one more column block of P.V, against
 // a B operand of ones, instead of a packed dot product and two cross-lane adds per key block on
 // the vector pipe (v_dot2 shares the matrix pipe and stalls it more than the two MFMAs cost).
-template <int D, int NK, int DV, bool HAS_DIV, int RG, int RPW, bool CM = false, int SPI = 1>
-__global__ __launch_bounds__(64 * RG, 2) void attn_stream_kernel(AttnParams const P) {
+template <int D, int NK, int DV, bool HAS_DIV, int RG, int RPW, bool CM = false, int SPI = 1, class Params = AttnParams>
+__global__ __launch_bounds__(64 * RG, 2) void attn_stream_kernel(Params const A) {
+  AttnParams const &P = attn_part(A);
   static_assert(SPI == 1 || !HAS_DIV, "strips of one iteration need the form without the division");
   constexpr bool MSUM = !HAS_DIV;
   constexpr int LDO = DV + 8;
@@ -997,6 +1055,8 @@ __global__ __launch_bounds__(64 * RG, 2) void attn_stream_kernel(AttnParams cons
   }
 
   // ---- store through LDS (the tile buffers are dead) ----------------------------------
+  AttnFold const next = next_fold<Params>();
+  bool const shared = next.tickets != nullptr;
   _Float16 *ow = buf + wave * RPW * 16 * LDO;
 #pragma unroll
   for (int rp = 0; rp < RPW; rp++) {
@@ -1008,6 +1068,15 @@ __global__ __launch_bounds__(64 * RG, 2) void attn_stream_kernel(AttnParams cons
       }
     }
   }
+  auto own_sum = [&](int rp) {  // of row 4 g + c, c < 4: every lane of a group holds the sums of rows 4g .. 4g + 3
+    return c == 0 ? racc[rp][0] : (c == 1 ? racc[rp][MSUM ? 1 : 0] : (c == 2 ? racc[rp][MSUM ? 2 : 0] : racc[rp][MSUM ? 3 : 0]));
+  };
+  if (!std::is_same_v<Params, AttnParams> && c < 4) {
+#pragma unroll
+    for (int rp = 0; rp < RPW; rp++) {
+      ow[(16 * rp + 4 * g + c) * LDO + DV] = own_sum(rp);  // (behind the row)
+    }
+  }
   __syncthreads();
   {
     _Float16 *og = static_cast<_Float16 *>(const_cast<void *>(P.o.ptr)) +
@@ -1015,20 +1084,20 @@ __global__ __launch_bounds__(64 * RG, 2) void attn_stream_kernel(AttnParams cons
     constexpr int CH = DV / 8;
     for (int e2 = lane; e2 < RPW * 16 * CH; e2 += 64) {
       int rr = e2 / CH, cc = (e2 % CH) * 8;
-      *reinterpret_cast<uint4v *>(og + (long long)rr * P.o.d_cols + cc) =
-          *reinterpret_cast<uint4v const *>(ow + rr * LDO + cc);
+      uint4v const v = *reinterpret_cast<uint4v const *>(ow + rr * LDO + cc);
+      store_result_16(og + (long long)rr * P.o.d_cols + cc, v, shared);
+      fold_chunk<Params>(next, bx, by, bz, row_base + rr, cc, v, [&] { return ow[rr * LDO + DV]; });
     }
     if (MSUM && c < 4) {
-      // every lane of a group holds the sums of rows 4g .. 4g + 3: lane c < 4 stores row 4g + c
       _Float16 *rgp = static_cast<_Float16 *>(const_cast<void *>(P.r.ptr)) +
                       tile_offset(P.r, bx, by, bz, 0);
 #pragma unroll
       for (int rp = 0; rp < RPW; rp++) {
-        _Float16 const v = c == 0 ? racc[rp][0] : (c == 1 ? racc[rp][MSUM ? 1 : 0] : (c == 2 ? racc[rp][MSUM ? 2 : 0] : racc[rp][MSUM ? 3 : 0]));
-        rgp[(long long)(row_base + 16 * rp + 4 * g + c) * P.r.d_cols] = v;
+        store_result_2(rgp + (long long)(row_base + 16 * rp + 4 * g + c) * P.r.d_cols, own_sum(rp), shared);
       }
     }
   }
+  fold_part<Params>(bx, by, bz, slice, slice * RG * RPW * 16, RG * RPW * 16, lds);
 }
 
 // Direct-staging variant: one row group of (up to) 16 query rows per workgroup, IP wavefronts
@@ -1076,11 +1145,11 @@ __device__ __forceinline__ void wait_vm() {
 // (IPS == 4) need every block to be 16 consecutive keys: they keep the plain key order and fetch
 // their V^T operand as two 8-byte reads.
 template <int D, int NK, int DV, bool HAS_DIV, int IP, int RPW, int NBUF, int NIT, int SPI, int IPS,
-          bool TRACE, bool CM>
-__global__ __launch_bounds__(64 * IP) void attn_direct_kernel(AttnParams const) {
+          bool TRACE, bool CM, class Params = AttnParams>
+__global__ __launch_bounds__(64 * IP) void attn_direct_kernel(Params const) {
   // (the argument block is read by hand, all of it at once; decode_block reads gridDim.z, so
   // the block counts behind the arguments exist and are fetched with them)
-  AttnParams const P = load_kernel_arguments<AttnParams, 3>();
+  AttnParams const P = load_kernel_arguments<AttnParams, 3, (int)sizeof(Params)>();
   constexpr bool PERM = CM && IPS != 4;  // permuted key order inside pairs of S^T blocks
   static_assert(D == 64 && NK == 64 && DV == 64, "the chunk swizzles assume rows of 128 bytes");
   static_assert((SPI == 1 || IPS == 1) && (SPI == 1 || SPI == 2 || SPI == 4) &&
@@ -1509,9 +1578,9 @@ __global__ __launch_bounds__(64 * IP) void attn_direct_kernel(AttnParams const) 
   if (TRACE) {
     t_joined = __builtin_amdgcn_s_memrealtime();
   }
-  // ---- ordered accumulation: every thread owns EPT consecutive columns of one row; the
-  // slots of up to four iterations are read before their (dependent) adds ---------------
+  // ---- ordered accumulation: every thread owns EPT consecutive columns of one row ---------
   {
+    AttnFold const next = next_fold<Params>();
     // fp16 sums, two per register: adding two fp16 numbers with one packed fp16 add gives their
     // exact sum rounded once, which is what adding in fp32 and rounding to fp16 gives
     half2v acc[EPT / 2];
@@ -1520,37 +1589,85 @@ __global__ __launch_bounds__(64 * IP) void attn_direct_kernel(AttnParams const) 
       acc[e] = half2v{(_Float16)0.0f, (_Float16)0.0f};
     }
     _Float16 const *all = reinterpret_cast<_Float16 const *>(lds) + out_row * LDO + out_col;
-    // iteration `it` is slice it % IPS of unit it / IPS, which wavefront unit % IP kept as its
-    // result number unit / IP
-    auto slot_of = [&](int it) {
-      int const unit = it / IPS;
-      return all + (unit % IP) * WAVE_HALFS + ((unit / IP) * IPS + it % IPS) * SLOT_HALFS;
+    // Iteration `it` is slice it % IPS of unit it / IPS, which wavefront unit % IP kept as its result number unit / IP:
+    // BLOCK iterations in a row have places that differ by constants.  They are read up to eight at a time, wanted or
+    // not (a slot no iteration filled holds whatever the tiles left there: it is read, never added), and added under
+    // one condition where all are wanted.  (A place worked out and a condition for each are a chain of some 30 cycles an
+    // iteration: prefill of 21 heads of 14 row blocks of 32, 14 tiles of 32 keys, 14.9 -> 13.1 us with the fold in both.)
+    constexpr int BLOCK = IP * IPS, BATCH = BLOCK < 8 ? BLOCK : 8;
+    auto in_order = [&](_Float16 const *from, auto &&words, auto &&add) {
+      constexpr int W = std::remove_reference_t<decltype(words)>::value;  // words of four bytes at each place (0: a half)
+#pragma unroll 1
+      for (int j = 0; j < NIT; j++) {
+        int const left = F - j * BLOCK;
+        _Float16 const *const block = from + j * (IPS * SLOT_HALFS);
+#pragma unroll
+        for (int c0 = 0; c0 < BLOCK; c0 += BATCH) {
+          if (c0 >= left) {
+            return;
+          }
+          uint32_t v[BATCH][W > 0 ? W : 1];
+#pragma unroll
+          for (int u = 0; u < BATCH; u++) {
+            _Float16 const *const src = block + (c0 + u) / IPS * WAVE_HALFS + (c0 + u) % IPS * SLOT_HALFS;
+#pragma unroll
+            for (int w = 0; w < W; w++) {
+              v[u][w] = *reinterpret_cast<uint32_t const *>(src + 2 * w);
+            }
+            if (W == 0) {
+              v[u][0] = __builtin_bit_cast(uint16_t, *src);
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < BATCH; u++) {
+#pragma unroll
+            for (int w = 0; w < (W > 0 ? W : 1); w++) {
+              asm volatile("" : "+v"(v[u][w]));  // (not sunk under the conditions, a trip to LDS each)
+            }
+          }
+          if (c0 + BATCH <= left) {
+#pragma unroll
+            for (int u = 0; u < BATCH; u++) {
+              add(v[u]);
+            }
+          } else {
+#pragma unroll
+            for (int u = 0; u < BATCH; u++) {
+              if (c0 + u < left) {
+                add(v[u]);
+              }
+            }
+          }
+        }
+      }
     };
-    // (a slot no iteration filled holds whatever the tiles left there: it is read, never added)
-    constexpr bool ALL = NIT == 1 && IPS == 1;  // one slot per wavefront: read them all at once
-    constexpr int BATCH = ALL ? IP : 4;
-    int const it_end = ALL ? IP : F;
+    if constexpr (NIT == 1 && IPS == 1) {  // one slot per wavefront: read them all at once
+      half2v v[IP][EPT / 2];
 #pragma unroll
-    for (int it0 = 0; it0 < it_end; it0 += BATCH) {
-      half2v v[BATCH][EPT / 2];
-#pragma unroll
-      for (int u = 0; u < BATCH; u++) {
-        _Float16 const *src = slot_of(ALL ? it0 + u : (it0 + u < F ? it0 + u : 0));
+      for (int u = 0; u < IP; u++) {
 #pragma unroll
         for (int e = 0; e < EPT / 2; e++) {
-          v[u][e] = *reinterpret_cast<half2v const *>(src + 2 * e);
+          v[u][e] = *reinterpret_cast<half2v const *>(all + u * WAVE_HALFS + 2 * e);
         }
       }
 #pragma unroll
-      for (int u = 0; u < BATCH; u++) {
-        if (it0 + u < F) {
+      for (int u = 0; u < IP; u++) {
+        if (u < F) {
 #pragma unroll
           for (int e = 0; e < EPT / 2; e++) {
             acc[e] = acc[e] + v[u][e];
           }
         }
       }
+    } else {
+      in_order(all, std::integral_constant<int, EPT / 2>{}, [&](uint32_t const (&v)[EPT / 2]) {
+#pragma unroll
+        for (int e = 0; e < EPT / 2; e++) {
+          acc[e] = acc[e] + __builtin_bit_cast(half2v, v[e]);
+        }
+      });
     }
+    bool const shared = next.tickets != nullptr;
     if (out_row < rows) {
       half2v out[EPT / 2];
 #pragma unroll
@@ -1561,27 +1678,39 @@ __global__ __launch_bounds__(64 * IP) void attn_direct_kernel(AttnParams const) 
         uint4v const w = {__builtin_bit_cast(uint32_t, out[0]), __builtin_bit_cast(uint32_t, out[1]),
                           __builtin_bit_cast(uint32_t, out[(EPT / 2 > 2) ? 2 : 0]),
                           __builtin_bit_cast(uint32_t, out[(EPT / 2 > 3) ? 3 : 0])};
-        *reinterpret_cast<uint4v *>(og) = w;
+        store_result_16(og, w, shared);
       } else if (EPT == 4) {
         uint2v const w = {__builtin_bit_cast(uint32_t, out[0]),
                           __builtin_bit_cast(uint32_t, out[(EPT / 2 > 1) ? 1 : 0])};
-        *reinterpret_cast<uint2v *>(og) = w;
+        store_result_8(og, w, shared);
       } else {
-        *reinterpret_cast<uint32_t *>(og) = __builtin_bit_cast(uint32_t, out[0]);
+        store_result_4(og, __builtin_bit_cast(uint32_t, out[0]), shared);
       }
     }
-    if (!HAS_DIV && tid < rows) {
-      _Float16 const *sums = reinterpret_cast<_Float16 const *>(lds) + ROWS * LDO + tid;
-      float ra = 0.0f;
-      for (int it = 0; it < F; it++) {
-        int const unit = it / IPS;
-        _Float16 const v = sums[(unit % IP) * WAVE_HALFS + ((unit / IP) * IPS + it % IPS) * SLOT_HALFS];
-        ra = static_cast<float>(static_cast<_Float16>(ra + static_cast<float>(v)));
+    auto total = [&](int row) {  // the sum of a row, in iteration order
+      _Float16 sum = (_Float16)0.0f;
+      in_order(reinterpret_cast<_Float16 const *>(lds) + ROWS * LDO + row, std::integral_constant<int, 0>{},
+               [&](uint32_t const (&v)[1]) { sum = sum + __builtin_bit_cast(_Float16, (uint16_t)v[0]); });
+      return sum;
+    };
+    _Float16 *const rgp = static_cast<_Float16 *>(const_cast<void *>(P.r.ptr)) + tile_offset(P.r, bx, by, bz, 0);
+    bool const own = !std::is_same_v<Params, AttnParams> && !shared;  // whole rows: the next operator's, from the same registers
+    if (own && out_row < rows) {
+      _Float16 const sum = total(out_row);
+      _Float16 *const to = next.o + fold_row(next, bx, by, bz, row_base + out_row) * next.o_cols + out_col;
+#pragma unroll
+      for (int e = 0; e < EPT / 2; e++) {
+        half2v const q = {fold_own(acc[e][0], sum), fold_own(acc[e][1], sum)};
+        store_result_4(to + 2 * e, __builtin_bit_cast(uint32_t, q), false);
       }
-      _Float16 *rgp = static_cast<_Float16 *>(const_cast<void *>(P.r.ptr)) +
-                      tile_offset(P.r, bx, by, bz, 0);
+      if (out_col == 0) {
+        store_result_2(rgp + (long long)(row_base + out_row) * P.r.d_cols, sum, false);
+      }
+    }
+    if (!HAS_DIV && !own && tid < rows) {
+      _Float16 const ra = total(tid);
       for (int c = 0; c < P.r_copies; c++) {
-        rgp[(long long)(row_base + tid) * P.r.d_cols + c * P.r_copy_stride] = static_cast<_Float16>(ra);
+        store_result_2(rgp + (long long)(row_base + tid) * P.r.d_cols + c * P.r_copy_stride, ra, shared);
       }
     }
   }
@@ -1596,6 +1725,7 @@ __global__ __launch_bounds__(64 * IP) void attn_direct_kernel(AttnParams const) 
     t[4] = t_joined;
     t[5] = __builtin_amdgcn_s_memrealtime();
   }
+  fold_part<Params>(bx, by, bz, slice, row_base, rows, lds);
 }
 
 }  // namespace mi355

@@ -56,12 +56,11 @@ constexpr int attn_tiles_lds(int D, int RPW, int ip, int rounds) {
 // 5.59 and 5.04; tiles of 80 keys, column-major, 10.87 and 9.72.  (Without strips, each
 // load straight to its operand: 3.25, 4.20 and 14.42; a lone block is worked on here as half of a pair.)
 typedef __attribute__((address_space(1))) uint4v global_chunk;
-typedef __attribute__((address_space(1))) _Float16 global_half;
 
-template <int D, bool HAS_DIV, bool CM, int RPW, int PAIRS>
+template <int D, bool HAS_DIV, bool CM, int RPW, int PAIRS, class Params = AttnParams>
 __global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
-    __attribute__((amdgpu_waves_per_eu(attn_tiles_lanes(D, PAIRS) == 8 ? 4 : 1))) void attn_tiles_kernel(AttnParams const) {
-  AttnParams const P = load_kernel_arguments<AttnParams, 4>();  // (blockDim.x is read)
+    __attribute__((amdgpu_waves_per_eu(attn_tiles_lanes(D, PAIRS) == 8 ? 4 : 1))) void attn_tiles_kernel(Params const) {
+  AttnParams const P = load_kernel_arguments<AttnParams, 4, (int)sizeof(Params)>();  // (blockDim.x is read)
   constexpr int DB = D / 16, DK = D / 32, ROWS = 16 * RPW, LD = D + 8, KLD = 40;  // pitches of rows of D and of keys
   constexpr int CPR = D / 8;                // 16-byte chunks of a row
   constexpr int CHUNKS = D / 16, KEYS = 64 / CPR;  // chunks a lane holds of a pair; keys per chunk of a wavefront
@@ -304,6 +303,15 @@ __global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
     int const n = (F - r0) < IP ? (F - r0) : IP;
     bool const first = r0 == 0, done = r0 + IP >= F;
     _Float16 *const og = static_cast<_Float16 *>(const_cast<void *>(P.o.ptr)) + tile_offset(P.o, bx, by, bz, 0);
+    AttnFold const next = done ? next_fold<Params>() : AttnFold{};
+    bool const shared = next.tickets != nullptr;
+    auto total = [&](int r) {  // the row's sum, of this round's and those before
+      _Float16 sum = first ? (_Float16)0.0f : sums[ROWS * LD + r];
+      for (int u = 0; u < n; u++) {
+        sum = sum + all[u * STRIP + ROWS * LD + r];
+      }
+      return sum;
+    };
     for (int e = tid; e < ROWS * CPR; e += NT) {
       int const r = e / CPR, at = r * LD + 8 * (e % CPR), row = row_base + r;
       uint4v sum = {0, 0, 0, 0};
@@ -321,19 +329,17 @@ __global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
       if (!done) {
         *reinterpret_cast<uint4v *>(sums + at) = sum;
       } else if (row < m) {
-        *(global_chunk *)(og + (long long)row * P.o.d_cols + 8 * (e % CPR)) = sum;
+        store_result_16(og + (long long)row * P.o.d_cols + 8 * (e % CPR), sum, shared);
+        fold_chunk<Params>(next, bx, by, bz, row, 8 * (e % CPR), sum, [&] { return total(r); });
       }
     }
     if (!HAS_DIV && tid < ROWS) {
-      _Float16 sum = first ? (_Float16)0.0f : sums[ROWS * LD + tid];
-      for (int u = 0; u < n; u++) {
-        sum = sum + all[u * STRIP + ROWS * LD + tid];
-      }
+      _Float16 const sum = total(tid);
       if (!done) {
         sums[ROWS * LD + tid] = sum;
       } else if (row_base + tid < m) {
         _Float16 *const rg = static_cast<_Float16 *>(const_cast<void *>(P.r.ptr)) + tile_offset(P.r, bx, by, bz, 0);
-        *(global_half *)(rg + (long long)(row_base + tid) * P.r.d_cols) = sum;
+        store_result_2(rg + (long long)(row_base + tid) * P.r.d_cols, sum, shared);
       }
     }
     if (!done) {
@@ -431,6 +437,7 @@ __global__ __launch_bounds__(attn_tiles_lanes(D, PAIRS) * 64)
       }
     }
   }
+  fold_part<Params>(bx, by, bz, slice, row_base, m - row_base < ROWS ? m - row_base : ROWS, lds);
 }
 
 }  // namespace mi355

@@ -23,6 +23,7 @@ public:
   virtual ~KNCustomizedOp();
   bool profile(ProfileResult &profile) override;
   void run(void);  // one fp16 launch on the backend stream, no synchronisation
+  void run_with(KNCustomizedOp &next);  // run(), next.run()
   bool fingerprint(void) override;
   operator json() const override;  // adds bgraph and plan (src/kernel/customized.cc:315-321)
 
@@ -33,6 +34,7 @@ private:
   // the kernel launches of run() [0] and fingerprint() [1] per backend queue, kept from one call
   // to the next
   std::shared_ptr<KeptLaunch> kept[2][4];
+  std::shared_ptr<KeptLaunch> kept_two[4];  // of run() and the next operator's together (execute_all)
   void launch(bool fingerprint);
   void add_output(mirage::threadblock::STensor const &stensor, int3 output_map);
 };
