@@ -455,7 +455,10 @@ double stream_ns(DevProgram const &P, GMatch const &G, StreamPlan const &plan, l
   return ns;
 }
 
-int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) {
+// `gate`: see GateRequest; *gated tells whether the launch takes care of it.  `R`: the program as the choice sees it, G but
+// for a row-major second operator of such a pair, which runs where it would run by itself: without its prologue no
+// kernel is slower than with it (2 rows x 576 x 6528 14.8 us before and so, 16.8 in the kernel of a plain product).
+int try_launch_lanes(DevProgram const &P, GMatch const &G, GMatch const &R, GemmParams const &A, _Float16 *gate, bool *gated) {
   State &s = state();
   // lora A comes in 16-rank pieces, the last one half full where its columns are rows in memory; two weights in
   // tiles of 64 columns and whole 64-k units only (programs printed for others are known to hold the tiles' kernel)
@@ -534,7 +537,7 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   long long const units = (long long)F * G.KT / 64;
   // (In 256-k iterations a piece's loads are waited for together: 8 x 4096 x 4096 column-major 12.0 / 11.4.  One range
   // of the other kernel has neither the slab nor its launch: 8 rows x 10112 x 768 9.3 / 5.8, 14336 x 832 12.7 / 6.2.)
-  StreamPlan const plan = G.whole && G.KT % 64 == 0 ? stream_plan(P, G) : StreamPlan{};
+  StreamPlan const plan = G.whole && G.KT % 64 == 0 ? stream_plan(P, R) : StreamPlan{};
   long long const here_ns = (1000 + (!G.wcm ? 225 : G.KT == 256 ? 185 : 142) * units) * ((blocks * S + 255) / 256);
   long long const there_ns = plan.ranges == 1 ? 4000 + blocks * units : 7000 + blocks * units + blocks * F * 7 / 10 + 15 * F;
   // Other tiles run on the any-size kernel or, in 96-k iterations of 64 columns, on the one with a barrier a step:
@@ -546,16 +549,16 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   bool there;
   if (G.whole && G.KT % 64 == 0) {
     there = blocks * S > (G.wcm ? 4096 : 1024) || weight_bytes > (most_mb << 20);
-    if (G.pro == PRO_SILU_MUL && G.M <= 16) {
+    if (R.pro == PRO_SILU_MUL && G.M <= 16) {
       there = units > 104 || here_ns > there_ns;
     }
-    if (plan.ranges > 0 && (G.pro != PRO_SILU_MUL || (G.wcm && plan.ranges == 1 && blocks * S > 256))) {
-      there = there || lanes_chain_ns(G, units, F, ip, lds, blocks * S) > stream_ns(P, G, plan, weight_bytes);
+    if (plan.ranges > 0 && (R.pro != PRO_SILU_MUL || (G.wcm && plan.ranges == 1 && blocks * S > 256))) {
+      there = there || lanes_chain_ns(R, units, F, ip, lds, blocks * S) > stream_ns(P, R, plan, weight_bytes);
     }
     // Row-major, the other kernel's whole blocks on more than half of the chip, and a prologue that is not done again
     // for every 16 columns (us, here / there: silu of 4 rows x 12416 x 640 7.6 / 6.5, lora 8576 x 768 7.5 / 6.4,
     // two weights of 8 x 13824 x 256 6.7 / 5.8).
-    if (!G.wcm && plan.ranges == 1 && blocks >= 128 && (G.pro != PRO_NONE || G.lora || G.nb == 2)) {
+    if (!G.wcm && plan.ranges == 1 && blocks >= 128 && (R.pro != PRO_NONE || G.lora || G.nb == 2)) {
       there = true;
     }
   } else if (G.wcm) {
@@ -577,6 +580,8 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
   L.pieces = pieces;
   L.rank = G.rank;
   L.slot_base = ip * wave_bytes;
+  L.g.gate = gate;
+  *gated = gate != nullptr;
   L.m_group = fast_div_magic(8 * S);
   L.m_pieces = fast_div_magic(S);
   L.m_columns = fast_div_magic(pieces);
@@ -611,7 +616,8 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GemmParams const &A) 
 int launch_combine(GemmParams const &A, int nb, dim3 blocks) {
   State &s = state();
   int const lds = A.forloop_range * 1024;
-  dim3 const fold_grid(blocks.x * nb * ((A.M + 7) / 8), blocks.y, blocks.z);
+  int const sets = A.gate != nullptr ? 2 : 1;  // weights of a workgroup
+  dim3 const fold_grid(blocks.x * (nb / sets) * ((A.M + 7) / 8), blocks.y, blocks.z);
   if (EmitSink *sink = emit_sink()) {
     bool const fold = lds <= s.max_lds;
     emit_launch(*sink, fold ? "gemm_fold_kernel" : "gemm_combine_kernel", emit_fmt("%d", nb), fold ? fold_grid : blocks, 256,
@@ -623,8 +629,8 @@ int launch_combine(GemmParams const &A, int nb, dim3 blocks) {
     return 1;
   }
   auto *fn = nb == 1 ? gemm_fold_kernel<1> : gemm_fold_kernel<2>;
-  MI355_GRANT_LDS(fn, lds);
-  MI355_HIP(launch_kernel(fn, fold_grid, 256, lds, s.stream(), A));
+  MI355_GRANT_LDS(fn, lds * sets);
+  MI355_HIP(launch_kernel(fn, fold_grid, 256 * sets, lds * sets, s.stream(), A));
   return 1;
 }
 
@@ -655,7 +661,7 @@ int launch_stream_pairs(StreamParams const &L, dim3 grid, int lds) {
 }
 
 // gemm_stream_kernel for this plan, or 0.
-int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A) {
+int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A, _Float16 *gate, bool *gated) {
   State &s = state();
   StreamPlan const plan = stream_plan(P, G);
   if (plan.ranges == 0 || (long long)P.grid[0] * plan.groups > 2147483647LL) {
@@ -672,6 +678,9 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A)
   }
   L.results = plan.ring;
   L.strips = plan.strips;
+  // (whole blocks of one weight meet in no workgroup, and no more do sums past the fold's LDS)
+  *gated = gate != nullptr && (plan.strips || (ks == 1 ? plan.pairs : P.forloop_range * 2048 <= s.max_lds));
+  L.g.gate = *gated ? gate : nullptr;
   dim3 const grid(P.grid[0] * plan.groups, P.grid[1], P.grid[2]);
   int rc = 0;
   if (plan.pairs) {
@@ -717,17 +726,73 @@ bool gemm_applicable(DevProgram const &P) {
   return gmatch(P, G);
 }
 
-int try_launch_gemm(DevProgram const &P) {
+// A gated MLP's operators: the first makes G and U, the second multiplies silu(G) * U.  Every block of columns of the
+// second, and in the one-launch kernel every 16 of them, makes that product of 16 x k values again, a chain of an
+// exponential, a reciprocal and a dozen instructions for each; where the first's kernel has both sums in a workgroup
+// it makes it once, into the queue's memory for operand copies, and the second is a plain product.  (G and U are
+// written as before.)  8 x 4096 x 14336, column-major: both 71.9 -> 68.0 us; 100 drawn gated MLPs 0.87 of the time in the
+// mean, 0.70 - 1.01.  A launch of its own for the product takes back what it gives (us, separate operators / with it, row-major:
+// 16 rows x 2496 x 5952 39.4 / 40.1, 8 x 1088 x 4288 17.6 / 19.1).
+// For-loops past what the fold keeps in LDS stay: the second's plain product then takes the one-launch kernel, where
+// result slots leave half the wavefronts (8 rows x 1408 x 14272 in 64-k iterations 19.6 us in ranges, 25.9 there).
+bool gate_pair(DevProgram const &first, DevProgram const &second, GateRequest &R) {
+  GMatch A, B;
+  if (!gmatch(first, A) || !gmatch(second, B) || A.nb != 2 || B.pro != PRO_SILU_MUL || A.M != B.M ||
+      second.forloop_range * 1024 > state().max_lds) {
+    return false;
+  }
+  DevOp const &o0 = first.ops[A.o0], &o1 = first.ops[A.o1], &g = second.ops[B.a0], &u = second.ops[B.a1];
+  if (first.out[o0.io] != second.in[g.io] || first.out[o1.io] != second.in[u.io]) {
+    return false;
+  }
+  // the first makes all of [M][columns] side by side, the second reads all of it iteration by iteration
+  int const columns = o0.d_cols;
+  int pieces = 1;
+  for (int i = 0; i < 3; i++) {
+    if (first.grid[i] > 1) {
+      if (o0.row_bs[i] != 0 || o0.g_bs[i] != 0 || o0.col_bs[i] != A.NC || o1.row_bs[i] != 0 || o1.g_bs[i] != 0 || o1.col_bs[i] != A.NC) {
+        return false;
+      }
+      pieces *= first.grid[i];
+    }
+    if (second.grid[i] > 1 && (g.row_bs[i] || g.col_bs[i] || g.g_bs[i] || u.row_bs[i] || u.col_bs[i] || u.g_bs[i])) {
+      return false;
+    }
+  }
+  int dims = (first.grid[0] > 1) + (first.grid[1] > 1) + (first.grid[2] > 1);
+  bool const walks = second.forloop_range == 1 || (g.col_fs == B.KT && g.row_fs == 0 && g.g_fs == 0 && u.col_fs == B.KT && u.row_fs == 0 && u.g_fs == 0);
+  if (dims > 1 || pieces * A.NC != columns || o1.d_cols != columns || g.d_cols != columns || u.d_cols != columns || !walks ||
+      second.forloop_range * B.KT != columns) {
+    return false;
+  }
+  R.elements = (size_t)A.M * columns;
+  return true;
+}
+
+int try_launch_gemm(DevProgram const &P, GateRequest *request, bool second) {
   GMatch G;
   if (!gmatch(P, G)) {
     return 0;
   }
   State &s = state();
+  _Float16 *const made = request != nullptr ? static_cast<_Float16 *>(request->h) : nullptr, *const gate = second ? nullptr : made;
+  bool gated = false;
+  GMatch by_itself = G;
+  if (second) {
+    G.pro = PRO_NONE;
+    G.a1 = -1;
+    if (G.wcm) {  // (column-major strips in one launch are what its prologue kept it from: 16 rows x 1408 x 6400 23.1 -> 16.8 us)
+      by_itself = G;
+    }
+  }
   GemmParams A{};
   int const extents[4] = {P.grid[0], P.grid[1], P.grid[2], P.forloop_range};
   bool fits = true;
   auto in_tile = [&](int i) { return gtile(P.ops[i], P.in[P.ops[i].io], extents, fits); };
   A.a0 = in_tile(G.a0);
+  if (second) {
+    A.a0.ptr = made;
+  }
   A.a1 = G.a1 >= 0 ? in_tile(G.a1) : A.a0;
   A.b0 = in_tile(G.b0);
   A.b1 = G.b1 >= 0 ? in_tile(G.b1) : A.b0;
@@ -741,14 +806,15 @@ int try_launch_gemm(DevProgram const &P) {
   A.M = G.M;
   A.KT = G.KT;
   A.forloop_range = P.forloop_range;
-  if (int const rc = try_launch_lanes(P, G, A)) {
-    return rc;
+  auto with_gate = [&](int rc) -> int { return rc == 1 && gate != nullptr && !gated ? 0 : rc; };
+  if (int const rc = try_launch_lanes(P, G, by_itself, A, gate, &gated)) {
+    return with_gate(rc);
   }
-  if (int const rc = try_launch_stream(P, G, A)) {
-    return rc;
+  if (int const rc = try_launch_stream(P, G, A, gate, &gated)) {
+    return with_gate(rc);
   }
   if (!G.whole || s.any_size_kernels) {
-    return launch_gemm_tiles(A, TileGemmPlan{{P.grid[0], P.grid[1], P.grid[2]}, G.pro, G.nb, G.rank, G.NC, G.wcm});
+    return with_gate(launch_gemm_tiles(A, TileGemmPlan{{P.grid[0], P.grid[1], P.grid[2]}, G.pro, G.nb, G.rank, G.NC, G.wcm}));
   }
   int const mt = G.M <= 16 ? 1 : (G.M <= 32 ? 2 : 4);
   long long const blocks = (long long)P.grid[0] * P.grid[1] * P.grid[2];
@@ -816,7 +882,7 @@ int try_launch_gemm(DevProgram const &P) {
     s.last().lds_bytes = lds;
     s.last().row_split = ksplit;
   }
-  return rc;
+  return with_gate(rc);
 }
 
 }  // namespace mi355

@@ -2002,22 +2002,38 @@ struct mi355_prepared {
   ~mi355_prepared() { drop_tickets(); }
 };
 
-// Two fp16 operators as one launch: 1 recorded, 0 not such a pair, < 0 an error.
+// Two fp16 operators that share work: 1 recorded, 0 not such a pair, < 0 an error.
 static int record_pair(mi355_prepared &p) {
   DevProgram first, second;
-  FoldRequest fold;
-  if (prepare(&p.op[0].plan, p.op[0].inputs, p.op[0].outputs, true, first) != MI355_OK || first.fused != 1 ||
-      prepare(&p.op[1].plan, p.op[1].inputs, p.op[1].outputs, true, second) != MI355_OK || second.fused != 3 ||
-      !combine_as_rows(second, fold.rows)) {
+  if (prepare(&p.op[0].plan, p.op[0].inputs, p.op[0].outputs, true, first) != MI355_OK ||
+      prepare(&p.op[1].plan, p.op[1].inputs, p.op[1].outputs, true, second) != MI355_OK) {
     return 0;
   }
-  fold.tickets = [&](int count) {
-    p.drop_tickets();
-    p.tickets = take_tickets(p.queue, count, p.tickets_life);
-    p.num_tickets = count;
-    return p.tickets;
-  };
-  return try_launch_attention(first, &fold);
+  FoldRequest fold;
+  if (first.fused == 1 && second.fused == 3 && combine_as_rows(second, fold.rows)) {
+    fold.tickets = [&](int count) {
+      p.drop_tickets();
+      p.tickets = take_tickets(p.queue, count, p.tickets_life);
+      p.num_tickets = count;
+      return p.tickets;
+    };
+    return try_launch_attention(first, &fold);
+  }
+  GateRequest gate;
+  if (first.fused == 2 && second.fused == 2 && gate_pair(first, second, gate)) {
+    // (in the queue's memory for operand copies: work of one queue is ordered)
+    if (state().planes() == nullptr || gate.elements * 2 > state().planes_bytes) {
+      return 0;
+    }
+    gate.h = state().planes();
+    int rc = try_launch_gemm(first, &gate, false);
+    rc = rc == 1 ? try_launch_gemm(second, &gate, true) : rc;
+    if (rc == 0) {
+      p.list.launches.clear();  // (what one of them recorded is not repeated)
+    }
+    return rc;
+  }
+  return 0;
 }
 
 static int record_prepared(mi355_prepared &p) {

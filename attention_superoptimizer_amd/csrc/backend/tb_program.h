@@ -122,7 +122,14 @@ struct PlanExtents {
 struct FoldRequest;
 int try_launch_attention(DevProgram const &prog, FoldRequest *fold = nullptr);
 bool attention_applicable(DevProgram const &prog);
-int try_launch_gemm(DevProgram const &prog);  // gemm_fused.hip, same convention
+// gemm_fused.hip, same convention.  `gate`: the program is the first (two weights) or the second (SiLU(a) * u of
+// the first's results) operator of a pair, whose first one leaves SiLU(a) * u in `h`, the second's activations.
+struct GateRequest {
+  void *h = nullptr;
+  size_t elements;  // of each of the first's results
+};
+bool gate_pair(DevProgram const &first, DevProgram const &second, GateRequest &R);
+int try_launch_gemm(DevProgram const &prog, GateRequest *gate = nullptr, bool second = false);
 bool gemm_applicable(DevProgram const &prog);
 int try_launch_combine(DevProgram const &prog);  // combine_fused.hip, same convention
 // A fold-and-divide program as what it does to a row: row r of the result, o_cols after the one before, is

@@ -761,17 +761,20 @@ static bool run_attention_rows(std::vector<KNOperator *> const &ops, size_t i) {
   return taken != 0;
 }
 
-// Customized operators of which the second takes what the first computes, two results (partial numerators
-// and denominators): the backend runs such a pair in one launch where it can.
+// Customized operators of which the second takes both results of the first (partial numerators and
+// denominators, a gated MLP's two products): the backend has such pairs share work where it can.
 static bool run_with_next(KNOperator *op, KNOperator *next) {
-  if (op->op_type != KN_CUSTOMIZED_OP || next->op_type != KN_CUSTOMIZED_OP || op->output_tensors.size() != 2 ||
-      next->input_tensors.size() != 2) {
+  if (op->op_type != KN_CUSTOMIZED_OP || next->op_type != KN_CUSTOMIZED_OP || op->output_tensors.size() != 2) {
     return false;
   }
-  int const a = next->input_tensors[0].guid, b = next->input_tensors[1].guid;
-  int const x = op->output_tensors[0].guid, y = op->output_tensors[1].guid;
-  if (!((a == x && b == y) || (a == y && b == x))) {
-    return false;
+  for (DTensor const &out : op->output_tensors) {
+    bool taken = false;
+    for (DTensor const &in : next->input_tensors) {
+      taken = taken || in.guid == out.guid;
+    }
+    if (!taken) {
+      return false;
+    }
   }
   static_cast<KNCustomizedOp *>(op)->run_with(*static_cast<KNCustomizedOp *>(next));
   return true;

@@ -43,6 +43,7 @@ struct GemmParams {
   int forloop_range;
   int ksplit;        // workgroups per logical block
   _Float16 *scratch; // [blocks][forloop_range][NB][M][64] fp16 product tiles (ksplit > 1)
+  _Float16 *gate;    // two weights: where silu(first) * second goes as well, in the places of the first result; or null
 };
 
 __device__ __forceinline__ long long gtile_offset(GTile const &t, int bx, int by, int bz, int it) {
@@ -63,6 +64,12 @@ __device__ __forceinline__ float prologue(int pro, float x) {
   // them.  Half the instructions of the full division, and for every fp16 x its result.
   float const d = 1.0f + __expf(-x), r = __builtin_amdgcn_rcpf(d), q = x * r;
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, x), r, q), d, x);
+}
+
+// The prologue silu(g) * u, with the roundings of the operators it is made of.
+__device__ __forceinline__ _Float16 gate_value(_Float16 g, _Float16 u) {
+  _Float16 const silu = static_cast<_Float16>(prologue(PRO_SILU, static_cast<float>(g)));
+  return static_cast<_Float16>(static_cast<float>(silu) * static_cast<float>(u));
 }
 
 // Transposing stage of a [R][C] tile (C contiguous, row stride ld) into dst[C][R]
@@ -536,18 +543,21 @@ __global__ __launch_bounds__(256) void gemm_combine_kernel(GemmParams const P) {
 // together into LDS, then added in order from there, so that the only trip to memory is one latency
 // long (61 rows, 20 iterations, 40 blocks: 22.1 -> 14.6 us for the plan; no slower at 8 rows).
 template <int NB>
-__global__ __launch_bounds__(256) void gemm_fold_kernel(GemmParams const P) {
+__global__ __launch_bounds__(256 * NB) void gemm_fold_kernel(GemmParams const P) {
   fetch_kernel_arguments<sizeof(GemmParams), 2>();  // (gridDim.x, .y are read)
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // [F][8][64] fp16
   typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-  int const tid = threadIdx.x, lane = tid % 64, wave = tid / 64, M = P.M, F = P.forloop_range;
-  int const groups = (M + 7) / 8, per_block = groups * NB;
+  int const tid = threadIdx.x % 256, lane = tid % 64, wave = tid / 64, M = P.M, F = P.forloop_range;
+  // with a gate a workgroup is twice as many threads and has both weights
+  int const sets = NB == 2 && P.gate != nullptr ? 2 : 1, set = threadIdx.x / 256;
+  int const groups = (M + 7) / 8, per_block = groups * (NB / sets);
   int const bx = blockIdx.x / per_block, by = blockIdx.y, bz = blockIdx.z;
-  int const part = blockIdx.x % per_block, b = part / groups, row0 = 8 * (part % groups);
+  int const part = blockIdx.x % per_block, b = sets == 2 ? set : part / groups, row0 = 8 * (part % groups);
   int const block_linear = bx + (gridDim.x / per_block) * (by + gridDim.y * bz);
   long long const slab = (long long)NB * M * 64;  // one iteration's tiles
   int const row = row0 + lane / 8 < M ? row0 + lane / 8 : M - 1;
   _Float16 const *src = P.scratch + (long long)block_linear * F * slab + (long long)b * M * 64 + row * 64 + 8 * (lane % 8);
+  unsigned char *const mine = lds + set * F * 1024;
   for (int it = wave; it < F; it += 16) {
     uint4v v[4];
 #pragma unroll
@@ -559,7 +569,7 @@ __global__ __launch_bounds__(256) void gemm_fold_kernel(GemmParams const P) {
 #pragma unroll
     for (int u = 0; u < 4; u++) {
       if (it + 4 * u < F) {
-        *reinterpret_cast<uint4v *>(lds + (it + 4 * u) * 1024 + 16 * lane) = v[u];
+        *reinterpret_cast<uint4v *>(mine + (it + 4 * u) * 1024 + 16 * lane) = v[u];
       }
     }
   }
@@ -568,12 +578,24 @@ __global__ __launch_bounds__(256) void gemm_fold_kernel(GemmParams const P) {
   half2v a = {(_Float16)0.0f, (_Float16)0.0f};
 #pragma unroll 8
   for (int it = 0; it < F; it++) {  // (a packed fp16 add is the exact sum rounded once)
-    a += *reinterpret_cast<half2v const *>(lds + it * 1024 + 128 * r + 2 * col);
+    a += *reinterpret_cast<half2v const *>(mine + it * 1024 + 128 * r + 2 * col);
   }
   if (row0 + r < M) {
     GTile const &ot = b == 0 ? P.o0 : P.o1;
     _Float16 *og = static_cast<_Float16 *>(const_cast<void *>(ot.ptr)) + gtile_offset(ot, bx, by, bz, 0);
     *reinterpret_cast<half2v *>(og + (long long)(row0 + r) * ot.d_cols + col) = a;
+  }
+  if (sets == 2) {
+    half2v *const other = reinterpret_cast<half2v *>(lds + F * 1024 + 128 * r + 2 * col);  // (the second set's, which only its thread has read)
+    if (set == 1) {
+      *other = a;
+    }
+    __syncthreads();
+    if (set == 0 && row0 + r < M) {
+      half2v const u = *other;
+      *reinterpret_cast<half2v *>(P.gate + gtile_offset(P.o0, bx, by, bz, 0) + (long long)(row0 + r) * P.o0.d_cols + col) =
+          half2v{gate_value(a[0], u[0]), gate_value(a[1], u[1])};
+    }
   }
 }
 
@@ -927,6 +949,20 @@ __global__ __launch_bounds__(64 * lanes_most(KT, LORA)) void gemm_lanes_kernel(L
       out[0] = static_cast<_Float16>(a0);
       out[1] = static_cast<_Float16>(a1);
       *reinterpret_cast<half2v *>(og + (long long)(16 * mt + r) * ot.d_cols + n0 + col) = out;
+    }
+    if (NB == 2 && P.gate != nullptr) {
+      *reinterpret_cast<half2v *>(slots + (b * 16 + r) * 16 + col) = half2v{(_Float16)a0, (_Float16)a1};  // (its own slot, which only it has read)
+    }
+  }
+  if (NB == 2 && P.gate != nullptr) {
+    __syncthreads();
+    _Float16 *const to = P.gate + gtile_offset(P.o0, bx, by, bz, 0);
+    for (int e = tid; e < 128; e += blockDim.x) {
+      int const r = e / 8, col = (e % 8) * 2;
+      half2v const x = *reinterpret_cast<half2v const *>(slots + r * 16 + col), u = *reinterpret_cast<half2v const *>(slots + (16 + r) * 16 + col);
+      if (16 * mt + r < M) {
+        *reinterpret_cast<half2v *>(to + (long long)(16 * mt + r) * P.o0.d_cols + n0 + col) = half2v{gate_value(x[0], u[0]), gate_value(x[1], u[1])};
+      }
     }
   }
 }
