@@ -292,6 +292,7 @@ int launch_kt(GemmParams const &A, dim3 grid, int lds) {
 struct StreamPlan {
   int ranges = 0;       // 0: not at all
   bool strips = false;  // 16 columns a workgroup
+  bool lone = false;    // of those, in one workgroup a compute unit at most
   bool pairs = false;   // both of two weights
   int mt = 0;           // 16-row groups
   int ring = 0, lds = 0, groups = 0;  // bytes of the slots, of LDS; workgroups of a block
@@ -316,10 +317,21 @@ StreamPlan stream_plan(DevProgram const &P, GMatch const &G) {
   // / ranges: 3840 columns x 4096, 240 workgroups, 7.6 / 10.7; 28672 39.9 / 51.6; two weights of 3072 x 8192
   // with a gated MLP's second product 37.9 / 40.1), but not where one weight's whole blocks fill it as well (below:
   // 4 rows x 12416 x 1536 9.7 / 8.0, 16 x 14656 x 1792 13.6 / 11.4, but 16 x 7360 x 1280, 115 blocks, 6.1 / 6.8).
-  int const eights = G.M <= 8 ? 1 : 2, strip_ring = 4 * columns_ring(eights) * columns_slot_bytes(eights);
+  int const eights = G.M <= 8 ? 1 : 2, strip_ring = 4 * columns_ring(eights, G.lora) * columns_slot_bytes(eights, G.lora);
   int const strip_lds = strip_ring + F * G.M * 32;
-  bool const strips = G.wcm && G.pro == PRO_NONE && !G.lora && G.M <= 16 && 4 * G.nb * blocks >= 192 && 2 * strip_lds <= s.max_lds &&
-                      !(G.nb == 1 && fits && blocks >= 192 && steps <= 8);
+  bool const narrow = G.wcm && G.pro == PRO_NONE && G.M <= 16;
+  bool strips = narrow && !G.lora && 4 * G.nb * blocks >= 192 && 2 * strip_lds <= s.max_lds && !(G.nb == 1 && fits && blocks >= 192 && steps <= 8);
+  // In 256-k iterations a 16-column strip asks for enough at a time that one workgroup a compute unit keeps up with
+  // memory, and one launch without a slab is ahead of both other kernels (us, the others / strips: LoRA 4096 columns x
+  // 4096 of 8 rows 10.9 / 8.0, x 1024 4.1 / 3.6, 3072 x 4096 8.2 / 7.2; one product of 16 rows 4096 x 8192 14.3 / 11.9,
+  // x 14336 26.6 / 24.9, 3072 x 4096 7.0 / 6.3), but not with fewer workgroups (LoRA of 2048 x 2048 4.75 / 4.9, one
+  // product of 16 x 2560 x 1536 3.9 / 4.2), where the wavefronts wait for one of them (5 iterations, 16 rows x 3072
+  // 3.4 / 3.9), in 64-k iterations, of which the ring holds a quarter (LoRA 4096 x 1024 of 8 rows 3.7 / 4.1), or where
+  // half the rows halve the others' slab, short of long loops (8 rows x 4096: 4096 7.5 / 7.8, 44 - 52 iterations 0.97 -
+  // 1.08 of the others' time, 56 - 112 0.88 - 1.02). A printed LoRA keeps the two launches that its readers know.
+  plan.lone = narrow && G.nb == 1 && G.KT == 256 && F >= 3 * ((F + 3) / 4) && 4 * blocks <= 256 && strip_lds <= s.max_lds &&
+              (G.lora ? blocks >= 40 && !emit_sink() : blocks >= 48 && (G.M > 8 || F > 52));
+  strips = strips || plan.lone;
   // One range per block where the blocks alone occupy the chip and a wavefront has a few steps to
   // make: no slab and no second launch (4 x 8192 x 2048 in 64-k iterations: 8.9 us against 12).
   // Otherwise four iterations, one per wavefront, to a range, as far as that many workgroups are
@@ -548,7 +560,7 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GMatch const &R, Gemm
   // 16 x 6400 x 3072 15.1 / 14.4).
   bool there;
   if (G.whole && G.KT % 64 == 0) {
-    there = blocks * S > (G.wcm ? 4096 : 1024) || weight_bytes > (most_mb << 20);
+    there = plan.lone || blocks * S > (G.wcm ? 4096 : 1024) || weight_bytes > (most_mb << 20);
     if (R.pro == PRO_SILU_MUL && G.M <= 16) {
       there = units > 104 || here_ns > there_ns;
     }

@@ -413,14 +413,18 @@ __device__ __forceinline__ void stream_block(StreamParams const &S) {
 // Bound by memory: two weights of 4096 x 14336 against 8 rows 42.9 us, ranges and their fold 47.2;
 // against 16 rows, and with a gated MLP's second product behind it, 79.5 against 82.5.  (With strips of 16 of one of
 // them a pair of workgroups took 42.8 us, with 8 of each and SiLU(a) * u 43.8, and the second product 25.2 instead of 29.4.)
-constexpr int columns_ring(int eights) { return eights == 1 ? 6 : 4; }  // slots per wavefront, two workgroups a compute unit
-constexpr int columns_slot_bytes(int eights) { return 2048 + 1024 * eights; }
+// A LoRA's A, 16 columns too, goes through the ring with every strip: 8 rows x 4096 x 4096 8.0 us, ranges and fold 11.1.
+// Slots per wavefront: for two workgroups on a compute unit.
+constexpr int columns_ring(int eights, bool lora) { return eights == 1 ? (lora ? 4 : 6) : (lora ? 3 : 4); }
+constexpr int columns_slot_bytes(int eights, bool lora) { return 2048 + 1024 * eights + (lora ? 2048 : 0); }
 
-template <int NB, int EIGHTS>
+template <int NB, int EIGHTS, bool LORA>
 __device__ __forceinline__ void stream_columns(StreamParams const &S) {
   GemmParams const &P = S.g;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  constexpr int W = 4, R = columns_ring(EIGHTS), SLOT = columns_slot_bytes(EIGHTS), LOADS = 2 + EIGHTS;
+  constexpr int W = 4, R = columns_ring(EIGHTS, LORA), SLOT = columns_slot_bytes(EIGHTS, LORA);
+  constexpr int LOADS = 2 + EIGHTS + (LORA ? 2 : 0), LA_AT = 2048 + 1024 * EIGHTS;
+  static_assert((R - 1) * LOADS < 64 && !(LORA && NB == 2), "loads in flight are counted in six bits");
   int const tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   int const g = lane / 16, c = lane % 16, l8 = lane / 8, ch8 = lane % 8;
   int const M = P.M, F = P.forloop_range, subs = P.KT / 64;
@@ -437,11 +441,15 @@ __device__ __forceinline__ void stream_columns(StreamParams const &S) {
   unsigned char *const mine = lds + wave * R * SLOT;
   uint32_t const mine_at = lane_lds_address(mine);
   auto swizzle = [](int row) { return (row >> 1) & 7; };
-  uint32_t w_off[2], x_off[EIGHTS];
+  uint32_t w_off[2], x_off[EIGHTS], la_off[2];
 #pragma unroll
   for (int j = 0; j < 2; j++) {  // (rows 8 - 15 of the LDS tile: the columns behind, or the other weight's)
     int const ld = NB == 2 && j == 1 ? P.b1.d_cols : P.b0.d_cols;
     w_off[j] = 2u * (uint32_t)((NB == 2 ? l8 : 8 * j + l8) * ld + 8 * (ch8 ^ swizzle(8 * j + l8)));
+  }
+#pragma unroll
+  for (int j = 0; j < 2; j++) {  // (lora A: 16 columns as well)
+    la_off[j] = LORA ? 2u * (uint32_t)((8 * j + l8) * P.la.d_cols + 8 * (ch8 ^ swizzle(8 * j + l8))) : 0u;
   }
 #pragma unroll
   for (int j = 0; j < EIGHTS; j++) {
@@ -464,6 +472,13 @@ __device__ __forceinline__ void stream_columns(StreamParams const &S) {
     for (int j = 0; j < EIGHTS; j++) {
       lane_dma16(x, x_off[j], at + (uint32_t)(2048 + 1024 * j));
     }
+    if (LORA) {
+      _Float16 const *la = static_cast<_Float16 const *>(P.la.ptr) + gtile_offset(P.la, bx, by, bz, it) + 64 * i_sub;
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        lane_dma16(la, la_off[j], at + (uint32_t)(LA_AT + 1024 * j));
+      }
+    }
     issued++;
     i_slot = i_slot + 1 == R ? 0 : i_slot + 1;
     i_sub++;
@@ -472,13 +487,20 @@ __device__ __forceinline__ void stream_columns(StreamParams const &S) {
       i_it = i_it + 1 == n_mine ? 0 : i_it + 1;
     }
   };
+  half4 lb_frag;  // lora B[4 g ..][16 piece + c], loop invariant
+  if (LORA) {
+    lb_frag = *reinterpret_cast<half4 const *>(static_cast<_Float16 const *>(P.lb.ptr) + gtile_offset(P.lb, bx, by, bz, 0) +
+                                               (long long)(16 * piece + c) * P.lb.d_cols + 4 * g);
+    stream_wait<0>();  // (before the counted loads begin)
+    asm volatile("" : "+v"(lb_frag));
+  }
   for (int s = 0; s < R && s < total; s++) {
     issue_next();
   }
   _Float16 *const all = reinterpret_cast<_Float16 *>(lds + S.results);  // [F][M][16]
   int slot = 0, step = 0;
   for (int i = 0; i < n_mine; i++) {
-    float4v o = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4v o = {0.0f, 0.0f, 0.0f, 0.0f}, d = o;
     for (int sub = 0; sub < subs; sub++, step++) {
       if (issued - step == R) {
         stream_wait<(R - 1) * LOADS>();
@@ -487,11 +509,14 @@ __device__ __forceinline__ void stream_columns(StreamParams const &S) {
       }
       unsigned char const *const at = mine + slot * SLOT;
       int const xr = EIGHTS == 2 ? c : c % 8;
-      half8 w[2], x[2];
+      half8 w[2], x[2], la[2];
 #pragma unroll
       for (int s = 0; s < 2; s++) {
         w[s] = *reinterpret_cast<half8 const *>(at + 128 * c + 16 * ((4 * s + g) ^ swizzle(c)));
         x[s] = *reinterpret_cast<half8 const *>(at + 2048 + 128 * xr + 16 * ((4 * s + g) ^ swizzle(xr)));
+        if (LORA) {
+          la[s] = *reinterpret_cast<half8 const *>(at + LA_AT + 128 * c + 16 * ((4 * s + g) ^ swizzle(c)));
+        }
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (issued < total) {
@@ -500,8 +525,15 @@ __device__ __forceinline__ void stream_columns(StreamParams const &S) {
       slot = slot + 1 == R ? 0 : slot + 1;
 #pragma unroll
       for (int s = 0; s < 2; s++) {
+        if (LORA) {
+          d = __builtin_amdgcn_mfma_f32_16x16x32_f16(la[s], x[s], d, 0, 0, 0);
+        }
         o = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[s], x[s], o, 0, 0, 0);
       }
+    }
+    if (LORA) {  // + [X.A] . B, as in stream_block
+      half4 const df = {(_Float16)d[0], (_Float16)d[1], (_Float16)d[2], (_Float16)d[3]};
+      o = __builtin_amdgcn_mfma_f32_16x16x16f16(lb_frag, df, o, 0, 0, 0);
     }
     int const j = i + rot, it = first + (j >= n_mine ? j - n_mine : j);
     if (c < M) {
@@ -534,12 +566,12 @@ __device__ __forceinline__ void stream_columns(StreamParams const &S) {
 template <int NB, int PRO, bool LORA, bool WCM, int MT>
 __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamParams const S) {
   fetch_kernel_arguments<sizeof(StreamParams), 2>();
-  if constexpr (PRO == PRO_NONE && !LORA && WCM && MT == 1) {
+  if constexpr (PRO == PRO_NONE && WCM && MT == 1) {
     if (S.strips) {
       if (S.g.M <= 8) {
-        stream_columns<NB, 1>(S);
+        stream_columns<NB, 1, LORA>(S);
       } else {
-        stream_columns<NB, 2>(S);
+        stream_columns<NB, 2, LORA>(S);
       }
       return;
     }

@@ -116,6 +116,43 @@ def test_strips_of_16_columns(rt, ranges, m, blocks, kt, loop, weights):
     _run(rt, spec, COL, f"strips {m} x {blocks}, {kt} x {loop}, {weights}", **({} if weights == 1 else {"std": 0.05}))
 
 
+@pytest.mark.parametrize("family,m,blocks,loop", [
+    ("plain", 9, 49, 7), ("plain", 16, 63, 3), ("plain", 15, 51, 33), ("plain", 16, 49, 56), ("plain", 7, 51, 53),
+    ("lora", 1, 41, 3), ("lora", 8, 63, 17), ("lora", 7, 49, 56), ("lora", 9, 41, 7), ("lora", 16, 63, 4), ("lora", 15, 51, 33)])
+def test_one_strip_a_compute_unit(rt, abi, family, m, blocks, loop):
+    """256-k iterations whose strips are at most one to a compute unit, on the ordinary rule: rows around 8 and 16, a
+    for-loop that the wavefronts share evenly and not, the fewest and many results; against the oracle, and bit for bit
+    what the one-launch kernel gives, infinities and NaN included."""
+    import numpy as np
+    from attention_superoptimizer_amd import workloads as W
+    from helpers import normal_f16
+    from test_gpu_f16 import _graph_f16
+    from test_gpu_launch_records import _kernel as launched
+    k, n = 256 * loop, 64 * blocks
+    if family == "lora":
+        spec, _ = W.config4_lora(m=m, d=k, r=16, grid=blocks, F=loop)
+        spec[1], spec[3] = W._inp([k, n], COL), W._inp([16, n], COL)
+    else:
+        spec, _ = W.tiled_matmul(m, n, k, (blocks, 1, 1), loop, (-1, -1, -1), (1, -1, -1), (1, -1, -1))
+    _run(rt, spec, COL, f"lone strips {family} {m} x {blocks}, {loop}", std=0.03)
+    assert launched()[1] == 4 * blocks
+    ins = {i: normal_f16(op["dims"], 1.0, 9 + i) for i, op in enumerate(spec) if op["op"] == "input"}
+    ins[0][m - 1, k - 1], ins[1][5, n - 1], ins[1][k - 3, 17] = np.inf, np.nan, -np.inf
+    want = None
+    for option in (0, 2):
+        assert abi.mi355_set_option(7, option) == 0
+        try:
+            got = _graph_f16(rt, spec, ins)[-1][0]
+        finally:
+            assert abi.mi355_set_option(7, 0) == 0
+        nan = np.isnan(got)
+        bits = np.where(nan, 0, got.view(np.uint16))
+        if want is not None:
+            np.testing.assert_array_equal(nan, want[0])
+            np.testing.assert_array_equal(bits, want[1])
+        want = (nan, bits)
+
+
 @pytest.mark.parametrize("order", [COL, ROW])
 @pytest.mark.parametrize("m,cols,blocks,kt,loop,rank", [
     (1, 16, 9, 64, 3, 0), (33, 48, 3, 128, 5, 0), (64, 128, 7, 256, 9, 0), (17, 80, 2, 64, 17, 0), (9, 32, 65, 256, 2, 0),
