@@ -127,6 +127,7 @@ ABI = {
     "mi355_f16_fill_normal": (_ci, [_vp, _sz, ctypes.c_float, _u64]),
     "mi355_f16_matmul": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci, _ci]),
     "mi355_f16_matmul_layout": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci, _ci, _ci, _ci]),
+    "mi355_f16_matmul_two": (_ci, [_vp, _ci, _ci, _ci, _ci, _ci, _ci, _vp, _vp, ctypes.POINTER(_ci)]),
     "mi355_f16_matmul_then": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci, _ci, _ci, _ci, _ci, _vp, _ci, _vp]),
     "mi355_f16_softmax_rows": (_ci, [_vp, _vp, _vp, _vp, _sz, _ci]),
     "mi355_f16_attention_rows": (_ci, [_vp] * 8 + [_ci] * 6 + [_vp]),

@@ -27,15 +27,22 @@ struct AnyGemm {
   _Float16 *C;
   _Float16 const *X;  // second operand of a binary consumer: [batch][m][n]
   _Float16 *E;        // the consumer's result
-  int epilogue;
+  int epilogue, epilogue2;  // of the first matrix of the batch; of the others
   int m, n, k;
-  int tiles_m, tiles_n, tiles_per_batch;
+  int tiles_m, tiles_n;
+  int group;       // tile rows that a column of tiles goes down (gemm_tile)
   unsigned total;  // workgroups
   // k in `ksplit` ranges, a workgroup each; with more than one a range's fp32 sums go to
   // partial[range][batch][m][n] and f16_gemm_fold_kernel adds them
   int ksplit, steps_per_range;
+  int a_rows;  // from a matrix of A to the next: m
   float *partial;
+  // elements from a matrix of the other operands to the next.  Two products of the same A are a batch of two with
+  // a_rows = 0 and these as the tensors happen to lie.
+  long long b_step, c_step, x_step, e_step;
 };
+// (two lines of kernel arguments, both asked for at the start: a field of a third, first read on the way out, was 0.1 us)
+static_assert(sizeof(AnyGemm) == 128, "two cache lines");
 
 __device__ __forceinline__ float f16_unary_value(bool exp, float x) { return exp ? __expf(x) : x / (1.0f + __expf(-x)); }
 
@@ -170,16 +177,19 @@ struct OperandStage {
 };
 
 // Which tile, batch and k range: an XCD (one L2) gets consecutive ids; the k ranges of a tile sit next to
-// each other, and tiles go down four tile rows before they move to the next columns.
+// each other, and tiles go down `group` tile rows before they move to the next columns: all of up to 512 rows where B
+// is larger than an L2, else four ([300, 2048] . [2048, 5504], five rows of tiles, whose columns a second group would
+// fetch again, 15.3 -> 14.1 us, [426, 128] . [128, 2575] 4.1 -> 4.3).
 __device__ __forceinline__ void gemm_tile(AnyGemm const &G, int bm, int bn, int &split, int &batch, int &row0, int &col0) {
   unsigned const xcd = blockIdx.x % 8, each = G.total / 8, more = G.total % 8;
   unsigned id = xcd * each + (xcd < more ? xcd : more) + blockIdx.x / 8;
   split = (int)(id % (unsigned)G.ksplit);
   id /= (unsigned)G.ksplit;
-  batch = (int)(id / (unsigned)G.tiles_per_batch);
-  int const t0 = (int)(id % (unsigned)G.tiles_per_batch);
-  int const per_group = 4 * G.tiles_n, first_m = 4 * (t0 / per_group);
-  int const gsz = (G.tiles_m - first_m) < 4 ? (G.tiles_m - first_m) : 4;
+  unsigned const tiles = (unsigned)(G.tiles_m * G.tiles_n);
+  batch = (int)(id / tiles);
+  int const t0 = (int)(id % tiles);
+  int const per_group = G.group * G.tiles_n, first_m = G.group * (t0 / per_group);
+  int const gsz = (G.tiles_m - first_m) < G.group ? (G.tiles_m - first_m) : G.group;
   row0 = (first_m + (t0 % per_group) % gsz) * bm;
   col0 = (t0 % per_group) / gsz * bn;
 }
@@ -193,7 +203,7 @@ __device__ __forceinline__ void gemm_store(AnyGemm const &G, float4v const (&acc
   int const g = lane / 16, c = lane % 16;
   if (G.ksplit > 1) {
     if (owner) {
-      int const batches = (int)(G.total / (unsigned)(G.ksplit * G.tiles_per_batch));
+      int const batches = (int)(G.total / (unsigned)(G.ksplit * G.tiles_m * G.tiles_n));
       float *const P = G.partial + ((size_t)split * batches + batch) * (size_t)G.m * G.n;
 #pragma unroll
       for (int i = 0; i < TM; i++) {
@@ -229,34 +239,36 @@ __device__ __forceinline__ void gemm_store(AnyGemm const &G, float4v const (&acc
     }
   }
   __syncthreads();
-  size_t const matrix = (size_t)batch * G.m * G.n;
+  _Float16 *const C = G.C + batch * G.c_step, *const E = G.E + batch * G.e_step;
+  _Float16 const *const X = G.X + batch * G.x_step;
+  int const epilogue = batch == 0 ? G.epilogue : G.epilogue2;
   for (int e = threadIdx.x; e < BM * (BN / 8); e += NT) {
     int const r = e / (BN / 8), c8 = 8 * (e % (BN / 8)), row = row0 + r, col = col0 + c8;
     if (row < G.m && col < G.n) {
       half8 const v = *reinterpret_cast<half8 const *>(tile + r * LDC + c8);
-      size_t const at = matrix + (size_t)row * G.n + col;
+      size_t const at = (size_t)row * G.n + col;
       if (col + 8 <= G.n) {
-        *reinterpret_cast<half8_any *>(G.C + at) = v;
-        if (G.epilogue != EPI_NONE) {
+        *reinterpret_cast<half8_any *>(C + at) = v;
+        if (epilogue != EPI_NONE) {
           half8 x = v;
-          if (G.epilogue >= EPI_ADD) {
-            x = *reinterpret_cast<half8_any const *>(G.X + at);
+          if (epilogue >= EPI_ADD) {
+            x = *reinterpret_cast<half8_any const *>(X + at);
           }
           half8 y;
 #pragma unroll
           for (int u = 0; u < 8; u++) {
-            y[u] = static_cast<_Float16>(epilogue_value(G.epilogue, static_cast<float>(v[u]), static_cast<float>(x[u])));
+            y[u] = static_cast<_Float16>(epilogue_value(epilogue, static_cast<float>(v[u]), static_cast<float>(x[u])));
           }
-          *reinterpret_cast<half8_any *>(G.E + at) = y;
+          *reinterpret_cast<half8_any *>(E + at) = y;
         }
       } else {
 #pragma unroll
         for (int u = 0; u < 7; u++) {
           if (col + u < G.n) {
-            G.C[at + u] = v[u];
-            if (G.epilogue != EPI_NONE) {
-              float const x = G.epilogue >= EPI_ADD ? static_cast<float>(G.X[at + u]) : 0.0f;
-              G.E[at + u] = static_cast<_Float16>(epilogue_value(G.epilogue, static_cast<float>(v[u]), x));
+            C[at + u] = v[u];
+            if (epilogue != EPI_NONE) {
+              float const x = epilogue >= EPI_ADD ? static_cast<float>(X[at + u]) : 0.0f;
+              E[at + u] = static_cast<_Float16>(epilogue_value(epilogue, static_cast<float>(v[u]), x));
             }
           }
         }
@@ -296,8 +308,8 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG) void f16_gemm_any_
 
   SA sa;
   SB sb;
-  sa.init(G.A + (size_t)batch * G.m * G.k, G.m, row0, G.k, tid);
-  sb.init(G.B + (size_t)batch * G.k * G.n, G.n, col0, G.k, tid);
+  sa.init(G.A + (size_t)batch * G.a_rows * G.k, G.m, row0, G.k, tid);
+  sb.init(G.B + batch * G.b_step, G.n, col0, G.k, tid);
 
   // This group's stages: whole stages [first, first + own) and, in the last range, the tail.
   int const whole = G.k / 64, tail = G.k % 64, ranges = G.ksplit * KG, range = split * KG + kg;
@@ -547,25 +559,33 @@ struct DirectStage {
 
 constexpr int kDirectRing = 3;
 
-template <int BM, int BN, int WM, int WN, bool B_KC>
+// Both of two products of one A (TWO): half of a tile's columns are of the second, a wavefront's all
+// of one, and each half leaves as a product by itself does.  A is fetched once, and a launch of 64 x 64 + 64 or
+// 128 + 128 columns has less to wait for than two: [300, 2048] . [2048, 5504] twice 26.1 us, one by one 2 x 17.8.  What
+// bounds it: the LDS traffic of a stage, 1100 cycles of 1600 with 128 columns of each.
+template <int BM, int BN, int WM, int WN, bool B_KC, bool TWO = false>
 __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void f16_gemm_direct_kernel(AnyGemm const G) {
-  constexpr int NT = 64 * (BM / WM) * (BN / WN), TM = WM / 16, TN = WN / 16;
+  constexpr int NT = 64 * (BM / WM) * (BN / WN), TM = WM / 16, TN = WN / 16, COLS = TWO ? BN / 2 : BN;
+  static_assert(COLS % WN == 0, "a wavefront has columns of one product");
   using SA = DirectStage<BM, NT, true>;
-  using SB = DirectStage<BN, NT, B_KC>;
-  constexpr int STAGE = SA::HALFS + SB::HALFS, LPS = SA::CH + SB::CH;
+  using SB = DirectStage<COLS, NT, B_KC>;
+  constexpr int STAGE = SA::HALFS + (TWO ? 2 : 1) * SB::HALFS, LPS = SA::CH + (TWO ? 2 : 1) * SB::CH;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   _Float16 *const ring = reinterpret_cast<_Float16 *>(lds);
   int const tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
 
   int split, batch, row0, col0;
-  gemm_tile(G, BM, BN, split, batch, row0, col0);
+  gemm_tile(G, BM, COLS, split, batch, row0, col0);
   SA sa;
-  SB sb;
-  sa.init(G.A + (size_t)batch * G.m * G.k, G.m, row0, G.k, tid);
-  sb.init(G.B + (size_t)batch * G.k * G.n, G.n, col0, G.k, tid);
+  SB sb, sb2;
+  sa.init(G.A + (size_t)batch * G.a_rows * G.k, G.m, row0, G.k, tid);
+  sb.init(G.B + batch * G.b_step, G.n, col0, G.k, tid);
+  if (TWO) {
+    sb2.init(G.B + G.b_step, G.n, col0, G.k, tid);
+  }
   int const whole = G.k / 64, first = split * G.steps_per_range < whole ? split * G.steps_per_range : whole;
   int const T = (whole - first) < G.steps_per_range ? (whole - first) : G.steps_per_range;
-  int const wm0 = (wave / (BN / WN)) * WM, wn0 = (wave % (BN / WN)) * WN;
+  int const wm0 = (wave / (BN / WN)) * WM, col = (wave % (BN / WN)) * WN, second = TWO ? col / COLS : 0, wn0 = col - second * COLS;
 
   float4v acc[TM][TN];
 #pragma unroll
@@ -580,6 +600,9 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void f16_gemm_direct_ke
     uint32_t const at = ring_at + 2u * (uint32_t)(slot * STAGE);
     sa.issue(first + t, at, wave);
     sb.issue(first + t, at + 2u * (uint32_t)SA::HALFS, wave);
+    if (TWO) {
+      sb2.issue(first + t, at + 2u * (uint32_t)(SA::HALFS + SB::HALFS), wave);
+    }
   };
   struct Operands {
     half8 a[TM], b[TN];
@@ -592,7 +615,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void f16_gemm_direct_ke
     }
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-      x.b[j] = SB::operand(buf + SA::HALFS, wn0 + 16 * j, s, lane);
+      x.b[j] = SB::operand(buf + SA::HALFS + second * SB::HALFS, wn0 + 16 * j, s, lane);
     }
   };
   auto multiply = [&](Operands const &x) {
@@ -649,7 +672,11 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void f16_gemm_direct_ke
     multiply(x1);
     __syncthreads();
   }
-  gemm_store<BM, BN, TM, TN, NT>(G, acc, ring, true, lane, split, batch, row0, col0, wm0, wn0);
+  gemm_store<BM, COLS, TM, TN, NT>(G, acc, ring, second == 0, lane, split, batch, row0, col0, wm0, wn0);
+  if (TWO) {  // (a thread stores the same elements of both: a consumer may read the first's)
+    __syncthreads();
+    gemm_store<BM, COLS, TM, TN, NT>(G, acc, ring, second == 1, lane, split, 1, row0, col0, wm0, wn0);
+  }
 }
 
 template <int BM, int BN>
@@ -740,8 +767,8 @@ __global__ __launch_bounds__(256) void f16_gemm_waves_kernel(AnyGemm const G) {
   gemm_tile(G, BM, BN, split, batch, row0, col0);
   SA sa;
   SB sb;
-  sa.init(G.A + (size_t)batch * G.m * G.k, G.m, row0, G.k, lane);
-  sb.init(G.B + (size_t)batch * G.k * G.n, G.n, col0, G.k, lane);
+  sa.init(G.A + (size_t)batch * G.a_rows * G.k, G.m, row0, G.k, lane);
+  sb.init(G.B + batch * G.b_step, G.n, col0, G.k, lane);
   // this range's steps [first, last); the wavefront's are first + wave, + 4, ..
   int const all = G.k / 32, first = split * G.steps_per_range < all ? split * G.steps_per_range : all;
   int const last = all - first < G.steps_per_range ? all : first + G.steps_per_range;

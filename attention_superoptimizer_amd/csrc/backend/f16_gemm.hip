@@ -317,35 +317,42 @@ __global__ __launch_bounds__(kThreads) void f16_transpose_kernel(_Float16 const 
 }
 
 // C[i] = fp16(sum over the k ranges of partial[s][i]), added in fp32 in range order, and the
-// consumer.  Four elements a thread: a 16-byte load per range.
+// consumer.  Four elements a thread: a 16-byte load per range.  `n` elements of a matrix; a batch is one of n elements
+// but where it is two products, whose second follows the first in the same thread: its consumer may read the first's.
+template <int PRODUCTS>
 __global__ void f16_gemm_fold_kernel(AnyGemm const G, size_t n) {
   size_t const stride = (size_t)gridDim.x * blockDim.x * 4;
   for (size_t i = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) * 4; i < n; i += stride) {
-    float4v r = {0.0f, 0.0f, 0.0f, 0.0f};
     int const left = n - i < 4 ? (int)(n - i) : 4;
-    for (int s = 0; s < G.ksplit; s++) {
-      float const *p = G.partial + (size_t)s * n + i;
-      if (left == 4) {
-        float4v const v = *reinterpret_cast<float4_any const *>(p);
+    for (int product = 0; product < PRODUCTS; product++) {
+      _Float16 *const C = G.C + product * G.c_step, *const E = G.E + product * G.e_step;
+      _Float16 const *const X = G.X + product * G.x_step;
+      int const epilogue = product == 0 ? G.epilogue : G.epilogue2;
+      float4v r = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int s = 0; s < G.ksplit; s++) {
+        float const *p = G.partial + ((size_t)s * PRODUCTS + product) * n + i;
+        if (left == 4) {
+          float4v const v = *reinterpret_cast<float4_any const *>(p);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          r[e] += v[e];
-        }
-      } else {
+          for (int e = 0; e < 4; e++) {
+            r[e] += v[e];
+          }
+        } else {
 #pragma unroll
-        for (int e = 0; e < 3; e++) {
-          r[e] += e < left ? p[e] : 0.0f;
+          for (int e = 0; e < 3; e++) {
+            r[e] += e < left ? p[e] : 0.0f;
+          }
         }
       }
-    }
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      if (e < left) {
-        _Float16 const v = static_cast<_Float16>(r[e]);
-        G.C[i + e] = v;
-        if (G.epilogue != EPI_NONE) {
-          float const x = G.epilogue >= EPI_ADD ? static_cast<float>(G.X[i + e]) : 0.0f;
-          G.E[i + e] = static_cast<_Float16>(epilogue_value(G.epilogue, static_cast<float>(v), x));
+      for (int e = 0; e < 4; e++) {
+        if (e < left) {
+          _Float16 const v = static_cast<_Float16>(r[e]);
+          C[i + e] = v;
+          if (epilogue != EPI_NONE) {
+            float const x = epilogue >= EPI_ADD ? static_cast<float>(X[i + e]) : 0.0f;
+            E[i + e] = static_cast<_Float16>(epilogue_value(epilogue, static_cast<float>(v), x));
+          }
         }
       }
     }
@@ -419,20 +426,28 @@ TileKernel tile_kernel_of(int i, bool a_kc, bool b_kc) {
   return b_kc ? tile_kernel_at<false, true>(i, Col{}) : tile_kernel_at<false, false>(i, Col{});
 }
 
-int launch_gemm_tiles(AnyGemm &G, int batch, bool a_kc, bool b_kc, GemmChoice const &choice) {
-  GemmTile const &t = (a_kc ? kGemmTiles : kGemmTilesColumnMajorA)[choice.tile];
-  TileKernel const kernel = tile_kernel_of(choice.tile, a_kc, b_kc);
+// The geometry of these tiles in so many ranges.
+int place_tiles(AnyGemm &G, int batch, GemmTile const &t, int ksplit) {
   G.tiles_m = (G.m + t.bm - 1) / t.bm;
   G.tiles_n = (G.n + t.bn - 1) / t.bn;
-  G.tiles_per_batch = G.tiles_m * G.tiles_n;
-  G.ksplit = choice.ksplit;
+  G.group = G.tiles_m * t.bm <= 512 && (size_t)G.k * G.n >= (2u << 20) ? G.tiles_m : 4;
+  G.ksplit = ksplit;
   G.steps_per_range = t.kind == WAVES ? (G.k / 32 + G.ksplit - 1) / G.ksplit : (G.k / 64 + G.ksplit * t.kg - 1) / (G.ksplit * t.kg);
   G.partial = static_cast<float *>(state().scratch());
-  long long const total = (long long)G.tiles_per_batch * batch * G.ksplit;
+  long long const total = (long long)G.tiles_m * G.tiles_n * batch * G.ksplit;
   if (total > 2147483647LL) {
     return fail(MI355_ERR_UNSUPPORTED, "matmul has too many output tiles");
   }
   G.total = (unsigned)total;
+  return MI355_OK;
+}
+
+int launch_gemm_tiles(AnyGemm &G, int batch, bool a_kc, bool b_kc, GemmChoice const &choice, bool two = false) {
+  GemmTile const &t = (a_kc ? kGemmTiles : kGemmTilesColumnMajorA)[choice.tile];
+  TileKernel const kernel = tile_kernel_of(choice.tile, a_kc, b_kc);
+  if (int rc = place_tiles(G, batch, t, choice.ksplit)) {
+    return rc;
+  }
   // Stages further ahead where a range is long (un-fused MLPs, us: 182 x 1830 x 1807 41.6 -> 33.3, 300 x 1027 x 2049 39.3
   // -> 33.9, 500 x 1999 x 3001 78.0 -> 75.1); a short one has them all in its last stages, which load under conditions
   // (from 6 on, 34 x 1455 x 790 27.7 -> 29.2).
@@ -440,9 +455,23 @@ int launch_gemm_tiles(AnyGemm &G, int batch, bool a_kc, bool b_kc, GemmChoice co
   MI355_GRANT_LDS(fn, kernel.lds);
   MI355_HIP(launch_kernel(fn, G.total, t.threads(), kernel.lds, state().stream(), G));
   if (G.ksplit > 1) {
-    size_t const n = (size_t)batch * G.m * G.n, blocks = (n / 4 + kThreads) / kThreads;
-    MI355_HIP(launch_kernel(f16_gemm_fold_kernel, (unsigned)std::min<size_t>(blocks, 4096), kThreads, 0, state().stream(), G, n));
+    size_t const n = (size_t)batch * G.m * G.n / (two ? 2 : 1), blocks = (n / 4 + kThreads) / kThreads;
+    MI355_HIP(launch_kernel(two ? f16_gemm_fold_kernel<2> : f16_gemm_fold_kernel<1>, (unsigned)std::min<size_t>(blocks, 4096), kThreads, 0,
+                            state().stream(), G, n));
   }
+  return MI355_OK;
+}
+
+// Both products in every workgroup, columns of each side by side.
+template <int HALF, int WN, bool B_KC>
+int launch_gemm_two(AnyGemm &G) {
+  auto *const fn = f16_gemm_direct_kernel<64, 2 * HALF, 32, WN, B_KC, true>;
+  constexpr int lds = direct_gemm_lds<64, 2 * HALF>();
+  if (int rc = place_tiles(G, 1, GemmTile{DIRECT, 64, HALF, 32, WN, 1}, 1)) {
+    return rc;
+  }
+  MI355_GRANT_LDS(fn, lds);
+  MI355_HIP(launch_kernel(fn, G.total, 64 * 2 * (2 * HALF / WN), lds, state().stream(), G));
   return MI355_OK;
 }
 
@@ -490,6 +519,10 @@ int run_matmul(AnyGemm G, int batch, int a_column_major, int b_column_major, boo
   }
   if (choice.route == GEMM_TILES) {
     *applied = true;
+    G.epilogue2 = G.epilogue;
+    G.a_rows = m;
+    G.b_step = (long long)k * n;
+    G.c_step = G.x_step = G.e_step = (long long)m * n;
     return launch_gemm_tiles(G, batch, !a_column_major || choice.copy_a, b_column_major != 0, choice);
   }
   dim3 grid((n + 63) / 64, (m + 63) / 64, batch);
@@ -522,6 +555,18 @@ extern "C" int mi355_f16_matmul(void const *A, void const *B, void *C, int batch
   return mi355_f16_matmul_layout(A, B, C, batch, m, n, k, 0, 0);
 }
 
+static bool consumer_of(int op, int x_first, int *epilogue) {
+  switch (op) {
+    case 0: *epilogue = EPI_NONE; return true;
+    case KN_EXP_OP: *epilogue = EPI_EXP; return true;
+    case KN_SILU_OP: *epilogue = EPI_SILU; return true;
+    case KN_ADD_OP: *epilogue = EPI_ADD; return true;
+    case KN_MUL_OP: *epilogue = EPI_MUL; return true;
+    case KN_DIV_OP: *epilogue = x_first ? EPI_RDIV : EPI_DIV; return true;
+    default: return false;
+  }
+}
+
 extern "C" int mi355_f16_matmul_then(void const *A, void const *B, void *C, int batch, int m, int n, int k,
                                      int a_column_major, int b_column_major, int op, void const *X, int x_first, void *E) {
   MI355_REQUIRE_INIT();
@@ -538,12 +583,7 @@ extern "C" int mi355_f16_matmul_then(void const *A, void const *B, void *C, int 
   G.m = m;
   G.n = n;
   G.k = k;
-  G.epilogue = op == KN_EXP_OP    ? EPI_EXP
-               : op == KN_SILU_OP ? EPI_SILU
-               : op == KN_ADD_OP  ? EPI_ADD
-               : op == KN_MUL_OP  ? EPI_MUL
-               : x_first          ? EPI_RDIV
-                                  : EPI_DIV;
+  consumer_of(op, x_first, &G.epilogue);
   bool applied;
   if (int rc = run_matmul(G, batch, a_column_major, b_column_major, &applied)) {
     return rc;
@@ -557,6 +597,55 @@ extern "C" int mi355_f16_matmul_then(void const *A, void const *B, void *C, int 
   }
   int const dims[3] = {batch, m, n};
   return mi355_f16_binary(op, x_first ? X : C, dims, x_first ? C : X, dims, E, dims, 3);
+}
+
+extern "C" int mi355_f16_matmul_two(void const *A, int a_column_major, int b_column_major, int batch, int m, int n, int k,
+                                    mi355_matmul_out const *first, mi355_matmul_out const *second, int *taken) {
+  MI355_REQUIRE_INIT();
+  *taken = 0;
+  AnyGemm G{};
+  G.A = static_cast<_Float16 const *>(A);
+  G.B = static_cast<_Float16 const *>(first->B);
+  G.C = static_cast<_Float16 *>(first->C);
+  G.X = static_cast<_Float16 const *>(first->X);
+  G.E = static_cast<_Float16 *>(first->E);
+  G.m = m;
+  G.n = n;
+  G.k = k;
+  if (!consumer_of(first->op, first->x_first, &G.epilogue) || !consumer_of(second->op, second->x_first, &G.epilogue2)) {
+    return fail(MI355_ERR_UNSUPPORTED, "op after a matmul");
+  }
+  uintptr_t const all = reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(first->B) | reinterpret_cast<uintptr_t>(second->B);
+  uintptr_t const results = reinterpret_cast<uintptr_t>(first->C) | reinterpret_cast<uintptr_t>(second->C) |
+                            reinterpret_cast<uintptr_t>(first->E) | reinterpret_cast<uintptr_t>(second->E) |
+                            reinterpret_cast<uintptr_t>(first->X) | reinterpret_cast<uintptr_t>(second->X);
+  if (batch != 1 || m <= 0 || n <= 0 || k <= 0 || ((all | results) & 1) != 0 || state().f16_matmul_route == 1) {
+    return MI355_OK;
+  }
+  auto elements = [](void const *from, void const *to) {
+    return (long long)(reinterpret_cast<intptr_t>(to) - reinterpret_cast<intptr_t>(from)) / 2;
+  };
+  G.a_rows = 0;
+  G.b_step = elements(first->B, second->B);
+  G.c_step = elements(first->C, second->C);
+  G.x_step = elements(first->X, second->X);
+  G.e_step = elements(first->E, second->E);
+  bool const reads_first = G.epilogue2 >= EPI_ADD && (second->X == first->C || (first->E != nullptr && second->X == first->E));
+  GemmTwoChoice const two = choose_gemm_two({1, m, n, k, a_column_major != 0, b_column_major != 0, (all & 15) == 0,
+                                             state().scratch() == nullptr ? 0 : state().scratch_bytes,
+                                             state().planes() == nullptr ? 0 : state().planes_bytes}, reads_first);
+  if (two.half != 0) {
+    *taken = 1;
+    if (two.half == 128) {
+      return b_column_major ? launch_gemm_two<128, 64, true>(G) : launch_gemm_two<128, 64, false>(G);
+    }
+    return b_column_major ? launch_gemm_two<64, 32, true>(G) : launch_gemm_two<64, 32, false>(G);
+  }
+  if (!two.tiles) {
+    return MI355_OK;
+  }
+  *taken = 1;
+  return launch_gemm_tiles(G, 2, !a_column_major, b_column_major != 0, two.choice, true);
 }
 
 extern "C" int mi355_f16_transpose(void const *in, void *out, int batch, int rows, int cols) {

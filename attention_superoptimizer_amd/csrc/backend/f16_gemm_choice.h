@@ -151,4 +151,65 @@ inline GemmChoice choose_gemm(GemmShape const &s) {
   return best;
 }
 
+// Two products of the same A and shape (a batch of one), both of them and what consumes them.
+struct GemmTwoChoice {
+  int half;    // columns of each that a workgroup of both has; 0: no such workgroups
+  bool tiles;  // each product's tiles as workgroups of one launch
+  GemmChoice choice;
+  double us;
+};
+// A workgroup of both (f16_gemm_direct_kernel, 64 rows), from timed launches: [300, 2048] . [2048, 5504] 26.1 us with 128
+// columns of each and 29.1 with 64, [700, 1024] . [1024, 2752] 15.4 and 16.1, [60, 1024] . [1024, 3000] 15.0 and 10.5.
+inline double gemm_two_cost(int half, int m, int n, int k) {
+  double const tiles = (double)((m + 63) / 64) * ((n + half - 1) / half), per_cu = std::ceil(tiles / 256.0);
+  double const stage = half == 128 ? 0.67 * per_cu : 0.38 * per_cu;
+  return 4.5 + k / 64 * stage + 1.5 * (per_cu - 1.0);
+}
+// Without either (half 0, no tiles) one after the other is expected to be faster.  reads_first: the second's consumer
+// takes what the first leaves, which whole products of different workgroups could not tell it.  With these
+// constants 218 un-fused gated MLPs of 1 - 1000 rows took 0.61 - 1.02 of their time one by one, 0.84 on average; the gain
+// is the second launch, the second fold and a chip that one product does not fill (us, one by one / two at a time, the
+// whole MLP: 6 x 1419 x 2111 34.6 / 22.7, 28 x 1169 x 1092 26.0 / 17.6, 512 x 2048 x 2048 35.4 / 27.6, 300 x 2048 x
+// 5504 56.7 / 47.1).  Not where tiles of one product fill the chip and none of both takes its sizes.
+inline GemmTwoChoice choose_gemm_two(GemmShape const &s, bool reads_first) {
+  GemmChoice const one = choose_gemm(s);
+  GemmTwoChoice best{0, false, one, one.route == GEMM_ELEMENTS ? 1e30 : 2.0 * one.us};
+  bool const a_kc = !s.a_column_major;
+  int const a_row = a_kc ? s.k : s.m, b_row = s.b_column_major ? s.k : s.n;
+  if (std::min(a_row, b_row) < 8 || std::max(a_row, b_row) >= (1 << 22)) {
+    return best;
+  }
+  bool const chunks = a_kc && (s.b_column_major || s.n % 8 == 0) && s.aligned;
+  for (int half : {64, 128}) {
+    if (chunks && s.k % 64 == 0) {
+      double const us = gemm_two_cost(half, s.m, s.n, s.k);
+      if (us < best.us) {
+        best = {half, false, one, us};
+      }
+    }
+  }
+  size_t const range_bytes = 2 * (size_t)s.m * s.n * sizeof(float);
+  GemmTile const *const tiles = a_kc ? kGemmTiles : kGemmTilesColumnMajorA;
+  int const count = (int)((a_kc ? sizeof(kGemmTiles) : sizeof(kGemmTilesColumnMajorA)) / sizeof(GemmTile));
+  for (int i = 0; i < count; i++) {
+    GemmTile const &t = tiles[i];
+    if (t.kind != STAGED && (!chunks || s.k % (t.kind == DIRECT ? 64 : 32) != 0)) {
+      continue;
+    }
+    for (int ranges : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      if (ranges > 1 && (s.k / 64 < ranges * (t.kind == WAVES ? 1 : t.kg) || range_bytes * ranges > s.scratch_bytes)) {
+        break;
+      }
+      if (ranges == 1 && reads_first) {
+        continue;
+      }
+      double const us = gemm_tile_cost(t, 2, s.m, s.n, s.k, ranges) * (a_kc ? 1.0 : 0.8) + 1.5;
+      if (us < best.us) {
+        best = {0, true, {GEMM_TILES, false, false, i, ranges, us}, us};
+      }
+    }
+  }
+  return best;
+}
+
 }  // namespace mi355

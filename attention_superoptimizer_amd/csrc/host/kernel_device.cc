@@ -635,14 +635,16 @@ static bool same_shape(DTensor const &a, DTensor const &b) {
   return same;
 }
 
-// a matmul and the element-wise operator after it that reads its result
-static bool run_matmul_then(KNOperator const *mm, KNOperator const *next) {
+// a matmul and, where `next` is an element-wise operator that reads its result, that operator
+static bool consumes(KNOperator const *mm, KNOperator const *next, mi355_matmul_out *p) {
+  DTensor const &C = mm->output_tensors[0];
+  *p = {mm->input_tensors[1].data_ptr, C.data_ptr, 0, 0, nullptr, nullptr};
   bool const unary = next->op_type == KN_EXP_OP || next->op_type == KN_SILU_OP;
   bool const binary = next->op_type == KN_ADD_OP || next->op_type == KN_MUL_OP || next->op_type == KN_DIV_OP;
-  if (mm->op_type != KN_MATMUL_OP || (!unary && !binary)) {
+  if (!unary && !binary) {
     return false;
   }
-  DTensor const &C = mm->output_tensors[0], &E = next->output_tensors[0];
+  DTensor const &E = next->output_tensors[0];
   DTensor const *X = nullptr;
   bool x_first = false;
   if (unary) {
@@ -663,11 +665,22 @@ static bool run_matmul_then(KNOperator const *mm, KNOperator const *next) {
   if (!same_shape(C, E) || column_major(C) || column_major(E)) {
     return false;
   }
+  p->op = next->op_type;
+  p->x_first = x_first ? 1 : 0;
+  p->X = X == nullptr ? nullptr : X->data_ptr;
+  p->E = E.data_ptr;
+  return true;
+}
+
+static bool run_matmul_then(KNOperator const *mm, KNOperator const *next) {
+  mi355_matmul_out p;
+  if (mm->op_type != KN_MATMUL_OP || !consumes(mm, next, &p)) {
+    return false;
+  }
   int batch, m, n, k;
   matmul_extents(mm->input_tensors[0], mm->input_tensors[1], batch, m, n, k);
-  MI355_CALL(mi355_f16_matmul_then(mm->input_tensors[0].data_ptr, mm->input_tensors[1].data_ptr, C.data_ptr, batch, m, n, k,
-                                   column_major(mm->input_tensors[0]) ? 1 : 0, column_major(mm->input_tensors[1]) ? 1 : 0,
-                                   next->op_type, X == nullptr ? nullptr : X->data_ptr, x_first ? 1 : 0, E.data_ptr));
+  MI355_CALL(mi355_f16_matmul_then(mm->input_tensors[0].data_ptr, p.B, p.C, batch, m, n, k, column_major(mm->input_tensors[0]) ? 1 : 0,
+                                   column_major(mm->input_tensors[1]) ? 1 : 0, p.op, p.X, p.x_first, p.E));
   return true;
 }
 
@@ -780,6 +793,35 @@ static bool run_with_next(KNOperator *op, KNOperator *next) {
   return true;
 }
 
+// Two matmuls of the same input with weights of one shape and storage order, each perhaps with the element-wise
+// operator that consumes it (a gated MLP's first half): how many of the operators from i on the backend took.
+static size_t run_two_matmuls(std::vector<KNOperator *> const &ops, size_t i) {
+  auto own_route = [&](size_t j) { return is_attention_rows(ops, j) || (j + 3 < ops.size() && is_softmax_rows(ops[j + 1], ops[j + 2], ops[j + 3])); };
+  mi355_matmul_out p[2];
+  size_t at = i;
+  KNOperator const *mm[2];
+  for (int which = 0; which < 2; which++) {
+    if (at >= ops.size() || ops[at]->op_type != KN_MATMUL_OP || own_route(at)) {
+      return 0;
+    }
+    mm[which] = ops[at];
+    if (column_major(mm[which]->output_tensors[0])) {
+      return 0;
+    }
+    p[which] = {mm[which]->input_tensors[1].data_ptr, mm[which]->output_tensors[0].data_ptr, 0, 0, nullptr, nullptr};
+    at += at + 1 < ops.size() && consumes(mm[which], ops[at + 1], &p[which]) ? 2 : 1;
+  }
+  DTensor const &A = mm[0]->input_tensors[0], &B = mm[0]->input_tensors[1], &B2 = mm[1]->input_tensors[1];
+  if (mm[1]->input_tensors[0].guid != A.guid || !same_shape(B, B2) || column_major(B) != column_major(B2) ||
+      B2.data_ptr == p[0].C || B2.data_ptr == p[0].E) {
+    return 0;
+  }
+  int batch, m, n, k, taken = 0;
+  matmul_extents(A, B, batch, m, n, k);
+  MI355_CALL(mi355_f16_matmul_two(A.data_ptr, column_major(A) ? 1 : 0, column_major(B) ? 1 : 0, batch, m, n, k, &p[0], &p[1], &taken));
+  return taken != 0 ? at - i : 0;
+}
+
 void execute_all(Graph const &graph) {
   require_device("execute_all");
   std::vector<KNOperator *> const &ops = graph.operators;
@@ -790,7 +832,9 @@ void execute_all(Graph const &graph) {
            !column_major(ops[i + 2]->output_tensors[0]);
   };
   for (size_t i = 0; i < n;) {
-    if (run_attention_rows(ops, i)) {
+    if (size_t const taken = run_two_matmuls(ops, i)) {
+      i += taken;
+    } else if (run_attention_rows(ops, i)) {
       i += 5;
     } else if (softmax_at(i)) {
       run_softmax_rows(ops[i], ops[i + 1], ops[i + 2]);

@@ -263,6 +263,18 @@ int mi355_fp_binary_many(int const *ops, uint16_t const *const *in1, int const *
 /* compute_reduction_fingerprint, src/kernel/cuda/reduction_kernel.cu:80-133 */
 int mi355_fp_reduce(uint16_t const *in, uint16_t *out, size_t n_out, int factor,
                     int in_stride, int out_stride);
+/* Two products of the same A and shapes, each with the element-wise operator that consumes it as above (op 0: none): C,
+ * E of the first, then of the second, whose X may be one of the first's.  *taken = 0 and nothing enqueued for
+ * batches and where one after the other is expected to be as fast. */
+typedef struct {
+  void const *B;
+  void *C;
+  int op, x_first;
+  void const *X;
+  void *E;
+} mi355_matmul_out;
+int mi355_f16_matmul_two(void const *A, int a_column_major, int b_column_major, int batch, int m, int n, int k,
+                         mi355_matmul_out const *first, mi355_matmul_out const *second, int *taken);
 /* E = exp(X), R[row] = sum of a row of E, P = E / R for `rows` rows of n elements: what mi355_fp_unary,
  * mi355_fp_reduce and mi355_fp_binary one after the other leave. */
 int mi355_fp_softmax_rows(uint16_t const *X, uint16_t *E, uint16_t *R, uint16_t *P, size_t rows, int n);
