@@ -17,16 +17,11 @@ using namespace mirage::type;
 
 // ---- operator base -----------------------------------------------------------
 KNOperator::KNOperator(KNOperatorType _type) : op_type(_type) {}
-KNOperator::KNOperator(KNOperatorType _type, DTensor const &a) : op_type(_type) {
-  input_tensors.push_back(a);
-}
+KNOperator::KNOperator(KNOperatorType _type, DTensor const &a) : op_type(_type), input_tensors{a} {}
 KNOperator::KNOperator(KNOperatorType _type, DTensor const &a, DTensor const &b)
-    : op_type(_type) {
-  input_tensors.push_back(a);
-  input_tensors.push_back(b);
-}
-KNOperator::KNOperator(KNOperatorType _type, std::vector<DTensor> const &inputs)
-    : op_type(_type), input_tensors(inputs) {}
+    : op_type(_type), input_tensors{a, b} {}
+KNOperator::KNOperator(KNOperatorType _type, std::vector<DTensor> inputs)
+    : op_type(_type), input_tensors(std::move(inputs)) {}
 KNOperator::~KNOperator() {}
 
 void KNOperator::release_outputs() {
@@ -397,10 +392,9 @@ KNOperator *Graph::create_customized_op(std::vector<DTensor> const &inputs,
   return new KNCustomizedOp(inputs, _graph);
 }
 
-// Appends one thread-block operator of kind `t` over `ins` to `bg`.
-static void append_tb_op(mirage::threadblock::Graph &bg, TBOperatorType t,
-                         std::vector<STensor> const &ins) {
-  auto arity = [&](size_t n) { MIRAGE_CHECK(ins.size() == n, "wrong operand count in plan"); };
+// Appends one thread-block operator of kind `t` over `count` operands to `bg`.
+static void append_tb_op(mirage::threadblock::Graph &bg, TBOperatorType t, STensor const *ins, size_t count) {
+  auto arity = [&](size_t n) { MIRAGE_CHECK(count == n, "wrong operand count in plan"); };
   if (t == TB_MATMUL_OP) {
     arity(2);
     bg.matmul(ins[0], ins[1]);
@@ -441,19 +435,25 @@ void KNCustomizedOp::add_output(STensor const &stensor, int3 output_map) {
   out->dtensor = output_tensors.back();
 }
 
-KNCustomizedOp::KNCustomizedOp(std::vector<DTensor> const &_inputs, ExecutionPlan const &_plan)
-    : KNOperator(KN_CUSTOMIZED_OP, _inputs), plan(_plan),
-      bgraph(_plan.grid_dim, _plan.block_dim, _plan.forloop_range, _plan.reduction_dimx) {
-  size_t const n = _inputs.size();
+// A search builds thousands of these: room for what is known to come is made once, and nothing is copied
+// that can be moved.
+KNCustomizedOp::KNCustomizedOp(std::vector<DTensor> _inputs, ExecutionPlan _plan)
+    : KNOperator(KN_CUSTOMIZED_OP, std::move(_inputs)), plan(std::move(_plan)),
+      bgraph(plan.grid_dim, plan.block_dim, plan.forloop_range, plan.reduction_dimx) {
+  size_t const n = input_tensors.size();
   MIRAGE_CHECK(plan.input_map.size() == n && plan.forloop_dim.size() == n &&
                    plan.input_smem_layouts.size() == n,
                "plan does not describe every input");
+  size_t const expected = n + plan.ops.size() + 2;  // operators of most plans: those given and up to two outputs
+  bgraph.operators.reserve(expected);
+  bgraph.allocated_tensors.reserve(expected);
   for (size_t i = 0; i < n; i++) {
     bgraph.new_input(input_tensors[i], plan.input_map[i], plan.forloop_dim[i],
                      plan.input_smem_layouts[i]);
   }
+  std::vector<STensor> ins;
   for (auto const &entry : plan.ops) {
-    std::vector<STensor> ins;
+    ins.clear();
     for (auto const &idx : entry.second) {
       MIRAGE_CHECK(idx.first >= 0 && idx.first < (int)bgraph.operators.size(),
                    "plan operand names a missing operator");
@@ -462,7 +462,7 @@ KNCustomizedOp::KNCustomizedOp(std::vector<DTensor> const &_inputs, ExecutionPla
                    "plan operand names a missing tensor");
       ins.push_back(outs[idx.second]);
     }
-    append_tb_op(bgraph, entry.first, ins);
+    append_tb_op(bgraph, entry.first, ins.data(), ins.size());
   }
   // every tile of a non-input operator that no later operator reads is an output
   size_t const num_ops = bgraph.operators.size();
@@ -528,7 +528,7 @@ KNCustomizedOp::KNCustomizedOp(std::vector<DTensor> const &_inputs,
       plan.output_map = out->output_map;
     } else {
       plan.ops.push_back({op->op_type, indices});
-      append_tb_op(bgraph, op->op_type, ins);
+      append_tb_op(bgraph, op->op_type, ins.data(), ins.size());
     }
   }
 }

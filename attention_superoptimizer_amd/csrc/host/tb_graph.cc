@@ -15,14 +15,9 @@ using mirage::kernel::DTensor;
 
 // ---- operator base --------------------------------------------------------------
 TBOperator::TBOperator(Graph *g, TBOperatorType t) : bgraph(g), op_type(t) {}
-TBOperator::TBOperator(Graph *g, TBOperatorType t, STensor const &a) : bgraph(g), op_type(t) {
-  input_tensors.push_back(a);
-}
+TBOperator::TBOperator(Graph *g, TBOperatorType t, STensor const &a) : bgraph(g), op_type(t), input_tensors{a} {}
 TBOperator::TBOperator(Graph *g, TBOperatorType t, STensor const &a, STensor const &b)
-    : bgraph(g), op_type(t) {
-  input_tensors.push_back(a);
-  input_tensors.push_back(b);
-}
+    : bgraph(g), op_type(t), input_tensors{a, b} {}
 TBOperator::TBOperator(Graph *g, TBOperatorType t, std::vector<STensor> const &ins)
     : bgraph(g), op_type(t), input_tensors(ins) {}
 TBOperator::~TBOperator() {}

@@ -1,9 +1,11 @@
 // _spec: builds a graph spec (workloads.py: a list of dicts) through the C facade of the host API.
 // A search builds a graph per candidate and drops it after one verification; through ctypes that was
 // a call, its argument conversions and a tensor query per operator: 18 us a graph, two thirds of a
-// candidate's cost.  Here the dicts are read where they are: 5 us.
+// candidate's cost.  Here the dicts are read where they are: 3.0 us (4.0 while the tensors' __init__ was called
+// and plans were copied into their operators).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <structmember.h>
 
 #include <cstring>
 #include <vector>
@@ -28,7 +30,7 @@ constexpr int kMaxOutputs = 4;
 struct Names {
   PyObject *op, *dims, *layout, *in, *dim, *size, *plan;
   PyObject *grid_dim, *block_dim, *output_map, *forloop_range, *reduction_dimx, *input_map, *forloop_dim,
-      *input_smem_layouts, *ops;
+      *input_smem_layouts, *ops, *h, *data_type, *guid;
 } names;
 
 struct Tables {  // of graph.py: name -> code
@@ -293,7 +295,30 @@ bool build_op(void *g, PyObject *op, Tables const &t, Built *built, int count) {
   return true;
 }
 
-PyObject *make_tensor(PyObject *type, void *handle) {
+// The slots of a tensor type, when all it does with its arguments is to keep them in __slots__: where they lie.
+struct TensorSlots {
+  Py_ssize_t at[4];  // _h, dims, data_type, guid
+  bool plain;
+};
+TensorSlots tensor_slots(PyObject *type) {
+  TensorSlots s = {{0, 0, 0, 0}, PyType_Check(type) != 0};
+  PyObject *const all[4] = {names.h, names.dims, names.data_type, names.guid};
+  PyTypeObject *const t = reinterpret_cast<PyTypeObject *>(type);
+  // (its own __init__ and no __new__: a class derived from it is called)
+  s.plain = s.plain && t->tp_base == &PyBaseObject_Type && t->tp_new == PyBaseObject_Type.tp_new;
+  for (int i = 0; s.plain && i < 4; i++) {
+    PyObject *const d = PyDict_GetItem(t->tp_dict, all[i]);
+    s.plain = d != nullptr && Py_IS_TYPE(d, &PyMemberDescr_Type);
+    if (s.plain) {
+      PyMemberDef const *const m = reinterpret_cast<PyMemberDescrObject *>(d)->d_member;
+      s.plain = m->type == T_OBJECT_EX;
+      s.at[i] = m->offset;
+    }
+  }
+  return s;
+}
+
+PyObject *make_tensor(PyObject *type, TensorSlots const &slots, void *handle) {
   int nd = 0, dims[4], dtype = 0, layout = 0;
   long long guid = 0;
   mirage_tensor_info(handle, &nd, dims, &dtype, &layout, &guid);
@@ -303,7 +328,15 @@ PyObject *make_tensor(PyObject *type, void *handle) {
   }
   PyObject *args[4] = {PyLong_FromVoidPtr(handle), shape, PyLong_FromLong(dtype), PyLong_FromLongLong(guid)};
   PyObject *x = nullptr;
-  if (args[0] != nullptr && args[1] != nullptr && args[2] != nullptr && args[3] != nullptr) {
+  bool const whole = args[0] != nullptr && args[1] != nullptr && args[2] != nullptr && args[3] != nullptr;
+  if (whole && slots.plain) {  // what its __init__ does, 0.2 us of interpreter a tensor
+    auto *const t = reinterpret_cast<PyTypeObject *>(type);
+    x = t->tp_alloc(t, 0);
+    for (int i = 0; x != nullptr && i < 4; i++) {
+      *reinterpret_cast<PyObject **>(reinterpret_cast<char *>(x) + slots.at[i]) = args[i];
+      args[i] = nullptr;
+    }
+  } else if (whole) {
     x = PyObject_Vectorcall(type, args, 4, nullptr);
   }
   for (PyObject *a : args) {
@@ -312,16 +345,29 @@ PyObject *make_tensor(PyObject *type, void *handle) {
   return x;
 }
 
-// build(graph handle, spec, tensor type, tables) -> list per operator of its output tensors
-PyObject *build(PyObject *, PyObject *args) {
-  unsigned long long graph;
-  PyObject *spec, *tensor;
-  Tables t;
-  if (!PyArg_ParseTuple(args, "KO!OO!O!O!O!O", &graph, &PyList_Type, &spec, &tensor, &PyDict_Type, &t.dmem_layout, &PyDict_Type,
-                        &t.smem_layout, &PyDict_Type, &t.kn_op, &PyDict_Type, &t.tb_op, &t.infeasible)) {
+// build(graph handle, spec, tensor type, four tables, exception) -> list per operator of its output tensors
+PyObject *build(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  if (nargs != 8 || !PyList_Check(args[1])) {
+    PyErr_SetString(PyExc_TypeError, "a graph handle, a list, a type, four dicts and an exception are expected");
     return nullptr;
   }
+  unsigned long long const graph = PyLong_AsUnsignedLongLong(args[0]);
+  if (graph == (unsigned long long)-1 && PyErr_Occurred()) {
+    return nullptr;
+  }
+  PyObject *const spec = args[1], *const tensor = args[2];
+  Tables t;
+  PyObject **const tables[4] = {&t.dmem_layout, &t.smem_layout, &t.kn_op, &t.tb_op};
+  for (int i = 0; i < 4; i++) {
+    *tables[i] = args[3 + i];
+    if (!PyDict_Check(*tables[i])) {
+      PyErr_SetString(PyExc_TypeError, "a table is a dict");
+      return nullptr;
+    }
+  }
+  t.infeasible = args[7];
   Py_ssize_t const n = PyList_GET_SIZE(spec);
+  TensorSlots const slots = tensor_slots(tensor);
   std::vector<Built> built((size_t)n);
   PyObject *all = PyList_New(n);
   if (all == nullptr) {
@@ -345,7 +391,7 @@ PyObject *build(PyObject *, PyObject *args) {
     }
     PyList_SET_ITEM(all, i, outs);
     for (int j = 0; j < built[i].n; j++) {
-      PyObject *x = make_tensor(tensor, built[i].out[j]);
+      PyObject *x = make_tensor(tensor, slots, built[i].out[j]);
       if (x == nullptr) {
         Py_DECREF(all);
         return nullptr;
@@ -356,7 +402,8 @@ PyObject *build(PyObject *, PyObject *args) {
   return all;
 }
 
-PyMethodDef methods[] = {{"build", build, METH_VARARGS, "Builds a graph spec; one list of output tensors per operator."},
+PyMethodDef methods[] = {{"build", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(build)), METH_FASTCALL,
+                          "Builds a graph spec; one list of output tensors per operator."},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_spec", "Graph specs read in native code.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
@@ -370,7 +417,7 @@ PyMODINIT_FUNC PyInit__spec(void) {
                    {&names.size, "size"}, {&names.plan, "plan"}, {&names.grid_dim, "grid_dim"}, {&names.block_dim, "block_dim"},
                    {&names.output_map, "output_map"}, {&names.forloop_range, "forloop_range"},
                    {&names.reduction_dimx, "reduction_dimx"}, {&names.input_map, "input_map"}, {&names.forloop_dim, "forloop_dim"},
-                   {&names.input_smem_layouts, "input_smem_layouts"}, {&names.ops, "ops"}};
+                   {&names.input_smem_layouts, "input_smem_layouts"}, {&names.ops, "ops"}, {&names.h, "_h"}, {&names.data_type, "data_type"}, {&names.guid, "guid"}};
   for (auto const &n : all) {
     *n.slot = PyUnicode_InternFromString(n.text);
     if (*n.slot == nullptr) {

@@ -16,8 +16,8 @@ public:
   // Builds the thread-block graph from a plan: one input loader per tensor, the
   // plan's operators in order, then one accumulating output per tile that no
   // later operator consumes (reference src/kernel/customized.cc:65-186).
-  KNCustomizedOp(std::vector<DTensor> const &inputs,
-                 mirage::threadblock::ExecutionPlan const &plan);
+  // (by value: a caller that has no more use for them moves them in)
+  KNCustomizedOp(std::vector<DTensor> inputs, mirage::threadblock::ExecutionPlan plan);
   // Rebuilds an existing thread-block graph over new inputs and recovers its plan.
   KNCustomizedOp(std::vector<DTensor> const &inputs, mirage::threadblock::Graph const &_graph);
   virtual ~KNCustomizedOp();

@@ -2,10 +2,12 @@
 mirage:: API (host-only runtime), lowering against the oracle's restatement, the
 soft-failure contract, the LIFO arena, and the C ABI's symbols."""
 import ctypes
+import gc
 import os
 import re
 import subprocess
 import sys
+import weakref
 
 import numpy as np
 import pytest
@@ -287,6 +289,30 @@ def _all_specs():
     for name in sorted(W.BASELINE_CONFIGS):
         yield from (s for s in W.BASELINE_CONFIGS[name]() if s is not None)
     yield from load_gqa_fixture()["generated_graphs"]
+
+
+def test_extension_makes_whole_tensors():
+    """Tensors made without their __init__ are like any others; a derived class has its own called."""
+    native, _ = _readers()
+    made = []
+
+    class Counted(G.DTensor):
+        def __init__(self, *args):
+            made.append(args)
+            super().__init__(*args)
+
+    spec = next(_all_specs())
+    with G.KNGraph() as g:
+        first = native(g, spec)[0][0]
+        assert (first.dims, first.data_type, first.guid, first.layout) == first._info()
+        gone, refs = weakref.ref(first), sys.getrefcount(G.DTensor)
+        assert gc.is_tracked(first)
+        del first
+        gc.collect()
+        assert gone() is None and sys.getrefcount(G.DTensor) <= refs
+    with G.KNGraph() as g:
+        vals = N.spec().build(g._g.value, spec, Counted, G.DMEM_LAYOUT, G.SMEM_LAYOUT, G.KN_OP, G.TB_OP, G.InfeasibleOperator)
+        assert len(made) == sum(len(v) for v in vals) and all(type(t) is Counted for v in vals for t in v)
 
 
 def test_readers_build_the_same_graphs():
