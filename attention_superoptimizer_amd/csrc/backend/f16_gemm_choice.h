@@ -19,7 +19,7 @@ struct GemmTile {
 constexpr GemmTile kGemmTiles[] = {
     {STAGED, 16, 64, 16, 16, 1}, {STAGED, 16, 64, 16, 16, 2},  {STAGED, 32, 64, 32, 16, 1},  {STAGED, 32, 64, 32, 16, 2},
     {STAGED, 64, 64, 32, 32, 1}, {STAGED, 64, 64, 32, 32, 2},  {STAGED, 64, 128, 32, 64, 1}, {STAGED, 64, 128, 32, 64, 2},
-    {STAGED, 128, 128, 64, 64, 1}, {DIRECT, 64, 64, 32, 32, 1}, {DIRECT, 64, 128, 32, 64, 1}, {DIRECT, 128, 64, 64, 32, 1},
+    {STAGED, 128, 128, 64, 64, 1}, {DIRECT, 64, 64, 32, 32, 1}, {DIRECT, 64, 128, 32, 32, 1}, {DIRECT, 128, 64, 64, 32, 1},
     {WAVES, 16, 64, 16, 64, 4},  {WAVES, 32, 64, 32, 64, 4}};
 // A column-major (a layout search may ask for one): the middle tiles
 constexpr GemmTile kGemmTilesColumnMajorA[] = {{STAGED, 64, 64, 32, 32, 1}, {STAGED, 64, 64, 32, 32, 2}};
@@ -46,7 +46,10 @@ struct GemmChoice {
 // with the compute units full, what they have to move: 128-byte rows through the vector cache, into
 // LDS and from there to the operands, and the matrix instructions.  k ranges need a second launch.
 // (The kernels that load LDS directly: 3.2 us, and 35 bytes a cycle per compute unit; a lone workgroup
-// waits 1.4 times as long for a stage, but not where wavefronts go their own ways.  15 shapes, within 15 %.
+// waits 1.4 times as long for a stage, but not where wavefronts go their own ways, and 1.25 with eight of them: two on
+// a SIMD read operands under each other's products (64 x 128 tiles by four wavefronts and by eight: [300, 2048] .
+// [2048, 5504] row-major 14.7 and 13.4 us, column-major 13.8 and 12.7, [300, 5504] . [5504, 2048] in three ranges 20.0
+// and 17.2; 64 x 64 there 14.1, 13.9 and 18.8; with 1.0 [256, 4096] . [4096, 4096] went to two ranges, 18.3 -> 19.4).  15 shapes, within 15 %.
 // The rings of f16_gemm_waves_kernel leave room for one or two workgroups on a compute unit: those that
 // queue there pay their first loads and the adding up again, 1.3 us: [200, 130, 96] . [200, 96, 130] 23.8 us
 // on it, 9 on 64 x 64.)
@@ -57,7 +60,7 @@ inline double gemm_tile_cost(GemmTile const &t, int batch, int m, int n, int k, 
     if (t.kind == WAVES || per_cu < 3.0) {
       per_cu = std::ceil(per_cu);  // (the compute unit with the most workgroups is the last to finish)
     }
-    double us = 3.2 + stages * stage * std::max(per_cu, t.kind == DIRECT ? 1.4 : 1.0) + per_cu * 0.9e-4 * t.bm * t.bn;
+    double us = 3.2 + stages * stage * std::max(per_cu, t.kind == WAVES ? 1.0 : t.threads() < 512 ? 1.4 : 1.25) + per_cu * 0.9e-4 * t.bm * t.bn;
     if (t.kind == WAVES) {
       int const resident = 160 * 1024 / (4 * kWavesRing * (t.bm + t.bn) * 64);
       us += 1.3 * (std::ceil(per_cu / resident) - 1.0);

@@ -48,6 +48,22 @@ def _matmul(abi, A, B, batch, m, n, k, a_cm, b_cm):
     return C[64:-64].view(batch, m, n).float(), torch.bmm(Af, Bf)
 
 
+@pytest.mark.parametrize("b_cm", [0, 1])
+@pytest.mark.parametrize("batch,m,n,k", [
+    (1, 129, 3336, 3264),  # 64 x 128 tiles of eight wavefronts in k ranges: a row and eight columns over
+    (1, 300, 5504, 2048),  # one range
+    (4, 166, 2616, 1024),
+    (2, 191, 3272, 1216),  # a row short of a tile, 19 stages
+])
+def test_wide_tiles_in_one_round(rt, abi, batch, m, n, k, b_cm):
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A = torch.randn(batch, m, k, device="cuda", generator=gen).half()
+    B = torch.randn((batch, n, k) if b_cm else (batch, k, n), device="cuda", generator=gen).half()
+    got, want = _matmul(abi, A, B, batch, m, n, k, 0, b_cm)
+    # a rounding to fp16, and a sum of k products in fp32: at most k roundings of partial sums of about sqrt(k)
+    assert (got - want).abs().max().item() <= 2**-11 * want.abs().max().item() + 2 * k * 2**-24 * k**0.5
+
+
 @pytest.mark.parametrize("batch,m,n,k,a_cm,b_cm", [
     (32, 500, 1000, 32, 0, 1),    # one step of the 256 x 256 kernel, ragged tiles
     (1, 4090, 4096, 64, 0, 1),    # two
