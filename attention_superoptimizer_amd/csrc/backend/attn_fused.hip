@@ -563,6 +563,7 @@ static bool make_fold(AttnParams const &A, Match const &M, DevProgram const &P, 
   out.X = R.X;
   out.o_cols = R.o_cols;
   out.mxv = fast_div_magic(R.X / 4);
+  out.after = R.mode == SUM_THEN_DIV ? -0.0f : 0.0f;
   out.tickets = nullptr;
   if (R.S > 1) {
     int const per_cu = std::max(1, std::min(state().max_lds / std::max(lds, 1), 1024 / threads));

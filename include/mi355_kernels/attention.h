@@ -1700,7 +1700,7 @@ __global__ __launch_bounds__(64 * IP) void attn_direct_kernel(Params const) {
       _Float16 *const to = next.o + fold_row(next, bx, by, bz, row_base + out_row) * next.o_cols + out_col;
 #pragma unroll
       for (int e = 0; e < EPT / 2; e++) {
-        half2v const q = {fold_own(acc[e][0], sum), fold_own(acc[e][1], sum)};
+        half2v const q = {fold_own(next, acc[e][0], sum), fold_own(next, acc[e][1], sum)};
         store_result_4(to + 2 * e, __builtin_bit_cast(uint32_t, q), false);
       }
       if (out_col == 0) {

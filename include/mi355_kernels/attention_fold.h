@@ -25,6 +25,7 @@ struct AttnFold {
   int arrivals;           // workgroups that have pieces of a row block
   int S, X, o_cols;
   uint32_t mxv;  // division magic of X / 4
+  float after;   // -0, what leaves a quotient as it is, or +0, what a sum or a saver behind the division begins with
 };
 
 // Memory as global memory (a flat access counts as an LDS operation too).  A result that a workgroup on another
@@ -72,10 +73,11 @@ __device__ __forceinline__ void store_result_2(_Float16 *p, _Float16 v, bool sha
 __device__ __forceinline__ long long fold_row(AttnFold const &F, int bx, int by, int bz, int row_base) {
   return (long long)bx * F.lin[0] + (long long)by * F.lin[1] + (long long)bz * F.lin[2] + row_base;
 }
-// combine_fused_kernel's arithmetic where it sums before it divides (with one piece its other forms come to the same).
-// One piece a row, this workgroup's own: the quotient of a column that it stores and of the row's sum.
-__device__ __forceinline__ _Float16 fold_own(_Float16 n, _Float16 sum) {
-  return static_cast<_Float16>((0.0f + static_cast<float>(n)) / (0.0f + static_cast<float>(sum)));
+// combine_fused_kernel's arithmetic.  One piece a row, this workgroup's own: the quotient of a column that it stores and
+// of the row's sum.  With one piece all its forms come to the same but for the sign of a zero (a negative number over
+// an infinite sum, or a quotient past the smallest number): what divides before it sums adds the quotient to +0.
+__device__ __forceinline__ _Float16 fold_own(AttnFold const &F, _Float16 n, _Float16 sum) {
+  return static_cast<_Float16>((0.0f + static_cast<float>(n)) / (0.0f + static_cast<float>(sum))) + static_cast<_Float16>(F.after);
 }
 __device__ __forceinline__ void fold_own_chunk(AttnFold const &F, long long row, int x, fold_uint4 n, _Float16 sum) {
   typedef _Float16 half8v __attribute__((ext_vector_type(8)));
@@ -83,12 +85,12 @@ __device__ __forceinline__ void fold_own_chunk(AttnFold const &F, long long row,
   half8v out;
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    out[j] = fold_own(v[j], sum);
+    out[j] = fold_own(F, v[j], sum);
   }
   store_result_16(F.o + row * F.o_cols + x, __builtin_bit_cast(fold_uint4, out), false);
 }
 
-// The same of S <= PIECES pieces a row, most of them other workgroups'.  All of a thread's loads go out together:
+// The same of S <= PIECES pieces a row, most of them other workgroups', summed before the division.  All of a thread's loads go out together:
 // from the memory that all XCDs share a trip is a microsecond.  `lds`: room for rows x S row sums.
 constexpr int kFoldPieces = 16;
 template <int PIECES>

@@ -99,6 +99,20 @@ def test_places_of_the_division(rt, ops, folds):
     _check(rt, _prefill(2, 64, 3, 64, 64, 5, COL, ops), folds)
 
 
+@pytest.mark.parametrize("order", [COL, ROW])
+@pytest.mark.parametrize("shape", [(2, 64, 3, 64, 64, 5), (3, 48, 3, 64, 48, 7), (16, 128, 32, 64, 64, 4), (2, 64, 3, 128, 64, 3)])
+@pytest.mark.parametrize("ops,sign", [
+    (W.COMBINE_OPS, True),
+    ([("tb_reduction_2_op", [(1, 0)]), ("tb_div_op", [(0, 0), (2, 0)])], False),
+    ([("tb_div_op", [(0, 0), (1, 0)])], False),
+    ([("tb_reduction_2_op", [(1, 0)]), ("tb_div_op", [(0, 0), (2, 0)]), ("tb_reduction_2_to_dimx_op", [(3, 0)])], False)])
+def test_signs_of_zero(rt, ops, sign, shape, order):
+    """Negative numerators over infinite row sums: the quotient is -0, and stays it where nothing is added to it
+    behind the division; a sum or a saver behind it begins with +0.  On every kernel that divides as it stores."""
+    out = _check(rt, _prefill(*shape, order, ops), True, std=0.7, passes=1).view(np.uint16)
+    assert (out == 0).any() and (out == 0x8000).any() == sign
+
+
 @pytest.mark.parametrize("spec", [_decode(2, 16, 64, 4, 4, COL), _prefill(4, 128, 2, 64, 64, 4, COL), _prefill(3, 48, 3, 64, 48, 3, ROW)])
 def test_infinities_and_nan(rt, spec):
     """Scores past the exponential's range: infinite row sums, infinity over infinity, zero over zero."""
