@@ -10,6 +10,7 @@
 #include "mirage/kernel/graph.h"
 #include "mirage/utils/hip_types.h"
 
+#include <algorithm>
 #include <cstring>
 
 using namespace mirage;
@@ -81,11 +82,12 @@ int mirage_graph_customized(void *g, void *const *inputs, int num_inputs, mirage
   plan.reduction_dimx = p->reduction_dimx;
   plan.output_map = {p->output_map[0], p->output_map[1], p->output_map[2]};
   std::vector<DTensor> ins;
-  ins.reserve(num_inputs);
-  plan.input_map.reserve(num_inputs);
-  plan.forloop_dim.reserve(num_inputs);
-  plan.input_smem_layouts.reserve(num_inputs);
-  plan.ops.reserve(p->num_ops);
+  auto room = [](int count) { return (size_t)std::max(count, 0); };  // (a negative count is none, and nothing is thrown from here)
+  ins.reserve(room(num_inputs));
+  plan.input_map.reserve(room(num_inputs));
+  plan.forloop_dim.reserve(room(num_inputs));
+  plan.input_smem_layouts.reserve(room(num_inputs));
+  plan.ops.reserve(room(p->num_ops));
   for (int i = 0; i < num_inputs; i++) {
     ins.push_back(*static_cast<DTensor *>(inputs[i]));
     plan.input_map.push_back({p->input_map[i][0], p->input_map[i][1], p->input_map[i][2]});
@@ -94,16 +96,13 @@ int mirage_graph_customized(void *g, void *const *inputs, int num_inputs, mirage
   }
   for (int i = 0; i < p->num_ops; i++) {
     std::vector<std::pair<int, int>> operands;
-    operands.reserve(p->op_num_operands[i]);
+    operands.reserve(room(p->op_num_operands[i]));
     for (int j = 0; j < p->op_num_operands[i]; j++) {
       operands.push_back({p->op_operands[i][j][0], p->op_operands[i][j][1]});
     }
     plan.ops.emplace_back((type::TBOperatorType)p->op_type[i], std::move(operands));
   }
   KNOperator *op = new kernel::KNCustomizedOp(std::move(ins), std::move(plan));
-  if (op == nullptr) {
-    return -1;
-  }
   G->operators.push_back(op);
   int n = (int)op->output_tensors.size();
   for (int i = 0; i < n && i < max_outputs; i++) {

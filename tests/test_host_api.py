@@ -291,6 +291,25 @@ def _all_specs():
     yield from load_gqa_fixture()["generated_graphs"]
 
 
+def test_negative_counts_are_none():
+    """A plan whose counts are negative has no operators (no inputs): it builds an operator without results, in a
+    process that goes on."""
+    code = """
+import ctypes
+from attention_superoptimizer_amd import graph as G, _native as N, workloads as W
+spec, _ = W.tiled_matmul(128, 256, 256, (2, 4, 1), 4, (0, -1, -1), (-1, 1, -1), (0, 1, -1))
+with G.KNGraph() as g:
+    ins = (ctypes.c_void_p * 2)(g.new_input((128, 256))._h, g.new_input((256, 256))._h)
+    outs = (ctypes.c_void_p * 4)()
+    for inputs in (2, 0, -1):
+        cp = G._c_plan(spec[2]["plan"])
+        cp.num_ops, cp.num_inputs = -1, inputs
+        print(N.runtime().mirage_graph_customized(g._g, ins, inputs, ctypes.byref(cp), outs, 4), end=" ")
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, env=dict(os.environ, MIRAGE_HOST_ONLY="1"))
+    assert r.returncode == 0 and r.stdout.split() == ["0", "0", "0"], r.stderr
+
+
 def test_extension_makes_whole_tensors():
     """Tensors made without their __init__ are like any others; a derived class has its own called."""
     native, _ = _readers()
