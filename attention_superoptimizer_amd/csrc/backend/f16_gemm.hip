@@ -602,6 +602,9 @@ extern "C" int mi355_f16_matmul_then(void const *A, void const *B, void *C, int 
 extern "C" int mi355_f16_matmul_two(void const *A, int a_column_major, int b_column_major, int batch, int m, int n, int k,
                                     mi355_matmul_out const *first, mi355_matmul_out const *second, int *taken) {
   MI355_REQUIRE_INIT();
+  if (first == nullptr || second == nullptr || taken == nullptr) {
+    return fail(MI355_ERR_INVALID, "no products or no place for the answer");
+  }
   *taken = 0;
   AnyGemm G{};
   G.A = static_cast<_Float16 const *>(A);

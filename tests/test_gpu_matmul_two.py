@@ -1,6 +1,8 @@
 """Two kernel-level matmuls of one input, with the element-wise operators that consume them, when a graph runs as a
 whole (KNGraph.execute_all): the products against the fp64 oracle, what consumes them bit for bit against the same
 operators run one by one on those products."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -10,6 +12,11 @@ from oracle import evaluate as orc
 
 pytestmark = pytest.mark.gpu
 ROW, COL = "DmemRowMajor", "DmemColumnMajor"
+
+
+class MatmulOut(ctypes.Structure):  # mi355_matmul_out
+    _fields_ = [("B", ctypes.c_void_p), ("C", ctypes.c_void_p), ("op", ctypes.c_int), ("x_first", ctypes.c_int),
+                ("X", ctypes.c_void_p), ("E", ctypes.c_void_p)]
 
 
 def _check(rt, b, m, n, k, order, form, a_order=ROW, ins=None, finite=True):
@@ -76,3 +83,10 @@ def test_infinities_and_nan(rt, m, n, k, order):
         np.testing.assert_array_equal(np.isnan(c[0]), np.isnan(want))
         inf = np.isinf(want)
         np.testing.assert_array_equal(c[0][inf], want[inf])
+
+
+def test_missing_products_and_place(rt, abi):
+    out, taken = MatmulOut(), ctypes.c_int()
+    for args in ((None, ctypes.byref(out), ctypes.byref(taken)), (ctypes.byref(out), None, ctypes.byref(taken)),
+                 (ctypes.byref(out), ctypes.byref(out), None)):
+        assert abi.mi355_f16_matmul_two(None, 0, 0, 1, 16, 64, 64, *args) == -3  # MI355_ERR_INVALID
