@@ -467,7 +467,7 @@ double stream_ns(DevProgram const &P, GMatch const &G, StreamPlan const &plan, l
   return ns;
 }
 
-// `gate`: see GateRequest; *gated tells whether the launch takes care of it.  `R`: the program as the choice sees it, G but
+// `gate`: see GateRequest; *gated tells whether a launch was made that takes care of it.  `R`: the program as the choice sees it, G but
 // for a row-major second operator of such a pair, which runs where it would run by itself: without its prologue no
 // kernel is slower than with it (2 rows x 576 x 6528 14.8 us before and so, 16.8 in the kernel of a plain product).
 int try_launch_lanes(DevProgram const &P, GMatch const &G, GMatch const &R, GemmParams const &A, _Float16 *gate, bool *gated) {
@@ -593,7 +593,6 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GMatch const &R, Gemm
   L.rank = G.rank;
   L.slot_base = ip * wave_bytes;
   L.g.gate = gate;
-  *gated = gate != nullptr;
   L.m_group = fast_div_magic(8 * S);
   L.m_pieces = fast_div_magic(S);
   L.m_columns = fast_div_magic(pieces);
@@ -615,6 +614,7 @@ int try_launch_lanes(DevProgram const &P, GMatch const &G, GMatch const &R, Gemm
   MI355_LANES_CASE(1, PRO_NONE, 2)
 #undef MI355_LANES_CASE
   if (rc == 1) {
+    *gated = gate != nullptr;
     s.last().kernel_id = MI355_KERNEL_F16_GEMM;
     s.last().workgroups = grid;
     s.last().threads = ip * 64;
@@ -691,8 +691,8 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A,
   L.results = plan.ring;
   L.strips = plan.strips;
   // (whole blocks of one weight meet in no workgroup, and no more do sums past the fold's LDS)
-  *gated = gate != nullptr && (plan.strips || (ks == 1 ? plan.pairs : P.forloop_range * 2048 <= s.max_lds));
-  L.g.gate = *gated ? gate : nullptr;
+  bool const takes_gate = gate != nullptr && (plan.strips || (ks == 1 ? plan.pairs : P.forloop_range * 2048 <= s.max_lds));
+  L.g.gate = takes_gate ? gate : nullptr;
   dim3 const grid(P.grid[0] * plan.groups, P.grid[1], P.grid[2]);
   int rc = 0;
   if (plan.pairs) {
@@ -720,6 +720,7 @@ int try_launch_stream(DevProgram const &P, GMatch const &G, GemmParams const &A,
     rc = launch_combine(L.g, G.nb, dim3(P.grid[0], P.grid[1], P.grid[2]));
   }
   if (rc == 1) {
+    *gated = takes_gate;
     s.last().kernel_id = MI355_KERNEL_F16_GEMM;
     s.last().workgroups = grid.x * grid.y * grid.z;
     s.last().threads = 256;
