@@ -30,7 +30,7 @@ constexpr int kMaxOutputs = 4;
 struct Names {
   PyObject *op, *dims, *layout, *in, *dim, *size, *plan;
   PyObject *grid_dim, *block_dim, *output_map, *forloop_range, *reduction_dimx, *input_map, *forloop_dim,
-      *input_smem_layouts, *ops, *h, *data_type, *guid;
+      *input_smem_layouts, *ops, *h, *data_type, *guid, *init, *keeping_init;
 } names;
 
 struct Tables {  // of graph.py: name -> code
@@ -295,7 +295,7 @@ bool build_op(void *g, PyObject *op, Tables const &t, Built *built, int count) {
   return true;
 }
 
-// The slots of a tensor type, when all it does with its arguments is to keep them in __slots__: where they lie.
+// The slots of a tensor type that says its __init__ only keeps its arguments in them: where they lie.
 struct TensorSlots {
   Py_ssize_t at[4];  // _h, dims, data_type, guid
   bool plain;
@@ -304,8 +304,13 @@ TensorSlots tensor_slots(PyObject *type) {
   TensorSlots s = {{0, 0, 0, 0}, PyType_Check(type) != 0};
   PyObject *const all[4] = {names.h, names.dims, names.data_type, names.guid};
   PyTypeObject *const t = reinterpret_cast<PyTypeObject *>(type);
-  // (its own __init__ and no __new__: a class derived from it is called)
-  s.plain = s.plain && t->tp_base == &PyBaseObject_Type && t->tp_new == PyBaseObject_Type.tp_new;
+  // (no other slots to fill, no __new__, and the __init__ it says so of is the one it has: any other type is called)
+  s.plain = s.plain && t->tp_base == &PyBaseObject_Type && t->tp_new == PyBaseObject_Type.tp_new &&
+            t->tp_basicsize == (Py_ssize_t)(sizeof(PyObject) + (4 + (t->tp_weaklistoffset != 0)) * sizeof(PyObject *));
+  if (s.plain) {
+    PyObject *const init = PyDict_GetItem(t->tp_dict, names.init);
+    s.plain = init != nullptr && init == PyDict_GetItem(t->tp_dict, names.keeping_init);
+  }
   for (int i = 0; s.plain && i < 4; i++) {
     PyObject *const d = PyDict_GetItem(t->tp_dict, all[i]);
     s.plain = d != nullptr && Py_IS_TYPE(d, &PyMemberDescr_Type);
@@ -417,7 +422,8 @@ PyMODINIT_FUNC PyInit__spec(void) {
                    {&names.size, "size"}, {&names.plan, "plan"}, {&names.grid_dim, "grid_dim"}, {&names.block_dim, "block_dim"},
                    {&names.output_map, "output_map"}, {&names.forloop_range, "forloop_range"},
                    {&names.reduction_dimx, "reduction_dimx"}, {&names.input_map, "input_map"}, {&names.forloop_dim, "forloop_dim"},
-                   {&names.input_smem_layouts, "input_smem_layouts"}, {&names.ops, "ops"}, {&names.h, "_h"}, {&names.data_type, "data_type"}, {&names.guid, "guid"}};
+                   {&names.input_smem_layouts, "input_smem_layouts"}, {&names.ops, "ops"}, {&names.h, "_h"}, {&names.data_type, "data_type"}, {&names.guid, "guid"},
+                   {&names.init, "__init__"}, {&names.keeping_init, "_keeping_init"}};
   for (auto const &n : all) {
     *n.slot = PyUnicode_InternFromString(n.text);
     if (*n.slot == nullptr) {

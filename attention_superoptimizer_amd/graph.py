@@ -63,6 +63,10 @@ class DTensor:
             dims, data_type, guid, _ = self._info()
         self.dims, self.data_type, self.guid = dims, data_type, guid
 
+    # Given all four, this __init__ keeps them in the slots and does nothing else: csrc/python/spec.cc then fills the
+    # slots itself and does not call it.  Not so any more?  Then this name goes.
+    _keeping_init = __init__
+
     def _info(self):
         nd, dt, lay = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         dims = (ctypes.c_int * 4)()

@@ -334,6 +334,42 @@ def test_extension_makes_whole_tensors():
         assert len(made) == sum(len(v) for v in vals) and all(type(t) is Counted for v in vals for t in v)
 
 
+def _build_as(cls):
+    spec = next(_all_specs())
+    with G.KNGraph() as g:
+        vals = N.spec().build(g._g.value, spec, cls, G.DMEM_LAYOUT, G.SMEM_LAYOUT, G.KN_OP, G.TB_OP, G.InfeasibleOperator)
+        return [(type(t), {n for n in ("_h", "dims", "data_type", "guid", "more") if hasattr(t, n)}) for v in vals for t in v]
+
+
+def test_extension_calls_an_init_that_does_more(monkeypatch):
+    """Only the __init__ that the class says keeps its arguments is passed by."""
+    _readers()
+    made = []
+
+    def slots(*more):
+        def init(self, handle, dims, data_type, guid):
+            made.append(guid)
+            self._h, self.dims, self.data_type, self.guid = handle, dims, data_type, guid
+            for name in more:
+                setattr(self, name, 0)
+        return {"__slots__": ("_h", "dims", "data_type", "guid", *more), "__init__": init}
+
+    kept = {"_h", "dims", "data_type", "guid"}
+    assert all(t == (G.DTensor, kept) for t in _build_as(G.DTensor)) and not made
+    other, wider = type("Other", (), slots()), type("Wider", (), slots("more"))
+    promising = slots("more")
+    promising = type("Promising", (), dict(promising, _keeping_init=promising["__init__"]))
+    for cls, names in ((other, kept), (wider, kept | {"more"}), (promising, kept | {"more"})):
+        made.clear()
+        tensors = _build_as(cls)
+        assert len(made) == len(tensors) and all(t == (cls, names) for t in tensors)
+    made.clear()
+    keep = G.DTensor.__init__
+    monkeypatch.setattr(G.DTensor, "__init__", lambda self, *args: (made.append(args), keep(self, *args))[1])
+    tensors = _build_as(G.DTensor)
+    assert len(made) == len(tensors) and all(t == (G.DTensor, kept) for t in tensors)
+
+
 def test_readers_build_the_same_graphs():
     native, python = _readers()
     n = 0
