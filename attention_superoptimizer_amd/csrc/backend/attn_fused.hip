@@ -508,14 +508,22 @@ bool attention_applicable(DevProgram const &P) {
 // What the next operator's fold of rows is to this launch: a workgroup's rows, and the places of its
 // results in them.  False where the operator is no fold of exactly these results, row by row.
 //
-// With whole rows in a workgroup it always pays: both launches of [12, 1040, 1040] in tiles of 80 18.8 -> 16.4 us, of
-// [32, 2048, 2048] at head size 128 78.8 -> 75.5 (both tensors' stores are what is left), 86 prefill plans 0.78 of the
-// time in the mean, 0.53 - 0.99.  Where the pieces come from several workgroups the last of them pays three trips to the
+// With whole rows in a workgroup it always pays: both launches of [12, 1040, 1040] in tiles of 80 18.8 -> 16.5 us, of
+// [32, 2048, 2048] at head size 128 78.5 -> 75.6 (both tensors' stores are what is left), 60 prefill plans 0.76 of the
+// time on the device in the mean, none above 1.  Where the pieces come from several workgroups the last of them pays three trips to the
 // memory that all XCDs share (its stores, its ticket, the pieces), 3 us against the 3.5 - 4.5 of a launch, and all others two while
 // they hold their place on a compute unit.  So: blocks that run in one round (64 groups of 16 blocks, two rounds, 50.8
 // us either way, folded 52.1), as many columns of threads as there are columns, and sixteen pieces, what a thread loads
-// together (7 groups of 16 rows, 20 pieces, one wavefront 8.8 us, folded 12.5).  135 split-KV plans 0.94 of the time
-// in the mean, 0.77 - 1.05; [5, 12, 64] against 12 pieces of 5 tiles of 48 keys 8.4 -> 7.7.
+// together (7 groups of 16 rows, 20 pieces, one wavefront 8.8 us, folded 12.5).
+// Nor where the other launch is short and many workgroups pay for it.  It adds up pieces in batches of four, or of sixteen
+// where there are so many (combine.h), and what is left over piece by piece: for four and sixteen, and for two, it has one
+// trip to make.  Of one row each there is little but that trip: from 32 workgroups on 46 plans of four or sixteen pieces take
+// 1.05 of the time on the device in the mean when folded (16 groups, 4 pieces of 10 tiles of 16 keys 8.23 / 8.73 us, 33
+// groups, 16 pieces of a tile of 48 7.85 / 8.96), 14 of two 1.01; other numbers of pieces less.  Of more rows so it is for
+// sixteen pieces and more than 128 workgroups, 40 plans 1.08 (20 groups of 16 rows, 7 tiles of 16 keys 9.11 / 11.02; 95 with
+// up to 128 0.97); for 4, 8 and 12 pieces and more than 192 workgroups it comes to the same, 0.90 - 1.14 of the time.
+// 435 other drawn split-KV plans 0.92 of the time on the device in the mean, 0.60 - 1.08, twenty above 1.01.
+// [5, 12, 64] against 12 pieces of 5 tiles of 48 keys 8.4 -> 7.9.
 static bool make_fold(AttnParams const &A, Match const &M, DevProgram const &P, int wg_rows, int threads, int lds, FoldRequest &f,
                       AttnFold &out) {
   RowFold const &R = f.rows;
@@ -568,8 +576,12 @@ static bool make_fold(AttnParams const &A, Match const &M, DevProgram const &P, 
   if (R.S > 1) {
     int const per_cu = std::max(1, std::min(state().max_lds / std::max(lds, 1), 1024 / threads));
     int const trips = (std::min(wg_rows, M.m) * R.X / 4 + threads - 1) / threads;
-    if (R.S > kFoldPieces || trips > (R.S <= 8 ? 2 : 1) || wg_rows * R.S * 2 + 16 > lds ||
-        (long long)P.grid[0] * P.grid[1] * P.grid[2] * A.split > 256 * per_cu) {
+    long long const workgroups = (long long)P.grid[0] * P.grid[1] * P.grid[2] * A.split;
+    if (R.S > kFoldPieces || trips > (R.S <= 8 ? 2 : 1) || wg_rows * R.S * 2 + 16 > lds || workgroups > 256 * per_cu) {
+      return false;
+    }
+    bool const one_trip = R.S == 2 || R.S == 4 || R.S == 16;  // of the other launch
+    if ((M.m == 1 && one_trip && workgroups >= 32) || (R.S == 16 && workgroups > 128) || (R.S % 4 == 0 && workgroups > 192)) {
       return false;
     }
     out.tickets = f.tickets(R.rows / M.m * A.split);

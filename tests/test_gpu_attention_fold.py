@@ -77,6 +77,15 @@ def test_pieces_of_several_workgroups(rt, groups, rows, keys, blocks, loop, fold
     _check(rt, _decode(groups, rows, keys, blocks, loop, order), folds)
 
 
+@pytest.mark.parametrize("groups,rows,keys,blocks,loop,folds", [
+    (7, 1, 64, 4, 5, True), (8, 1, 64, 4, 5, False), (8, 1, 64, 5, 5, True), (16, 1, 48, 2, 3, False), (2, 1, 32, 16, 3, False),
+    (1, 1, 32, 16, 3, True), (8, 16, 64, 16, 4, True), (9, 16, 64, 16, 4, False), (9, 2, 80, 16, 2, False), (9, 2, 80, 15, 2, True),
+    (24, 8, 64, 8, 4, True), (25, 8, 64, 8, 4, False), (25, 8, 64, 9, 4, True)])
+def test_where_the_other_launch_is_short(rt, groups, rows, keys, blocks, loop, folds):
+    """Few pieces of one row, and sixteen of more: two launches from so many workgroups on."""
+    _check(rt, _decode(groups, rows, keys, blocks, loop, ROW), folds)
+
+
 # heads, row tile, row blocks, head size, key tile, for-loop: the streaming kernel (128- and 64-row slabs, 256-row
 # ones, wide key tiles), the one for whole tiles, the one with a tile pair a wavefront, the one for any size
 PREFILL = [(16, 128, 32, 64, 64, 4), (32, 128, 16, 128, 64, 2), (32, 64, 16, 64, 64, 3), (4, 256, 130, 64, 64, 2), (4, 128, 8, 128, 256, 2),
