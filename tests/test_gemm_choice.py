@@ -1,8 +1,11 @@
 """The kernel a kernel-level fp16 matmul is given (csrc/backend/f16_gemm_choice.h), without a device."""
 import os
+import random
 import subprocess
 
 import pytest
+
+from test_gpu_matmul_two import COL, SHAPES, TAKEN
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 STAGED, DIRECT, WAVES = 0, 1, 2
@@ -10,12 +13,16 @@ SCRATCH, COPIES = 64 << 20, 128 << 20  # what a queue has
 
 
 @pytest.fixture(scope="module")
-def choose(tmp_path_factory):
+def exe(tmp_path_factory):
     exe = tmp_path_factory.mktemp("choice") / "gemm_choice"
     subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-I",
                            os.path.join(ROOT, "attention_superoptimizer_amd", "csrc", "backend"), "-o", str(exe),
                            os.path.join(ROOT, "tests", "cpp", "gemm_choice.cc")])
+    return exe
 
+
+@pytest.fixture(scope="module")
+def choose(exe):
     def one(batch, m, n, k, a_cm=0, b_cm=1, aligned=1, scratch=SCRATCH, copies=COPIES):
         out = subprocess.run([str(exe)], input=f"{batch} {m} {n} {k} {a_cm} {b_cm} {aligned} {scratch} {copies}\n", capture_output=True,
                              text=True, check=True).stdout.split()
@@ -107,3 +114,52 @@ def test_ranges_fit_the_scratch_memory(choose):
     assert choose(1, 300, 512, 5504, scratch=0)["ksplit"] == 1
     c = choose(1, 300, 512, 5504, scratch=3 * 300 * 512 * 4)
     assert c["ksplit"] <= 3
+
+
+# ---- two products of one A ---------------------------------------------------------------------
+@pytest.fixture(scope="module")
+def choose_two(exe):
+    def many(shapes):
+        """Of (m, n, k, a_cm, b_cm, aligned, scratch, reads_first): what both products are given."""
+        lines = "".join(f"1 {m} {n} {k} {a_cm} {b_cm} {aligned} {scratch} {COPIES} {reads_first}\n"
+                        for m, n, k, a_cm, b_cm, aligned, scratch, reads_first in shapes)
+        out = subprocess.run([str(exe), "two"], input=lines, capture_output=True, text=True, check=True).stdout.splitlines()
+        return [dict(zip(("half", "tiles", "kind", "bm", "bn", "ksplit", "us", "one_us"), [int(x) for x in line.split()[:6]] +
+                         [float(x) for x in line.split()[6:]])) for line in out]
+
+    return many
+
+
+def test_two_products_take_the_kernels_their_gpu_test_names(choose_two):
+    """... test_gpu_matmul_two.py's shapes: 64 or 128 columns of both, tiles as (kind, k ranges), or none of these."""
+    for reads_first in (0, 1):
+        got = choose_two([(m, n, k, int(a == COL), int(order == COL), 1, SCRATCH, reads_first) for b, m, n, k, order, a in SHAPES])
+        for shape, c, want in zip(SHAPES, got, TAKEN):
+            route = c["half"] or ((c["kind"], c["ksplit"]) if c["tiles"] else None)
+            assert shape[0] > 1 or route == want[reads_first], (shape, reads_first, c)
+    routes = {r for w in TAKEN for r in w}
+    assert {64, 128, None} < routes and {r[0] for r in routes if isinstance(r, tuple)} == {STAGED, DIRECT, WAVES}
+    assert any(isinstance(r, tuple) and r[1] > 1 for r in routes)
+
+
+def test_two_products_of_drawn_shapes(choose_two):
+    """A second consumer that reads what the first leaves never has tiles of one range (each in a workgroup of its own);
+    ranges of both fit the scratch memory; a workgroup of both wants whole stages and chunks; and what is taken is
+    expected to be faster than one after the other."""
+    rng = random.Random(5)
+    near = lambda lo, hi: int(round(lo * (hi / lo) ** rng.random()))  # noqa: E731
+    shapes = [(near(1, 1024), rng.choice([1, 1, 8]) * near(1, 700), rng.choice([1, 8, 64]) * near(1, 32), rng.choice([0, 0, 0, 1]), rng.randint(0, 1),
+               rng.choice([0, 1, 1]), rng.choice([0, 1 << 20, SCRATCH]), rng.randint(0, 1)) for _ in range(4000)]
+    seen = set()
+    for (m, n, k, a_cm, b_cm, aligned, scratch, reads_first), c in zip(shapes, choose_two(shapes)):
+        what = (m, n, k, a_cm, b_cm, aligned, scratch, reads_first, c)
+        if c["half"]:
+            assert not a_cm and aligned and k % 64 == 0 and (b_cm or n % 8 == 0), what
+        elif c["tiles"]:
+            assert c["ksplit"] > 1 or not reads_first, what
+            assert c["ksplit"] == 1 or 2 * m * n * 4 * c["ksplit"] <= scratch, what
+            assert c["kind"] == STAGED or (not a_cm and aligned and (b_cm or n % 8 == 0) and k % (64 if c["kind"] == DIRECT else 32) == 0), what
+        if c["half"] or c["tiles"]:
+            assert c["us"] <= 2 * c["one_us"] + 0.01 or c["one_us"] == 0, what  # (0: a product with no tiles of its own)
+        seen.add((c["half"], c["tiles"], c["tiles"] and c["ksplit"] > 1))
+    assert {(0, 0, 0), (64, 0, 0), (128, 0, 0), (0, 1, False), (0, 1, True)} <= seen

@@ -6,6 +6,7 @@ import ctypes
 import numpy as np
 import pytest
 
+from attention_superoptimizer_amd import _native as N
 from attention_superoptimizer_amd import graph as G
 from helpers import assert_f16_close, normal_f16
 from oracle import evaluate as orc
@@ -19,7 +20,21 @@ class MatmulOut(ctypes.Structure):  # mi355_matmul_out
                 ("X", ctypes.c_void_p), ("E", ctypes.c_void_p)]
 
 
-def _check(rt, b, m, n, k, order, form, a_order=ROW, ins=None, finite=True):
+def _taken(A, B, B2, X, C, E, C2, E2, form, b, m, n, k):
+    """Whether the backend runs these two products as one launch (it does so here, once more)."""
+    at = lambda t: None if t is None else t.device_ptr(False)  # noqa: E731
+    op = {"gate": ("silu", "mul"), "add first": ("silu", "add"), "others": ("div", "exp"), "plain": (None, None)}[form]
+    op = [G.KN_OP.get(name, 0) for name in op]
+    first = MatmulOut(at(B), at(C), op[0], int(form == "others"), at(X) if form == "others" else None, at(E))
+    second = MatmulOut(at(B2), at(C2), op[1], int(form == "gate"), at({"gate": E, "add first": C}.get(form)), at(E2))
+    taken = ctypes.c_int(-1)
+    rc = N.backend().mi355_f16_matmul_two(at(A), int(A.column_major), int(B.column_major), b, m, n, k, ctypes.byref(first),
+                                          ctypes.byref(second), ctypes.byref(taken))
+    assert rc == 0, N.last_error()
+    return taken.value
+
+
+def _check(rt, b, m, n, k, order, form, a_order=ROW, ins=None, finite=True, taken=None):
     g = G.KNGraph()
     try:
         A = g.new_input((b, m, k), layout=a_order)
@@ -41,6 +56,8 @@ def _check(rt, b, m, n, k, order, form, a_order=ROW, ins=None, finite=True):
                 t.write_data(np.full(t.dims, -7, np.float16))
             g.execute_all()
         got = [t.read_data() for t in made]
+        if taken is not None:
+            assert _taken(A, B, B2, X, C, E, C2, E2, form, b, m, n, k) == taken
         if finite:
             what = f"{b} x {m} x {k} x {n} {order} {form}"
             assert_f16_close(got[0], orc.f16_matmul(ins[0], ins[1]), what=what)
@@ -61,12 +78,19 @@ SHAPES = [(1, 1, 8, 64, ROW, ROW), (1, 65, 72, 192, ROW, ROW), (1, 64, 513, 128,
           (1, 300, 3332, 128, COL, ROW), (1, 300, 1032, 1024, COL, ROW), (1, 3, 7, 515, COL, ROW), (1, 17, 130, 65, ROW, ROW),
           (1, 33, 513, 1030, ROW, ROW), (1, 5, 72, 1024, ROW, ROW), (1, 130, 72, 1024, COL, ROW), (2, 33, 256, 128, ROW, ROW),
           (1, 40, 72, 520, COL, COL), (1, 257, 1032, 8, COL, COL), (1, 1, 1, 1, COL, ROW)]
+# what these are given (test_gemm_choice.py): columns of both in a workgroup, or a kind of tile and its k ranges, or None:
+# where the second's consumer reads nothing of the first's, and where it does
+STAGED, DIRECT, WAVES = 0, 1, 2
+TAKEN = [((STAGED, 1), 64), ((STAGED, 1), 64), ((STAGED, 1), 64), (128, 128), (128, 128), ((DIRECT, 1), 64), ((STAGED, 1), (STAGED, 2)),
+         ((STAGED, 1), None), ((STAGED, 1), (STAGED, 4)), ((WAVES, 1), (STAGED, 4)), ((WAVES, 1), (STAGED, 4)), (None, None),
+         ((STAGED, 1), (STAGED, 4)), ((STAGED, 1), None), (None, None)]
 
 
 @pytest.mark.parametrize("form", ["gate", "add first", "others", "plain"])
 @pytest.mark.parametrize("b,m,n,k,order,a_order", SHAPES)
 def test_two_matmuls_of_one_input(rt, b, m, n, k, order, a_order, form):
-    _check(rt, b, m, n, k, order, form, a_order)
+    route = TAKEN[SHAPES.index((b, m, n, k, order, a_order))][form in ("gate", "add first")]
+    _check(rt, b, m, n, k, order, form, a_order, taken=int(route is not None))
 
 
 @pytest.mark.parametrize("m,n,k,order", [(5, 72, 192, ROW), (3, 130, 1030, COL), (385, 2440, 64, ROW)])
