@@ -508,8 +508,8 @@ bool attention_applicable(DevProgram const &P) {
 // What the next operator's fold of rows is to this launch: a workgroup's rows, and the places of its
 // results in them.  False where the operator is no fold of exactly these results, row by row.
 //
-// With whole rows in a workgroup it always pays: both launches of [12, 1040, 1040] in tiles of 80 18.8 -> 16.5 us, of
-// [32, 2048, 2048] at head size 128 78.5 -> 75.6 (both tensors' stores are what is left), 60 prefill plans 0.76 of the
+// With whole rows in a workgroup it always pays: both launches of [12, 1040, 1040] in tiles of 80 18.9 -> 16.7 us, of
+// [32, 2048, 2048] at head size 128 80.2 -> 77.6 (both tensors' stores are what is left), 60 prefill plans 0.76 of the
 // time on the device in the mean, none above 1.  Where the pieces come from several workgroups the last of them pays three trips to the
 // memory that all XCDs share (its stores, its ticket, the pieces), 3 us against the 3.5 - 4.5 of a launch, and all others two while
 // they hold their place on a compute unit.  So: blocks that run in one round (64 groups of 16 blocks, two rounds, 50.8

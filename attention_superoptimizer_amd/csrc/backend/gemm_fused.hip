@@ -328,7 +328,10 @@ StreamPlan stream_plan(DevProgram const &P, GMatch const &G) {
   // product of 16 x 2560 x 1536 3.9 / 4.2), where the wavefronts wait for one of them (5 iterations, 16 rows x 3072
   // 3.4 / 3.9), in 64-k iterations, of which the ring holds a quarter (LoRA 4096 x 1024 of 8 rows 3.7 / 4.1), or where
   // half the rows halve the others' slab, short of long loops (8 rows x 4096: 4096 7.5 / 7.8, 44 - 52 iterations 0.97 -
-  // 1.08 of the others' time, 56 - 112 0.88 - 1.02). A printed LoRA keeps the two launches that its readers know.
+  // 1.08 of the others' time, 53 of 58 and more blocks 1.02 - 1.05 (fewer 1.0), 54 - 63 0.92 - 1.03, 64 - 112 0.88 - 1.02).
+  // Iterations of 128 and of 512 k were not timed in these strips: they keep the kernels they had.  Nor does a printed program
+  // change: the text of a LoRA's is what programs built around it know (two launches and a workspace that it allocates;
+  // tests/test_generated_hip.py pins it), the same bits, 11.2 us for 16 rows x 4096 x 4096 where the strips take 7.9.
   plan.lone = narrow && G.nb == 1 && G.KT == 256 && F >= 3 * ((F + 3) / 4) && 4 * blocks <= 256 && strip_lds <= s.max_lds &&
               (G.lora ? blocks >= 40 && !emit_sink() : blocks >= 48 && (G.M > 8 || F > 52));
   strips = strips || plan.lone;
