@@ -519,7 +519,11 @@ bool attention_applicable(DevProgram const &P) {
 // where there are so many (combine.h), and what is left over piece by piece: for four and sixteen, and for two, it has one
 // trip to make.  Of one row each there is little but that trip: from 32 workgroups on 46 plans of four or sixteen pieces take
 // 1.05 of the time on the device in the mean when folded (16 groups, 4 pieces of 10 tiles of 16 keys 8.23 / 8.73 us, 33
-// groups, 16 pieces of a tile of 48 7.85 / 8.96), 14 of two 1.01; other numbers of pieces less.  Of more rows so it is for
+// groups, 16 pieces of a tile of 48 7.85 / 8.96), 14 of two 1.01; other numbers of pieces less.  From eight iterations on the
+// host's second launch is hidden by the device's work, and the line is nearer: 24 workgroups (7 groups, 4 pieces of 13 tiles of 32
+// keys, passes back to back, 8.50 / 8.93), 48 where the other launch makes two or three trips (18 groups, 5 pieces of 16 tiles of 32 9.40 /
+// 9.78, 12 groups, 8 of 11 tiles of 16 8.93 / 9.28; four trips and more, 7 pieces, 21 groups of 12 tiles of 64, 12.73 / 12.08).  Below
+// these lines 86 plans of one row take 0.98 of the time of two launches, 0.88 - 1.02.  Of more rows so it is for
 // sixteen pieces and more than 128 workgroups, 40 plans 1.08 (20 groups of 16 rows, 7 tiles of 16 keys 9.11 / 11.02; 95 with
 // up to 128 0.97); for 4, 8 and 12 pieces and more than 192 workgroups it comes to the same, 0.90 - 1.14 of the time.
 // 435 other drawn split-KV plans 0.92 of the time on the device in the mean, 0.60 - 1.08, twenty above 1.01.
@@ -580,8 +584,10 @@ static bool make_fold(AttnParams const &A, Match const &M, DevProgram const &P, 
     if (R.S > kFoldPieces || trips > (R.S <= 8 ? 2 : 1) || wg_rows * R.S * 2 + 16 > lds || workgroups > 256 * per_cu) {
       return false;
     }
-    bool const one_trip = R.S == 2 || R.S == 4 || R.S == 16;  // of the other launch
-    if ((M.m == 1 && one_trip && workgroups >= 32) || (R.S == 16 && workgroups > 128) || (R.S % 4 == 0 && workgroups > 192)) {
+    int const other = R.S == 16 ? 1 : R.S / 4 + R.S % 4;  // trips of the other launch
+    bool const one_trip = R.S == 2 || other == 1;         // (of two the first is loaded ahead)
+    int const most = one_trip ? (P.forloop_range < 8 ? 32 : 24) : other <= 3 && P.forloop_range >= 8 ? 48 : 1 << 30;
+    if ((M.m == 1 && workgroups >= most) || (R.S == 16 && workgroups > 128) || (R.S % 4 == 0 && workgroups > 192)) {
       return false;
     }
     out.tickets = f.tickets(R.rows / M.m * A.split);

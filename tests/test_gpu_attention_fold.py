@@ -80,9 +80,12 @@ def test_pieces_of_several_workgroups(rt, groups, rows, keys, blocks, loop, fold
 @pytest.mark.parametrize("groups,rows,keys,blocks,loop,folds", [
     (7, 1, 64, 4, 5, True), (8, 1, 64, 4, 5, False), (8, 1, 64, 5, 5, True), (16, 1, 48, 2, 3, False), (2, 1, 32, 16, 3, False),
     (1, 1, 32, 16, 3, True), (8, 16, 64, 16, 4, True), (9, 16, 64, 16, 4, False), (9, 2, 80, 16, 2, False), (9, 2, 80, 15, 2, True),
-    (24, 8, 64, 8, 4, True), (25, 8, 64, 8, 4, False), (25, 8, 64, 9, 4, True)])
+    (24, 8, 64, 8, 4, True), (25, 8, 64, 8, 4, False), (25, 8, 64, 9, 4, True), (7, 1, 32, 4, 7, True), (7, 1, 32, 4, 8, False),
+    (5, 1, 32, 4, 13, True), (6, 1, 32, 4, 13, False), (18, 1, 32, 5, 7, True), (18, 1, 32, 5, 16, False), (9, 1, 32, 5, 16, True),
+    (6, 1, 16, 8, 11, False), (5, 1, 16, 8, 11, True), (16, 1, 32, 3, 8, False), (15, 1, 32, 3, 8, True), (21, 1, 32, 7, 12, True),
+    (7, 2, 32, 4, 13, True)])
 def test_where_the_other_launch_is_short(rt, groups, rows, keys, blocks, loop, folds):
-    """Few pieces of one row, and sixteen of more: two launches from so many workgroups on."""
+    """Few pieces of one row, and sixteen of more: two launches from so many workgroups on, fewer in long loops."""
     _check(rt, _decode(groups, rows, keys, blocks, loop, ROW), folds)
 
 
